@@ -629,6 +629,295 @@ __device__ float4 forward_row(const DScene &S, const float4 *colours, uint32_t k
     return C;
 }
 
+// ---------------------------------------------------------------------------
+// Coverage by cells.  A block owns a tile of blockDim.x pixels (64 to
+// TILE_MAX) of one row of one image and takes the image's paths SEG at a
+// time.  One thread per row piece adds the piece's coverage *differences* to
+// the path's row of LDS cells: only the columns the piece's ramp touches, so
+// a piece costs its x extent instead of the tile's width, and a 64-lane
+// prefix sum then gives every pixel's coverage.  (Evaluating every piece that
+// touches a wavefront's columns on all of its pixels took 3.84 ms for 64
+// images of 256x256 with 17,500 paths, most of it on pixels outside the
+// ramp; this form takes 1.27 ms, and 91 us instead of 297 for one 512x512
+// image of 256 paths.  What is left is VALU work: per path and pixel about 9
+// instructions of prefix sum and 9 of composite.)
+//
+// Cells are integers in units of 2^-24 (an i32 add): the sum does not depend
+// on the order of the pieces, so the same inputs give the same canvas
+// whichever kernel computes it, and each column's value is rounded once, at
+// 2^-25, where a float sum rounds at every piece.  i32 holds |A| < 128; a
+// (path, row) with more than HEAVY pieces takes 64-bit cells instead.
+//
+// Every 64-column chunk of a row stands alone: a piece left of a chunk adds
+// its whole signed height to the chunk's first cell, so no carry passes
+// between wavefronts.
+// ---------------------------------------------------------------------------
+constexpr uint32_t SEG = 16;         // paths per round
+// Pixels per block.  At 93 VGPRs a SIMD holds 5 wavefronts, and blocks of 4
+// wavefronts fill them where blocks of 8 leave one empty: a 1000x600 image
+// takes 229 us a call with 256, 250 with 512, 233 with 128.
+constexpr uint32_t TILE_MAX = 256;
+constexpr uint32_t ROW_PATHS = 256;  // paths whose cell counts are staged at once
+constexpr uint32_t HEAVY = 120;      // pieces of one path in one row past which cells are 64-bit
+constexpr int RAMP_LANE = 8;         // ramps of at most this many columns are walked by one lane
+constexpr float CELL_ONE = 16777216.0f;  // 2^24
+
+struct RowLds {
+    __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of the staged paths' piece counts, then the total
+    uint32_t dl[ROW_PATHS];                    // list position of a path's piece e: dl + e
+    uint32_t vb[ROW_PATHS + 1];                // first vertices
+    uint32_t marks[ROW_PATHS / SEG];           // per round: bit j, path j has pieces; bit 16 + j, it is heavy
+    uint32_t poison[2];                        // per round parity: bit j, path j has a piece that is no number here
+};
+
+// Counts and list offsets of row Y for the n <= ROW_PATHS paths from global
+// path kbase.  Every thread calls it, between barriers of the caller.
+__device__ void stage_row(const DScene &S, uint32_t kbase, uint32_t n, int Y, RowLds &R) {
+    const uint32_t lane = threadIdx.x;
+    if (lane < 64) {
+        uint32_t c[4], o[4], sum = 0, nib = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t p = 4 * lane + i;
+            const uint64_t cell = (uint64_t)(kbase + (p < n ? p : 0u)) * S.H + (uint32_t)Y;
+            c[i] = p < n ? S.cell_cnt[cell] : 0u;
+            o[i] = S.cell_off[cell];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            sum += c[i];
+            nib |= ((c[i] ? 1u : 0u) | (c[i] > HEAVY ? 0x10000u : 0u)) << i;
+        }
+        const uint32_t incl = wave_incl_dpp<false>(sum);
+        uint32_t pre = incl - sum;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            R.pb[4 * lane + i] = pre;
+            R.dl[4 * lane + i] = o[i] - pre;
+            pre += c[i];
+        }
+        if (lane == 63) R.pb[ROW_PATHS] = incl;
+        uint32_t h = nib << (4 * (lane & 3));
+        h |= (uint32_t)__shfl_xor((int)h, 1, 64);
+        h |= (uint32_t)__shfl_xor((int)h, 2, 64);
+        if ((lane & 3) == 0) R.marks[lane >> 2] = h;
+        if (lane < 2) R.poison[lane] = 0;
+    }
+    for (uint32_t p = threadIdx.x; p <= n; p += blockDim.x) R.vb[p] = S.vtx_off[kbase + p];
+}
+
+// Piece e of round s (staged paths [s * SEG, s * SEG + SEG)).
+struct PieceRef {
+    uint32_t j;     // path within the round, NO_IDX: none
+    uint32_t edge;  // the path's edge
+};
+
+__device__ __forceinline__ PieceRef piece_ref(const DScene &S, const RowLds &R, uint32_t s, uint32_t e) {
+    const uint32_t end = R.pb[(s + 1) * SEG];
+    PieceRef r;
+    r.j = NO_IDX;
+    r.edge = 0;
+    if (e >= end) return r;
+    uint32_t j = 0;  // the last path of the round that starts at or before e
+#pragma unroll
+    for (uint32_t i = 0; i < SEG; i += 4) {
+        const uint4 q = *reinterpret_cast<const uint4 *>(&R.pb[s * SEG + i]);
+        j += (q.x <= e ? 1u : 0u) + (q.y <= e ? 1u : 0u) + (q.z <= e ? 1u : 0u) + (q.w <= e ? 1u : 0u);
+    }
+    r.j = j - 1;
+    r.edge = S.cell_edge[R.dl[s * SEG + r.j] + e];
+    return r;
+}
+
+// The two vertices of a piece's edge and their indices.
+struct PieceVtx {
+    float2 p, q;
+    uint32_t ip, iq;
+};
+
+__device__ __forceinline__ PieceVtx piece_vtx(const DScene &S, const RowLds &R, uint32_t s, const PieceRef &r,
+                                              uint32_t &bad) {
+    const uint32_t t = s * SEG + (r.j != NO_IDX ? r.j : 0u);
+    const uint32_t vb = R.vb[t], V = R.vb[t + 1] - vb;
+    bad |= r.edge < V ? 0u : 1u;
+    const uint32_t e = r.edge < V ? r.edge : 0u;
+    PieceVtx v;
+    v.ip = vb + e;
+    v.iq = vb + (e + 1 < V ? e + 1 : 0u);
+    v.p = S.vtx[v.ip];
+    v.q = S.vtx[v.iq];
+    return v;
+}
+
+// A piece against the tile: its coverage M is 0 left of its ramp, 1 right of
+// it.  [c0, c1) are the ramp's columns within the tile (c1 <= c0: none), and
+// from column max(c0, c1) on the piece counts whole.
+struct Ramp {
+    float lo, hi, inv, z;  // x range, 1 / (hi - lo), signed height
+    int c0, c1;
+    bool live, nan;
+};
+
+__device__ __forceinline__ Ramp ramp_of(const Piece &r, float xb0, int tw) {
+    Ramp m;
+    m.lo = r.xa < r.xb ? r.xa : r.xb;
+    m.hi = r.xa < r.xb ? r.xb : r.xa;
+    m.z = r.sign * r.h;
+    const float w = m.hi - m.lo;
+    m.nan = r.live & !(w < __builtin_inff());  // a NaN or unbounded x
+    m.live = r.live & !m.nan & (m.lo < xb0 + (float)tw);
+    m.inv = w < EPS_W ? 0.0f : 1.0f / w;  // 0: narrow, the midpoint's value
+    const float f0 = floorf(m.lo) - xb0, f1 = ceilf(m.hi) - xb0;
+    m.c0 = f0 > 0.0f ? (f0 < (float)tw ? (int)f0 : tw) : 0;
+    m.c1 = f1 > 0.0f ? (f1 < (float)tw ? (int)f1 : tw) : 0;
+    return m;
+}
+
+// M at the pixel whose right border is X1, within the ramp (as mean_clamp).
+__device__ __forceinline__ float ramp_cover(const Ramp &m, float X1) {
+    const float lo = X1 - m.hi, hi = X1 - m.lo;
+    if (m.inv == 0.0f) return clamp01((lo + hi) * 0.5f);
+    const float a = clamp01(lo), b = clamp01(hi);
+    return ((b - a) * (a + b) * 0.5f + (hi > 1.0f ? hi - 1.0f : 0.0f)) * m.inv;
+}
+
+template <typename T>
+__device__ __forceinline__ T cell_of(float zs, float M) {
+    return (T)__float2int_rn(zs * M);  // |zs * M| <= 2^24
+}
+template <typename T>
+__device__ __forceinline__ void cell_add(T *c, T v) {
+    if constexpr (sizeof(T) == 8)
+        atomicAdd(reinterpret_cast<unsigned long long *>(c), (unsigned long long)v);
+    else
+        atomicAdd(c, v);
+}
+
+// Adds one piece per lane to its path's row of cells (row; the wavefront's
+// lanes all call it, those without a piece with m.live false).  A ramp of
+// more than RAMP_LANE columns is evaluated by the whole wavefront, one column
+// per lane, so that one long near-horizontal piece does not hold up 63 lanes.
+template <typename T>
+__device__ __forceinline__ void scatter_piece(T *cells, uint32_t row_at, const Ramp &m, float xb0, int tw) {
+    const float zs = m.z * CELL_ONE;
+    const int n = m.c1 - m.c0;
+    const bool wide = m.live & (n > RAMP_LANE);
+    T prev = 0;
+    if (m.live & !wide) {
+        for (int c = m.c0; c < m.c1; ++c) {
+            const T q = cell_of<T>(zs, ramp_cover(m, xb0 + (float)(c + 1)));
+            cell_add(&cells[row_at + c], q - ((c & 63) ? prev : (T)0));
+            prev = q;
+        }
+    }
+    unsigned long long todo = __ballot(wide);
+    while (todo) {
+        const int l = __ffsll((long long)todo) - 1;
+        todo &= todo - 1;
+        auto bc = [l](float v) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+        };
+        Ramp w;
+        w.lo = bc(m.lo);
+        w.hi = bc(m.hi);
+        w.inv = bc(m.inv);
+        const float wz = bc(zs);
+        const int w0 = __builtin_amdgcn_readlane(m.c0, l), w1 = __builtin_amdgcn_readlane(m.c1, l);
+        const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)row_at, l);
+        const int lane = threadIdx.x & 63;
+        for (int c = w0 + lane; c < w1; c += 64) {
+            const T q = cell_of<T>(wz, ramp_cover(w, xb0 + (float)(c + 1)));
+            const T b = ((c > w0) & ((c & 63) != 0)) ? cell_of<T>(wz, ramp_cover(w, xb0 + (float)c)) : (T)0;
+            cell_add(&cells[at + c], q - b);
+        }
+    }
+    if (!m.live) return;
+    if (wide) prev = cell_of<T>(zs, ramp_cover(m, xb0 + (float)m.c1));  // the last ramp column's value
+    // from the column after the ramp on: whole
+    const T whole = cell_of<T>(zs, 1.0f);
+    const int t = m.c1 > m.c0 ? m.c1 : m.c0;
+    if (t < tw) cell_add(&cells[row_at + t], whole - ((t & 63) ? prev : (T)0));
+    for (int c = (t | 63) + 1; c < tw; c += 64) cell_add(&cells[row_at + c], whole);
+}
+
+// Coverage A[j] of round s's paths at this thread's pixel, from the first
+// blockDim.x pieces (ref, v: one per thread, loaded by the caller ahead of
+// time) and any further ones.  cells: SEG rows of pitch `pitch`, zero on
+// entry and on exit (the exit barrier included).  Every thread calls it.
+__device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t s, const PieceRef &ref,
+                                            const PieceVtx &v, const Piece &first, int Y, float xb0, int *cells,
+                                            uint32_t pitch, float A[SEG], uint32_t &bad) {
+    const int tid = threadIdx.x, tw = (int)blockDim.x;
+    const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];
+    const uint32_t heavy = R.marks[s] >> 16;
+#pragma unroll
+    for (uint32_t j = 0; j < SEG; ++j) A[j] = 0.0f;
+    if (heavy) {  // (uniform) one heavy path at a time, in 64-bit cells over the same LDS
+        long long *c64 = reinterpret_cast<long long *>(cells);
+        for (uint32_t j = 0; j < SEG; ++j) {
+            if (!((heavy >> j) & 1u)) continue;
+            c64[tid] = 0;
+            __syncthreads();
+            const uint32_t e0 = R.pb[s * SEG + j], e1 = R.pb[s * SEG + j + 1];
+            for (uint32_t eb = e0; eb < e1; eb += (uint32_t)tw) {  // whole blocks: scatter_piece is collective
+                const uint32_t e = eb + (uint32_t)tid;
+                PieceRef r = piece_ref(S, R, s, e < e1 ? e : NO_IDX);
+                const PieceVtx u = piece_vtx(S, R, s, r, bad);
+                Piece pc = piece_of(u.p, u.q, Y);
+                pc.live &= r.j != NO_IDX;
+                const Ramp m = ramp_of(pc, xb0, tw);
+                if (m.nan) atomicOr(&R.poison[s & 1], 1u << j);
+                scatter_piece<long long>(c64, 0u, m, xb0, tw);
+            }
+            __syncthreads();
+            const long long sum = (long long)wave_incl_t<unsigned long long, false>((unsigned long long)c64[tid]);
+            const float a = (float)sum * (1.0f / CELL_ONE);
+#pragma unroll
+            for (uint32_t k = 0; k < SEG; ++k) A[k] = k == j ? a : A[k];
+            __syncthreads();
+        }
+        c64[tid] = 0;
+        __syncthreads();
+    }
+    for (uint32_t eb = base; eb < end; eb += (uint32_t)tw) {
+        PieceRef r = ref;
+        Piece pc = first;
+        if (eb != base) {
+            r = piece_ref(S, R, s, eb + (uint32_t)tid);
+            const PieceVtx u = piece_vtx(S, R, s, r, bad);
+            pc = piece_of(u.p, u.q, Y);
+        }
+        pc.live &= r.j != NO_IDX;
+        const uint32_t j = r.j != NO_IDX ? r.j : 0u;
+        pc.live &= ((heavy >> j) & 1u) == 0u;
+        const Ramp m = ramp_of(pc, xb0, tw);
+        if (m.nan) atomicOr(&R.poison[s & 1], 1u << j);
+        scatter_piece<int>(cells, j * pitch, m, xb0, tw);
+    }
+    __syncthreads();
+    uint32_t c[SEG];
+#pragma unroll
+    for (uint32_t j = 0; j < SEG; ++j) {
+        c[j] = (uint32_t)cells[j * pitch + tid];
+        cells[j * pitch + tid] = 0;
+    }
+    const uint32_t poison = R.poison[s & 1];
+    if (tid == 0) R.poison[(s + 1) & 1] = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < SEG; ++j) {
+        const float a = (float)(int)wave_incl_dpp<false>(c[j]) * (1.0f / CELL_ONE);
+        A[j] = ((heavy >> j) & 1u) ? A[j] : a;
+    }
+    // a piece without an x takes its path's whole row (coverage past 1, and so no gradient)
+    if (poison) {
+#pragma unroll
+        for (uint32_t j = 0; j < SEG; ++j) A[j] = ((poison >> j) & 1u) ? 2.0f : A[j];
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ float alpha_cover(float A) { return __builtin_amdgcn_fmed3f(fabsf(A), 0.0f, 1.0f); }
+
 #define DIFF_STAGE_LDS(VI, PQ)                                          \
     __shared__ uint32_t s_cnt[PCHUNK], s_off[PCHUNK], s_pb[PCHUNK];    \
     __shared__ float4 s_col[PCHUNK];                                    \
@@ -637,22 +926,79 @@ __device__ float4 forward_row(const DScene &S, const float4 *colours, uint32_t k
     __shared__ uint32_t s_w[DBLOCK / 64];                               \
     const Stage sg{s_cnt, s_off, s_pb, s_col, s_pc, s_ev, VI, PQ, s_w}
 
-// With ck non-null it also leaves what k_backward's replay would write: the
-// canvas before every KSEG-th path, and each path's coverage when cov is
-// non-null (same slots as k_backward).
-__global__ __launch_bounds__(DBLOCK) void k_forward(DScene S, const float4 *colours, float4 *canvas, float4 *ck,
-                                                    uint64_t ck_stride, float *cov, DevStatus *st) {
-    DIFF_STAGE_LDS(nullptr, nullptr);
+// Colour of the image's path j, or zero where `on` is 0 (a path without
+// pieces in the row does not touch it, whatever its colour).  Uniform: scalar
+// loads, and no branch between a round's paths.
+__device__ __forceinline__ float4 round_colour(const float4 *__restrict__ colours, uint32_t k0, uint32_t np,
+                                               uint32_t j, uint32_t on) {
+    const float4 c = colours[k0 + (j < np ? j : np - 1)];
+    const uint32_t m = 0u - on;
+    auto sel = [m](float v) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & m); };
+    return make_float4(sel(c.x), sel(c.y), sel(c.z), sel(c.w));
+}
+
+// The canvas of one tile of one row: the image's paths composited over
+// transparent pixels, SEG at a time, with the next round's pieces loaded
+// while a round is composited.  With ck it also leaves the canvas before
+// every KSEG-th path and, with cov, each path's coverage (paths with no piece
+// in the row are left out, as their coverage is 0) at slot
+// (image row) * ck_pitch + X.
+__global__ __launch_bounds__(TILE_MAX) void k_forward(DScene S, const float4 *__restrict__ colours,
+                                                      float4 *__restrict__ canvas, float4 *__restrict__ ck,
+                                                      uint32_t ck_pitch, uint64_t ck_stride,
+                                                      float *__restrict__ cov, DevStatus *st) {
+    extern __shared__ __align__(16) int s_cells[];
+    __shared__ RowLds R;
     if (run_failed(st)) return;
-    const int X = (int)(blockIdx.x * DBLOCK + threadIdx.x), Y = (int)blockIdx.y;
-    const uint32_t im = blockIdx.z;
-    const uint32_t k0 = S.img_first[im], k1 = S.img_first[im + 1];
-    const uint64_t slot = ((uint64_t)blockIdx.z * gridDim.y + blockIdx.y) * (gridDim.x * DBLOCK) +
-                          (uint64_t)blockIdx.x * DBLOCK + threadIdx.x;
+    const uint32_t tw = blockDim.x, pitch = tw + 1;
+    const uint32_t X = blockIdx.x * tw + threadIdx.x, Y = blockIdx.y, im = blockIdx.z;
+    const float xb0 = (float)(blockIdx.x * tw);
+    const uint32_t k0 = S.img_first[im], np = S.img_first[im + 1] - k0;
+    const uint64_t slot = ((uint64_t)im * S.H + Y) * ck_pitch + X;
+    const bool in = X < S.W;
     uint32_t bad = 0;
-    const float4 C = forward_row(S, colours, k0, k1 - k0, X, Y, slot, ck, ck_stride, ck ? cov : nullptr, sg, bad);
+    float4 C = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (uint32_t i = threadIdx.x; i < SEG * pitch; i += tw) s_cells[i] = 0;
+    for (uint32_t ja = 0; ja < np; ja += ROW_PATHS) {
+        const uint32_t n = np - ja < ROW_PATHS ? np - ja : ROW_PATHS;
+        const uint32_t rounds = (n + SEG - 1) / SEG;
+        __syncthreads();  // the previous paths' staging is no longer read
+        stage_row(S, k0 + ja, n, (int)Y, R);
+        __syncthreads();
+        PieceRef ref = piece_ref(S, R, 0, R.pb[0] + threadIdx.x);
+        PieceVtx v = piece_vtx(S, R, 0, ref, bad);
+        PieceRef nref = ref;
+        if (rounds > 1) nref = piece_ref(S, R, 1, R.pb[SEG] + threadIdx.x);
+        for (uint32_t s = 0; s < rounds; ++s) {
+            const Piece first = piece_of(v.p, v.q, (int)Y);
+            const PieceRef cur = ref;
+            const PieceVtx cv = v;
+            if (s + 1 < rounds) {  // the next round's vertices, and the one after's edge
+                ref = nref;
+                v = piece_vtx(S, R, s + 1, ref, bad);
+                if (s + 2 < rounds) nref = piece_ref(S, R, s + 2, R.pb[(s + 2) * SEG] + threadIdx.x);
+            }
+            float A[SEG];
+            round_cover(S, R, s, cur, cv, first, (int)Y, xb0, s_cells, pitch, A, bad);
+            const uint32_t j0 = ja + s * SEG;
+            const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
+            if (cov && in) {
+#pragma unroll
+                for (uint32_t j = 0; j < SEG; ++j)
+                    if ((some >> j) & 1u) cov[(uint64_t)(j0 + j) * ck_stride + slot] = A[j];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < SEG; ++j) {
+                if (ck && j % KSEG == 0 && j0 + j < np && in) ck[(uint64_t)((j0 + j) / KSEG) * ck_stride + slot] = C;
+                const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
+                const float al = alpha_cover(A[j]), keep = fmaf(-c.w, al, 1.0f);
+                C = make_float4(fmaf(C.x, keep, c.x * al), fmaf(C.y, keep, c.y * al), fmaf(C.z, keep, c.z * al),
+                                fmaf(C.w, keep, c.w * al));
+            }
+        }
+    }
     if (bad) raise_err(st, FT_EDEVICE);
-    if ((uint32_t)X < S.W) canvas[((uint64_t)im * S.H + (uint32_t)Y) * S.W + (uint32_t)X] = C;
+    if (in) canvas[((uint64_t)im * S.H + Y) * S.W + X] = C;
 }
 
 // loss partials per block (sum of squared differences); grad = 2 (C - T) / N.
@@ -692,7 +1038,8 @@ __global__ __launch_bounds__(BLOCK) void k_loss(const float *canvas, const float
 // forms its vertex gradients from S1..S3 with global atomics; the colour
 // gradients are flushed once per segment.
 __global__ __launch_bounds__(DBLOCK) void k_backward(DScene S, const float4 *colours, const float4 *grad_canvas,
-                                                     float4 *ck, uint64_t ck_stride, float *cov, uint32_t replayed,
+                                                     float4 *ck, uint32_t ck_pitch, uint64_t ck_stride, float *cov,
+                                                     uint32_t replayed,
                                                      float2 *gvtx, float *gcol, DevStatus *st) {
     __shared__ uint2 s_vi[ECAP];
     __shared__ float4 s_pq[ECAP];
@@ -713,8 +1060,7 @@ __global__ __launch_bounds__(DBLOCK) void k_backward(DScene S, const float4 *col
     const float Xf = (float)X, xw0 = (float)(X - lane);
     const uint32_t im = blockIdx.z;
     const bool active = (uint32_t)X < S.W;
-    const uint64_t slot = ((uint64_t)blockIdx.z * gridDim.y + blockIdx.y) * (gridDim.x * DBLOCK) +
-                          (uint64_t)blockIdx.x * DBLOCK + tid;
+    const uint64_t slot = ((uint64_t)im * S.H + (uint32_t)Y) * ck_pitch + (uint32_t)X;
     const uint32_t k0 = S.img_first[im], np = S.img_first[im + 1] - k0;
     uint32_t bad = 0;
     if (!replayed) (void)forward_row(S, colours, k0, np, X, Y, slot, ck, ck_stride, cov, sg, bad);
@@ -762,7 +1108,7 @@ __global__ __launch_bounds__(DBLOCK) void k_backward(DScene S, const float4 *col
         uint32_t w_lo = 0, w_n = 0;  // staged window: pieces [w_lo, w_lo + w_n) of the segment
         if (cov) {
             for (uint32_t j = 0; j < ns; ++j)
-                if (s_cnt[j]) s_A[j][tid] = cov[(uint64_t)(j0 + j) * ck_stride + slot];
+                if (active && s_cnt[j]) s_A[j][tid] = cov[(uint64_t)(j0 + j) * ck_stride + slot];
         } else {
             const int wid = tid >> 6;
             const float xb0 = (float)(blockIdx.x * DBLOCK);
@@ -825,7 +1171,7 @@ __global__ __launch_bounds__(DBLOCK) void k_backward(DScene S, const float4 *col
         // composite from the checkpoint for each path)
         float4 Cbs[KSEG];
         {
-            float4 C = ck[(uint64_t)seg * ck_stride + slot];
+            float4 C = active ? ck[(uint64_t)seg * ck_stride + slot] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
             for (uint32_t i = 0; i < (uint32_t)KSEG; ++i) {
                 Cbs[i] = C;
@@ -1000,7 +1346,8 @@ struct ft_diff {
     size_t cap_tiles = 0;
     unsigned long long *d_lb = nullptr;  // scan look-back words
     float4 *d_ck = nullptr;
-    uint64_t ck_stride = 0;
+    uint32_t ck_pitch = 0;  // checkpoint pixels per row
+    uint64_t ck_stride = 0;  // and per checkpoint
     float *d_cov = nullptr;  // [max_paths][ck_stride] kept coverage (FT_DIFF_KEEP_COVERAGE), or null: recomputed
     double *d_partial = nullptr;  // [LOSS_GRID] loss partials, then [LOSS_GRID] their sum
     double *h_loss = nullptr;     // pinned: the summed loss
@@ -1097,14 +1444,23 @@ ft_status grow_pairs(ft_diff *d) {
 
 dim3 raster_grid(const ft_diff *d) { return dim3((d->W + DBLOCK - 1) / DBLOCK, d->H, d->n_images); }
 
+// Forward tiles: at most TILE_MAX pixels of a row, in whole wavefronts.
+ft_status launch_forward(ft_diff *d, const float *colours, float *canvas, bool keep) {
+    const uint32_t tiles = (d->W + TILE_MAX - 1) / TILE_MAX;
+    const uint32_t tw = ((d->W + tiles - 1) / tiles + 63) / 64 * 64;
+    const size_t lds = (size_t)SEG * (tw + 1) * sizeof(int);
+    k_forward<<<dim3(tiles, d->H, d->n_images), tw, lds, d->stream>>>(
+        scene_of(d), reinterpret_cast<const float4 *>(colours), reinterpret_cast<float4 *>(canvas),
+        keep ? d->d_ck : nullptr, d->ck_pitch, d->ck_stride, keep ? d->d_cov : nullptr, d->d_status);
+    FD_HIP(hipGetLastError());
+    return FT_OK;
+}
+
 ft_status run_forward(ft_diff *d, const float *points, const float *colours, float *canvas) {
     for (int attempt = 0; attempt < 3; ++attempt) {
         ft_status st = launch_geometry(d, points, false, nullptr);
         if (st) return st;
-        k_forward<<<raster_grid(d), DBLOCK, 0, d->stream>>>(scene_of(d), reinterpret_cast<const float4 *>(colours),
-                                                             reinterpret_cast<float4 *>(canvas), nullptr,
-                                                             d->ck_stride, nullptr, d->d_status);
-        FD_HIP(hipGetLastError());
+        if ((st = launch_forward(d, colours, canvas, false))) return st;
         st = finish(d);
         if (st != (ft_status)0x100) return st;
         if ((st = grow_pairs(d))) return st;
@@ -1138,7 +1494,7 @@ ft_status launch_backward(ft_diff *d, const float *colours, const float *grad_ca
     DScene S = scene_of(d);
     k_backward<<<raster_grid(d), DBLOCK, 0, d->stream>>>(
         S, reinterpret_cast<const float4 *>(colours), reinterpret_cast<const float4 *>(grad_canvas), d->d_ck,
-        d->ck_stride, d->d_cov, replayed ? 1u : 0u, d->d_gvtx, grad_colours, d->d_status);
+        d->ck_pitch, d->ck_stride, d->d_cov, replayed ? 1u : 0u, d->d_gvtx, grad_colours, d->d_status);
     k_point_grad<<<grid_of(d->n_pts), BLOCK, 0, d->stream>>>(S, d->d_gvtx, reinterpret_cast<float2 *>(grad_points),
                                                              d->n_pts, d->d_pt_path);
     FD_HIP(hipGetLastError());
@@ -1166,10 +1522,7 @@ ft_status run_step(ft_diff *d, const float *points, const float *colours, const 
     for (int attempt = 0; attempt < 3; ++attempt) {
         ft_status st = launch_geometry(d, points, true, grad_colours);
         if (st) return st;
-        k_forward<<<raster_grid(d), DBLOCK, 0, d->stream>>>(scene_of(d), reinterpret_cast<const float4 *>(colours),
-                                                             reinterpret_cast<float4 *>(canvas), d->d_ck,
-                                                             d->ck_stride, d->d_cov, d->d_status);
-        FD_HIP(hipGetLastError());
+        if ((st = launch_forward(d, colours, canvas, true))) return st;
         if ((st = launch_loss(d, canvas, target, grad_canvas))) return st;
         if ((st = launch_backward(d, colours, grad_canvas, grad_points, grad_colours, true))) return st;
         st = finish(d, true);
@@ -1230,7 +1583,8 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
     d->n_cells = cells;
     d->canvas_floats = 4ull * L->n_images * L->width * L->height;
     const dim3 g = raster_grid(d);
-    d->ck_stride = (uint64_t)g.x * g.y * g.z * DBLOCK;
+    d->ck_pitch = g.x * DBLOCK;
+    d->ck_stride = (uint64_t)d->ck_pitch * g.y * g.z;
     const uint64_t n_ck = std::max<uint64_t>(1, (max_paths + KSEG - 1) / KSEG);
     d->cap_tiles = (cells + SCAN_TILE_MIN - 1) / SCAN_TILE_MIN + 1;
     d->cap_pairs = (uint32_t)std::min<uint64_t>(0xFFFFFFF0ull, 8 * nv + 4096);

@@ -8,18 +8,16 @@
 //   k_rows       each edge adds +1/-1 at the ends of its row range per path
 //   scan, scan   -> edges per (path, row) cell, CSR offsets
 //   k_fill_cells, k_sort_cells   edge lists per cell, in edge order
-//   k_forward    one lane per pixel: coverage of every path of the image from
-//                its cell's edges, composite, write the canvas
+//   k_forward    one lane per pixel of a row tile: coverage of the image's
+//                paths, 16 per round, from integer LDS cells and a prefix sum,
+//                composite, the canvas and (in a step) its value before every
+//                round, which the backward starts from
 //   k_loss, k_loss_sum   L2 against a target: d loss / d canvas and the loss,
 //                summed on the device in a fixed order
-//   k_backward   one lane per pixel: replays the forward into canvas
-//                checkpoints every KSEG paths (inside ft_diff_step k_forward
-//                has written them), walks each segment's paths backwards with
-//                their coverage recomputed into LDS (or read from the kept
-//                coverage buffer, FT_DIFF_KEEP_COVERAGE), reduces the per-edge
-//                and per-colour gradients over the wavefront and gathers them
-//                per block in LDS before one atomic add per touched vertex and
-//                colour channel
+//   k_backward   the rounds last to first: coverage again, d loss / d alpha
+//                per pixel and path, the colours' gradients summed over the
+//                tile, and one lane per edge piece gathering its gradient from
+//                the columns it touches
 //   k_point_grad vertex gradients -> control point gradients
 #include <algorithm>
 #include <cstring>
@@ -32,9 +30,6 @@ namespace diff {
 
 constexpr int DSEG = 16;          // segments per cubic
 constexpr float EPS_W = 1e-5f;    // narrower pieces use the midpoint value
-constexpr int DBLOCK = 256;       // pixels of one row per block (four wavefronts)
-constexpr int KSEG = 8;           // paths per checkpoint segment
-constexpr uint64_t COV_MAX_BYTES = 16ull << 30;  // largest kept-coverage buffer
 
 struct DScene {
     uint32_t n_images, W, H, n_paths;
@@ -60,40 +55,7 @@ __device__ inline void bern(int j, float w[4]) {
     w[3] = t * t * t / 4096.0f;
 }
 
-__device__ inline float clamp01(float u) { return u < 0.0f ? 0.0f : (u > 1.0f ? 1.0f : u); }
-
-// Mean of clamp(u, 0, 1) for u moving linearly from ua to ub, and its partials.
-__device__ inline float mean_clamp(float ua, float ub, float &d_ua, float &d_ub) {
-    const float lo = ua < ub ? ua : ub, hi = ua < ub ? ub : ua;
-    float m, dlo = 0.0f, dhi = 0.0f;
-    if (hi <= 0.0f) {
-        m = 0.0f;
-    } else if (lo >= 1.0f) {
-        m = 1.0f;
-    } else {
-        const float w = hi - lo;
-        if (w < EPS_W) {
-            const float mid = (lo + hi) * 0.5f;
-            if (mid <= 0.0f) {
-                m = 0.0f;
-            } else if (mid >= 1.0f) {
-                m = 1.0f;
-            } else {
-                m = mid;
-                dlo = dhi = 0.5f;
-            }
-        } else {
-            const float a = clamp01(lo), b = clamp01(hi);
-            const float integral = (b - a) * (a + b) * 0.5f + (hi > 1.0f ? hi - 1.0f : 0.0f);
-            m = integral / w;
-            dhi = (b - m) / w;
-            dlo = (m - a) / w;
-        }
-    }
-    d_ua = ua <= ub ? dlo : dhi;
-    d_ub = ua <= ub ? dhi : dlo;
-    return m;
-}
+__device__ __forceinline__ float clamp01(float u) { return __builtin_amdgcn_fmed3f(u, 0.0f, 1.0f); }
 
 // The row piece of an edge: its part within row Y, oriented top to bottom.
 struct Piece {
@@ -162,21 +124,9 @@ __device__ __forceinline__ float dpp_add(float v) {
     return v + __builtin_bit_cast(float, src);
 }
 
-// Sum over the 64 lanes (all active), returned to every lane: an inclusive
-// scan with DPP (row_shr 1, 2, 4, 8 within rows of 16 lanes, then
-// row_bcast:15 and row_bcast:31), read from lane 63.  The same lanes add in
-// the same order on every call.
-__device__ inline float wave_sum(float v) {
-    v = dpp_add<0x111, 0xf>(v);
-    v = dpp_add<0x112, 0xf>(v);
-    v = dpp_add<0x114, 0xf>(v);
-    v = dpp_add<0x118, 0xf>(v);
-    v = dpp_add<0x142, 0xa>(v);
-    v = dpp_add<0x143, 0xc>(v);
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
-
-// Three sums at once (their DPP steps interleave).
+// Sums over the 64 lanes (all active), returned to every lane: inclusive
+// scans with DPP (row_shr 1, 2, 4, 8 within rows of 16 lanes, then
+// row_bcast:15 and row_bcast:31), read from lane 63.
 __device__ inline void wave_sum3(float &a, float &b, float &c) {
 #define FT_DPP3(CTRL, RM) a = dpp_add<CTRL, RM>(a); b = dpp_add<CTRL, RM>(b); c = dpp_add<CTRL, RM>(c);
     FT_DPP3(0x111, 0xf)
@@ -189,21 +139,6 @@ __device__ inline void wave_sum3(float &a, float &b, float &c) {
     a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 63));
     b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, b), 63));
     c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c), 63));
-}
-
-__device__ inline float alpha_of(float A, float &dadA) {
-    const float m = fabsf(A);
-    if (m < 1.0f) {
-        dadA = A > 0.0f ? 1.0f : (A < 0.0f ? -1.0f : 0.0f);
-        return m;
-    }
-    dadA = 0.0f;
-    return 1.0f;
-}
-
-__device__ inline float4 over(float4 c, float al, float4 C) {
-    const float keep = 1.0f - c.w * al;
-    return make_float4(c.x * al + C.x * keep, c.y * al + C.y * keep, c.z * al + C.z * keep, c.w * al + C.w * keep);
 }
 
 // ---------------------------------------------------------------------------
@@ -472,163 +407,6 @@ __global__ __launch_bounds__(BLOCK) void k_sort_cells(DScene S, DevStatus *st) {
 // ---------------------------------------------------------------------------
 // Forward, loss, backward
 // ---------------------------------------------------------------------------
-// Row staging.  A block owns DBLOCK pixels of one row of one image.  It
-// stages the (cell count, list offset, colour) of a run of the image's paths
-// for its row (stage_paths) and then their row pieces in windows of ECAP
-// (one thread per piece: edge index, two vertices, piece_of), so that the
-// per-pixel loops read every piece and colour from LDS with one broadcast
-// load instead of a chain of dependent global loads per edge and path.
-constexpr uint32_t PCHUNK = DBLOCK;  // paths staged per round (one per thread)
-constexpr uint32_t ECAP = 512;       // pieces staged per window
-constexpr uint32_t LAST_BIT = 0x80000000u, LIVE_BIT = 0x40000000u, J_MASK = 0x3FFFFFFFu;
-
-struct Stage {
-    uint32_t *cnt;  // [PCHUNK] pieces of each staged path in the row
-    uint32_t *off;  // [PCHUNK] its cell's list offset
-    uint32_t *pb;   // [PCHUNK] exclusive scan of cnt
-    float4 *col;    // [PCHUNK] its colour
-    float4 *pc;     // [ECAP] piece: x at top, x at bottom, sign * height, 0
-    uint32_t *ev;   // [ECAP] staged path index | LAST_BIT | LIVE_BIT
-    uint2 *vi;      // [ECAP] global indices of the edge's two vertices (or null: not staged)
-    float4 *pq;     // [ECAP] their coordinates (or null)
-    uint32_t *w;    // [DBLOCK / 64] scan scratch
-};
-
-// Counts, offsets and colours of row Y for the n <= PCHUNK paths from global
-// path kbase; returns their total number of pieces.  Every thread calls it.
-__device__ uint32_t stage_paths(const DScene &S, const float4 *colours, uint32_t kbase, uint32_t n, int Y,
-                                const Stage &sg) {
-    const uint32_t t = threadIdx.x;
-    const bool in = t < n;
-    const uint64_t cell = (uint64_t)(kbase + (in ? t : 0u)) * S.H + (uint32_t)Y;
-    const uint32_t c = in ? S.cell_cnt[cell] : 0u;
-    const uint32_t o = in ? S.cell_off[cell] : 0u;
-    const float4 col = colours[kbase + (in ? t : 0u)];
-    const uint32_t incl = wave_incl_dpp<false>(c);
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 63) sg.w[wid] = incl;
-    __syncthreads();
-    uint32_t pre = incl - c, total = 0;
-#pragma unroll
-    for (int w = 0; w < DBLOCK / 64; ++w) {
-        pre += w < wid ? sg.w[w] : 0u;
-        total += sg.w[w];
-    }
-    if (in) {
-        sg.cnt[t] = c;
-        sg.off[t] = o;
-        sg.pb[t] = pre;
-        sg.col[t] = col;
-    }
-    __syncthreads();
-    return total;
-}
-
-// Pieces [e0, e0 + n) (n <= ECAP) of the np staged paths into the piece
-// arrays at [0, n).  Piece e belongs to the last staged path t with
-// pb[t] <= e.  The caller synchronises before and after.
-__device__ void stage_pieces(const DScene &S, uint32_t kbase, uint32_t np, int Y, uint32_t e0, uint32_t n,
-                             const Stage &sg, uint32_t &bad) {
-    for (uint32_t i = threadIdx.x; i < n; i += DBLOCK) {
-        const uint32_t e = e0 + i;
-        uint32_t lo = 0, hi = np;  // pb[lo] <= e < pb[hi] (pb[np] taken as the total)
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (sg.pb[mid] <= e)
-                lo = mid;
-            else
-                hi = mid;
-        }
-        const uint32_t q = e - sg.pb[lo];
-        const uint32_t k = kbase + lo;
-        const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
-        const uint32_t edge = S.cell_edge[sg.off[lo] + q];
-        bad |= edge < V ? 0u : 1u;
-        const uint32_t i0 = edge < V ? edge : 0u;
-        const uint32_t i1 = i0 + 1 < V ? i0 + 1 : 0u;
-        const float2 a = S.vtx[vb + i0], b = S.vtx[vb + i1];
-        const Piece r = piece_of(a, b, Y);
-        sg.pc[i] = make_float4(r.xa, r.xb, r.live ? r.sign * r.h : 0.0f, 0.0f);
-        sg.ev[i] = lo | (q + 1 == sg.cnt[lo] ? LAST_BIT : 0u) | (r.live ? LIVE_BIT : 0u);
-        if (sg.vi) {
-            sg.vi[i] = make_uint2(vb + i0, vb + i1);
-            sg.pq[i] = make_float4(a.x, a.y, b.x, b.y);
-        }
-    }
-}
-
-// sign * h * M of a staged piece at pixel X, M = mean_clamp(X + 1 - xa,
-// X + 1 - xb).  A wavefront whose pixels [xw0, xw0 + 63] all lie left of the
-// piece (X + 1 <= min x: M = 0) or all right of it (X >= max x: M = 1) takes
-// the answer without evaluating M; these are exactly the values mean_clamp
-// returns there.
-__device__ inline float piece_cover(float4 pc, float Xf, float xw0) {
-    const float lo = fminf(pc.x, pc.y), hi = fmaxf(pc.x, pc.y);
-    if (xw0 + 64.0f <= lo) return 0.0f;
-    if (xw0 >= hi) return pc.z;
-    float da, db;
-    return pc.z * mean_clamp(Xf + 1.0f - pc.x, Xf + 1.0f - pc.y, da, db);
-}
-
-// The image's np paths (from global path k0) composited over a transparent
-// pixel (X, Y).  With ck it also writes the canvas before every KSEG-th path
-// (the backward's checkpoints) and, with cov, each path's coverage (paths
-// with no piece in the row are left out, as their coverage is 0).  Every
-// thread of the block calls it.
-__device__ float4 forward_row(const DScene &S, const float4 *colours, uint32_t k0, uint32_t np, int X, int Y,
-                              uint64_t slot, float4 *ck, uint64_t ck_stride, float *cov, const Stage &sg,
-                              uint32_t &bad) {
-    float4 C = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float A = 0.0f;
-    uint32_t next_ck = 0;
-    const float Xf = (float)X;
-    const float xw0 = (float)(X - (int)(threadIdx.x & 63));
-    for (uint32_t ja = 0; ja < np; ja += PCHUNK) {
-        const uint32_t n = np - ja < PCHUNK ? np - ja : PCHUNK;
-        __syncthreads();  // the previous round's staging is no longer read
-        const uint32_t total = stage_paths(S, colours, k0 + ja, n, Y, sg);
-        for (uint32_t e0 = 0; e0 < total; e0 += ECAP) {
-            const uint32_t ne = total - e0 < ECAP ? total - e0 : ECAP;
-            __syncthreads();
-            stage_pieces(S, k0 + ja, n, Y, e0, ne, sg, bad);
-            __syncthreads();
-            auto close_path = [&](uint32_t ev) {  // the path's last piece: composite it
-                const uint32_t t = ev & J_MASK, j = ja + t;
-                if (ck)
-                    for (; next_ck * KSEG <= j; ++next_ck) ck[(uint64_t)next_ck * ck_stride + slot] = C;
-                if (ck && cov) cov[(uint64_t)j * ck_stride + slot] = A;  // j < max_paths, slot < ck_stride
-                float dadA;
-                C = over(sg.col[t], alpha_of(A, dadA), C);
-                A = 0.0f;
-            };
-            // four pieces' loads at a time, their covers added in order
-            uint32_t i = 0;
-            for (; i + 4 <= ne; i += 4) {
-                const float4 p0 = sg.pc[i], p1 = sg.pc[i + 1], p2 = sg.pc[i + 2], p3 = sg.pc[i + 3];
-                const uint4 ev = *reinterpret_cast<const uint4 *>(sg.ev + i);
-                const float c0 = piece_cover(p0, Xf, xw0), c1 = piece_cover(p1, Xf, xw0);
-                const float c2 = piece_cover(p2, Xf, xw0), c3 = piece_cover(p3, Xf, xw0);
-                A += c0;
-                if (ev.x & LAST_BIT) close_path(ev.x);
-                A += c1;
-                if (ev.y & LAST_BIT) close_path(ev.y);
-                A += c2;
-                if (ev.z & LAST_BIT) close_path(ev.z);
-                A += c3;
-                if (ev.w & LAST_BIT) close_path(ev.w);
-            }
-            for (; i < ne; ++i) {
-                A += piece_cover(sg.pc[i], Xf, xw0);
-                const uint32_t ev = sg.ev[i];
-                if (ev & LAST_BIT) close_path(ev);
-            }
-        }
-    }
-    if (ck)
-        for (; next_ck * KSEG < np; ++next_ck) ck[(uint64_t)next_ck * ck_stride + slot] = C;
-    return C;
-}
-
 // ---------------------------------------------------------------------------
 // Coverage by cells.  A block owns a tile of blockDim.x pixels (64 to
 // TILE_MAX) of one row of one image and takes the image's paths SEG at a
@@ -642,11 +420,13 @@ __device__ float4 forward_row(const DScene &S, const float4 *colours, uint32_t k
 // image of 256 paths.  What is left is VALU work: per path and pixel about 9
 // instructions of prefix sum and 9 of composite.)
 //
-// Cells are integers in units of 2^-24 (an i32 add): the sum does not depend
+// Cells are integers in units of 2^-26 (an i32 add): the sum does not depend
 // on the order of the pieces, so the same inputs give the same canvas
 // whichever kernel computes it, and each column's value is rounded once, at
-// 2^-25, where a float sum rounds at every piece.  i32 holds |A| < 128; a
-// (path, row) with more than HEAVY pieces takes 64-bit cells instead.
+// 2^-27, where a float sum rounds at every piece.  (At 2^-24 a pixel that an
+// edge covers by less than 2^-25 lost its gradient: 8.2e-6 from FP64 on a
+// 512x512 scene whose gradients are 4.4e-6 off otherwise.)  i32 holds
+// |A| < 32; a (path, row) with more than HEAVY pieces takes 64-bit cells.
 //
 // Every 64-column chunk of a row stands alone: a piece left of a chunk adds
 // its whole signed height to the chunk's first cell, so no carry passes
@@ -658,9 +438,9 @@ constexpr uint32_t SEG = 16;         // paths per round
 // takes 229 us a call with 256, 250 with 512, 233 with 128.
 constexpr uint32_t TILE_MAX = 256;
 constexpr uint32_t ROW_PATHS = 256;  // paths whose cell counts are staged at once
-constexpr uint32_t HEAVY = 120;      // pieces of one path in one row past which cells are 64-bit
+constexpr uint32_t HEAVY = 31;       // pieces of one path in one row past which cells are 64-bit
 constexpr int RAMP_LANE = 8;         // ramps of at most this many columns are walked by one lane
-constexpr float CELL_ONE = 16777216.0f;  // 2^24
+constexpr float CELL_ONE = 67108864.0f;  // 2^26
 
 struct RowLds {
     __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of the staged paths' piece counts, then the total
@@ -753,7 +533,7 @@ __device__ __forceinline__ PieceVtx piece_vtx(const DScene &S, const RowLds &R, 
 // it.  [c0, c1) are the ramp's columns within the tile (c1 <= c0: none), and
 // from column max(c0, c1) on the piece counts whole.
 struct Ramp {
-    float lo, hi, inv, z;  // x range, 1 / (hi - lo), signed height
+    float lo, hi, w, inv, z;  // x range, its width, 1 / w (0: narrow, the midpoint's value), signed height
     int c0, c1;
     bool live, nan;
 };
@@ -763,27 +543,38 @@ __device__ __forceinline__ Ramp ramp_of(const Piece &r, float xb0, int tw) {
     m.lo = r.xa < r.xb ? r.xa : r.xb;
     m.hi = r.xa < r.xb ? r.xb : r.xa;
     m.z = r.sign * r.h;
-    const float w = m.hi - m.lo;
-    m.nan = r.live & !(w < __builtin_inff());  // a NaN or unbounded x
+    m.w = m.hi - m.lo;
+    m.nan = r.live & !(m.w < __builtin_inff());  // a NaN or unbounded x
     m.live = r.live & !m.nan & (m.lo < xb0 + (float)tw);
-    m.inv = w < EPS_W ? 0.0f : 1.0f / w;  // 0: narrow, the midpoint's value
+    m.inv = m.w < EPS_W ? 0.0f : 1.0f / m.w;
     const float f0 = floorf(m.lo) - xb0, f1 = ceilf(m.hi) - xb0;
     m.c0 = f0 > 0.0f ? (f0 < (float)tw ? (int)f0 : tw) : 0;
     m.c1 = f1 > 0.0f ? (f1 < (float)tw ? (int)f1 : tw) : 0;
     return m;
 }
 
-// M at the pixel whose right border is X1, within the ramp (as mean_clamp).
-__device__ __forceinline__ float ramp_cover(const Ramp &m, float X1) {
+// M at the pixel whose right border is X1, within the ramp: the mean of
+// clamp(u, 0, 1) for u from X1 - hi to X1 - lo; a and b are the clamped ends.
+// The quotient is the correctly rounded one (a product with 1 / w corrected
+// by its remainder): M close to 0 or 1 decides whether a pixel has a
+// gradient.
+__device__ __forceinline__ float ramp_mean(const Ramp &m, float X1, float &a, float &b) {
     const float lo = X1 - m.hi, hi = X1 - m.lo;
+    a = clamp01(lo);
+    b = clamp01(hi);
     if (m.inv == 0.0f) return clamp01((lo + hi) * 0.5f);
-    const float a = clamp01(lo), b = clamp01(hi);
-    return ((b - a) * (a + b) * 0.5f + (hi > 1.0f ? hi - 1.0f : 0.0f)) * m.inv;
+    const float I = (b - a) * (a + b) * 0.5f + fmaxf(hi - 1.0f, 0.0f);
+    const float q = I * m.inv;
+    return fmaf(fmaf(-q, m.w, I), m.inv, q);
+}
+__device__ __forceinline__ float ramp_cover(const Ramp &m, float X1) {
+    float a, b;
+    return ramp_mean(m, X1, a, b);
 }
 
 template <typename T>
 __device__ __forceinline__ T cell_of(float zs, float M) {
-    return (T)__float2int_rn(zs * M);  // |zs * M| <= 2^24
+    return (T)__float2int_rn(zs * M);  // |zs * M| <= 2^26
 }
 template <typename T>
 __device__ __forceinline__ void cell_add(T *c, T v) {
@@ -820,6 +611,7 @@ __device__ __forceinline__ void scatter_piece(T *cells, uint32_t row_at, const R
         Ramp w;
         w.lo = bc(m.lo);
         w.hi = bc(m.hi);
+        w.w = w.hi - w.lo;
         w.inv = bc(m.inv);
         const float wz = bc(zs);
         const int w0 = __builtin_amdgcn_readlane(m.c0, l), w1 = __builtin_amdgcn_readlane(m.c1, l);
@@ -841,11 +633,13 @@ __device__ __forceinline__ void scatter_piece(T *cells, uint32_t row_at, const R
 }
 
 // Coverage A[j] of round s's paths at this thread's pixel, from the first
-// blockDim.x pieces (ref, v: one per thread, loaded by the caller ahead of
+// blockDim.x pieces (ref, first: one per thread, loaded by the caller ahead of
 // time) and any further ones.  cells: SEG rows of pitch `pitch`, zero on
-// entry and on exit (the exit barrier included).  Every thread calls it.
+// entry; with ZERO zero again on exit, behind a barrier, else the caller's to
+// use: each thread has read its own column.  Every thread calls it.
+template <bool ZERO>
 __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t s, const PieceRef &ref,
-                                            const PieceVtx &v, const Piece &first, int Y, float xb0, int *cells,
+                                            const Piece &first, int Y, float xb0, int *cells,
                                             uint32_t pitch, float A[SEG], uint32_t &bad) {
     const int tid = threadIdx.x, tw = (int)blockDim.x;
     const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];
@@ -899,7 +693,7 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
 #pragma unroll
     for (uint32_t j = 0; j < SEG; ++j) {
         c[j] = (uint32_t)cells[j * pitch + tid];
-        cells[j * pitch + tid] = 0;
+        if (ZERO) cells[j * pitch + tid] = 0;
     }
     const uint32_t poison = R.poison[s & 1];
     if (tid == 0) R.poison[(s + 1) & 1] = 0;
@@ -913,18 +707,10 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
 #pragma unroll
         for (uint32_t j = 0; j < SEG; ++j) A[j] = ((poison >> j) & 1u) ? 2.0f : A[j];
     }
-    __syncthreads();
+    if (ZERO) __syncthreads();
 }
 
 __device__ __forceinline__ float alpha_cover(float A) { return __builtin_amdgcn_fmed3f(fabsf(A), 0.0f, 1.0f); }
-
-#define DIFF_STAGE_LDS(VI, PQ)                                          \
-    __shared__ uint32_t s_cnt[PCHUNK], s_off[PCHUNK], s_pb[PCHUNK];    \
-    __shared__ float4 s_col[PCHUNK];                                    \
-    __shared__ float4 s_pc[ECAP];                                       \
-    __shared__ __align__(16) uint32_t s_ev[ECAP];                       \
-    __shared__ uint32_t s_w[DBLOCK / 64];                               \
-    const Stage sg{s_cnt, s_off, s_pb, s_col, s_pc, s_ev, VI, PQ, s_w}
 
 // Colour of the image's path j, or zero where `on` is 0 (a path without
 // pieces in the row does not touch it, whatever its colour).  Uniform: scalar
@@ -940,13 +726,11 @@ __device__ __forceinline__ float4 round_colour(const float4 *__restrict__ colour
 // The canvas of one tile of one row: the image's paths composited over
 // transparent pixels, SEG at a time, with the next round's pieces loaded
 // while a round is composited.  With ck it also leaves the canvas before
-// every KSEG-th path and, with cov, each path's coverage (paths with no piece
-// in the row are left out, as their coverage is 0) at slot
-// (image row) * ck_pitch + X.
+// every round but the first, at slot (image row) * ck_pitch + X; canvas may
+// be null.
 __global__ __launch_bounds__(TILE_MAX) void k_forward(DScene S, const float4 *__restrict__ colours,
                                                       float4 *__restrict__ canvas, float4 *__restrict__ ck,
-                                                      uint32_t ck_pitch, uint64_t ck_stride,
-                                                      float *__restrict__ cov, DevStatus *st) {
+                                                      uint32_t ck_pitch, uint64_t ck_stride, DevStatus *st) {
     extern __shared__ __align__(16) int s_cells[];
     __shared__ RowLds R;
     if (run_failed(st)) return;
@@ -970,26 +754,20 @@ __global__ __launch_bounds__(TILE_MAX) void k_forward(DScene S, const float4 *__
         PieceRef nref = ref;
         if (rounds > 1) nref = piece_ref(S, R, 1, R.pb[SEG] + threadIdx.x);
         for (uint32_t s = 0; s < rounds; ++s) {
-            const Piece first = piece_of(v.p, v.q, (int)Y);
             const PieceRef cur = ref;
-            const PieceVtx cv = v;
+            const Piece first = piece_of(v.p, v.q, (int)Y);
             if (s + 1 < rounds) {  // the next round's vertices, and the one after's edge
                 ref = nref;
                 v = piece_vtx(S, R, s + 1, ref, bad);
                 if (s + 2 < rounds) nref = piece_ref(S, R, s + 2, R.pb[(s + 2) * SEG] + threadIdx.x);
             }
             float A[SEG];
-            round_cover(S, R, s, cur, cv, first, (int)Y, xb0, s_cells, pitch, A, bad);
+            round_cover<true>(S, R, s, cur, first, (int)Y, xb0, s_cells, pitch, A, bad);
             const uint32_t j0 = ja + s * SEG;
             const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
-            if (cov && in) {
-#pragma unroll
-                for (uint32_t j = 0; j < SEG; ++j)
-                    if ((some >> j) & 1u) cov[(uint64_t)(j0 + j) * ck_stride + slot] = A[j];
-            }
+            if (ck && j0 && in) ck[(uint64_t)(j0 / SEG) * ck_stride + slot] = C;
 #pragma unroll
             for (uint32_t j = 0; j < SEG; ++j) {
-                if (ck && j % KSEG == 0 && j0 + j < np && in) ck[(uint64_t)((j0 + j) / KSEG) * ck_stride + slot] = C;
                 const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
                 const float al = alpha_cover(A[j]), keep = fmaf(-c.w, al, 1.0f);
                 C = make_float4(fmaf(C.x, keep, c.x * al), fmaf(C.y, keep, c.y * al), fmaf(C.z, keep, c.z * al),
@@ -998,7 +776,7 @@ __global__ __launch_bounds__(TILE_MAX) void k_forward(DScene S, const float4 *__
         }
     }
     if (bad) raise_err(st, FT_EDEVICE);
-    if (in) canvas[((uint64_t)im * S.H + Y) * S.W + X] = C;
+    if (canvas && in) canvas[((uint64_t)im * S.H + Y) * S.W + X] = C;
 }
 
 // loss partials per block (sum of squared differences); grad = 2 (C - T) / N.
@@ -1023,249 +801,233 @@ __global__ __launch_bounds__(BLOCK) void k_loss(const float *canvas, const float
     }
 }
 
-// One lane per pixel.  Pass 1 replays the forward into the checkpoints
-// (skipped when k_forward of the same inputs has written them: `replayed`).
-// Pass 2 walks the checkpoint segments last to first.  Per segment: the
-// segment's paths (counts, offsets, colours) and their coverage per pixel
-// into LDS (recomputed from the staged pieces, or read from the kept
-// coverage buffer); then its paths last to first, with no block barrier: the
-// canvas under path j re-composited from the segment's checkpoint, the colour
-// gradient (wave sums into LDS), and per piece of path j the sums S1 = sum
-// dA M, S2 = sum dA dM/dua, S3 = sum dA dM/dub over the block's pixels (a
-// wavefront wholly right of the piece adds its dA total to S1 alone, one
-// wholly left adds nothing), accumulated in LDS.  When the walk leaves the
-// staged window of pieces (and at the segment's end) one thread per piece
-// forms its vertex gradients from S1..S3 with global atomics; the colour
-// gradients are flushed once per segment.
-__global__ __launch_bounds__(DBLOCK) void k_backward(DScene S, const float4 *colours, const float4 *grad_canvas,
-                                                     float4 *ck, uint32_t ck_pitch, uint64_t ck_stride, float *cov,
-                                                     uint32_t replayed,
-                                                     float2 *gvtx, float *gcol, DevStatus *st) {
-    __shared__ uint2 s_vi[ECAP];
-    __shared__ float4 s_pq[ECAP];
-    DIFF_STAGE_LDS(s_vi, s_pq);
-    __shared__ float s_A[KSEG][DBLOCK];  // coverage of the segment's paths; each thread uses its own column
-    __shared__ float4 s_S[ECAP];         // per staged piece: S1, S2, S3
-    __shared__ float s_gc[KSEG][4];      // colour gradients of the segment's paths
-    // coverage recompute, per staged window: each wavefront's sum of the
-    // pieces wholly left of it per path, and its list of the pieces that
-    // touch its columns
-    constexpr int NW = DBLOCK / 64;
-    __shared__ float s_Lw[KSEG][NW];
-    __shared__ uint16_t s_tl[NW][ECAP];
-    __shared__ uint32_t s_tn[NW];
+// Sums of 64 values over the wavefront's lanes at once, as a tree that
+// halves the number of registers at each level instead of reducing every
+// value on its own (141 instructions for 64 values; 6 DPP adds each would be
+// 384).  sum2 takes two values: lanes below 32 of the result hold a's sums
+// over lane pairs (l, l + 32), the others b's; sum_rows does the same over
+// row pairs of 16 lanes, and sum_dpp within a row, where the DPP pattern
+// CTRL mirrors the lanes and `hi` is the lane bit that decides.
+__device__ __forceinline__ float sum2(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+__device__ __forceinline__ float sum_rows(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ float sum_dpp(float a, float b, bool hi) {
+    const float give = hi ? a : b;
+    const int got = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), CTRL, 0xf, 0xf, true);
+    return (hi ? b : a) + __builtin_bit_cast(float, got);
+}
+
+// Inclusive prefix sum over the 64 lanes.
+__device__ __forceinline__ float wave_incl_f32(float v) {
+    v = dpp_add<0x111, 0xf>(v);
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);
+    return dpp_add<0x143, 0xc>(v);
+}
+
+// A piece's S1 = sum dA M, S2 = sum dA dM/dx_lo, S3 = sum dA dM/dx_hi terms
+// of one column (dA: the pixel's d loss / d coverage; the partials are with
+// respect to u = X1 - x, so S2 goes with the larger x).
+__device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, float &S1, float &S2, float &S3) {
+    float a, b;
+    const float M = ramp_mean(m, X1, a, b);
+    S1 = fmaf(g, M, S1);
+    if (m.inv == 0.0f) {  // narrow: half of the slope each
+        const float half = ((M > 0.0f) & (M < 1.0f)) ? 0.5f : 0.0f;
+        S2 += g * half;
+        S3 += g * half;
+        return;
+    }
+    S2 = fmaf(g, (M - a) * m.inv, S2);
+    S3 = fmaf(g, (b - M) * m.inv, S3);
+}
+
+// One tile of one row, the image's rounds of SEG paths last to first.  With f
+// the pixel's d loss / d canvas, everything the paths' gradients need of the
+// canvas is the scalar q_j = f . (canvas under path j), and of the paths above
+// the scalar T_j, the product of their 1 - alpha (the same for every channel):
+//     d loss / d alpha_j  = T_j (f . c_j - c_j.w q_j)
+//     d loss / d c_j      = sum over pixels of T_j alpha_j (f.x, f.y, f.z, f.w - q_j)
+// q starts from the round's checkpoint (k_forward's) and runs forward over
+// the round; T runs backward.  So a path costs a pixel about 20 operations
+// beside its coverage, where re-compositing four channels cost twice that.
+//
+// The paths' dA and its prefix sums per 64-column chunk go to LDS, and one
+// thread per piece gathers its sums: the ramp's columns one by one, and all
+// columns right of it from the prefix sums.  (Evaluating each piece on all 64
+// pixels of every wavefront it touches and reducing the three sums over the
+// wavefront took 18.4 ms for 64 images of 256x256 with 17,500 paths; this
+// form takes 4.4 ms, and 320 us instead of 869 for one 512x512 image of 256
+// paths; about 1.1 ms and 90 us of that are the vertex gradients' atomics.)  Four wavefronts per SIMD are asked for: without, the kernel takes
+// 156 VGPRs, a CU holds three blocks, and the 1,024 blocks of a 512x512 image
+// run in two passes (370 us).
+__global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4 *__restrict__ colours,
+                                                       const float4 *__restrict__ grad_canvas,
+                                                       const float4 *__restrict__ ck, uint32_t ck_pitch,
+                                                       uint64_t ck_stride, float2 *__restrict__ gvtx,
+                                                       float *__restrict__ gcol, DevStatus *st) {
+    extern __shared__ __align__(16) int s_cells[];  // cells, then the prefix sums of dA; then dA
+    __shared__ RowLds R;
+    __shared__ float s_gc[64];  // the round's colour gradients, in sum-tree order
     if (run_failed(st)) return;
+    const uint32_t tw = blockDim.x, pitch = tw + 1;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int X = (int)(blockIdx.x * DBLOCK + tid), Y = (int)blockIdx.y;
-    const float Xf = (float)X, xw0 = (float)(X - lane);
-    const uint32_t im = blockIdx.z;
-    const bool active = (uint32_t)X < S.W;
-    const uint64_t slot = ((uint64_t)im * S.H + (uint32_t)Y) * ck_pitch + (uint32_t)X;
+    const uint32_t X = blockIdx.x * tw + threadIdx.x, Y = blockIdx.y, im = blockIdx.z;
+    const float xb0 = (float)(blockIdx.x * tw);
     const uint32_t k0 = S.img_first[im], np = S.img_first[im + 1] - k0;
+    const uint64_t slot = ((uint64_t)im * S.H + Y) * ck_pitch + X;
+    const bool in = X < S.W;
+    float *const s_pre = reinterpret_cast<float *>(s_cells);
+    float *const s_dA = s_pre + SEG * pitch;
     uint32_t bad = 0;
-    if (!replayed) (void)forward_row(S, colours, k0, np, X, Y, slot, ck, ck_stride, cov, sg, bad);
-    float4 g = active ? grad_canvas[((uint64_t)im * S.H + (uint32_t)Y) * S.W + (uint32_t)X]
-                      : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    // the vertex gradients of the staged window's pieces [0, n) from their
-    // sums (then cleared); every thread calls it
-    // (every thread owns staged pieces tid and tid + DBLOCK; both are loaded
-    // before either's gradient is formed)
-    static_assert(ECAP == 2 * DBLOCK, "two staged pieces per thread");
-    auto flush_pieces = [&](uint32_t n) {
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float4 f = in ? grad_canvas[((uint64_t)im * S.H + Y) * S.W + X] : zero;
+    float T = 1.0f;
+    for (uint32_t i = threadIdx.x; i < SEG * pitch; i += tw) s_cells[i] = 0;
+    if (tid < 64) s_gc[tid] = 0.0f;
+    for (uint32_t chunk = (np + ROW_PATHS - 1) / ROW_PATHS; chunk-- > 0;) {
+        const uint32_t ja = chunk * ROW_PATHS;
+        const uint32_t n = np - ja < ROW_PATHS ? np - ja : ROW_PATHS;
+        const uint32_t rounds = (n + SEG - 1) / SEG;
+        __syncthreads();  // the previous paths' staging is no longer read
+        stage_row(S, k0 + ja, n, (int)Y, R);
         __syncthreads();
-        const uint32_t ia = tid, ib = tid + DBLOCK;
-        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        const float4 Sa = ia < n ? s_S[ia] : zero, Sb = ib < n ? s_S[ib] : zero;
-        const uint32_t ea = s_ev[ia], eb = s_ev[ib];
-        const float4 pqa = s_pq[ia], pqb = s_pq[ib];
-        const uint2 via = s_vi[ia], vib = s_vi[ib];
-        auto grad_of = [&](float4 Sm, uint32_t ev, float4 pq, uint2 vi) {
-            if (((Sm.x != 0.0f) | (Sm.y != 0.0f) | (Sm.z != 0.0f)) && (ev & LIVE_BIT)) {
-                float gr[4];
-                piece_grad(make_float2(pq.x, pq.y), make_float2(pq.z, pq.w), Y, Sm.x, Sm.y, Sm.z, gr);
-                atomicAdd(&gvtx[vi.x].x, gr[0]);
-                atomicAdd(&gvtx[vi.x].y, gr[1]);
-                atomicAdd(&gvtx[vi.y].x, gr[2]);
-                atomicAdd(&gvtx[vi.y].y, gr[3]);
+        PieceRef ref = piece_ref(S, R, rounds - 1, R.pb[(rounds - 1) * SEG] + threadIdx.x);
+        PieceVtx v = piece_vtx(S, R, rounds - 1, ref, bad);
+        PieceRef nref = ref;
+        if (rounds > 1) nref = piece_ref(S, R, rounds - 2, R.pb[(rounds - 2) * SEG] + threadIdx.x);
+        for (uint32_t s = rounds; s-- > 0;) {
+            const uint32_t j0 = ja + s * SEG;
+            const float4 C = in && j0 ? ck[(uint64_t)(j0 / SEG) * ck_stride + slot] : zero;
+            const PieceRef cur = ref;
+            const PieceVtx cv = v;
+            if (s > 0) {  // the next round's vertices, and the one after's edge
+                ref = nref;
+                v = piece_vtx(S, R, s - 1, ref, bad);
+                if (s > 1) nref = piece_ref(S, R, s - 2, R.pb[(s - 2) * SEG] + threadIdx.x);
             }
-        };
-        grad_of(Sa, ea, pqa, via);
-        grad_of(Sb, eb, pqb, vib);
-        if (ia < n) s_S[ia] = zero;
-        if (ib < n) s_S[ib] = zero;
-        __syncthreads();
-    };
-    for (uint32_t i = tid; i < ECAP; i += DBLOCK) s_S[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const uint32_t n_seg = (np + KSEG - 1) / KSEG;
-    for (uint32_t seg = n_seg; seg-- > 0;) {
-        const uint32_t j0 = seg * KSEG, j1 = j0 + KSEG < np ? j0 + KSEG : np;
-        const uint32_t ns = j1 - j0;
-        __syncthreads();  // the previous segment's staging is no longer read
-        const uint32_t total = stage_paths(S, colours, k0 + j0, ns, Y, sg);
-        if (tid < KSEG * 4) s_gc[tid >> 2][tid & 3] = 0.0f;
-        // the segment's coverage per path
-        for (uint32_t j = 0; j < ns; ++j) s_A[j][tid] = 0.0f;
-        uint32_t w_lo = 0, w_n = 0;  // staged window: pieces [w_lo, w_lo + w_n) of the segment
-        if (cov) {
-            for (uint32_t j = 0; j < ns; ++j)
-                if (active && s_cnt[j]) s_A[j][tid] = cov[(uint64_t)(j0 + j) * ck_stride + slot];
-        } else {
-            const int wid = tid >> 6;
-            const float xb0 = (float)(blockIdx.x * DBLOCK);
-            for (uint32_t e0 = 0; e0 < total; e0 += ECAP) {
-                const uint32_t ne = total - e0 < ECAP ? total - e0 : ECAP;
-                __syncthreads();
-                stage_pieces(S, k0 + j0, ns, Y, e0, ne, sg, bad);
-                if (tid < KSEG * NW) s_Lw[tid / NW][tid % NW] = 0.0f;
-                if (tid < NW) s_tn[tid] = 0;
-                __syncthreads();
-                w_lo = e0;
-                w_n = ne;
-                // each staged piece against each wavefront's 64 columns (the
-                // tests of piece_cover): wholly right adds nothing, wholly
-                // left its full sign * height, else it goes on the list
-                for (uint32_t i = tid; i < ne; i += DBLOCK) {
-                    const float4 pc = s_pc[i];
-                    const uint32_t ev = s_ev[i];
-                    if (!(ev & LIVE_BIT)) continue;  // no coverage
-                    const float lo = fminf(pc.x, pc.y), hi = fmaxf(pc.x, pc.y);
-                    const uint32_t j = ev & J_MASK;
+            float A[SEG];
+            round_cover<false>(S, R, s, cur, piece_of(cv.p, cv.q, (int)Y), (int)Y, xb0, s_cells, pitch, A, bad);
+            const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
+            float q[SEG], d[SEG];  // f . canvas under path j, and f . c_j - c_j.w q_j
+            float qr = fmaf(f.w, C.w, fmaf(f.z, C.z, fmaf(f.y, C.y, f.x * C.x)));
 #pragma unroll
-                    for (int w = 0; w < NW; ++w) {
-                        const float x0 = xb0 + 64.0f * (float)w;
-                        if (x0 + 64.0f <= lo) continue;
-                        if (x0 >= hi) {
-                            atomicAdd(&s_Lw[j][w], pc.z);
-                        } else {
-                            const uint32_t at = atomicAdd(&s_tn[w], 1u);
-                            s_tl[w][at] = (uint16_t)i;
-                        }
+            for (uint32_t j = 0; j < SEG; ++j) {
+                const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
+                const float fc = fmaf(f.w, c.w, fmaf(f.z, c.z, fmaf(f.y, c.y, f.x * c.x)));
+                const float al = alpha_cover(A[j]);
+                q[j] = qr;
+                d[j] = fmaf(-c.w, qr, fc);
+                qr = fmaf(al, d[j], qr);  // = al f . c_j + (1 - c_j.w al) q_j
+            }
+            float z[SEG / 2];
+            const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0, b1 = (lane & 2) != 0, b0 = (lane & 1) != 0;
+#pragma unroll
+            for (uint32_t jp = SEG / 2; jp-- > 0;) {
+                float r[2][4];
+#pragma unroll
+                for (uint32_t h = 2; h-- > 0;) {
+                    const uint32_t j = 2 * jp + h;
+                    const float cw = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u).w;
+                    const float al = alpha_cover(A[j]);
+                    const float dal = T * d[j], V = T * al;
+                    const bool part = (fabsf(A[j]) < 1.0f) & (A[j] != 0.0f);
+                    const float dA = part ? (A[j] > 0.0f ? dal : -dal) : 0.0f;
+                    r[h][0] = V * f.x;
+                    r[h][1] = V * f.y;
+                    r[h][2] = V * f.z;
+                    r[h][3] = V * (f.w - q[j]);
+                    T *= fmaf(-cw, al, 1.0f);
+                    s_dA[j * pitch + tid] = dA;
+                    s_pre[j * pitch + tid] = wave_incl_f32(dA);
+                }
+                const float x0 = sum2(r[0][0], r[1][0]), x1 = sum2(r[0][1], r[1][1]);
+                const float x2 = sum2(r[0][2], r[1][2]), x3 = sum2(r[0][3], r[1][3]);
+                z[jp] = sum_dpp<0x140>(sum_rows(x0, x1), sum_rows(x2, x3), b3);  // row_mirror
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) z[i] = sum_dpp<0x141>(z[2 * i], z[2 * i + 1], b2);  // row_half_mirror
+#pragma unroll
+            for (uint32_t i = 0; i < 2; ++i) z[i] = sum_dpp<0x1B>(z[2 * i], z[2 * i + 1], b1);  // quad_perm 3,2,1,0
+            // lane: path 2 (4 b0 + 2 b1 + b2) + (lane >> 5), channel 2 b3 + (lane >> 4 & 1)
+            const float gc = sum_dpp<0xB1>(z[0], z[1], b0);  // quad_perm 1,0,3,2
+            if (gc != 0.0f) atomicAdd(&s_gc[lane], gc);
+            __syncthreads();
+            if (tid < 64) {
+                const float g = s_gc[tid];
+                const uint32_t j = 2 * (4 * (tid & 1) + (tid & 2) + ((tid >> 2) & 1)) + (tid >> 5);
+                const uint32_t ch = ((tid >> 2) & 2) + ((tid >> 4) & 1);
+                s_gc[tid] = 0.0f;
+                if (g != 0.0f && j0 + j < np) atomicAdd(&gcol[4 * (uint64_t)(k0 + j0 + j) + ch], g);
+            }
+            // the pieces' gradients
+            const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];
+            for (uint32_t eb = base; eb < end; eb += tw) {
+                PieceRef pr = cur;
+                PieceVtx pv = cv;
+                if (eb != base) {
+                    pr = piece_ref(S, R, s, eb + threadIdx.x);
+                    pv = piece_vtx(S, R, s, pr, bad);
+                }
+                Piece pc = piece_of(pv.p, pv.q, (int)Y);
+                pc.live &= pr.j != NO_IDX;
+                const Ramp m = ramp_of(pc, xb0, (int)tw);
+                const uint32_t at = (pr.j != NO_IDX ? pr.j : 0u) * pitch;
+                const bool wide = m.live & (m.c1 - m.c0 > RAMP_LANE);
+                float S1 = 0.0f, S2 = 0.0f, S3 = 0.0f;
+                if (m.live & !wide)
+                    for (int c = m.c0; c < m.c1; ++c) ramp_grad(m, xb0 + (float)(c + 1), s_dA[at + c], S1, S2, S3);
+                unsigned long long todo = __ballot(wide);
+                while (todo) {  // a long ramp: one column per lane
+                    const int l = __ffsll((long long)todo) - 1;
+                    todo &= todo - 1;
+                    auto bc = [l](float u) {
+                        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, u), l));
+                    };
+                    Ramp w;
+                    w.lo = bc(m.lo);
+                    w.hi = bc(m.hi);
+                    w.w = w.hi - w.lo;
+                    w.inv = bc(m.inv);
+                    const int w0 = __builtin_amdgcn_readlane(m.c0, l), w1 = __builtin_amdgcn_readlane(m.c1, l);
+                    const uint32_t wat = (uint32_t)__builtin_amdgcn_readlane((int)at, l);
+                    float a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+                    for (int c = w0 + lane; c < w1; c += 64)
+                        ramp_grad(w, xb0 + (float)(c + 1), s_dA[wat + c], a1, a2, a3);
+                    wave_sum3(a1, a2, a3);
+                    S1 = lane == l ? a1 : S1;
+                    S2 = lane == l ? a2 : S2;
+                    S3 = lane == l ? a3 : S3;
+                }
+                if (m.live) {  // the columns right of the ramp
+                    const int t = m.c1 > m.c0 ? m.c1 : m.c0;
+                    if (t < (int)tw) S1 += s_pre[at + (t | 63)] - ((t & 63) ? s_pre[at + t - 1] : 0.0f);
+                    for (int c = (t | 63) + 64; c < (int)tw; c += 64) S1 += s_pre[at + c];
+                    if ((S1 != 0.0f) | (S2 != 0.0f) | (S3 != 0.0f)) {
+                        float gr[4];
+                        const bool flip = pc.xa < pc.xb;  // S2 goes with the larger x
+                        piece_grad(pv.p, pv.q, (int)Y, S1, flip ? S3 : S2, flip ? S2 : S3, gr);
+                        atomicAdd(&gvtx[pv.ip].x, gr[0]);
+                        atomicAdd(&gvtx[pv.ip].y, gr[1]);
+                        atomicAdd(&gvtx[pv.iq].x, gr[2]);
+                        atomicAdd(&gvtx[pv.iq].y, gr[3]);
                     }
                 }
-                __syncthreads();
-                // the window's coverage of each path at this lane's pixel
-                for (uint32_t j = 0; j < ns; ++j) s_A[j][tid] += s_Lw[j][wid];
-                const uint32_t nt = s_tn[wid];
-                uint32_t k = 0;
-                for (; k + 2 <= nt; k += 2) {
-                    const uint32_t ia = s_tl[wid][k], ib = s_tl[wid][k + 1];
-                    const float4 pa = s_pc[ia], pb = s_pc[ib];
-                    const uint32_t ja = s_ev[ia] & J_MASK, jb = s_ev[ib] & J_MASK;
-                    float da, db;
-                    const float ca = pa.z * mean_clamp(Xf + 1.0f - pa.x, Xf + 1.0f - pa.y, da, db);
-                    const float cb = pb.z * mean_clamp(Xf + 1.0f - pb.x, Xf + 1.0f - pb.y, da, db);
-                    s_A[ja][tid] += ca;
-                    s_A[jb][tid] += cb;
-                }
-                if (k < nt) {
-                    const uint32_t i = s_tl[wid][k];
-                    const float4 pc = s_pc[i];
-                    float da, db;
-                    s_A[s_ev[i] & J_MASK][tid] += pc.z * mean_clamp(Xf + 1.0f - pc.x, Xf + 1.0f - pc.y, da, db);
-                }
             }
-        }
-        __syncthreads();  // s_gc cleared before the walk's atomics
-        // the canvas under each of the segment's paths, composited once from
-        // the checkpoint (the same operations, in the same order, as a
-        // composite from the checkpoint for each path)
-        float4 Cbs[KSEG];
-        {
-            float4 C = active ? ck[(uint64_t)seg * ck_stride + slot] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            __syncthreads();
 #pragma unroll
-            for (uint32_t i = 0; i < (uint32_t)KSEG; ++i) {
-                Cbs[i] = C;
-                if (i + 1 < ns) {
-                    float d;
-                    C = over(s_col[i], alpha_of(s_A[i][tid], d), C);
-                }
-            }
-        }
-        for (uint32_t jl = ns; jl-- > 0;) {
-            float4 Cb = Cbs[0];  // canvas before path j
-#pragma unroll
-            for (uint32_t k = 1; k < (uint32_t)KSEG; ++k)
-                if (k == jl) Cb = Cbs[k];
-            const float A = s_A[jl][tid];
-            float dadA;
-            const float al = alpha_of(A, dadA);
-            const float4 cc = s_col[jl];
-            const float dal = g.x * (cc.x - cc.w * Cb.x) + g.y * (cc.y - cc.w * Cb.y) + g.z * (cc.z - cc.w * Cb.z) +
-                              g.w * (cc.w - cc.w * Cb.w);
-            const float gdotC = g.x * Cb.x + g.y * Cb.y + g.z * Cb.z + g.w * Cb.w;
-            if (__ballot(al != 0.0f)) {
-                float r0 = g.x * al, r1 = g.y * al, r2 = g.z * al;
-                float r3 = g.w * al - al * gdotC;
-                wave_sum3(r0, r1, r2);
-                r3 = wave_sum(r3);
-                if (lane == 0) {
-                    atomicAdd(&s_gc[jl][0], r0);
-                    atomicAdd(&s_gc[jl][1], r1);
-                    atomicAdd(&s_gc[jl][2], r2);
-                    atomicAdd(&s_gc[jl][3], r3);
-                }
-            }
-            const float keep = 1.0f - cc.w * al;
-            g = make_float4(g.x * keep, g.y * keep, g.z * keep, g.w * keep);
-            const float dA = active ? dal * dadA : 0.0f;
-            // s_cnt and s_pb are the same for the whole block, so the window
-            // decisions (and the barriers in them) are too
-            const uint32_t cnt = s_cnt[jl], pb = s_pb[jl];
-            if (!cnt) continue;
-            const bool wave_on = __ballot(dA != 0.0f) != 0;
-            const float Tw = wave_sum(dA);  // the wavefront's dA total
-            // the path's pieces [pb, pb + cnt), in windows from the top
-            for (uint32_t e_hi = pb + cnt; e_hi > pb;) {
-                const uint32_t e_lo = e_hi - pb > ECAP ? e_hi - ECAP : pb;
-                if (!(e_lo >= w_lo && e_hi <= w_lo + w_n)) {
-                    // the walk leaves the staged window: its pieces' gradients, then
-                    // a window ending at e_hi (pieces of this path and the ones before)
-                    flush_pieces(w_n);
-                    const uint32_t lo = e_hi > ECAP ? e_hi - ECAP : 0u;
-                    stage_pieces(S, k0 + j0, ns, Y, lo, e_hi - lo, sg, bad);
-                    __syncthreads();
-                    w_lo = lo;
-                    w_n = e_hi - lo;
-                }
-                // a piece's sums: S1 = Σ dA·M, S2 = Σ dA·∂M/∂u_a, S3 = Σ dA·∂M/∂u_b
-                // over the wavefront
-                auto piece_sums = [&](uint32_t i, float4 pc, uint32_t ev) {
-                    if (!(ev & LIVE_BIT)) return;
-                    const float lo = fminf(pc.x, pc.y), hi = fmaxf(pc.x, pc.y);
-                    if (xw0 + 64.0f <= lo) return;  // M = 0 on every pixel of the wavefront
-                    if (xw0 >= hi) {               // M = 1, dM = 0
-                        if (lane == 0) atomicAdd(&s_S[i].x, Tw);
-                        return;
-                    }
-                    float mua, mub;
-                    const float M = mean_clamp(Xf + 1.0f - pc.x, Xf + 1.0f - pc.y, mua, mub);
-                    float S1 = dA * M, S2 = dA * mua, S3 = dA * mub;
-                    wave_sum3(S1, S2, S3);
-                    if (lane == 0) {
-                        atomicAdd(&s_S[i].x, S1);
-                        atomicAdd(&s_S[i].y, S2);
-                        atomicAdd(&s_S[i].z, S3);
-                    }
-                };
-                // four pieces' loads at a time
-                uint32_t e = e_lo;
-                for (; wave_on && e + 4 <= e_hi; e += 4) {
-                    const uint32_t i = e - w_lo;
-                    const float4 p0 = s_pc[i], p1 = s_pc[i + 1], p2 = s_pc[i + 2], p3 = s_pc[i + 3];
-                    const uint32_t v0 = s_ev[i], v1 = s_ev[i + 1], v2 = s_ev[i + 2], v3 = s_ev[i + 3];
-                    piece_sums(i, p0, v0);
-                    piece_sums(i + 1, p1, v1);
-                    piece_sums(i + 2, p2, v2);
-                    piece_sums(i + 3, p3, v3);
-                }
-                for (; wave_on && e < e_hi; ++e) piece_sums(e - w_lo, s_pc[e - w_lo], s_ev[e - w_lo]);
-                e_hi = e_lo;
-            }
-        }
-        flush_pieces(w_n);  // the segment's last window (and its barrier before the colours)
-        if (tid < (int)ns * 4) {
-            const float a = s_gc[tid >> 2][tid & 3];
-            if (a != 0.0f) atomicAdd(&gcol[4 * (uint64_t)(k0 + j0 + (tid >> 2)) + (tid & 3)], a);
+            for (uint32_t j = 0; j < SEG; ++j) s_cells[j * pitch + tid] = 0;
+            __syncthreads();
         }
     }
     if (bad) raise_err(st, FT_EDEVICE);
@@ -1348,7 +1110,6 @@ struct ft_diff {
     float4 *d_ck = nullptr;
     uint32_t ck_pitch = 0;  // checkpoint pixels per row
     uint64_t ck_stride = 0;  // and per checkpoint
-    float *d_cov = nullptr;  // [max_paths][ck_stride] kept coverage (FT_DIFF_KEEP_COVERAGE), or null: recomputed
     double *d_partial = nullptr;  // [LOSS_GRID] loss partials, then [LOSS_GRID] their sum
     double *h_loss = nullptr;     // pinned: the summed loss
     DevStatus *d_status = nullptr, *h_status = nullptr;
@@ -1442,16 +1203,21 @@ ft_status grow_pairs(ft_diff *d) {
     return FT_OK;
 }
 
-dim3 raster_grid(const ft_diff *d) { return dim3((d->W + DBLOCK - 1) / DBLOCK, d->H, d->n_images); }
+// Tiles of the forward and the backward: at most TILE_MAX pixels of a row, in
+// whole wavefronts.
+uint32_t tiles_of(const ft_diff *d) { return (d->W + TILE_MAX - 1) / TILE_MAX; }
+uint32_t tile_width(const ft_diff *d) {
+    const uint32_t n = tiles_of(d);
+    return ((d->W + n - 1) / n + 63) / 64 * 64;
+}
 
-// Forward tiles: at most TILE_MAX pixels of a row, in whole wavefronts.
+// canvas may be null; keep: also the checkpoints that the backward needs.
 ft_status launch_forward(ft_diff *d, const float *colours, float *canvas, bool keep) {
-    const uint32_t tiles = (d->W + TILE_MAX - 1) / TILE_MAX;
-    const uint32_t tw = ((d->W + tiles - 1) / tiles + 63) / 64 * 64;
+    const uint32_t tw = tile_width(d);
     const size_t lds = (size_t)SEG * (tw + 1) * sizeof(int);
-    k_forward<<<dim3(tiles, d->H, d->n_images), tw, lds, d->stream>>>(
+    k_forward<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
         scene_of(d), reinterpret_cast<const float4 *>(colours), reinterpret_cast<float4 *>(canvas),
-        keep ? d->d_ck : nullptr, d->ck_pitch, d->ck_stride, keep ? d->d_cov : nullptr, d->d_status);
+        keep ? d->d_ck : nullptr, d->ck_pitch, d->ck_stride, d->d_status);
     FD_HIP(hipGetLastError());
     return FT_OK;
 }
@@ -1487,14 +1253,16 @@ ft_status run_loss(ft_diff *d, const float *canvas, const float *target, float *
     return st;
 }
 
-// Enqueues the backward kernels.  replayed: k_forward with checkpoints of the
-// same points and colours ran just before on the same geometry.
+// Enqueues the backward kernels, after a forward of the same points and
+// colours that left its checkpoints.
 ft_status launch_backward(ft_diff *d, const float *colours, const float *grad_canvas, float *grad_points,
-                          float *grad_colours, bool replayed) {
+                          float *grad_colours) {
     DScene S = scene_of(d);
-    k_backward<<<raster_grid(d), DBLOCK, 0, d->stream>>>(
+    const uint32_t tw = tile_width(d);
+    const size_t lds = 2 * (size_t)SEG * (tw + 1) * sizeof(float);
+    k_backward<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
         S, reinterpret_cast<const float4 *>(colours), reinterpret_cast<const float4 *>(grad_canvas), d->d_ck,
-        d->ck_pitch, d->ck_stride, d->d_cov, replayed ? 1u : 0u, d->d_gvtx, grad_colours, d->d_status);
+        d->ck_pitch, d->ck_stride, d->d_gvtx, grad_colours, d->d_status);
     k_point_grad<<<grid_of(d->n_pts), BLOCK, 0, d->stream>>>(S, d->d_gvtx, reinterpret_cast<float2 *>(grad_points),
                                                              d->n_pts, d->d_pt_path);
     FD_HIP(hipGetLastError());
@@ -1505,7 +1273,8 @@ ft_status run_backward(ft_diff *d, const float *points, const float *colours, co
                        float *grad_points, float *grad_colours) {
     for (int attempt = 0; attempt < 3; ++attempt) {
         ft_status st = launch_geometry(d, points, true, grad_colours);
-        if (!st) st = launch_backward(d, colours, grad_canvas, grad_points, grad_colours, false);
+        if (!st) st = launch_forward(d, colours, nullptr, true);
+        if (!st) st = launch_backward(d, colours, grad_canvas, grad_points, grad_colours);
         if (st) return st;
         st = finish(d);
         if (st != (ft_status)0x100) return st;
@@ -1524,7 +1293,7 @@ ft_status run_step(ft_diff *d, const float *points, const float *colours, const 
         if (st) return st;
         if ((st = launch_forward(d, colours, canvas, true))) return st;
         if ((st = launch_loss(d, canvas, target, grad_canvas))) return st;
-        if ((st = launch_backward(d, colours, grad_canvas, grad_points, grad_colours, true))) return st;
+        if ((st = launch_backward(d, colours, grad_canvas, grad_points, grad_colours))) return st;
         st = finish(d, true);
         if (st == FT_OK && loss) *loss = *d->h_loss / (double)d->canvas_floats;
         if (st != (ft_status)0x100) return st;
@@ -1582,10 +1351,9 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
     for (uint32_t k = 0; k < L->n_paths; ++k) d->max_path_vtx = std::max(d->max_path_vtx, vtx_off[k + 1] - vtx_off[k]);
     d->n_cells = cells;
     d->canvas_floats = 4ull * L->n_images * L->width * L->height;
-    const dim3 g = raster_grid(d);
-    d->ck_pitch = g.x * DBLOCK;
-    d->ck_stride = (uint64_t)d->ck_pitch * g.y * g.z;
-    const uint64_t n_ck = std::max<uint64_t>(1, (max_paths + KSEG - 1) / KSEG);
+    d->ck_pitch = (d->W + 15) / 16 * 16;
+    d->ck_stride = (uint64_t)d->ck_pitch * d->H * d->n_images;
+    const uint64_t n_ck = std::max<uint64_t>(1, (max_paths + SEG - 1) / SEG);
     d->cap_tiles = (cells + SCAN_TILE_MIN - 1) / SCAN_TILE_MIN + 1;
     d->cap_pairs = (uint32_t)std::min<uint64_t>(0xFFFFFFF0ull, 8 * nv + 4096);
     ft_status st;
@@ -1612,15 +1380,6 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
         st = FT_EDEVICE;
     else
         st = FT_OK;
-    // By default the backward recomputes every path's coverage.  On request
-    // (FT_DIFF_KEEP_COVERAGE) the forward keeps it, 4 B per path and pixel,
-    // which spares the second evaluation; without room for the buffer the
-    // handle recomputes anyway.
-    const uint64_t cov_elems = (L->flags & FT_DIFF_KEEP_COVERAGE) ? (uint64_t)max_paths * d->ck_stride : 0;
-    if (!st && cov_elems && cov_elems <= COV_MAX_BYTES / sizeof(float) && dalloc(d->d_cov, cov_elems)) {
-        d->d_cov = nullptr;
-        (void)hipGetLastError();  // the failed optional allocation is not an error of a later call
-    }
     if (st) {
         ft_diff_free(d);
         return st;
@@ -1633,7 +1392,7 @@ void ft_diff_free(ft_diff *d) {
     if (!d) return;
     void *bufs[] = {d->d_pt_off,   d->d_vtx_off,  d->d_vtx_path, d->d_pt_path,   d->d_img_first, d->d_vtx,
                     d->d_gvtx,     d->d_cell_cnt, d->d_cell_off, d->d_cell_cur,  d->d_cell_edge, d->d_lb,
-                    d->d_ck,       d->d_cov,       d->d_partial,   d->d_status};
+                    d->d_ck,       d->d_partial,  d->d_status};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (d->h_loss) (void)hipHostFree(d->h_loss);

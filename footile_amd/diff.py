@@ -37,9 +37,8 @@ def device_array(a):
 class DiffRenderer:
     """A scene layout and its device workspace (ft_diff).
 
-    By default the backward recomputes every path's coverage; keep_coverage
-    (FT_DIFF_KEEP_COVERAGE) keeps it from the forward instead, at 4 B per path
-    and pixel."""
+    keep_coverage (FT_DIFF_KEEP_COVERAGE) is accepted and changes nothing: the
+    backward always recomputes the paths' coverage."""
 
     def __init__(self, n_images, width, height, path_image, path_cubics, keep_coverage=False):
         self.n_images, self.width, self.height = int(n_images), int(width), int(height)

@@ -259,10 +259,10 @@ ft_status ft_memset_d(void *dst, int value, size_t bytes);
  * ------------------------------------------------------------------------ */
 typedef struct ft_diff ft_diff;
 /* ft_diff_layout.flags */
-#define FT_DIFF_KEEP_COVERAGE 1u /* opt-in: keep each path's coverage from the
-                                    forward for the backward (4 B per path and
-                                    pixel, see ft_diff_backward) instead of
-                                    recomputing it */
+#define FT_DIFF_KEEP_COVERAGE 1u /* accepted; the results are the same.  Coverage is
+                                    always recomputed in the backward: that takes
+                                    less time than reading 4 B per path and pixel
+                                    back */
 typedef struct ft_diff_layout {
     uint32_t n_images, width, height;
     uint32_t n_paths;
@@ -277,13 +277,11 @@ ft_status ft_diff_info(const ft_diff *d, uint64_t *n_points, uint64_t *n_paths, 
 ft_status ft_diff_forward(ft_diff *d, const float *points, const float *colours, float *canvas);
 /* loss = mean((canvas - target)^2); grad_canvas (may be NULL) = d loss / d canvas */
 ft_status ft_diff_loss(ft_diff *d, const float *canvas, const float *target, float *grad_canvas, double *loss);
-/* Vector-Jacobian product: grad_canvas -> d/d points, d/d colours.  Replays
- * the forward into canvas checkpoints every 8 paths (16 B per pixel of every
- * image per checkpoint, max_paths / 8 rounded up of them, max_paths the most
+/* Vector-Jacobian product: grad_canvas -> d/d points, d/d colours.  Runs the
+ * forward into canvas checkpoints every 16 paths (16 B per pixel of every
+ * image per checkpoint, max_paths / 16 rounded up of them, max_paths the most
  * paths of one image) and recomputes each path's coverage while it walks the
- * paths backwards.  With FT_DIFF_KEEP_COVERAGE (and when the buffer fits in
- * 16 GiB) the replay also keeps every path's coverage, max_paths x 4 B per
- * pixel of every image, and the walk reads it instead. */
+ * paths backwards. */
 ft_status ft_diff_backward(ft_diff *d, const float *points, const float *colours, const float *grad_canvas,
                            float *grad_points, float *grad_colours);
 /* forward + loss + backward (one optimisation step's gradient) with one host

@@ -4,10 +4,8 @@
 // in path order) is specified by the FP64 oracle the tests compare against.
 //
 // Per step:
-//   k_vertices   control points -> polygon vertices (16 per cubic, Bernstein)
-//   k_rows       each edge adds +1/-1 at the ends of its row range per path
-//   scan, scan   -> edges per (path, row) cell, CSR offsets
-//   k_fill_cells, k_sort_cells   edge lists per cell, in edge order
+//   k_geometry   control points -> polygon vertices (16 per cubic, Bernstein),
+//                edge lists per (path, row)
 //   k_forward    one lane per pixel of a row tile: coverage of the image's
 //                paths, 16 per round, from integer LDS cells and a prefix sum,
 //                composite, the canvas and (in a step) its value before every
@@ -144,6 +142,18 @@ __device__ inline void wave_sum3(float &a, float &b, float &c) {
 // ---------------------------------------------------------------------------
 // Geometry
 // ---------------------------------------------------------------------------
+// Vertex v of a path with control points P: the start point, then the points
+// t = 1/16 .. 1 of each cubic.
+__device__ __forceinline__ float2 path_vertex(const float2 *P, uint32_t v) {
+    if (!v) return P[0];
+    const uint32_t c = (v - 1) / DSEG;
+    float w[4];
+    bern((int)((v - 1) % DSEG) + 1, w);
+    const float2 p0 = P[3 * c], p1 = P[3 * c + 1], p2 = P[3 * c + 2], p3 = P[3 * c + 3];
+    return make_float2(w[0] * p0.x + w[1] * p1.x + w[2] * p2.x + w[3] * p3.x,
+                       w[0] * p0.y + w[1] * p1.y + w[2] * p2.y + w[3] * p3.y);
+}
+
 __global__ __launch_bounds__(BLOCK) void k_vertices(DScene S, const float2 *points, DevStatus *st) {
     for (uint32_t v = blockIdx.x * BLOCK + threadIdx.x; v < S.n_vtx; v += gridDim.x * BLOCK) {
         const uint32_t k = S.vtx_path[v];
@@ -151,20 +161,14 @@ __global__ __launch_bounds__(BLOCK) void k_vertices(DScene S, const float2 *poin
             raise_err(st, FT_EDEVICE);
             continue;
         }
-        const uint32_t local = v - S.vtx_off[k];
-        const float2 *P = points + S.pt_off[k];
-        float2 r = P[0];
-        if (local) {
-            const uint32_t c = (local - 1) / DSEG;
-            const int j = (int)((local - 1) % DSEG) + 1;
-            float w[4];
-            bern(j, w);
-            const float2 p0 = P[3 * c], p1 = P[3 * c + 1], p2 = P[3 * c + 2], p3 = P[3 * c + 3];
-            r.x = w[0] * p0.x + w[1] * p1.x + w[2] * p2.x + w[3] * p3.x;
-            r.y = w[0] * p0.y + w[1] * p1.y + w[2] * p2.y + w[3] * p3.y;
-        }
-        S.vtx[v] = r;
+        S.vtx[v] = path_vertex(points + S.pt_off[k], v - S.vtx_off[k]);
     }
+}
+
+// Clears a run's look-back words and status.
+__global__ __launch_bounds__(BLOCK) void k_clear_run(unsigned long long *lb, uint32_t n_lb, DevStatus *st) {
+    for (uint32_t i = threadIdx.x; i < n_lb; i += BLOCK) lb[i] = 0;
+    if (threadIdx.x < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
 }
 
 // Rows [r0, r1] an edge overlaps within [0, H); false when none.
@@ -222,94 +226,143 @@ __global__ __launch_bounds__(BLOCK) void k_rows(DScene S, DevStatus *st) {
     }
 }
 
-// Edge lists per (path, row) in edge order, one block per path, without
-// atomics or a sort: the block stages its edges' row ranges in LDS; each
-// wavefront takes every fourth row of the path's span and walks the edges in
-// chunks of 64, giving each crossing edge its slot by a ballot count of the
-// crossing edges before it.  Paths of more than CELL_EDGES edges take the
-// atomic fill and the sort below instead.
-constexpr uint32_t CELL_EDGES = 2048;
-
-__global__ __launch_bounds__(BLOCK) void k_cells(DScene S, DevStatus *st) {
-    __shared__ uint2 s_rows[CELL_EDGES];
-    __shared__ uint32_t s_lo[BLOCK / 64], s_hi[BLOCK / 64];
-    if (run_failed(st)) return;
-    if (st->n_pairs > S.cap_pairs) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            atomicOr(&st->overflow, 2u);
-            st->need_pairs = st->n_pairs;
-        }
-        return;
+// Exclusive scan of x over the block's BLOCK threads, and the total.  Every
+// thread calls it; s_w is free again when it returns.
+__device__ __forceinline__ uint32_t block_excl(uint32_t x, uint32_t *s_w, uint32_t &total) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const uint32_t incl = wave_incl_dpp<false>(x);
+    if (lane == 63) s_w[wid] = incl;
+    __syncthreads();
+    uint32_t pre = incl - x;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; ++w) {
+        pre += w < wid ? s_w[w] : 0u;
+        total += s_w[w];
     }
-    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    for (uint32_t k = blockIdx.x; k < S.n_paths; k += gridDim.x) {
+    __syncthreads();
+    return pre;
+}
+
+// The whole geometry in one launch, for layouts whose paths have at most
+// GEOM_EDGES edges and images at most GEOM_ROWS rows: a block takes `per`
+// consecutive paths, writes their vertices and counts their (edge, row)
+// pairs, takes its place in the pair list by look-back, and then per path
+// counts the rows' edges in LDS, scans them into the cells' list offsets and
+// hands out the list slots with LDS cursors.  Order within a list is free:
+// coverage is an integer sum.  It also clears the gradients (gvtx null:
+// none).  It replaces a clear over all cells, a vertex pass, atomics per edge
+// on the cells, two scans over all cells and a kernel that tested every edge
+// of a path against every row: 545 -> 168 us of a 64-image step with 17,500
+// paths, 85 us in six launches -> 19 us in two for 256 paths, 110 -> 17 us for
+// a 1000x600 image of 128 paths.  A path's work is a chain of a few barriers,
+// so a launch of few paths is bound by latency.
+constexpr uint32_t GEOM_EDGES = 2048, GEOM_ROWS = 8192, GEOM_BLOCKS = 1024;
+constexpr uint32_t EDGE_LANES = 4;  // threads per edge in the fill, on every fourth of its rows
+
+__global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *points, float2 *gvtx, float *gcol,
+                                                    uint32_t per, unsigned long long *lb, DevStatus *st) {
+    extern __shared__ uint32_t s_row[];  // [H + 1]: differences, counts, then list cursors
+    __shared__ uint32_t s_w[BLOCK / 64], s_tk;
+    __shared__ unsigned long long s_base;
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0) s_tk = lookback_ticket(lb);
+    __syncthreads();
+    const uint32_t b = s_tk;
+    const uint32_t k0 = b * per, k1 = k0 + per < S.n_paths ? k0 + per : S.n_paths;
+    // vertices, then the pairs of the paths' edges
+    for (uint32_t k = k0; k < k1; ++k) {
         const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
-        if (V > CELL_EDGES) continue;  // uniform: left to the atomic fill
-        uint32_t lo = 0xFFFFFFFFu, hi = 0;
-        for (uint32_t e = threadIdx.x; e < V; e += BLOCK) {
-            uint32_t r0 = 1, r1 = 0;
-            const float2 a = S.vtx[vb + e], b = S.vtx[vb + (e + 1 < V ? e + 1 : 0u)];
-            if (!edge_row_range(a, b, S.H, r0, r1)) {
-                r0 = 1;
-                r1 = 0;
-            }
-            s_rows[e] = make_uint2(r0, r1);
-            if (r0 <= r1) {
-                lo = r0 < lo ? r0 : lo;
-                hi = r1 > hi ? r1 : hi;
-            }
+        for (uint32_t v = tid; v < V; v += BLOCK) {
+            S.vtx[vb + v] = path_vertex(points + S.pt_off[k], v);
+            if (gvtx) gvtx[vb + v] = make_float2(0.0f, 0.0f);
         }
+        if (gcol && tid < 4) gcol[4 * (uint64_t)k + tid] = 0.0f;
+    }
+    __syncthreads();
+    unsigned long long mine = 0;
+    for (uint32_t k = k0; k < k1; ++k) {
+        const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
+        for (uint32_t e = tid; e < V; e += BLOCK) {
+            uint32_t r0, r1;
+            if (edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) mine += r1 - r0 + 1;
+        }
+    }
+    // at most GEOM_EDGES edges of GEOM_ROWS rows per path: one path's pairs fit 32 bits, a block's need not
+    const unsigned long long wsum = wave_incl_t<unsigned long long, false>(mine);
+    __shared__ unsigned long long s_sum[BLOCK / 64];
+    if ((tid & 63) == 63) s_sum[tid >> 6] = wsum;
+    __syncthreads();
+    if (tid < 64) {
+        unsigned long long tot = 0;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint32_t l2 = __shfl_xor(lo, o, 64), h2 = __shfl_xor(hi, o, 64);
-            lo = l2 < lo ? l2 : lo;
-            hi = h2 > hi ? h2 : hi;
-        }
-        if (lane == 0) {
-            s_lo[wid] = lo;
-            s_hi[wid] = hi;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < BLOCK / 64; ++w) {
-            lo = s_lo[w] < lo ? s_lo[w] : lo;
-            hi = s_hi[w] > hi ? s_hi[w] : hi;
-        }
-        const uint64_t c0 = (uint64_t)k * S.H;
-        uint32_t bad = 0;
-        for (uint32_t rb = lo + wid * 64; lo <= hi && rb <= hi; rb += BLOCK) {
-            // the list offsets of this wavefront's next 64 rows rb, rb + 1, ...
-            // (rows interleave over the wavefronts in runs of 64)
-            const uint32_t my_row = rb + lane;
-            const uint32_t my_off = my_row <= hi ? S.cell_off[c0 + my_row] : 0u;
-            const uint32_t n_r = hi - rb + 1 < 64u ? hi - rb + 1 : 64u;
-            for (uint32_t i = 0; i < n_r; ++i) {
-                const uint32_t r = rb + i;
-                const uint32_t base = (uint32_t)__shfl((int)my_off, (int)i, 64);
-                uint32_t run = 0;
-                for (uint32_t e0 = 0; e0 < V; e0 += 64) {
-                    const uint32_t e = e0 + lane;
-                    const uint2 rr = e < V ? s_rows[e] : make_uint2(1u, 0u);
-                    const bool x = (rr.x <= r) & (r <= rr.y);
-                    const unsigned long long m = __ballot(x);
-                    if (x) {
-                        const uint32_t at = base + run +
-                                            __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                        if (at < S.cap_pairs)
-                            S.cell_edge[at] = e;
-                        else
-                            bad = 1;
-                    }
-                    run += (uint32_t)__popcll(m);
+        for (int w = 0; w < BLOCK / 64; ++w) tot += s_sum[w];
+        const unsigned long long pre = lookback_prefix<unsigned long long, false>(lb, b, tot, st);
+        if (tid == 0) {
+            s_base = pre + tot <= S.cap_pairs ? pre : ~0ull;
+            if (k1 == S.n_paths && k0 < S.n_paths) {  // the run's total
+                const unsigned long long all = pre + tot;
+                st->n_pairs = all < 0xFFFFFFFFull ? (uint32_t)all : 0xFFFFFFFFu;
+                if (all > S.cap_pairs) {
+                    atomicOr(&st->overflow, 2u);
+                    st->need_pairs = all < 0xFFFFFFFFull ? (uint32_t)all : 0xFFFFFFFFu;
                 }
             }
         }
-        if (bad) raise_err(st, FT_EDEVICE);
-        __syncthreads();  // s_rows and s_lo / s_hi are the next path's
+    }
+    __syncthreads();
+    if (s_base == ~0ull) return;  // no room: the run is repeated with more
+    uint32_t base = (uint32_t)s_base;
+    const uint32_t rows_per = (S.H + BLOCK - 1) / BLOCK;
+    for (uint32_t k = k0; k < k1; ++k) {
+        const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
+        for (uint32_t r = tid; r <= S.H; r += BLOCK) s_row[r] = 0;
+        __syncthreads();
+        for (uint32_t e = tid; e < V; e += BLOCK) {
+            uint32_t r0, r1;
+            if (!edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) continue;
+            atomicAdd(&s_row[r0], 1u);
+            atomicAdd(&s_row[r1 + 1], 0xFFFFFFFFu);
+        }
+        __syncthreads();
+        // thread t's rows [a, z): counts from the differences, then offsets
+        const uint32_t a = tid * rows_per < S.H ? tid * rows_per : S.H;
+        const uint32_t z = a + rows_per < S.H ? a + rows_per : S.H;
+        uint32_t d = 0, total;
+        for (uint32_t r = a; r < z; ++r) d += s_row[r];
+        uint32_t cnt = block_excl(d, s_w, total);
+        const uint32_t before = cnt;
+        uint32_t sum = 0;
+        for (uint32_t r = a; r < z; ++r) {
+            cnt += s_row[r];
+            sum += cnt;
+        }
+        uint32_t at = base + block_excl(sum, s_w, total);
+        cnt = before;
+        const uint64_t c0 = (uint64_t)k * S.H;
+        for (uint32_t r = a; r < z; ++r) {
+            cnt += s_row[r];
+            S.cell_cnt[c0 + r] = cnt;
+            S.cell_off[c0 + r] = at;
+            s_row[r] = at;
+            at += cnt;
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < V * EDGE_LANES; i += BLOCK) {
+            const uint32_t e = i / EDGE_LANES;
+            uint32_t r0, r1;
+            if (!edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) continue;
+            for (uint32_t r = r0 + i % EDGE_LANES; r <= r1; r += EDGE_LANES)
+                S.cell_edge[atomicAdd(&s_row[r], 1u)] = e;
+        }
+        base += total;
+        __syncthreads();
     }
 }
 
+// The general form, for longer paths and taller images: k_vertices, k_rows
+// (differences on the cells), two scans over the cells, and k_fill_cells.
+//
 // FILL_LANES threads per edge, each taking every FILL_LANES-th run of
 // FILL_ROWS rows, with the run's FILL_ROWS slot reservations (returning
 // atomics on the cells' cursors) in flight together: a tall edge does not
@@ -331,7 +384,6 @@ __global__ __launch_bounds__(BLOCK) void k_fill_cells(DScene S, DevStatus *st) {
         uint32_t k, r0, r1;
         float2 a, b;
         edge_at(S, v, k, a, b);
-        if (S.vtx_off[k + 1] - S.vtx_off[k] <= CELL_EDGES) continue;  // k_cells has the path
         if (!edge_row_range(a, b, S.H, r0, r1)) continue;
         const uint32_t local = v - S.vtx_off[k];
         const uint64_t c0 = (uint64_t)k * S.H;
@@ -347,58 +399,6 @@ __global__ __launch_bounds__(BLOCK) void k_fill_cells(DScene S, DevStatus *st) {
                     S.cell_edge[at[u]] = local;
                 else
                     raise_err(st, FT_EDEVICE);
-            }
-        }
-    }
-}
-
-// Each cell's edges in ascending order, so that sums run in edge order.  A
-// cell of 2 to 16 edges is loaded into registers (all loads in flight),
-// sorted by an odd-even transposition network of 8 or 16 places and stored
-// back; longer cells are sorted in place.
-template <uint32_t N>
-__device__ inline void sort_cell_regs(uint32_t *e, uint32_t n) {
-    uint32_t x[N];
-#pragma unroll
-    for (uint32_t i = 0; i < N; ++i) x[i] = i < n ? e[i] : 0xFFFFFFFFu;
-#pragma unroll
-    for (uint32_t pass = 0; pass < N; ++pass) {
-#pragma unroll
-        for (uint32_t i = pass & 1u; i + 1 < N; i += 2) {
-            const uint32_t lo = x[i] < x[i + 1] ? x[i] : x[i + 1];
-            const uint32_t hi = x[i] < x[i + 1] ? x[i + 1] : x[i];
-            x[i] = lo;
-            x[i + 1] = hi;
-        }
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < N; ++i)
-        if (i < n) e[i] = x[i];
-}
-
-__global__ __launch_bounds__(BLOCK) void k_sort_cells(DScene S, DevStatus *st) {
-    if (run_failed(st)) return;
-    for (uint32_t c = blockIdx.x * BLOCK + threadIdx.x; c < S.n_cells; c += gridDim.x * BLOCK) {
-        const uint32_t off = S.cell_off[c], n = S.cell_cnt[c];
-        if ((uint64_t)off + n > S.cap_pairs) {
-            raise_err(st, FT_EDEVICE);
-            continue;
-        }
-        if (n < 2 || S.vtx_off[c / S.H + 1] - S.vtx_off[c / S.H] <= CELL_EDGES) continue;  // k_cells: in order
-        uint32_t *e = S.cell_edge + off;
-        if (n <= 8) {
-            sort_cell_regs<8>(e, n);
-        } else if (n <= 16) {
-            sort_cell_regs<16>(e, n);
-        } else {
-            for (uint32_t i = 1; i < n; ++i) {
-                const uint32_t x = e[i];
-                uint32_t j = i;
-                while (j > 0 && e[j - 1] > x) {
-                    e[j] = e[j - 1];
-                    --j;
-                }
-                e[j] = x;
             }
         }
     }
@@ -1161,23 +1161,29 @@ uint32_t grid_of(uint64_t n) {
 ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, float *gcol) {
     hipStream_t s = d->stream;
     DScene S = scene_of(d);
+    float2 *const gvtx = clear_grads ? d->d_gvtx : nullptr;
+    if (!clear_grads) gcol = nullptr;
+    const float2 *const pts = reinterpret_cast<const float2 *>(points);
+    if (d->max_path_vtx <= GEOM_EDGES && d->H <= GEOM_ROWS && d->n_paths) {
+        const uint32_t per = (d->n_paths + GEOM_BLOCKS - 1) / GEOM_BLOCKS;
+        const uint32_t blocks = (d->n_paths + per - 1) / per;
+        k_clear_run<<<1, BLOCK, 0, s>>>(d->d_lb, (uint32_t)lookback_words(blocks), d->d_status);
+        k_geometry<<<blocks, BLOCK, (d->H + 1) * sizeof(uint32_t), s>>>(S, pts, gvtx, gcol, per, d->d_lb, d->d_status);
+        FD_HIP(hipGetLastError());
+        return FT_OK;
+    }
     const uint32_t n_lb = (uint32_t)(4 * d->cap_tiles);  // look-back words of the two cell scans
     const uint64_t n_clear = std::max<uint64_t>(std::max<uint64_t>(d->n_cells, d->n_vtx),
                                                 std::max<uint64_t>(4ull * d->n_paths, n_lb));
-    k_clear_cells<<<grid_of(n_clear), BLOCK, 0, s>>>(S, clear_grads ? d->d_gvtx : nullptr,
-                                                     clear_grads ? gcol : nullptr, d->d_lb, n_lb, d->d_status);
-    k_vertices<<<grid_of(d->n_vtx), BLOCK, 0, s>>>(S, reinterpret_cast<const float2 *>(points), d->d_status);
+    k_clear_cells<<<grid_of(n_clear), BLOCK, 0, s>>>(S, gvtx, gcol, d->d_lb, n_lb, d->d_status);
+    k_vertices<<<grid_of(d->n_vtx), BLOCK, 0, s>>>(S, pts, d->d_status);
     k_rows<<<grid_of(d->n_vtx), BLOCK, 0, s>>>(S, d->d_status);
     const uint32_t nc = (uint32_t)d->n_cells;
     scan_launch<uint32_t, false>(s, scan_resident_blocks(), d->d_cell_cnt, d->d_cell_cnt, nullptr, nc, nc, d->d_lb,
                                  nullptr, d->d_status, false, true);
     scan_launch<uint32_t, false>(s, scan_resident_blocks(), d->d_cell_cnt, d->d_cell_off, nullptr, nc, nc,
                                  d->d_lb + 2 * d->cap_tiles, &d->d_status->n_pairs, d->d_status, false, false);
-    k_cells<<<(uint32_t)std::min<size_t>(std::max<size_t>(d->n_paths, 1), 65535), BLOCK, 0, s>>>(S, d->d_status);
-    if (d->max_path_vtx > CELL_EDGES) {
-        k_fill_cells<<<grid_of((size_t)d->n_vtx * FILL_LANES), BLOCK, 0, s>>>(S, d->d_status);
-        k_sort_cells<<<grid_of(d->n_cells), BLOCK, 0, s>>>(S, d->d_status);
-    }
+    k_fill_cells<<<grid_of((size_t)d->n_vtx * FILL_LANES), BLOCK, 0, s>>>(S, d->d_status);
     FD_HIP(hipGetLastError());
     return FT_OK;
 }
@@ -1363,7 +1369,7 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
              (st = dalloc(d->d_img_first, L->n_images + 1)) || (st = dalloc(d->d_vtx, nv)) ||
              (st = dalloc(d->d_gvtx, nv)) || (st = dalloc(d->d_cell_cnt, cells)) ||
              (st = dalloc(d->d_cell_off, cells)) || (st = dalloc(d->d_cell_cur, cells)) ||
-             (st = dalloc(d->d_cell_edge, d->cap_pairs)) || (st = dalloc(d->d_lb, 4 * d->cap_tiles)) ||
+             (st = dalloc(d->d_cell_edge, d->cap_pairs)) || (st = dalloc(d->d_lb, std::max<size_t>(4 * d->cap_tiles, lookback_words(GEOM_BLOCKS)))) ||
              (st = dalloc(d->d_ck, n_ck * d->ck_stride)) || (st = dalloc(d->d_partial, LOSS_GRID + 1)) ||
              (st = dalloc(d->d_status, 1)))
         ;

@@ -62,6 +62,40 @@ def test_tile_and_round_edges(oracle, w, h, paths, cubics, images):
     _check(_scene(w + paths, w, h, paths, cubics, images))
 
 
+@pytest.mark.parametrize("w,h,paths,cubics", [
+    (8, 4, 1024, 1), (8, 4, 1025, 1), (8, 3, 2500, 1),  # one and several paths per geometry block
+    (4, 255, 3, 2), (4, 257, 3, 2),  # one and two rows per thread
+    (20, 10, 3, 127), (20, 10, 3, 128)])  # 2,033 and 2,049 edges: either side of the one-launch limit
+def test_geometry_sizes(oracle, w, h, paths, cubics):
+    _check(_scene(w + h + paths, w, h, paths, cubics), pieces=0.6 * cubics + 17.0 * cubics / h)
+
+
+def _canvas(sc):
+    from footile_amd.diff import DiffRenderer, device_array
+    r = DiffRenderer.for_scene(sc)
+    canvas = r.new_canvas()
+    r.forward(device_array(sc.points), device_array(sc.colours), canvas)
+    return canvas.download(dtype=np.float32).reshape(r.canvas_shape)
+
+
+def test_geometry_forms_agree(oracle):
+    """The one-launch geometry and the general form (images past 8,192 rows,
+    paths past 2,048 edges) give the same bytes: coverage does not depend on
+    the order of a row's pieces."""
+    import dataclasses
+    tall = _scene(11, 5, 8192, 6, 3)
+    assert np.array_equal(_canvas(tall)[0], _canvas(dataclasses.replace(tall, height=8193))[0, :8192])
+    sc = _scene(12, 90, 40, 30, 4)
+    # one more path, last, of 2,081 edges and outside the image
+    g = np.random.default_rng(13)
+    far = g.uniform(200.0, 300.0, size=(1 + 3 * 130, 2)).astype(np.float32)
+    more = dataclasses.replace(sc, path_image=np.append(sc.path_image, 0).astype(np.uint32),
+                               path_cubics=np.append(sc.path_cubics, 130).astype(np.uint32),
+                               points=np.concatenate([sc.points, far]),
+                               colours=np.concatenate([sc.colours, sc.colours[:1]]))
+    assert np.array_equal(_canvas(sc), _canvas(more))
+
+
 def test_wide_and_narrow_ramps(oracle):
     """Outlines whose edges cross hundreds of columns in a row or none."""
     def points(g, n):

@@ -83,36 +83,37 @@ __device__ inline Piece piece_of(float2 p, float2 q, int Y) {
     return r;
 }
 
-// d(sign * h * M) / d(x_top, y_top, x_bot, y_bot) given S1 = sum dA M,
-// S2 = sum dA dM/dua, S3 = sum dA dM/dub over the pixels of the row.
-__device__ inline void piece_grad(float2 p, float2 q, int Y, float S1, float S2, float S3, float g[4]) {
+// Gradients of one piece's sign * h * M, given S1 = sum dA M, Sa = sum dA
+// dM/du_a, Sb = sum dA dM/du_b over the pixels of the row (u = X1 - x at the
+// piece's top and bottom).  x_a and x_b are linear in the edge's ends, so
+// over all the rows between them d/dy of an end is -slope times its d/dx: a
+// piece adds the d/dx of both ends, and only the row that holds an end adds
+// that end's own d/dy terms.  The slope enters once per edge (vertex_grad).
+// That is 2.2 atomics per piece instead of 4.
+struct EdgeGrad {
+    float xp, xq;  // d/dx of the first and second vertex
+    float yp, yq;  // their rows' own d/dy terms
+    bool has_p, has_q;
+};
+
+__device__ __forceinline__ EdgeGrad piece_grad(float2 p, float2 q, int Y, float S1, float Sa, float Sb) {
     const bool down = q.y > p.y;
     const float2 t = down ? p : q, b = down ? q : p;
-    const float sign = down ? 1.0f : -1.0f;
-    const bool clip_top = !(t.y > (float)Y), clip_bot = !(b.y < (float)(Y + 1));
-    const float ya = clip_top ? (float)Y : t.y, yb = clip_bot ? (float)(Y + 1) : b.y;
-    const float dy = b.y - t.y, dx = b.x - t.x;
-    const float sl = dx / dy;
-    // partials of ya, yb, sl w.r.t. (xt, yt, xb, yb_end)
-    const float dya[4] = {0.0f, clip_top ? 0.0f : 1.0f, 0.0f, 0.0f};
-    const float dyb[4] = {0.0f, 0.0f, 0.0f, clip_bot ? 0.0f : 1.0f};
-    const float dsl[4] = {-1.0f / dy, sl / dy, 1.0f / dy, -sl / dy};
-    const float ra = ya - t.y, rb = yb - t.y;
-    float gd[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float dt = i == 1 ? 1.0f : 0.0f, dxt = i == 0 ? 1.0f : 0.0f;
-        const float dra = dya[i] - dt, drb = dyb[i] - dt;
-        const float dxa = dxt + dra * sl + ra * dsl[i];
-        const float dxb = dxt + drb * sl + rb * dsl[i];
-        const float dh = dyb[i] - dya[i];
-        gd[i] = sign * (dh * S1 - (yb - ya) * (dxa * S2 + dxb * S3));
-    }
-    // back to (x_p, y_p, x_q, y_q)
-    g[0] = down ? gd[0] : gd[2];
-    g[1] = down ? gd[1] : gd[3];
-    g[2] = down ? gd[2] : gd[0];
-    g[3] = down ? gd[3] : gd[1];
+    const bool top = t.y > (float)Y, bot = b.y < (float)(Y + 1);  // the ends lie inside the row
+    const float ya = top ? t.y : (float)Y, yb = bot ? b.y : (float)(Y + 1);
+    const float dy = b.y - t.y, h = yb - ya, idy = 1.0f / dy, hsl = h * ((b.x - t.x) / dy);
+    const float fa = (ya - t.y) * idy, fb = (yb - t.y) * idy;  // where the piece lies on the edge
+    const float s = down ? 1.0f : -1.0f, sh = -s * h;
+    const float xt = sh * fmaf(1.0f - fa, Sa, (1.0f - fb) * Sb), xb = sh * fmaf(fa, Sa, fb * Sb);
+    const float yt = -s * fmaf(hsl, Sa, S1), yz = s * fmaf(-hsl, Sb, S1);
+    EdgeGrad g;
+    g.xp = down ? xt : xb;
+    g.xq = down ? xb : xt;
+    g.yp = down ? yt : yz;
+    g.yq = down ? yz : yt;
+    g.has_p = down ? top : bot;
+    g.has_q = down ? bot : top;
+    return g;
 }
 
 // One DPP step of a wavefront float scan: v + (v of the source lane, or 0).
@@ -194,7 +195,7 @@ __device__ inline void edge_at(const DScene &S, uint32_t v, uint32_t &k, float2 
 
 // Clears the cell counters, the scans' look-back words, the status and (when
 // given) the gradients.
-__global__ __launch_bounds__(BLOCK) void k_clear_cells(DScene S, float2 *gvtx, float *gcol, unsigned long long *lb,
+__global__ __launch_bounds__(BLOCK) void k_clear_cells(DScene S, float4 *gedge, float *gcol, unsigned long long *lb,
                                                        uint32_t n_lb, DevStatus *st) {
     uint32_t n = S.n_cells > S.n_vtx ? S.n_cells : S.n_vtx;
     n = n > 4 * S.n_paths ? n : 4 * S.n_paths;
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(BLOCK) void k_clear_cells(DScene S, float2 *gvtx, f
             S.cell_cnt[i] = 0;
             S.cell_cur[i] = 0;
         }
-        if (gvtx && i < S.n_vtx) gvtx[i] = make_float2(0.0f, 0.0f);
+        if (gedge && i < S.n_vtx) gedge[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (gcol && i < 4 * S.n_paths) gcol[i] = 0.0f;
     }
     if (blockIdx.x == 0 && threadIdx.x < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
@@ -250,7 +251,7 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t x, uint32_t *s_w, uint32
 // pairs, takes its place in the pair list by look-back, and then per path
 // counts the rows' edges in LDS, scans them into the cells' list offsets and
 // hands out the list slots with LDS cursors.  Order within a list is free:
-// coverage is an integer sum.  It also clears the gradients (gvtx null:
+// coverage is an integer sum.  It also clears the gradients (gedge null:
 // none).  It replaces a clear over all cells, a vertex pass, atomics per edge
 // on the cells, two scans over all cells and a kernel that tested every edge
 // of a path against every row: 545 -> 168 us of a 64-image step with 17,500
@@ -260,7 +261,7 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t x, uint32_t *s_w, uint32
 constexpr uint32_t GEOM_EDGES = 2048, GEOM_ROWS = 8192, GEOM_BLOCKS = 1024;
 constexpr uint32_t EDGE_LANES = 4;  // threads per edge in the fill, on every fourth of its rows
 
-__global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *points, float2 *gvtx, float *gcol,
+__global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *points, float4 *gedge, float *gcol,
                                                     uint32_t per, unsigned long long *lb, DevStatus *st) {
     extern __shared__ uint32_t s_row[];  // [H + 1]: differences, counts, then list cursors
     __shared__ uint32_t s_w[BLOCK / 64], s_tk;
@@ -275,7 +276,7 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
         const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
         for (uint32_t v = tid; v < V; v += BLOCK) {
             S.vtx[vb + v] = path_vertex(points + S.pt_off[k], v);
-            if (gvtx) gvtx[vb + v] = make_float2(0.0f, 0.0f);
+            if (gedge) gedge[vb + v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
         if (gcol && tid < 4) gcol[4 * (uint64_t)k + tid] = 0.0f;
     }
@@ -509,10 +510,10 @@ __device__ __forceinline__ PieceRef piece_ref(const DScene &S, const RowLds &R, 
     return r;
 }
 
-// The two vertices of a piece's edge and their indices.
+// The two vertices of a piece's edge.
 struct PieceVtx {
     float2 p, q;
-    uint32_t ip, iq;
+    uint32_t ip;  // index of the first
 };
 
 __device__ __forceinline__ PieceVtx piece_vtx(const DScene &S, const RowLds &R, uint32_t s, const PieceRef &r,
@@ -523,9 +524,8 @@ __device__ __forceinline__ PieceVtx piece_vtx(const DScene &S, const RowLds &R, 
     const uint32_t e = r.edge < V ? r.edge : 0u;
     PieceVtx v;
     v.ip = vb + e;
-    v.iq = vb + (e + 1 < V ? e + 1 : 0u);
     v.p = S.vtx[v.ip];
-    v.q = S.vtx[v.iq];
+    v.q = S.vtx[vb + (e + 1 < V ? e + 1 : 0u)];
     return v;
 }
 
@@ -674,6 +674,7 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
         __syncthreads();
     }
     for (uint32_t eb = base; eb < end; eb += (uint32_t)tw) {
+        if (eb + ((uint32_t)tid & ~63u) >= end) break;  // no piece for this wavefront
         PieceRef r = ref;
         Piece pc = first;
         if (eb != base) {
@@ -697,10 +698,15 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
     }
     const uint32_t poison = R.poison[s & 1];
     if (tid == 0) R.poison[(s + 1) & 1] = 0;
+    float light[SEG];
 #pragma unroll
-    for (uint32_t j = 0; j < SEG; ++j) {
-        const float a = (float)(int)wave_incl_dpp<false>(c[j]) * (1.0f / CELL_ONE);
-        A[j] = ((heavy >> j) & 1u) ? A[j] : a;
+    for (uint32_t j = 0; j < SEG; ++j) light[j] = (float)(int)wave_incl_dpp<false>(c[j]) * (1.0f / CELL_ONE);
+    if (heavy) {
+#pragma unroll
+        for (uint32_t j = 0; j < SEG; ++j) A[j] = ((heavy >> j) & 1u) ? A[j] : light[j];
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < SEG; ++j) A[j] = light[j];
     }
     // a piece without an x takes its path's whole row (coverage past 1, and so no gradient)
     if (poison) {
@@ -728,7 +734,7 @@ __device__ __forceinline__ float4 round_colour(const float4 *__restrict__ colour
 // while a round is composited.  With ck it also leaves the canvas before
 // every round but the first, at slot (image row) * ck_pitch + X; canvas may
 // be null.
-__global__ __launch_bounds__(TILE_MAX) void k_forward(DScene S, const float4 *__restrict__ colours,
+__global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 *__restrict__ colours,
                                                       float4 *__restrict__ canvas, float4 *__restrict__ ck,
                                                       uint32_t ck_pitch, uint64_t ck_stride, DevStatus *st) {
     extern __shared__ __align__(16) int s_cells[];
@@ -867,14 +873,15 @@ __device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, floa
 // columns right of it from the prefix sums.  (Evaluating each piece on all 64
 // pixels of every wavefront it touches and reducing the three sums over the
 // wavefront took 18.4 ms for 64 images of 256x256 with 17,500 paths; this
-// form takes 4.4 ms, and 320 us instead of 869 for one 512x512 image of 256
-// paths; about 1.1 ms and 90 us of that are the vertex gradients' atomics.)  Four wavefronts per SIMD are asked for: without, the kernel takes
+// form takes 3.8 ms, and 252 us instead of 869 for one 512x512 image of 256
+// paths.  Adding four vertex gradients per piece instead of EdgeGrad's two and
+// its ends took 4.5 ms and 332 us.)  Four wavefronts per SIMD are asked for: without, the kernel takes
 // 156 VGPRs, a CU holds three blocks, and the 1,024 blocks of a 512x512 image
 // run in two passes (370 us).
 __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4 *__restrict__ colours,
                                                        const float4 *__restrict__ grad_canvas,
                                                        const float4 *__restrict__ ck, uint32_t ck_pitch,
-                                                       uint64_t ck_stride, float2 *__restrict__ gvtx,
+                                                       uint64_t ck_stride, float4 *__restrict__ gedge,
                                                        float *__restrict__ gcol, DevStatus *st) {
     extern __shared__ __align__(16) int s_cells[];  // cells, then the prefix sums of dA; then dA
     __shared__ RowLds R;
@@ -973,6 +980,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
             // the pieces' gradients
             const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];
             for (uint32_t eb = base; eb < end; eb += tw) {
+                if (eb + ((uint32_t)tid & ~63u) >= end) break;  // no piece for this wavefront
                 PieceRef pr = cur;
                 PieceVtx pv = cv;
                 if (eb != base) {
@@ -1014,13 +1022,13 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                     if (t < (int)tw) S1 += s_pre[at + (t | 63)] - ((t & 63) ? s_pre[at + t - 1] : 0.0f);
                     for (int c = (t | 63) + 64; c < (int)tw; c += 64) S1 += s_pre[at + c];
                     if ((S1 != 0.0f) | (S2 != 0.0f) | (S3 != 0.0f)) {
-                        float gr[4];
                         const bool flip = pc.xa < pc.xb;  // S2 goes with the larger x
-                        piece_grad(pv.p, pv.q, (int)Y, S1, flip ? S3 : S2, flip ? S2 : S3, gr);
-                        atomicAdd(&gvtx[pv.ip].x, gr[0]);
-                        atomicAdd(&gvtx[pv.ip].y, gr[1]);
-                        atomicAdd(&gvtx[pv.iq].x, gr[2]);
-                        atomicAdd(&gvtx[pv.iq].y, gr[3]);
+                        const EdgeGrad g =
+                            piece_grad(pv.p, pv.q, (int)Y, S1, flip ? S3 : S2, flip ? S2 : S3);
+                        atomicAdd(&gedge[pv.ip].x, g.xp);
+                        atomicAdd(&gedge[pv.ip].y, g.xq);
+                        if (g.has_p) atomicAdd(&gedge[pv.ip].z, g.yp);
+                        if (g.has_q) atomicAdd(&gedge[pv.ip].w, g.yq);
                     }
                 }
             }
@@ -1050,16 +1058,32 @@ __global__ __launch_bounds__(BLOCK) void k_loss_sum(const double *partial, uint3
     }
 }
 
-// Control point gradients from vertex gradients (one thread per point).
-__global__ __launch_bounds__(BLOCK) void k_point_grad(DScene S, const float2 *gvtx, float2 *gpts, uint32_t n_pts,
+// The edge gradients of a path's edge e, with the y gradients completed by
+// the slope's share: (x, y) of its first vertex, (x, y) of its second.
+__device__ __forceinline__ float4 edge_grad(const DScene &S, const float4 *gedge, uint32_t vb, uint32_t V,
+                                            uint32_t e) {
+    const float4 g = gedge[vb + e];
+    const float2 p = S.vtx[vb + e], q = S.vtx[vb + (e + 1 < V ? e + 1 : 0u)];
+    const float sl = (q.x - p.x) / (q.y - p.y);
+    // (an edge without pieces, a horizontal one among them, has no gradient)
+    return make_float4(g.x, g.x != 0.0f ? fmaf(-sl, g.x, g.z) : g.z, g.y, g.y != 0.0f ? fmaf(-sl, g.y, g.w) : g.w);
+}
+
+// Control point gradients from edge gradients (one thread per point): the sum
+// over the point's cubics' vertices of their Bernstein weights times the
+// vertex's gradient, which is its two edges' shares.
+__global__ __launch_bounds__(BLOCK) void k_point_grad(DScene S, const float4 *gedge, float2 *gpts, uint32_t n_pts,
                                                       const uint32_t *pt_path) {
     for (uint32_t m = blockIdx.x * BLOCK + threadIdx.x; m < n_pts; m += gridDim.x * BLOCK) {
         const uint32_t k = pt_path[m];
         const uint32_t local = m - S.pt_off[k];
         const uint32_t n_cub = (S.pt_off[k + 1] - S.pt_off[k] - 1) / 3;
-        const uint32_t vb = S.vtx_off[k];
+        const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
         float2 acc = make_float2(0.0f, 0.0f);
-        if (local == 0) acc = gvtx[vb];
+        if (local == 0) {
+            const float4 g = edge_grad(S, gedge, vb, V, 0), l = edge_grad(S, gedge, vb, V, V - 1);
+            acc = make_float2(g.x + l.z, g.y + l.w);
+        }
         // the point is control r of cubic c (and control 0 of cubic c + 1 when r == 3)
         for (int pass = 0; pass < 2; ++pass) {
             uint32_t c, r;
@@ -1073,12 +1097,15 @@ __global__ __launch_bounds__(BLOCK) void k_point_grad(DScene S, const float2 *gv
                 r = 0;
                 if (c >= n_cub) continue;
             }
+            float4 in = edge_grad(S, gedge, vb, V, c * DSEG);  // the edge into vertex c * DSEG + 1
+#pragma unroll 4
             for (int j = 1; j <= DSEG; ++j) {
+                const float4 out = edge_grad(S, gedge, vb, V, c * DSEG + (uint32_t)j);
                 float w[4];
                 bern(j, w);
-                const float2 gv = gvtx[vb + 1 + c * DSEG + (uint32_t)(j - 1)];
-                acc.x += w[r] * gv.x;
-                acc.y += w[r] * gv.y;
+                acc.x += w[r] * (in.z + out.x);
+                acc.y += w[r] * (in.w + out.y);
+                in = out;
             }
         }
         gpts[m] = acc;
@@ -1102,7 +1129,8 @@ struct ft_diff {
     uint64_t n_cells = 0, canvas_floats = 0;
     uint32_t *d_pt_off = nullptr, *d_vtx_off = nullptr, *d_vtx_path = nullptr, *d_img_first = nullptr,
              *d_pt_path = nullptr;
-    float2 *d_vtx = nullptr, *d_gvtx = nullptr;
+    float2 *d_vtx = nullptr;
+    float4 *d_gedge = nullptr;  // per edge: see EdgeGrad
     uint32_t *d_cell_cnt = nullptr, *d_cell_off = nullptr, *d_cell_cur = nullptr, *d_cell_edge = nullptr;
     uint32_t cap_pairs = 0;
     size_t cap_tiles = 0;
@@ -1161,21 +1189,21 @@ uint32_t grid_of(uint64_t n) {
 ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, float *gcol) {
     hipStream_t s = d->stream;
     DScene S = scene_of(d);
-    float2 *const gvtx = clear_grads ? d->d_gvtx : nullptr;
+    float4 *const gedge = clear_grads ? d->d_gedge : nullptr;
     if (!clear_grads) gcol = nullptr;
     const float2 *const pts = reinterpret_cast<const float2 *>(points);
     if (d->max_path_vtx <= GEOM_EDGES && d->H <= GEOM_ROWS && d->n_paths) {
         const uint32_t per = (d->n_paths + GEOM_BLOCKS - 1) / GEOM_BLOCKS;
         const uint32_t blocks = (d->n_paths + per - 1) / per;
         k_clear_run<<<1, BLOCK, 0, s>>>(d->d_lb, (uint32_t)lookback_words(blocks), d->d_status);
-        k_geometry<<<blocks, BLOCK, (d->H + 1) * sizeof(uint32_t), s>>>(S, pts, gvtx, gcol, per, d->d_lb, d->d_status);
+        k_geometry<<<blocks, BLOCK, (d->H + 1) * sizeof(uint32_t), s>>>(S, pts, gedge, gcol, per, d->d_lb, d->d_status);
         FD_HIP(hipGetLastError());
         return FT_OK;
     }
     const uint32_t n_lb = (uint32_t)(4 * d->cap_tiles);  // look-back words of the two cell scans
     const uint64_t n_clear = std::max<uint64_t>(std::max<uint64_t>(d->n_cells, d->n_vtx),
                                                 std::max<uint64_t>(4ull * d->n_paths, n_lb));
-    k_clear_cells<<<grid_of(n_clear), BLOCK, 0, s>>>(S, gvtx, gcol, d->d_lb, n_lb, d->d_status);
+    k_clear_cells<<<grid_of(n_clear), BLOCK, 0, s>>>(S, gedge, gcol, d->d_lb, n_lb, d->d_status);
     k_vertices<<<grid_of(d->n_vtx), BLOCK, 0, s>>>(S, pts, d->d_status);
     k_rows<<<grid_of(d->n_vtx), BLOCK, 0, s>>>(S, d->d_status);
     const uint32_t nc = (uint32_t)d->n_cells;
@@ -1268,8 +1296,8 @@ ft_status launch_backward(ft_diff *d, const float *colours, const float *grad_ca
     const size_t lds = 2 * (size_t)SEG * (tw + 1) * sizeof(float);
     k_backward<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
         S, reinterpret_cast<const float4 *>(colours), reinterpret_cast<const float4 *>(grad_canvas), d->d_ck,
-        d->ck_pitch, d->ck_stride, d->d_gvtx, grad_colours, d->d_status);
-    k_point_grad<<<grid_of(d->n_pts), BLOCK, 0, d->stream>>>(S, d->d_gvtx, reinterpret_cast<float2 *>(grad_points),
+        d->ck_pitch, d->ck_stride, d->d_gedge, grad_colours, d->d_status);
+    k_point_grad<<<grid_of(d->n_pts), BLOCK, 0, d->stream>>>(S, d->d_gedge, reinterpret_cast<float2 *>(grad_points),
                                                              d->n_pts, d->d_pt_path);
     FD_HIP(hipGetLastError());
     return FT_OK;
@@ -1367,7 +1395,7 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
     else if ((st = dalloc(d->d_pt_off, L->n_paths + 1)) || (st = dalloc(d->d_vtx_off, L->n_paths + 1)) ||
              (st = dalloc(d->d_vtx_path, nv)) || (st = dalloc(d->d_pt_path, np)) ||
              (st = dalloc(d->d_img_first, L->n_images + 1)) || (st = dalloc(d->d_vtx, nv)) ||
-             (st = dalloc(d->d_gvtx, nv)) || (st = dalloc(d->d_cell_cnt, cells)) ||
+             (st = dalloc(d->d_gedge, nv)) || (st = dalloc(d->d_cell_cnt, cells)) ||
              (st = dalloc(d->d_cell_off, cells)) || (st = dalloc(d->d_cell_cur, cells)) ||
              (st = dalloc(d->d_cell_edge, d->cap_pairs)) || (st = dalloc(d->d_lb, std::max<size_t>(4 * d->cap_tiles, lookback_words(GEOM_BLOCKS)))) ||
              (st = dalloc(d->d_ck, n_ck * d->ck_stride)) || (st = dalloc(d->d_partial, LOSS_GRID + 1)) ||
@@ -1397,7 +1425,7 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
 void ft_diff_free(ft_diff *d) {
     if (!d) return;
     void *bufs[] = {d->d_pt_off,   d->d_vtx_off,  d->d_vtx_path, d->d_pt_path,   d->d_img_first, d->d_vtx,
-                    d->d_gvtx,     d->d_cell_cnt, d->d_cell_off, d->d_cell_cur,  d->d_cell_edge, d->d_lb,
+                    d->d_gedge,     d->d_cell_cnt, d->d_cell_off, d->d_cell_cur,  d->d_cell_edge, d->d_lb,
                     d->d_ck,       d->d_partial,  d->d_status};
     for (void *b : bufs)
         if (b) (void)hipFree(b);

@@ -1418,6 +1418,9 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
     if (SPLIT && threadIdx.x == 0) *q_n = 0;
     __syncthreads();
     const int32_t shift = top_row < 0 ? top_row : 0;
+    // the group's rows in 32 bits: an edge's rows are within +-2^16, so a
+    // raster row past 2^31 - 1 has none either way
+    const int32_t g0 = ry0 < 0x7FFFFFFFu ? (int32_t)ry0 : 0x7FFFFFFF, g1 = y1 < 0x7FFFFFFFu ? (int32_t)y1 : 0x7FFFFFFF;
     if (!list_ok && threadIdx.x == 0) raise_err(st, FT_EDEVICE);
     // Cell pass, taller groups: the block takes CR list entries at a time; their
     // (edge, row) pairs are laid out by a scan of the rows per edge and spread
@@ -1441,26 +1444,30 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
                 const bool in = ei < L.cap_points;
                 if (!in) raise_err(st, FT_EDEVICE);
                 const EdgeRec E = edges[in ? ei : 0u];
-                const int64_t a = (int64_t)fx_int(E.y_upper) - shift, b = (int64_t)fx_int(E.y_lower) - shift;
-                if (in & ((E.flags & 1u) != 0) & (a < (int64_t)y1) & (b >= (int64_t)ry0))
+                const int32_t a = fx_int(E.y_upper) - shift, b = fx_int(E.y_lower) - shift;
+                if (in & ((E.flags & 1u) != 0) & (a < g1) & (b >= g0))
                     s_list[atomicAdd(s_nl, 1u)] = ei;
             }
             __syncthreads();
             const uint32_t n_pairs = *s_nl * rows;
             for (uint32_t p = threadIdx.x; p < n_pairs; p += BLOCK) {
-                const EdgeRec E = edges[s_list[p / rows]];
-                const int64_t r = (int64_t)ry0 + p % rows;
-                if ((r < (int64_t)fx_int(E.y_upper) - shift) | (r > (int64_t)fx_int(E.y_lower) - shift)) continue;
+                // p / rows, rows <= DIRECT_ROWS
+                static_assert(DIRECT_ROWS == 4, "quotients by 1 to 4");
+                const uint32_t pe = rows == 3 ? __umulhi(p, 0xAAAAAAABu) >> 1 : p >> (rows >> 1);
+                const uint32_t pr = p - mul24_u(pe, rows);  // the pair's row of the group
+                const EdgeRec E = edges[s_list[pe]];
+                const int32_t r = g0 + (int32_t)pr;
+                if ((r < fx_int(E.y_upper) - shift) | (r > fx_int(E.y_lower) - shift)) continue;
                 const int32_t ed = ((int)((E.flags >> 1) & 1u) == fwd) ? 1 : -1;
-                const RowCells c = row_setup(E, (int32_t)(r + shift), (int32_t)W);
-                int32_t *const at = s_cells + (size_t)(r - ry0) * Wp + c.x_s;
+                const RowCells c = row_setup(E, r + shift, (int32_t)W);
+                int32_t *const at = s_cells + (size_t)pr * Wp + c.x_s;
                 ++n_pairs_acc;
                 if (row_cells_exceed(c, LONG_CELLS)) {
                     const uint32_t qi = atomicAdd(q_n, 1u);
                     if (qi < LONG_QUEUE) {
                         LongWalk w;
                         w.c = c;
-                        w.at = (int32_t)((uint32_t)(r - ry0) * Wp + (uint32_t)c.x_s);
+                        w.at = (int32_t)(pr * Wp + (uint32_t)c.x_s);
                         w.ed = ed;
                         q[qi] = w;
                         continue;
@@ -1497,12 +1504,12 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
         for (int j = 0; j < EB; ++j) {
             if (!ok[j]) continue;
             const int32_t ed = ((int)((E[j].flags >> 1) & 1u) == fwd) ? 1 : -1;
-            int64_t a = (int64_t)fx_int(E[j].y_upper) - shift, b = (int64_t)fx_int(E[j].y_lower) - shift;
-            a = a < (int64_t)ry0 ? (int64_t)ry0 : a;
-            b = b > (int64_t)y1 - 1 ? (int64_t)y1 - 1 : b;
-            for (int64_t r = a; r <= b; ++r) {  // edge_row_cells, counted
-                const RowCells c = row_setup(E[j], (int32_t)(r + shift), (int32_t)W);
-                int32_t *const at = s_cells + (size_t)(r - ry0) * Wp + c.x_s;
+            int32_t a = fx_int(E[j].y_upper) - shift, b = fx_int(E[j].y_lower) - shift;
+            a = a < g0 ? g0 : a;
+            b = b > g1 - 1 ? g1 - 1 : b;
+            for (int32_t r = a; r <= b; ++r) {  // edge_row_cells, counted
+                const RowCells c = row_setup(E[j], r + shift, (int32_t)W);
+                int32_t *const at = s_cells + (size_t)(uint32_t)(r - g0) * Wp + c.x_s;
                 ++n_pairs_acc;
                 row_walk(c, [&](int32_t jj, int32_t d) {
                     if (d) {
@@ -1521,9 +1528,9 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
         okk = okk & (ei < L.cap_points);
         const EdgeRec E = edges[okk ? ei : 0u];
         okk = okk & ((E.flags & 1u) != 0);  // a point without an edge (path edge lists)
-        int64_t ra = (int64_t)fx_int(E.y_upper) - shift, rb = (int64_t)fx_int(E.y_lower) - shift;
-        ra = ra < (int64_t)ry0 ? (int64_t)ry0 : ra;
-        rb = rb > (int64_t)y1 - 1 ? (int64_t)y1 - 1 : rb;
+        int32_t ra = fx_int(E.y_upper) - shift, rb = fx_int(E.y_lower) - shift;
+        ra = ra < g0 ? g0 : ra;
+        rb = rb > g1 - 1 ? g1 - 1 : rb;
         const uint32_t nr = (okk & (ra <= rb)) ? (uint32_t)(rb - ra + 1) : 0u;
         const uint32_t incl = wave_incl_u32(nr);
         if (lane == 63) s_segsum[wid] = incl;
@@ -1545,11 +1552,11 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
             for (uint32_t step = CR / 2; step; step >>= 1) lo += s_pair0[lo + step] <= p ? step : 0u;
             const EdgeRec Eo = s_edge[lo];
             int32_t r_first = fx_int(Eo.y_upper) - shift;
-            r_first = r_first < (int32_t)ry0 ? (int32_t)ry0 : r_first;
+            r_first = r_first < g0 ? g0 : r_first;
             const int32_t row = r_first + (int32_t)(p - s_pair0[lo]);  // raster row in [ry0, y1)
             const int32_t ed = ((int)((Eo.flags >> 1) & 1u) == fwd) ? 1 : -1;
             const RowCells c = row_setup(Eo, row + shift, (int32_t)W);
-            int32_t *const cr = s_cells + (size_t)(row - (int32_t)ry0) * Wp + c.x_s;
+            int32_t *const cr = s_cells + (size_t)(uint32_t)(row - g0) * Wp + c.x_s;
             ++n_pairs_acc;
             row_walk(c, [&](int32_t j, int32_t d) {
                 if (d) {

@@ -763,7 +763,8 @@ FT_HD inline EdgeRec make_edge(I2 q, I2 q1) {
     E.step = dx != 0 ? step : 0;
     E.y_upper = up.y;
     E.y_lower = lo.y;
-    E.x_bot0 = wadd(up.x, fx_mul(E.inv, wsub(fx_floor(wadd(up.y, FX_ONE)), up.y)));
+    // down to the next row: fx_floor(up.y + ONE) - up.y is ONE - fract
+    E.x_bot0 = wadd(up.x, fx_mul_frac(E.inv, FX_ONE - fx_fract(up.y)));
     E.flags = 1u | (fwd ? 2u : 0u);
     return E;
 }
@@ -919,7 +920,7 @@ FT_HD inline bool path_forward(const PathState &s, const Limits &L, const I2 *pt
 // including the first pixel where x_pix reaches cov, or the raster's right
 // edge.  row_setup describes the row; row_walk produces its cells in order.
 struct RowCells {
-    int64_t xc0, st;  // x_cov at step k: min(xc0 + k * st, ONE)
+    int32_t xc0, st;  // x_cov at step k: min(xc0 + k * st, ONE); 0 <= xc0 <= ONE, 0 < st <= ONE
     int32_t cov;      // the row's coverage, 1..256
     int32_t x_s;      // first cell
     int32_t k_s;      // step of the first cell
@@ -940,19 +941,21 @@ FT_HD inline RowCells row_setup(const EdgeRec &E, int32_t sr, int32_t W) {
     c.cov = cov;
     if (cov <= 0) return c;
     const int32_t x_bot = (int32_t)((uint32_t)E.x_bot0 + (uint32_t)(sr - r0) * (uint32_t)E.inv);
-    const int32_t x0 = starting ? wsub(x_bot, fx_mul(E.inv, wsub(FX_ONE, fx_fract(E.y_upper)))) : wsub(x_bot, E.inv);
-    const int32_t x1 = ending ? wsub(x_bot, fx_mul(E.inv, wsub(fx_ceil(E.y_lower), E.y_lower))) : x_bot;
+    // x at the top and bottom of the edge's part of the row: x_bot less the
+    // slope's share of the row below the top (a whole row unless it starts
+    // here) and of the row below the bottom (none unless it ends here)
+    const int32_t x0 = wsub(x_bot, fx_mul_frac(E.inv, starting ? FX_ONE - fx_fract(E.y_upper) : FX_ONE));
+    const int32_t x1 = wsub(x_bot, fx_mul_frac(E.inv, ending ? (int32_t)((0u - (uint32_t)E.y_lower) & 0xFFFFu) : 0));
     const int32_t min_x = x0 < x1 ? x0 : x1, max_x = x0 < x1 ? x1 : x0;
     const int32_t min_pix = fx_int(min_x), max_pix = fx_int(max_x);
     const int32_t full = cov << 8;  // Fixed::from(cov as f32 / 256.0), exact
-    const int32_t r = (min_pix == max_pix) ? fx_mul(wsub(FX_ONE, fx_fract(fx_avg(max_x, min_x))), full)
-                                           : fx_mul(wsub(FX_ONE, fx_fract(min_x)), FX_HALF);
-    c.xc0 = E.step > 0 ? fx_mul(r, E.step) : r;
+    const int32_t r = (min_pix == max_pix) ? fx_mul_unit(FX_ONE - fx_fract(fx_avg(max_x, min_x)), full)
+                                           : (FX_ONE - fx_fract(min_x)) >> 1;  // times HALF
+    c.xc0 = E.step > 0 ? fx_mul_unit(r, E.step) : r;
     c.st = E.step > 0 ? E.step : FX_ONE;
     if (min_pix >= W) return c;
     // every step at x <= 0 adds to cell 0: their sum is x_pix at x = 0
-    const int64_t k0 = min_pix < 0 ? -(int64_t)min_pix : 0;
-    c.k_s = (int32_t)(k0 < 65537 ? k0 : 65537);
+    c.k_s = min_pix < 0 ? -min_pix : 0;  // (below 2^15 + 1)
     c.x_s = min_pix < 0 ? 0 : min_pix;
     c.n = W - c.x_s;
     return c;
@@ -966,9 +969,12 @@ FT_HD inline RowCells row_setup(const EdgeRec &E, int32_t sr, int32_t W) {
 // (u + 128) >> 8, which reaches 256 >= cov at ONE, so the walk ends.
 template <class F>
 FT_HD inline void row_walk(const RowCells &c, F &&f) {
-    const int64_t xk = c.xc0 + (int64_t)c.k_s * c.st;
-    int32_t xc = xk < FX_ONE ? (int32_t)xk : FX_ONE;
-    const int32_t st = (int32_t)c.st;
+    const int32_t st = c.st;
+    int32_t xc = c.xc0;
+    if (c.k_s > 0) {  // starts left of the raster
+        const int64_t xk = c.xc0 + (int64_t)c.k_s * st;
+        xc = xk < FX_ONE ? (int32_t)xk : FX_ONE;
+    }
     int32_t prev = 0;
     for (int32_t j = 0; j < c.n; ++j) {
         const int32_t xp = (xc + 128) >> 8;

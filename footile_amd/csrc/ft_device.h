@@ -14,6 +14,7 @@
 #else
 #define FT_HD
 #endif
+#define FT_INLINE FT_HD inline __attribute__((always_inline))
 
 namespace ft {
 

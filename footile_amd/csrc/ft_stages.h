@@ -123,6 +123,31 @@ FT_HD uint32_t flatten_walk(const Curve &root, float tol_sq, uint32_t max_depth,
     }
 }
 
+// flatten_walk with the first LEVELS levels below `root` walked by direct
+// recursion, the right child kept while the left subtree is walked: the same
+// nodes in the same order, but the levels that most subtrees end in are not
+// replayed from the root for every sibling.
+template <int LEVELS, class Curve, class Emit>
+FT_INLINE uint32_t flatten_tree(const Curve &root, float tol_sq, uint32_t max_depth, uint32_t &leaves, Emit &&emit) {
+    if constexpr (LEVELS == 0) {
+        return flatten_walk(root, tol_sq, max_depth, leaves, emit);
+    } else {
+        Curve L, R;
+        if (split(root, tol_sq, L, R)) {
+            if (++leaves > FT_FLATTEN_MAX_LEAVES) return FT_ERANGE;
+            emit(end_of(root));
+            return 0;
+        }
+        if (max_depth == 0) return FT_ERANGE;
+        const uint32_t rc = flatten_tree<LEVELS - 1>(L, tol_sq, max_depth - 1, leaves, emit);
+        return rc ? rc : flatten_tree<LEVELS - 1>(R, tol_sq, max_depth - 1, leaves, emit);
+    }
+}
+// One level: a 16,384-path atlas launch takes 1,490 us (1,505 with none, 1,479
+// with two, 1,504 with three) and a plain 256x256 stroke 49.1 us (50.0, 50.8,
+// 67.6: its one block's code outgrows the instruction cache).
+constexpr int TREE_LEVELS = 1;
+
 // A curve is flattened by 2^sp lanes (OP_LANES in the pipeline, sp =
 // FLAT_SPLIT).  Lane s takes the subtree sp levels below the root whose
 // left/right choices are the bits of s, most significant first; a node that
@@ -148,7 +173,7 @@ FT_HD uint32_t flatten_share(const Curve &root, float tol_sq, uint32_t s, uint32
         }
         cur = ((s >> (sp - 1 - lv)) & 1u) ? R : L;
     }
-    return flatten_walk(cur, tol_sq, FT_FLATTEN_MAX_DEPTH - sp, leaves, emit);
+    return flatten_tree<TREE_LEVELS>(cur, tol_sq, FT_FLATTEN_MAX_DEPTH - sp, leaves, emit);
 }
 
 // Index of the op that last set the pen before op i (plotter.rs:128-130,
@@ -233,7 +258,7 @@ constexpr uint32_t LEAF_CACHE = 8;
 // sp / last_lane: a curve's lanes split its tree sp levels down, and the
 // op's last lane (which emits the path's final close) is last_lane; the
 // pipeline gives every op OP_LANES lanes.
-FT_HD inline OpCount count_op(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
+FT_INLINE OpCount count_op(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
                               uint32_t s, uint32_t mode, const uint32_t *lastpw, I2 *cache = nullptr,
                               size_t stride = 0, uint32_t sp = FLAT_SPLIT, uint32_t last_lane = OP_LANES - 1,
                               uint32_t cap = LEAF_CACHE) {
@@ -360,7 +385,7 @@ struct EventSink {
 // `cache` / `cached`: the lane's points kept by count_op (point k at
 // cache[k * stride]) and their number (used in fill runs when it is at most
 // the cache's capacity `cap`).
-FT_HD inline uint32_t emit_op(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
+FT_INLINE uint32_t emit_op(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
                               uint32_t s, uint32_t mode, const uint32_t *lastpw, unsigned long long off,
                               EventSink em, const I2 *cache = nullptr, uint32_t cached = 0, size_t stride = 0,
                               uint32_t sp = FLAT_SPLIT, uint32_t last_lane = OP_LANES - 1,

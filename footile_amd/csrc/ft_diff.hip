@@ -166,10 +166,15 @@ __global__ __launch_bounds__(BLOCK) void k_vertices(DScene S, const float2 *poin
     }
 }
 
-// Clears a run's look-back words and status.
-__global__ __launch_bounds__(BLOCK) void k_clear_run(unsigned long long *lb, uint32_t n_lb, DevStatus *st) {
+// Clears a run's look-back words and status.  Needed before the first run and
+// after a failed one only: k_forward leaves the words clear for the next
+// k_geometry, and a run without errors leaves no error (2 us and a gap per
+// call of some 110 us otherwise).
+__global__ __launch_bounds__(BLOCK) void k_clear_run(unsigned long long *lb, uint32_t n_lb, DevStatus *st,
+                                                     uint32_t *host_err) {
     for (uint32_t i = threadIdx.x; i < n_lb; i += BLOCK) lb[i] = 0;
     if (threadIdx.x < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
+    if (threadIdx.x == 0) st->host_err = host_err;  // (one wavefront: after the words above)
 }
 
 // Rows [r0, r1] an edge overlaps within [0, H); false when none.
@@ -196,7 +201,7 @@ __device__ inline void edge_at(const DScene &S, uint32_t v, uint32_t &k, float2 
 // Clears the cell counters, the scans' look-back words, the status and (when
 // given) the gradients.
 __global__ __launch_bounds__(BLOCK) void k_clear_cells(DScene S, float4 *gedge, float *gcol, unsigned long long *lb,
-                                                       uint32_t n_lb, DevStatus *st) {
+                                                       uint32_t n_lb, DevStatus *st, uint32_t *host_err) {
     uint32_t n = S.n_cells > S.n_vtx ? S.n_cells : S.n_vtx;
     n = n > 4 * S.n_paths ? n : 4 * S.n_paths;
     n = n > n_lb ? n : n_lb;
@@ -210,6 +215,7 @@ __global__ __launch_bounds__(BLOCK) void k_clear_cells(DScene S, float4 *gedge, 
         if (gcol && i < 4 * S.n_paths) gcol[i] = 0.0f;
     }
     if (blockIdx.x == 0 && threadIdx.x < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->host_err = host_err;  // (one wavefront: after the words above)
 }
 
 __global__ __launch_bounds__(BLOCK) void k_rows(DScene S, DevStatus *st) {
@@ -733,12 +739,19 @@ __device__ __forceinline__ float4 round_colour(const float4 *__restrict__ colour
 // transparent pixels, SEG at a time, with the next round's pieces loaded
 // while a round is composited.  With ck it also leaves the canvas before
 // every round but the first, at slot (image row) * ck_pitch + X; canvas may
-// be null.
+// be null.  One block also clears the n_lb look-back words of the geometry
+// (done by now) for the next run and, with `report`, reports the status.
 __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 *__restrict__ colours,
                                                       float4 *__restrict__ canvas, float4 *__restrict__ ck,
-                                                      uint32_t ck_pitch, uint64_t ck_stride, DevStatus *st) {
+                                                      uint32_t ck_pitch, uint64_t ck_stride, DevStatus *st,
+                                                      unsigned long long *__restrict__ lb, uint32_t n_lb,
+                                                      HostStatus *__restrict__ report) {
     extern __shared__ __align__(16) int s_cells[];
     __shared__ RowLds R;
+    if ((blockIdx.x | blockIdx.y | blockIdx.z) == 0) {
+        if (report) report_status(report, st, nullptr, nullptr, 0);
+        for (uint32_t i = threadIdx.x; i < n_lb; i += blockDim.x) lb[i] = 0;
+    }
     if (run_failed(st)) return;
     const uint32_t tw = blockDim.x, pitch = tw + 1;
     const uint32_t X = blockIdx.x * tw + threadIdx.x, Y = blockIdx.y, im = blockIdx.z;
@@ -1072,8 +1085,12 @@ __device__ __forceinline__ float4 edge_grad(const DScene &S, const float4 *gedge
 // Control point gradients from edge gradients (one thread per point): the sum
 // over the point's cubics' vertices of their Bernstein weights times the
 // vertex's gradient, which is its two edges' shares.
+// One block also reports the run's status, every other kernel of the run
+// being done.
 __global__ __launch_bounds__(BLOCK) void k_point_grad(DScene S, const float4 *gedge, float2 *gpts, uint32_t n_pts,
-                                                      const uint32_t *pt_path) {
+                                                      const uint32_t *pt_path, const DevStatus *st,
+                                                      HostStatus *report) {
+    if (blockIdx.x == 0) report_status(report, st, nullptr, nullptr, 0);
     for (uint32_t m = blockIdx.x * BLOCK + threadIdx.x; m < n_pts; m += gridDim.x * BLOCK) {
         const uint32_t k = pt_path[m];
         const uint32_t local = m - S.pt_off[k];
@@ -1138,9 +1155,11 @@ struct ft_diff {
     float4 *d_ck = nullptr;
     uint32_t ck_pitch = 0;  // checkpoint pixels per row
     uint64_t ck_stride = 0;  // and per checkpoint
-    double *d_partial = nullptr;  // [LOSS_GRID] loss partials, then [LOSS_GRID] their sum
-    double *h_loss = nullptr;     // pinned: the summed loss
-    DevStatus *d_status = nullptr, *h_status = nullptr;
+    double *d_partial = nullptr;  // [LOSS_GRID] loss partials
+    double *h_loss = nullptr;     // pinned: the summed loss, written by k_loss_sum
+    DevStatus *d_status = nullptr;
+    HostStatus *h_status = nullptr;  // pinned: written by a run's last kernel
+    bool clean = false;  // d_lb and d_status are as k_clear_run leaves them
 };
 
 namespace {
@@ -1185,6 +1204,13 @@ uint32_t grid_of(uint64_t n) {
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(g, GRID_MAX));
 }
 
+// Blocks of k_geometry (0: the scene takes the general form).
+uint32_t geometry_blocks(const ft_diff *d) {
+    if (d->max_path_vtx > GEOM_EDGES || d->H > GEOM_ROWS || !d->n_paths) return 0;
+    const uint32_t per = (d->n_paths + GEOM_BLOCKS - 1) / GEOM_BLOCKS;
+    return (d->n_paths + per - 1) / per;
+}
+
 // Geometry for one parameter set: vertices, per-(path, row) edge lists.
 ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, float *gcol) {
     hipStream_t s = d->stream;
@@ -1192,10 +1218,13 @@ ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, flo
     float4 *const gedge = clear_grads ? d->d_gedge : nullptr;
     if (!clear_grads) gcol = nullptr;
     const float2 *const pts = reinterpret_cast<const float2 *>(points);
-    if (d->max_path_vtx <= GEOM_EDGES && d->H <= GEOM_ROWS && d->n_paths) {
+    uint32_t *const host_err = &d->h_status->late_err;
+    const bool clean = d->clean;
+    d->clean = false;  // until this run is known to have left them so
+    if (const uint32_t blocks = geometry_blocks(d)) {
         const uint32_t per = (d->n_paths + GEOM_BLOCKS - 1) / GEOM_BLOCKS;
-        const uint32_t blocks = (d->n_paths + per - 1) / per;
-        k_clear_run<<<1, BLOCK, 0, s>>>(d->d_lb, (uint32_t)lookback_words(blocks), d->d_status);
+        if (!clean)
+            k_clear_run<<<1, BLOCK, 0, s>>>(d->d_lb, (uint32_t)lookback_words(blocks), d->d_status, host_err);
         k_geometry<<<blocks, BLOCK, (d->H + 1) * sizeof(uint32_t), s>>>(S, pts, gedge, gcol, per, d->d_lb, d->d_status);
         FD_HIP(hipGetLastError());
         return FT_OK;
@@ -1203,7 +1232,7 @@ ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, flo
     const uint32_t n_lb = (uint32_t)(4 * d->cap_tiles);  // look-back words of the two cell scans
     const uint64_t n_clear = std::max<uint64_t>(std::max<uint64_t>(d->n_cells, d->n_vtx),
                                                 std::max<uint64_t>(4ull * d->n_paths, n_lb));
-    k_clear_cells<<<grid_of(n_clear), BLOCK, 0, s>>>(S, gedge, gcol, d->d_lb, n_lb, d->d_status);
+    k_clear_cells<<<grid_of(n_clear), BLOCK, 0, s>>>(S, gedge, gcol, d->d_lb, n_lb, d->d_status, host_err);
     k_vertices<<<grid_of(d->n_vtx), BLOCK, 0, s>>>(S, pts, d->d_status);
     k_rows<<<grid_of(d->n_vtx), BLOCK, 0, s>>>(S, d->d_status);
     const uint32_t nc = (uint32_t)d->n_cells;
@@ -1216,19 +1245,22 @@ ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, flo
     return FT_OK;
 }
 
-// The run's one host wait: status (and, with loss, the device-summed loss).
-ft_status finish(ft_diff *d, bool loss = false) {
-    FD_HIP(hipMemcpyAsync(d->h_status, d->d_status, sizeof(DevStatus), hipMemcpyDeviceToHost, d->stream));
-    if (loss)
-        FD_HIP(hipMemcpyAsync(d->h_loss, d->d_partial + LOSS_GRID, sizeof(double), hipMemcpyDeviceToHost, d->stream));
+// The run's one host wait.  Its kernels have written the status (and the
+// summed loss) to host memory: two copies behind the last kernel cost 8 us of
+// a 390 us step.
+ft_status finish(ft_diff *d) {
     FD_HIP(hipStreamSynchronize(d->stream));
-    if (d->h_status->err) return (ft_status)d->h_status->err;
-    if (d->h_status->overflow) return (ft_status)0x100;
+    const uint32_t late = d->h_status->late_err;
+    d->h_status->late_err = 0;
+    if (d->h_status->st.err) return (ft_status)d->h_status->st.err;
+    if (late) return (ft_status)late;
+    if (d->h_status->st.overflow) return (ft_status)0x100;
+    d->clean = geometry_blocks(d) != 0;
     return FT_OK;
 }
 
 ft_status grow_pairs(ft_diff *d) {
-    const uint64_t need = (uint64_t)d->h_status->need_pairs;
+    const uint64_t need = (uint64_t)d->h_status->st.need_pairs;
     const uint64_t cap = need + need / 4 + 4096;
     if (cap >= 0xFFFFFFFFull) return FT_ENOMEM;
     ft_status st = dalloc(d->d_cell_edge, cap);
@@ -1245,13 +1277,16 @@ uint32_t tile_width(const ft_diff *d) {
     return ((d->W + n - 1) / n + 63) / 64 * 64;
 }
 
-// canvas may be null; keep: also the checkpoints that the backward needs.
-ft_status launch_forward(ft_diff *d, const float *colours, float *canvas, bool keep) {
+// canvas may be null; keep: also the checkpoints that the backward needs;
+// last: no later kernel reports the run's status.
+ft_status launch_forward(ft_diff *d, const float *colours, float *canvas, bool keep, bool last) {
+    const uint32_t blocks = geometry_blocks(d);
     const uint32_t tw = tile_width(d);
     const size_t lds = (size_t)SEG * (tw + 1) * sizeof(int);
     k_forward<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
         scene_of(d), reinterpret_cast<const float4 *>(colours), reinterpret_cast<float4 *>(canvas),
-        keep ? d->d_ck : nullptr, d->ck_pitch, d->ck_stride, d->d_status);
+        keep ? d->d_ck : nullptr, d->ck_pitch, d->ck_stride, d->d_status, d->d_lb,
+        blocks ? (uint32_t)lookback_words(blocks) : 0u, last ? d->h_status : nullptr);
     FD_HIP(hipGetLastError());
     return FT_OK;
 }
@@ -1260,7 +1295,7 @@ ft_status run_forward(ft_diff *d, const float *points, const float *colours, flo
     for (int attempt = 0; attempt < 3; ++attempt) {
         ft_status st = launch_geometry(d, points, false, nullptr);
         if (st) return st;
-        if ((st = launch_forward(d, colours, canvas, false))) return st;
+        if ((st = launch_forward(d, colours, canvas, false, true))) return st;
         st = finish(d);
         if (st != (ft_status)0x100) return st;
         if ((st = grow_pairs(d))) return st;
@@ -1268,10 +1303,10 @@ ft_status run_forward(ft_diff *d, const float *points, const float *colours, flo
     return FT_ENOMEM;
 }
 
-// Enqueues the loss partials and their fixed-order sum (at d_partial[LOSS_GRID]).
+// Enqueues the loss partials and their fixed-order sum (to h_loss).
 ft_status launch_loss(ft_diff *d, const float *canvas, const float *target, float *grad) {
     k_loss<<<LOSS_GRID, BLOCK, 0, d->stream>>>(canvas, target, grad, d->canvas_floats, d->d_partial);
-    k_loss_sum<<<1, BLOCK, 0, d->stream>>>(d->d_partial, LOSS_GRID, d->d_partial + LOSS_GRID);
+    k_loss_sum<<<1, BLOCK, 0, d->stream>>>(d->d_partial, LOSS_GRID, d->h_loss);
     FD_HIP(hipGetLastError());
     return FT_OK;
 }
@@ -1279,8 +1314,6 @@ ft_status launch_loss(ft_diff *d, const float *canvas, const float *target, floa
 ft_status run_loss(ft_diff *d, const float *canvas, const float *target, float *grad, double *loss) {
     ft_status st = launch_loss(d, canvas, target, grad);
     if (!st) {
-        FD_HIP(hipMemcpyAsync(d->h_loss, d->d_partial + LOSS_GRID, sizeof(double), hipMemcpyDeviceToHost,
-                              d->stream));
         FD_HIP(hipStreamSynchronize(d->stream));
         if (loss) *loss = *d->h_loss / (double)d->canvas_floats;
     }
@@ -1298,7 +1331,7 @@ ft_status launch_backward(ft_diff *d, const float *colours, const float *grad_ca
         S, reinterpret_cast<const float4 *>(colours), reinterpret_cast<const float4 *>(grad_canvas), d->d_ck,
         d->ck_pitch, d->ck_stride, d->d_gedge, grad_colours, d->d_status);
     k_point_grad<<<grid_of(d->n_pts), BLOCK, 0, d->stream>>>(S, d->d_gedge, reinterpret_cast<float2 *>(grad_points),
-                                                             d->n_pts, d->d_pt_path);
+                                                             d->n_pts, d->d_pt_path, d->d_status, d->h_status);
     FD_HIP(hipGetLastError());
     return FT_OK;
 }
@@ -1307,7 +1340,7 @@ ft_status run_backward(ft_diff *d, const float *points, const float *colours, co
                        float *grad_points, float *grad_colours) {
     for (int attempt = 0; attempt < 3; ++attempt) {
         ft_status st = launch_geometry(d, points, true, grad_colours);
-        if (!st) st = launch_forward(d, colours, nullptr, true);
+        if (!st) st = launch_forward(d, colours, nullptr, true, false);
         if (!st) st = launch_backward(d, colours, grad_canvas, grad_points, grad_colours);
         if (st) return st;
         st = finish(d);
@@ -1325,10 +1358,10 @@ ft_status run_step(ft_diff *d, const float *points, const float *colours, const 
     for (int attempt = 0; attempt < 3; ++attempt) {
         ft_status st = launch_geometry(d, points, true, grad_colours);
         if (st) return st;
-        if ((st = launch_forward(d, colours, canvas, true))) return st;
+        if ((st = launch_forward(d, colours, canvas, true, false))) return st;
         if ((st = launch_loss(d, canvas, target, grad_canvas))) return st;
         if ((st = launch_backward(d, colours, grad_canvas, grad_points, grad_colours))) return st;
-        st = finish(d, true);
+        st = finish(d);
         if (st == FT_OK && loss) *loss = *d->h_loss / (double)d->canvas_floats;
         if (st != (ft_status)0x100) return st;
         if ((st = grow_pairs(d))) return st;
@@ -1398,12 +1431,12 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
              (st = dalloc(d->d_gedge, nv)) || (st = dalloc(d->d_cell_cnt, cells)) ||
              (st = dalloc(d->d_cell_off, cells)) || (st = dalloc(d->d_cell_cur, cells)) ||
              (st = dalloc(d->d_cell_edge, d->cap_pairs)) || (st = dalloc(d->d_lb, std::max<size_t>(4 * d->cap_tiles, lookback_words(GEOM_BLOCKS)))) ||
-             (st = dalloc(d->d_ck, n_ck * d->ck_stride)) || (st = dalloc(d->d_partial, LOSS_GRID + 1)) ||
+             (st = dalloc(d->d_ck, n_ck * d->ck_stride)) || (st = dalloc(d->d_partial, LOSS_GRID)) ||
              (st = dalloc(d->d_status, 1)))
         ;
-    else if (hipHostMalloc(reinterpret_cast<void **>(&d->h_loss), sizeof(double), hipHostMallocDefault) !=
+    else if (hipHostMalloc(reinterpret_cast<void **>(&d->h_loss), sizeof(double), hipHostMallocCoherent) !=
                  hipSuccess ||
-             hipHostMalloc(reinterpret_cast<void **>(&d->h_status), sizeof(DevStatus), hipHostMallocDefault) !=
+             hipHostMalloc(reinterpret_cast<void **>(&d->h_status), sizeof(HostStatus), hipHostMallocCoherent) !=
                  hipSuccess)
         st = FT_ENOMEM;
     else if (hipMemcpy(d->d_pt_off, pt_off.data(), pt_off.size() * 4, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1412,8 +1445,10 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
              hipMemcpy(d->d_pt_path, pt_path.data(), np * 4, hipMemcpyHostToDevice) != hipSuccess ||
              hipMemcpy(d->d_img_first, img_first.data(), img_first.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
         st = FT_EDEVICE;
-    else
+    else {
+        *d->h_status = HostStatus{};
         st = FT_OK;
+    }
     if (st) {
         ft_diff_free(d);
         return st;

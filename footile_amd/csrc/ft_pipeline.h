@@ -140,6 +140,7 @@ struct Workspace {
     std::vector<PathState> h_pstate_store;
     bool pstate_copied = false;  // the status copy since the last launch included the path states
     bool status_owed = false;    // eager launches left their status on the device: ws_finish copies it
+    bool status_reported = false;  // the last eager launch's raster writes it to h_status itself
     bool edges_counted = false;  // PathState::n_edges holds the last run's counts
     // band / LDS geometry of the next ws_set_batch
     Tuning tuning;

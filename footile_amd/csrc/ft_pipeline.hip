@@ -83,7 +83,7 @@ __device__ inline void block_reduce_keyed(bool has, uint32_t key, T v, T identit
 __global__ __launch_bounds__(BLOCK) void k_clear(PathState *ps, unsigned long long *top_rep, uint32_t n_paths,
                                                  uint32_t *band_cnt, uint32_t *band_cur, uint32_t n_slots,
                                                  unsigned long long *lb, uint32_t n_lb, DevStatus *st,
-                                                 uint32_t keep_failed) {
+                                                 uint32_t keep_failed, uint32_t *host_err) {
     uint32_t n = n_paths * TOP_REPS > n_slots ? n_paths * TOP_REPS : n_slots;
     n = n > n_lb ? n : n_lb;
     for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
@@ -113,6 +113,7 @@ __global__ __launch_bounds__(BLOCK) void k_clear(PathState *ps, unsigned long lo
     if (blockIdx.x == 0 && threadIdx.x < sizeof(DevStatus) / 4) {
         const bool failed = (keep_failed != 0u) & ((st->err | st->overflow) != 0u);
         if (!failed) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
+        if (threadIdx.x == 0) st->host_err = host_err;  // (one wavefront: after the words above)
     }
 }
 
@@ -1676,10 +1677,12 @@ __global__ __launch_bounds__(BLOCK) void k_raster(Limits L0, const PathDev *path
                                                   uint32_t first_block, uint32_t band_shift,
                                                   const uint32_t *band_off, const uint32_t *band_list,
                                                   const EdgeRec *edges, const PathState *ps, DevStatus *st,
-                                                  unsigned long long *stats) {
+                                                  unsigned long long *stats, HostStatus *report, PathState *report_ps) {
     extern __shared__ uint4 s_dyn[];
     __shared__ uint32_t s_segsum[BLOCK / 64];
     __shared__ uint32_t s_stat[2 * BLOCK / 64];
+    // (blocks are ordered largest first: the last one has time to report)
+    if (report && blockIdx.x == gridDim.x - 1) report_status(report, st, report_ps, ps, L0.n_paths);
     if (run_failed(st)) return;
     const Limits L = run_limits(st, L0.n_ops, L0.n_paths, L0.n_bands, L0.cap_points);
     const uint4 rb = rblock[first_block + blockIdx.x];
@@ -2116,11 +2119,14 @@ __device__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, uint32_t n_sev, St
 template <bool STROKE>
 __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, SmallOps inl, uint32_t n_ops,
                                                         PathDev P, StrokeParams sp, EdgeRec *edges, PathState *ps,
-                                                        DevStatus *st) {
+                                                        DevStatus *st, HostStatus *host, PathState *host_ps) {
     __shared__ SmallLds S;
     const uint32_t tid = threadIdx.x;
     if (tid < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[tid] = 0;
     if (tid == 0) {
+        st->host_err = &host->late_err;  // (one wavefront: after the words above)
+        host->st.err = 0;
+        host->st.overflow = 0;
         S.path = P;
         S.flag = 0;
     }
@@ -2155,7 +2161,7 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
                            s_leaf, s_nleaf);
     }
     if (!ok) {
-        if (tid == 0) atomicOr(&st->overflow, SMALL_NOT_HANDLED);
+        if (tid == 0) st->overflow = host->st.overflow = SMALL_NOT_HANDLED;
         return;
     }
     Limits L{};
@@ -2252,13 +2258,14 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
     }
     __syncthreads();
     if (S.flag) {  // an index check failed: let the full pipeline run (and report)
-        if (tid == 0) atomicOr(&st->overflow, SMALL_NOT_HANDLED);
+        if (tid == 0) st->overflow = host->st.overflow = SMALL_NOT_HANDLED;
         return;
     }
     // 6. the edge list and the path's state for the raster blocks
     for (uint32_t i = tid; i < n_kept; i += SBLOCK) edges[i] = S.a.edges[i];
     if (tid == 0) {
         ps[0] = S.ps;
+        host_ps[0] = S.ps;
         st->n_events = n_events;
         st->n_closes = n_runs;
         st->n_kept = n_kept;
@@ -2409,13 +2416,14 @@ ft_status ws_init_arena(Workspace &ws, void *arena, size_t bytes, hipStream_t st
 // The status + path-state blocks (device and pinned host) for n_paths paths;
 // the previous blocks are freed.
 constexpr size_t STATUS_BYTES = 256;
-static_assert(sizeof(DevStatus) <= STATUS_BYTES, "the status fits in front of the path states");
+static_assert(sizeof(HostStatus) <= STATUS_BYTES, "the status fits in front of the path states");
 
 static ft_status sp_grow(Workspace &ws, size_t n_paths) {
     const size_t bytes = STATUS_BYTES + n_paths * sizeof(PathState);
     uint8_t *d = nullptr, *h = nullptr;
     if (hipMalloc(reinterpret_cast<void **>(&d), bytes) != hipSuccess) return FT_ENOMEM;
-    if (hipHostMalloc(reinterpret_cast<void **>(&h), bytes, hipHostMallocDefault) != hipSuccess) {
+    // (coherent: kernels report into it, report_status)
+    if (hipHostMalloc(reinterpret_cast<void **>(&h), bytes, hipHostMallocCoherent) != hipSuccess) {
         (void)hipFree(d);
         return FT_ENOMEM;
     }
@@ -2913,7 +2921,23 @@ static inline uint32_t grid_for(size_t n) {
 }
 
 static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool with_pstate, bool copy_status,
-                            bool keep_failed);
+                            bool keep_failed, HostStatus *report);
+
+// Whether a run's raster kernel reports the status and the path states: its
+// blocks must not be several kernels' (one pixel format, no tile scheduler),
+// and the report is one block's stores over the bus, so the path states are
+// few: REPORT_PATHS of 40 bytes each (a copy costs the same from one path to
+// some hundreds).
+constexpr size_t REPORT_PATHS = 16;
+static bool reports_itself(const Workspace &ws, uint32_t mode) {
+    if (ws.arena || ws.fstream || !ws.d_sp || (mode != MODE_FILL && mode != MODE_STROKE)) return false;
+    int kernels = 0;
+    for (int f = 0; f < 3; ++f) {
+        if (ws.n_bands && ws.rb_count[f]) ++kernels;
+        if (ws.it_count[f]) return false;
+    }
+    return kernels == 1 && ws.n_paths && ws.n_paths <= REPORT_PATHS;
+}
 
 // Enqueue one run.  In graph mode a fill run is captured once into a HIP
 // graph (the launch sequence has no memset nodes and no host waits) and then
@@ -2942,16 +2966,20 @@ ft_status ws_launch(Workspace &ws, uint32_t mode) {
     if (!(ws.graph && mode == MODE_FILL) || ws.fstream) {
         // An eager run leaves its status (and path states) on the device:
         // ws_finish copies them once for all the launches before it, and a
-        // failed launch stays failed until then (keep_failed).
+        // failed launch stays failed until then (keep_failed).  Where the
+        // raster is one kernel over few paths on the workspace's one stream,
+        // that kernel reports them itself (k_raster, report_status).
         const bool keep = ws.status_owed;
-        const ft_status st = ws_enqueue(ws, mode, ev, false, false, keep);
+        HostStatus *const report = reports_itself(ws, mode) ? reinterpret_cast<HostStatus *>(ws.h_status) : nullptr;
+        const ft_status st = ws_enqueue(ws, mode, ev, false, false, keep, report);
         ws.status_owed = true;
+        ws.status_reported = report && !st;
         return st;
     }
     if (!ws.gexec) {
         hipGraph_t g = nullptr;
         FT_HIP(hipStreamBeginCapture(ws.stream, hipStreamCaptureModeThreadLocal));
-        const ft_status st = ws_enqueue(ws, mode, nullptr, false, true, false);
+        const ft_status st = ws_enqueue(ws, mode, nullptr, false, true, false, nullptr);
         const hipError_t e = hipStreamEndCapture(ws.stream, &g);
         if (st) {
             if (g) (void)hipGraphDestroy(g);
@@ -2975,7 +3003,7 @@ ft_status ws_launch(Workspace &ws, uint32_t mode) {
 }
 
 static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool with_pstate, bool copy_status,
-                            bool keep_failed) {
+                            bool keep_failed, HostStatus *report) {
     if (mode == MODE_STROKE) {
         const ft_status e = ensure_stroke_capacity(ws);
         if (e) return e;
@@ -3007,10 +3035,11 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
     // dispatch (ev[0] at k_clear's start, ev[1] / ev[2] around the raster), so
     // no marker packet stalls the stream between kernels.
     const size_t n_slots = ws.n_bands << ws.band_shift;
+    uint32_t *const host_err = report ? &report->late_err : nullptr;
     hipExtLaunchKernelGGL(k_clear, dim3(grid_for(std::max(std::max(ws.n_paths * TOP_REPS, n_slots), (size_t)n_lb))),
                           dim3(BLOCK), 0, s, ev ? ev[0] : nullptr, nullptr, 0, ws.d_pstate, ws.d_top_rep,
                           (uint32_t)ws.n_paths, ws.d_band_cnt, ws.d_band_cur, (uint32_t)n_slots, lb, n_lb, st,
-                          keep_failed ? 1u : 0u);
+                          keep_failed ? 1u : 0u, host_err);
     const uint32_t *lastpw = nullptr;
     if (mode != MODE_FILL && n_ops) {
         k_pen_width_mark<<<grid_for(n_ops), BLOCK, 0, s>>>(ws.d_ops, n_ops, ws.d_op_pw);
@@ -3198,17 +3227,18 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
             if (f == FT_MATTE8)
                 hipExtLaunchKernelGGL(k_raster<false, FMT_MATTE8>, grid, dim3(BLOCK), lds, s, e0, e1, 0, L0,
                                       ws.d_paths, ws.d_rblock, ws.rb_first[f], ws.band_shift, ws.d_band_off,
-                                      ws.d_band_list, ws.d_edges, ws.d_pstate, st, stats);
+                                      ws.d_band_list, ws.d_edges, ws.d_pstate, st, stats, report,
+                                      ws.h_pstate);
             else if (f == FT_RGBA8P)
                 hipExtLaunchKernelGGL(pf ? k_raster<true, FMT_RGBA8P> : k_raster<false, FMT_RGBA8P>, grid,
                                       dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_rblock, ws.rb_first[f],
                                       ws.band_shift, ws.d_band_off, ws.d_band_list, ws.d_edges, ws.d_pstate, st,
-                                      stats);
+                                      stats, report, ws.h_pstate);
             else
                 hipExtLaunchKernelGGL(pf ? k_raster<true, FMT_GRAYA8P> : k_raster<false, FMT_GRAYA8P>, grid,
                                       dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_rblock, ws.rb_first[f],
                                       ws.band_shift, ws.d_band_off, ws.d_band_list, ws.d_edges, ws.d_pstate, st,
-                                      stats);
+                                      stats, report, ws.h_pstate);
         }
         if (ev && n_rl == 0) {
             FT_HIP(hipEventRecord(ev[1], s));
@@ -3225,8 +3255,21 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
     return FT_OK;
 }
 
+// The late error word of the host status block, cleared (the stream is idle).
+static uint32_t take_late_err(Workspace &ws) {
+    if (ws.arena || !ws.h_sp) return 0;  // (no such word: the status is always copied)
+    HostStatus *const h = reinterpret_cast<HostStatus *>(ws.h_sp);
+    const uint32_t e = h->late_err;
+    h->late_err = 0;
+    return e;
+}
+
 ft_status ws_finish(Workspace &ws, bool read_pstate) {
-    if (ws.status_owed) {  // the eager launches' status, with the path states when they share its block
+    const bool reported = ws.status_owed && ws.status_reported;
+    if (reported) {  // the last launch's raster wrote both to the host block
+        ws.pstate_copied = true;
+        ws.status_owed = ws.status_reported = false;
+    } else if (ws.status_owed) {  // the eager launches' status, with the path states when they share its block
         const bool with_ps = read_pstate && ws.d_sp && ws.n_paths;
         const size_t back = with_ps ? STATUS_BYTES + ws.n_paths * sizeof(PathState) : sizeof(DevStatus);
         FT_HIP(hipMemcpyAsync(ws.h_status, ws.d_status, back, hipMemcpyDeviceToHost, ws.stream));
@@ -3251,7 +3294,9 @@ ft_status ws_finish(Workspace &ws, bool read_pstate) {
     }
     ws.n_pending = 0;
     const DevStatus &h = *ws.h_status;
+    const uint32_t late = take_late_err(ws);
     if (h.err) return (ft_status)h.err;
+    if (reported && late) return (ft_status)late;
     if (h.overflow) return (ft_status)0x100;  // internal: capacity exceeded
     return FT_OK;
 }
@@ -3365,12 +3410,13 @@ ft_status ws_small_fill(Workspace &ws, const ft_path_op *ops, size_t n_ops, cons
     sp.join = ws.join;
     sp.miter = ws.miter;
     sp.tol_sq = ws.stroke_tol_sq;
+    HostStatus *const host = reinterpret_cast<HostStatus *>(ws.h_status);
     if (mode == MODE_STROKE)
         k_small_front<true><<<1, SBLOCK, 0, ws.stream>>>(d_ops, inl, (uint32_t)n_ops, P, sp, ws.d_edges,
-                                                         ws.d_pstate, ws.d_status);
+                                                         ws.d_pstate, ws.d_status, host, ws.h_pstate);
     else
         k_small_front<false><<<1, SBLOCK, 0, ws.stream>>>(d_ops, inl, (uint32_t)n_ops, P, sp, ws.d_edges,
-                                                          ws.d_pstate, ws.d_status);
+                                                          ws.d_pstate, ws.d_status, host, ws.h_pstate);
     if (d.fmt == FT_MATTE8)
         k_small_raster<FMT_MATTE8><<<groups, BLOCK, lds, ws.stream>>>(P, ws.d_edges, ws.d_pstate, ws.d_status);
     else if (d.fmt == FT_RGBA8P)
@@ -3378,12 +3424,11 @@ ft_status ws_small_fill(Workspace &ws, const ft_path_op *ops, size_t n_ops, cons
     else
         k_small_raster<FMT_GRAYA8P><<<groups, BLOCK, lds, ws.stream>>>(P, ws.d_edges, ws.d_pstate, ws.d_status);
     FT_HIP(hipGetLastError());
-    FT_HIP(hipMemcpyAsync(ws.h_status, ws.d_status, STATUS_BYTES + sizeof(PathState), hipMemcpyDeviceToHost,
-                          ws.stream));
     FT_HIP(hipStreamSynchronize(ws.stream));
-    const DevStatus &h = *ws.h_status;
-    if (h.overflow & SMALL_NOT_HANDLED) return FT_OK;
-    if (h.err) return (ft_status)h.err;
+    // (k_small_front wrote the status and the path state to the host block)
+    const uint32_t late = take_late_err(ws);
+    if (ws.h_status->overflow & SMALL_NOT_HANDLED) return FT_OK;
+    if (late) return (ft_status)late;
     *handled = true;
     if (offered) *offered = ws.h_pstate[0].offered;
     if (stored) *stored = ws.h_pstate[0].stored;

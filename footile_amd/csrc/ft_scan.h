@@ -55,7 +55,29 @@ struct DevAtom {
     __device__ static void add_cell(int32_t *p, int32_t v) { atomicAdd(p, v); }
 };
 
-__device__ inline void raise_err(DevStatus *st, uint32_t code) { atomicCAS(&st->err, 0u, code); }
+__device__ inline void raise_err(DevStatus *st, uint32_t code) {
+    atomicCAS(&st->err, 0u, code);
+    uint32_t *const h = st->host_err;
+    if (h) __hip_atomic_store(h, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The status in pinned host memory, written by a kernel of the run itself: a
+// copy after the last kernel is one more dispatch between the raster and the
+// host's wait (2.5 to 4 us of a 36 us small fill).  The block that reports
+// runs beside blocks that may still raise an error, which then reaches the
+// host through DevStatus::host_err (late_err), a word the report never writes.
+struct HostStatus {
+    DevStatus st;
+    uint32_t late_err;
+};
+// Called by one block: every word of the status (and of n_ps path states).
+__device__ inline void report_status(HostStatus *h, const DevStatus *st, PathState *h_ps, const PathState *ps,
+                                     uint32_t n_ps) {
+    uint32_t *const d0 = reinterpret_cast<uint32_t *>(&h->st), *const d1 = reinterpret_cast<uint32_t *>(h_ps);
+    const uint32_t *const s0 = reinterpret_cast<const uint32_t *>(st), *const s1 = reinterpret_cast<const uint32_t *>(ps);
+    for (uint32_t i = threadIdx.x; i < sizeof(DevStatus) / 4; i += blockDim.x) d0[i] = s0[i];
+    for (uint32_t i = threadIdx.x; i < n_ps * (sizeof(PathState) / 4); i += blockDim.x) d1[i] = s1[i];
+}
 // A kernel's early exit after an earlier kernel of the run failed: plain
 // loads (the previous kernels have completed), both issued before either is
 // tested, so the check costs one memory round trip.

@@ -83,7 +83,8 @@ struct DevStatus {
     unsigned long long stroke_total;  // stroker outline: events << 32 | closes
     uint32_t st_subs, st_items;       // sub-strokes kept; outline items
     uint32_t spin_fail;
-    uint32_t pad[3];
+    uint32_t pad;
+    uint32_t *host_err;  // a pinned host word that also receives `err` when it is raised (null: none)
 };
 
 struct EdgeRec {

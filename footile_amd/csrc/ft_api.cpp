@@ -357,15 +357,19 @@ ft_status ft_batch_set_tuning(ft_batch *b, const ft_tuning *t) {
     tu.dst_prefetch = t->dst_prefetch ? 1u : 0u;
     tu.tile_groups = t->tile_groups;
     const ft::Tuning old = b->ws.tuning;
+    const bool was_tuned = b->ws.tuned;
     b->ws.tuning = tu;
+    b->ws.tuned = true;
     ft_status s = ft::ws_set_batch(b->ws, b->ops.data(), b->ops.size(), b->descs.data(), b->descs.size());
     if (s) {
         b->ws.tuning = old;
+        b->ws.tuned = was_tuned;
         (void)ft::ws_set_batch(b->ws, b->ops.data(), b->ops.size(), b->descs.data(), b->descs.size());
         return s;
     }
     for (int k = 1; k < b->depth && !s; ++k) {
         b->slot(k).tuning = tu;
+        b->slot(k).tuned = true;
         s = ft::ws_set_batch(b->slot(k), b->ops.data(), b->ops.size(), b->descs.data(), b->descs.size());
     }
     return s ? s : twin_follow(b);
@@ -414,6 +418,7 @@ ft_status ft_batch_set_pipeline(ft_batch *b, int depth) {
         if (!s) s = ft::ws_pipe_attach(w, b->ws.stream);
         if (!s) {
             w.tuning = b->ws.tuning;
+            w.tuned = b->ws.tuned;
             w.timing = b->ws.timing;
             s = ft::ws_set_batch(w, b->ops.data(), b->ops.size(), b->descs.data(), b->descs.size());
         }

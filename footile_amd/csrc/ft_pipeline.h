@@ -142,8 +142,10 @@ struct Workspace {
     bool status_owed = false;    // eager launches left their status on the device: ws_finish copies it
     bool status_reported = false;  // the last eager launch's raster writes it to h_status itself
     bool edges_counted = false;  // PathState::n_edges holds the last run's counts
-    // band / LDS geometry of the next ws_set_batch
+    // band / LDS geometry of the next ws_set_batch: `tuning` as it stands when
+    // `tuned` (ft_batch_set_tuning), else default_tuning's per path
     Tuning tuning;
+    bool tuned = false;
     // graph mode: fill runs replay a captured graph of the launch sequence
     bool graph = false;
     hipGraphExec_t gexec = nullptr;

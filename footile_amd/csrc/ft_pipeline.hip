@@ -1233,20 +1233,22 @@ __device__ __forceinline__ void chunk_out(const uint32_t *v, uint32_t base, uint
 
 // Prefix-sum the cells [xb, xe) of one raster row (one wavefront) from
 // `carry`, map coverage and store / composite CPT pixels per lane per chunk.
-// `loaded`: the pipe already holds the segment's first DST_DEPTH chunks.
 template <int FMT, int CPT, uint32_t RULE, bool FRESH>
 __device__ __forceinline__ void row_pass(const int32_t *cells, uint32_t xb, uint32_t xe, gbyte *row,
-                                         const uint4 *lut, uint32_t clr, uint32_t carry, DstPipe &pp, bool loaded) {
+                                         const uint4 *lut, uint32_t clr, uint32_t carry) {
     constexpr bool RMW = FMT != FMT_MATTE8 && !FRESH;
     constexpr uint32_t chunk = 64u * CPT;
     const uint32_t nck = (xe - xb + chunk - 1) / chunk;
+    // (Loading the first chunks before the cell pass made every raster slower:
+    // it holds 16 VGPRs through the pass, 82 against 68, and a CU then has five
+    // blocks instead of seven: 78 against 62 us for two 4096x4096 Rgba8p fills.)
+    DstPipe pp;
+    pp.q0 = pp.q1 = pp.q2 = pp.q3 = make_uint4(0, 0, 0, 0);
     if constexpr (RMW) {
-        if (!loaded) {
-            pp.q0 = dst_load<FMT, CPT>(row, xb, xe, 0, nck);
-            pp.q1 = dst_load<FMT, CPT>(row, xb, xe, 1, nck);
-            pp.q2 = dst_load<FMT, CPT>(row, xb, xe, 2, nck);
-            pp.q3 = dst_load<FMT, CPT>(row, xb, xe, 3, nck);
-        }
+        pp.q0 = dst_load<FMT, CPT>(row, xb, xe, 0, nck);
+        pp.q1 = dst_load<FMT, CPT>(row, xb, xe, 1, nck);
+        pp.q2 = dst_load<FMT, CPT>(row, xb, xe, 2, nck);
+        pp.q3 = dst_load<FMT, CPT>(row, xb, xe, 3, nck);
     }
     const uint32_t lx = (uint32_t)(threadIdx.x & 63) * CPT;
     for (uint32_t k = 0; k < nck; k += DST_DEPTH) {
@@ -1270,12 +1272,11 @@ __device__ __forceinline__ void row_pass(const int32_t *cells, uint32_t xb, uint
 
 template <int FMT, int CPT, bool FRESH>
 __device__ __forceinline__ void row_pass_rule(uint32_t rule, const int32_t *cells, uint32_t xb, uint32_t xe,
-                                              gbyte *row, const uint4 *lut, uint32_t clr, uint32_t carry,
-                                              DstPipe &pp, bool loaded) {
+                                              gbyte *row, const uint4 *lut, uint32_t clr, uint32_t carry) {
     if (rule)
-        row_pass<FMT, CPT, 1, FRESH>(cells, xb, xe, row, lut, clr, carry, pp, loaded);
+        row_pass<FMT, CPT, 1, FRESH>(cells, xb, xe, row, lut, clr, carry);
     else
-        row_pass<FMT, CPT, 0, FRESH>(cells, xb, xe, row, lut, clr, carry, pp, loaded);
+        row_pass<FMT, CPT, 0, FRESH>(cells, xb, xe, row, lut, clr, carry);
 }
 
 template <int FMT, int LPR>
@@ -1339,7 +1340,7 @@ constexpr size_t SPLIT_LIST_BYTES = SPLIT_LIST * sizeof(uint32_t);
 // queued (up to LONG_QUEUE of them; a lane walks the rest itself) and every
 // wavefront then takes queued walks, one cell per lane (row_cell_delta).
 // The listed order does not matter: the cell adds are integer adds.
-template <bool PF, int FMT, class Src, bool SPLIT = false>
+template <int FMT, class Src, bool SPLIT = false>
 __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, const PathState &S, int fwd,
                                              uint32_t y0, uint32_t y1, Src src, uint32_t cnt, bool list_ok,
                                              const EdgeRec *edges, uint4 *s_dyn, uint32_t *s_segsum,
@@ -1390,28 +1391,8 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
         xb = (wid % seg) * seg_len;
         xe = xb + seg_len < W ? xb + seg_len : W;
     }
-    // the first destination chunks of a read-modify-write format, now
-    DstPipe pp;
-    pp.q0 = pp.q1 = pp.q2 = pp.q3 = make_uint4(0, 0, 0, 0);
-    const bool rmw = !fresh & (fmt != FMT_MATTE8);
     // Narrow rows: LPR lanes per row, 64 / LPR rows per wavefront at once.
     const uint32_t lpr = seg > 1 ? 64u : (W <= 16u * cpt ? 16u : (W <= 32u * cpt ? 32u : 64u));
-    const bool pre = PF & rmw & (xb < xe) & (r0 < rows) & (lpr == 64u);
-    if constexpr (PF && FMT != FMT_MATTE8) if (pre) {
-        const gbyte *row = base + (size_t)(ry0 + r0) * P.pitch;
-        const uint32_t nck = (xe - xb + chunk - 1) / chunk;
-        if constexpr (FMT == FMT_RGBA8P) {
-            pp.q0 = dst_load<FMT_RGBA8P, 4>(row, xb, xe, 0, nck);
-            pp.q1 = dst_load<FMT_RGBA8P, 4>(row, xb, xe, 1, nck);
-            pp.q2 = dst_load<FMT_RGBA8P, 4>(row, xb, xe, 2, nck);
-            pp.q3 = dst_load<FMT_RGBA8P, 4>(row, xb, xe, 3, nck);
-        } else {
-            pp.q0 = dst_load<FMT_GRAYA8P, 8>(row, xb, xe, 0, nck);
-            pp.q1 = dst_load<FMT_GRAYA8P, 8>(row, xb, xe, 1, nck);
-            pp.q2 = dst_load<FMT_GRAYA8P, 8>(row, xb, xe, 2, nck);
-            pp.q3 = dst_load<FMT_GRAYA8P, 8>(row, xb, xe, 3, nck);
-        }
-    }
     for (uint32_t c = threadIdx.x; c < rows * Wp / 4; c += BLOCK)
         reinterpret_cast<int4 *>(s_cells)[c] = make_int4(0, 0, 0, 0);
     uint32_t *const q_n = reinterpret_cast<uint32_t *>(s_dyn);
@@ -1618,28 +1599,26 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
         }
         return;
     }
-    bool loaded = pre;
     for (uint32_t r = r0; r < rows; r += rstep) {
         if (xb >= xe) break;
         const int32_t *cells = s_cells + (size_t)r * Wp;
         gbyte *row = base + (size_t)(ry0 + r) * P.pitch;
         if constexpr (FMT == FMT_MATTE8) {
             if (cpt == 16)
-                row_pass_rule<FMT_MATTE8, 16, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry, pp, false);
+                row_pass_rule<FMT_MATTE8, 16, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry);
             else
-                row_pass_rule<FMT_MATTE8, 4, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry, pp, false);
+                row_pass_rule<FMT_MATTE8, 4, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry);
         } else if constexpr (FMT == FMT_RGBA8P) {
             if (fresh)
-                row_pass_rule<FMT_RGBA8P, 4, true>(P.rule, cells, xb, xe, row, lut, P.clr, carry, pp, false);
+                row_pass_rule<FMT_RGBA8P, 4, true>(P.rule, cells, xb, xe, row, lut, P.clr, carry);
             else
-                row_pass_rule<FMT_RGBA8P, 4, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry, pp, loaded);
+                row_pass_rule<FMT_RGBA8P, 4, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry);
         } else {
             if (fresh)
-                row_pass_rule<FMT_GRAYA8P, 8, true>(P.rule, cells, xb, xe, row, lut, P.clr, carry, pp, false);
+                row_pass_rule<FMT_GRAYA8P, 8, true>(P.rule, cells, xb, xe, row, lut, P.clr, carry);
             else
-                row_pass_rule<FMT_GRAYA8P, 8, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry, pp, loaded);
+                row_pass_rule<FMT_GRAYA8P, 8, false>(P.rule, cells, xb, xe, row, lut, P.clr, carry);
         }
-        loaded = false;
     }
 }
 
@@ -1672,7 +1651,7 @@ __device__ inline void block_stats(uint32_t a, uint32_t b, unsigned long long *s
 // from `first`, ordered largest first.  The block accumulates the band's listed edges for its G rows
 // in LDS and scans each row into the raster; the band's other groups are
 // other blocks.
-template <bool PF, int FMT>
+template <int FMT>
 __global__ __launch_bounds__(BLOCK) void k_raster(Limits L0, const PathDev *paths, const uint4 *rblock,
                                                   uint32_t first_block, uint32_t band_shift,
                                                   const uint32_t *band_off, const uint32_t *band_list,
@@ -1705,7 +1684,7 @@ __global__ __launch_bounds__(BLOCK) void k_raster(Limits L0, const PathDev *path
     if (y0 < y1) {
         const PathState S = ps[p];
         const bool list_ok = (off <= end) & (end <= L.n_pairs);
-        raster_group<PF, FMT>(L, P, S, (int)S.fwd, y0, y1, BandListSrc{band_list, off},
+        raster_group<FMT>(L, P, S, (int)S.fwd, y0, y1, BandListSrc{band_list, off},
                               list_ok ? end - off : 0u, list_ok, edges, s_dyn, s_segsum, st, n_pairs, n_adds);
     }
     block_stats(n_pairs, n_adds, stats, first_block + blockIdx.x, s_stat);
@@ -1719,7 +1698,7 @@ __global__ __launch_bounds__(BLOCK) void k_raster(Limits L0, const PathDev *path
 // tile-mode path has no bands: an item reads the path's own stored points as
 // its edge list (one edge per point, in point order), so nothing is binned.
 // The winding direction (Fig::get_dir) is evaluated per item.
-template <bool PF, int FMT>
+template <int FMT>
 __global__ __launch_bounds__(BLOCK) void k_tiles(Limits L0, const PathDev *paths, const uint2 *items,
                                                  uint32_t first_item, uint32_t n_items, const EdgeRec *edges,
                                                  const I2 *pts, const uint32_t *pt_run, const uint32_t *run_start,
@@ -1754,7 +1733,7 @@ __global__ __launch_bounds__(BLOCK) void k_tiles(Limits L0, const PathDev *paths
         const bool list_ok = ((uint64_t)S.pt_base + S.stored) <= L.cap_points;
         __syncthreads();  // s_fwd
         if (y0 < y1)
-            raster_group<PF, FMT>(L, P, S, (int)s_fwd, y0, y1, PathEdgeSrc{S.pt_base},
+            raster_group<FMT>(L, P, S, (int)s_fwd, y0, y1, PathEdgeSrc{S.pt_base},
                                   (has_pts && list_ok) ? S.stored : 0u, list_ok, edges, s_dyn, s_segsum, st,
                                   n_pairs, n_adds);
         __syncthreads();  // the next item reuses the LDS and s_fwd
@@ -2296,7 +2275,7 @@ __global__ __launch_bounds__(BLOCK) void k_small_raster(PathDev P, const EdgeRec
     const bool has_pts = S.topkey != NO_KEY && S.topidx != NO_IDX && n_kept <= SMALL_EVENTS;
     uint32_t n_pairs = 0, n_adds = 0;
     if (y0 < y1)
-        raster_group<false, FMT, PathEdgeSrc, true>(L, P, S, (int)S.fwd, y0, y1, PathEdgeSrc{0u},
+        raster_group<FMT, PathEdgeSrc, true>(L, P, S, (int)S.fwd, y0, y1, PathEdgeSrc{0u},
                                                     has_pts ? n_kept : 0u, true, edges, s_dyn, s_segsum, st, n_pairs,
                                                     n_adds);
 }
@@ -2656,11 +2635,11 @@ static uint32_t tile_grid_for(const Workspace &ws, int f, uint32_t cells) {
     int per_cu = 0;
     hipError_t e;
     if (f == FT_MATTE8)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiles<false, FMT_MATTE8>, BLOCK, lds);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiles<FMT_MATTE8>, BLOCK, lds);
     else if (f == FT_RGBA8P)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiles<true, FMT_RGBA8P>, BLOCK, lds);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiles<FMT_RGBA8P>, BLOCK, lds);
     else
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiles<true, FMT_GRAYA8P>, BLOCK, lds);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiles<FMT_GRAYA8P>, BLOCK, lds);
     if (e != hipSuccess || per_cu < 1) per_cu = 1;
     const uint64_t cus = ws.scan_resident ? ws.scan_resident / 4 : 64;
     const uint64_t g = cus * (uint64_t)per_cu;
@@ -2694,6 +2673,9 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
     std::vector<uint64_t> rcost_f[3];  // estimated work of each raster block
     std::vector<uint64_t> cost_f[3];  // estimated work of each item, for the largest-first order
     uint32_t lds = 0;
+    uint64_t n_cells = 0;  // of the whole batch
+    for (size_t k = 0; k < n_paths; ++k)
+        if (paths[k].width <= FT_MAX_WIDTH) n_cells += (uint64_t)cell_stride(paths[k].width) * paths[k].height;
     for (size_t k = 0; k < n_paths; ++k) {
         const ft_fill_desc &d = paths[k];
         if (d.op_begin > n_ops || d.op_count > n_ops - d.op_begin) return FT_EINVAL;
@@ -2707,14 +2689,15 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
             op_path[i] = (uint32_t)k;
         }
         PathDev &P = pd[k];
-        P = path_from_desc(d, extra_flags, ws.tuning);
+        const Tuning tuning = ws.tuned || ws.arena ? ws.tuning : default_tuning(d.width, d.height, n_cells, ws.tuning);
+        P = path_from_desc(d, extra_flags, tuning);
         // Tile mode: a path of at most tuning.tile_groups LDS groups (rows
         // whose cells fit lds_cells) is rastered by the tile scheduler, one
         // work item per group, with no bands.
         const uint32_t wp = cell_stride(d.width);
-        const uint32_t gt = wp ? std::max(1u, ws.tuning.lds_cells / wp) : 1u;
+        const uint32_t gt = wp ? std::max(1u, tuning.lds_cells / wp) : 1u;
         const uint64_t tgroups = d.height ? ((uint64_t)d.height + gt - 1) / gt : 0;
-        if (ws.tuning.tile_groups && d.width && d.height && tgroups <= ws.tuning.tile_groups) {
+        if (tuning.tile_groups && d.width && d.height && tgroups <= tuning.tile_groups) {
             P.flags |= PATH_TILE;
             P.n_bands = 0;
             P.band_rows = d.height;
@@ -2732,7 +2715,7 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
             continue;
         }
         uint32_t rows, group, nb, cells;
-        band_geometry(d.width, d.height, ws.tuning, &rows, &group, &nb, &cells);
+        band_geometry(d.width, d.height, tuning, &rows, &group, &nb, &cells);
         nb = P.n_bands;
         P.band_base = (uint32_t)band_path.size();
         if (nb && cells > lds) lds = cells;
@@ -2859,7 +2842,9 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
             if ((s = ensure_event_capacity(ws, 16 * n_ops + 1024))) return s;
         }
         if (!ws.d_band_list) {
-            size_t cap = 4 * (16 * n_ops + 1024);
+            // (an edge lies in up to three times as many bands of default_tuning's
+            // rows as of the nominal ones)
+            size_t cap = (ws.tuned ? 4 : 12) * (16 * n_ops + 1024);
             if ((s = dev_alloc(ws, ws.d_band_list, cap))) return s;
             ws.cap_pairs = cap;
         }
@@ -3196,7 +3181,6 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
             if (ws.n_bands && ws.rb_count[f]) rl[n_rl++] = {f, false};
         for (int f = 0; f < 3; ++f)
             if (ws.it_count[f] && ws.tile_grid[f]) rl[n_rl++] = {f, true};
-        const bool pf = ws.tuning.dst_prefetch != 0;
         unsigned long long *const stats = ws.stats ? ws.d_stats : nullptr;
         uint32_t tile_slot = (uint32_t)ws.n_rblocks;  // per-block stats: band blocks, then tile blocks
         for (int k = 0; k < n_rl; ++k) {
@@ -3207,16 +3191,16 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
                 const dim3 grid(ws.tile_grid[f]);
                 const uint32_t nf = ws.it_first[f], ni = ws.it_count[f];
                 if (f == FT_MATTE8)
-                    hipExtLaunchKernelGGL(k_tiles<false, FMT_MATTE8>, grid, dim3(BLOCK), lds, s, e0, e1, 0, L0,
+                    hipExtLaunchKernelGGL(k_tiles<FMT_MATTE8>, grid, dim3(BLOCK), lds, s, e0, e1, 0, L0,
                                           ws.d_paths, ws.d_items, nf, ni, ws.d_edges, ws.d_pts, ws.d_pt_run,
                                           ws.d_run_start, ws.d_run_end, ws.d_pstate, st, stats, tile_slot);
                 else if (f == FT_RGBA8P)
-                    hipExtLaunchKernelGGL(pf ? k_tiles<true, FMT_RGBA8P> : k_tiles<false, FMT_RGBA8P>, grid,
+                    hipExtLaunchKernelGGL(k_tiles<FMT_RGBA8P>, grid,
                                           dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_items, nf, ni,
                                           ws.d_edges, ws.d_pts, ws.d_pt_run, ws.d_run_start, ws.d_run_end,
                                           ws.d_pstate, st, stats, tile_slot);
                 else
-                    hipExtLaunchKernelGGL(pf ? k_tiles<true, FMT_GRAYA8P> : k_tiles<false, FMT_GRAYA8P>, grid,
+                    hipExtLaunchKernelGGL(k_tiles<FMT_GRAYA8P>, grid,
                                           dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_items, nf, ni,
                                           ws.d_edges, ws.d_pts, ws.d_pt_run, ws.d_run_start, ws.d_run_end,
                                           ws.d_pstate, st, stats, tile_slot);
@@ -3225,17 +3209,17 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
             }
             const dim3 grid(ws.rb_count[f]);
             if (f == FT_MATTE8)
-                hipExtLaunchKernelGGL(k_raster<false, FMT_MATTE8>, grid, dim3(BLOCK), lds, s, e0, e1, 0, L0,
+                hipExtLaunchKernelGGL(k_raster<FMT_MATTE8>, grid, dim3(BLOCK), lds, s, e0, e1, 0, L0,
                                       ws.d_paths, ws.d_rblock, ws.rb_first[f], ws.band_shift, ws.d_band_off,
                                       ws.d_band_list, ws.d_edges, ws.d_pstate, st, stats, report,
                                       ws.h_pstate);
             else if (f == FT_RGBA8P)
-                hipExtLaunchKernelGGL(pf ? k_raster<true, FMT_RGBA8P> : k_raster<false, FMT_RGBA8P>, grid,
+                hipExtLaunchKernelGGL(k_raster<FMT_RGBA8P>, grid,
                                       dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_rblock, ws.rb_first[f],
                                       ws.band_shift, ws.d_band_off, ws.d_band_list, ws.d_edges, ws.d_pstate, st,
                                       stats, report, ws.h_pstate);
             else
-                hipExtLaunchKernelGGL(pf ? k_raster<true, FMT_GRAYA8P> : k_raster<false, FMT_GRAYA8P>, grid,
+                hipExtLaunchKernelGGL(k_raster<FMT_GRAYA8P>, grid,
                                       dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_rblock, ws.rb_first[f],
                                       ws.band_shift, ws.d_band_off, ws.d_band_list, ws.d_edges, ws.d_pstate, st,
                                       stats, report, ws.h_pstate);

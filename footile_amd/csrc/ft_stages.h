@@ -1087,7 +1087,7 @@ constexpr uint32_t CELL_ALIGN = 16;   // row stride of cells in LDS
 struct Tuning {
     uint32_t band_rows_min = BAND_ROWS_MIN;  // 1 .. 256
     uint32_t lds_cells = LDS_CELLS;          // 1024 .. 32768, a multiple of CELL_ALIGN (and fitting LDS)
-    uint32_t dst_prefetch = 1;               // raster blocks load their destination chunks first
+    uint32_t dst_prefetch = 1;               // accepted and reported; changes nothing
     uint32_t tile_groups = 0;                // paths of at most this many LDS groups go to the tile
                                              // scheduler (0: none)
 };
@@ -1116,6 +1116,29 @@ FT_HD inline void band_geometry(uint32_t width, uint32_t height, const Tuning &t
     *group = g;
     *n_bands = height ? (height + r - 1) / r : 0;
     *cells = g * wp;
+}
+
+// The geometry of one path of a batch nobody has tuned, `n_cells` cells in
+// all.  Measured on whole launches with the rows and cells swept:
+//  - batches of at most SMALL_CELLS cells: 2,048 cells a block, since with
+//    4,096 there are too few blocks to hide their row chains (a 1237x771
+//    Graya8p drawing's raster takes 12.5 us, 17.4 with 4,096; 384 glyph tiles
+//    11.0 and 12.3).
+//  - larger ones: 3,072, at which a CU holds eight Matte8 blocks (16,384 atlas
+//    tiles: 504 us, 559 with 4,096, 596 with 2,048), but two rows of a raster
+//    up to 3,072 wide (3000x2200 Rgba8p: 20.8 us, 23.4 with one row).
+//  - bands of 8 rows up to a height of SHORT_ROWS (the atlas: 504 us, 550 with
+//    16; 8,000 cubics over 700x700: 14.8 and 19.3), 16 above, where an edge
+//    crosses many bands (4096x4096 with 300 segments: 74 us a launch, 78 with
+//    8).
+constexpr uint64_t SMALL_CELLS = 4u << 20;
+constexpr uint32_t SHORT_ROWS = 1024;
+inline Tuning default_tuning(uint32_t width, uint32_t height, uint64_t n_cells, Tuning t) {
+    const uint32_t wp = cell_stride(width);
+    const uint32_t two = 2 * wp < 6144u ? (2 * wp + CELL_ALIGN - 1) / CELL_ALIGN * CELL_ALIGN : 3072u;
+    t.lds_cells = n_cells <= SMALL_CELLS ? 2048u : (two > 3072u ? two : 3072u);
+    t.band_rows_min = height <= SHORT_ROWS ? 8u : BAND_ROWS_MIN;
+    return t;
 }
 
 // Device form of one batch path (ft_fill_desc -> PathDev); band_base is set

@@ -2,8 +2,7 @@
 
 Candidates are (band_rows_min, lds_cells, dst_prefetch, tile_groups): band
 height for edge binning, the LDS cell budget that fixes the rows per raster
-block, (for read-modify-write rasters) whether raster blocks load their
-destination before the cell pass, and the largest path (in LDS row groups)
+block, a flag that changes nothing, and the largest path (in LDS row groups)
 the tile scheduler takes instead of the bands.  Each
 candidate is timed on the batch itself with device events (whole launch
 sequence, median of a few launches after one warm-up run); the fastest wins.
@@ -84,9 +83,7 @@ def autotune(batch, descs, n_ops, cache=DEFAULT_CACHE, reps=3, candidates=None, 
         e = table[key]
         batch.set_tuning(e["band_rows_min"], e["lds_cells"], e.get("dst_prefetch", True), e.get("tile_groups", 0))
         return dict(e, cached=True, tried=0)
-    # the destination prefetch only matters for read-modify-write rasters
-    rmw = any(int(d.c.fmt) != 0 and not int(d.c.fresh) for d in descs)
-    prefetch = (True, False) if rmw else (True,)
+    prefetch = (False,)
     cands = candidates or ([(b, c, p, 0) for b in BAND_ROWS for c in LDS_CELLS for p in prefetch] +
                            _tile_candidates(descs, prefetch))
     best = None

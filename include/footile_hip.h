@@ -176,13 +176,16 @@ ft_status ft_batch_counts(ft_batch *b, uint64_t *offered, uint64_t *stored, uint
  * most tile_groups such groups (0: none) skips the bands: the atlas tile
  * scheduler, one persistent launch per pixel format, rasters its groups from
  * the path's own edges, largest work items first.  Setting it re-lays the
- * batch out.  No reference counterpart: the autotuner (footile_amd.tune)
- * picks it per workload. */
+ * batch out.  Until it is set, each path's geometry follows its size (and
+ * ft_batch_get_tuning reports the nominal 16 rows and 4,096 cells).  No
+ * reference counterpart: the autotuner (footile_amd.tune) picks it per
+ * workload. */
 typedef struct ft_tuning {
     uint32_t band_rows_min;
     uint32_t lds_cells;
-    uint32_t dst_prefetch; /* 1: raster blocks of Rgba8p/Graya8p read their
-                              destination before the cell pass */
+    uint32_t dst_prefetch; /* accepted and reported; changes nothing (reading
+                              the destination before the cell pass was slower
+                              at every size measured) */
     uint32_t tile_groups;
 } ft_tuning;
 ft_status ft_batch_set_tuning(ft_batch *b, const ft_tuning *t);

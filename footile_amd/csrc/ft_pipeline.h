@@ -65,6 +65,7 @@ struct Workspace {
     std::vector<uint4> h_rblock;
     bool uploads_pending = false;  // a layout's uploads may not have run yet (cleared by a stream sync)
     uint8_t *h_pin = nullptr;      // pinned staging of the layout's uploads
+    std::vector<uint8_t> h_stage;  // the same in arena mode, in plain memory
     size_t cap_pin = 0;
     bool op_ordered = false;
     // the kept flags take the ingest pass (pushed marks and their running
@@ -129,15 +130,15 @@ struct Workspace {
     // results
     PathState *d_pstate = nullptr;
     unsigned long long *d_top_rep = nullptr;  // per path: TOP_REPS partial top keys
-    // Outside arena mode the status and the path states are one device block
-    // and one pinned host block (status first, STATUS_BYTES long), so that a
+    // The status and the path states are one device block and one host block
+    // (status first, STATUS_BYTES long; pinned outside arena mode), so that a
     // run's final copy can bring both back at once.
     DevStatus *d_status = nullptr;
     DevStatus *h_status = nullptr;  // pinned
-    PathState *h_pstate = nullptr;  // host copy of d_pstate (pinned, or h_pstate_store in arena mode)
+    PathState *h_pstate = nullptr;  // host copy of d_pstate (pinned, or h_sp_store in arena mode)
     uint8_t *d_sp = nullptr, *h_sp = nullptr;
     size_t cap_sp_paths = 0;
-    std::vector<PathState> h_pstate_store;
+    std::vector<uint64_t> h_sp_store;  // h_status and h_pstate in arena mode
     bool pstate_copied = false;  // the status copy since the last launch included the path states
     bool status_owed = false;    // eager launches left their status on the device: ws_finish copies it
     bool status_reported = false;  // the last eager launch's raster writes it to h_status itself
@@ -162,10 +163,9 @@ struct Workspace {
     // [arena, arena + arena_bytes), nothing is allocated or freed, each
     // ws_set_batch carves afresh, and a run that outgrows its carved
     // capacities fails with FT_ENOMEM instead of growing.  The stream is the
-    // caller's and the status is read back into h_status_store.
+    // caller's and the status is read back into h_sp_store.
     uint8_t *arena = nullptr;
     size_t arena_bytes = 0, arena_used = 0;
-    DevStatus h_status_store{};
 };
 
 // Allocate the stream and status buffers.

@@ -2387,7 +2387,6 @@ ft_status ws_init_arena(Workspace &ws, void *arena, size_t bytes, hipStream_t st
     ws.arena = reinterpret_cast<uint8_t *>(arena);
     ws.arena_bytes = bytes;
     ws.arena_used = 0;
-    ws.h_status = &ws.h_status_store;
     ws.tickets = true;  // the caller's stream: other waiting kernels may run beside
     return FT_OK;
 }
@@ -2569,9 +2568,8 @@ ft_status ws_upload_ops(Workspace &ws, const ft_path_op *ops, size_t n_ops) {
     return FT_OK;
 }
 
-// Arena mode: forget every carved buffer (the next layout carves afresh) and
-// carve the status block first.
-static ft_status arena_rewind(Workspace &ws) {
+// Arena mode: forget every carved buffer (the next layout carves afresh).
+static void arena_rewind(Workspace &ws) {
     ws.arena_used = 0;
     void **ptrs[] = {(void **)&ws.d_lay, (void **)&ws.d_ops, (void **)&ws.d_op_path, (void **)&ws.d_op_order,
                      (void **)&ws.d_paths,
@@ -2590,7 +2588,22 @@ static ft_status arena_rewind(Workspace &ws) {
     for (void **p : ptrs) *p = nullptr;
     ws.cap_ops = ws.cap_paths = ws.cap_events = ws.cap_stroke = ws.cap_lay = 0;
     ws.cap_band_slots = ws.cap_pairs = ws.cap_tiles = 0;
-    return arena_carve(ws, ws.d_status, 1);
+    ws.d_sp = nullptr;
+}
+
+// Arena mode: the status and the path states as one block, on the device and
+// on the host (plain memory here), so that one copy brings both back.
+static ft_status arena_sp(Workspace &ws, size_t n_paths) {
+    const size_t bytes = STATUS_BYTES + n_paths * sizeof(PathState);
+    const ft_status s = arena_carve(ws, ws.d_sp, bytes);
+    if (s) return s;
+    ws.h_sp_store.resize((bytes + 7) / 8);
+    ws.d_status = reinterpret_cast<DevStatus *>(ws.d_sp);
+    ws.d_pstate = reinterpret_cast<PathState *>(ws.d_sp + STATUS_BYTES);
+    uint8_t *const h = reinterpret_cast<uint8_t *>(ws.h_sp_store.data());
+    ws.h_status = reinterpret_cast<DevStatus *>(h);
+    ws.h_pstate = reinterpret_cast<PathState *>(h + STATUS_BYTES);
+    return FT_OK;
 }
 
 // Arena mode: the rest of the arena, after the layout's fixed buffers and the
@@ -2656,10 +2669,7 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
     // staging is only rewritten once the previous layout's uploads are done
     if (ws.uploads_pending) FT_HIP(hipStreamSynchronize(ws.stream));
     ws.uploads_pending = false;
-    if (ws.arena) {
-        const ft_status s = arena_rewind(ws);
-        if (s) return s;
-    }
+    if (ws.arena) arena_rewind(ws);
     std::vector<uint32_t> &op_path = ws.h_op_path;
     std::vector<PathDev> &pd = ws.h_paths;
     std::vector<uint32_t> &band_path = ws.h_band_path;
@@ -2776,7 +2786,7 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
     if (n_paths > ws.cap_paths || !ws.d_pstate) {  // per-path results
         const size_t cap = n_paths ? n_paths : 1;
         if (ws.arena)
-            s = dev_alloc(ws, ws.d_pstate, cap);
+            s = arena_sp(ws, cap);
         else if (cap > ws.cap_sp_paths)
             s = sp_grow(ws, cap);
         if (s || (s = dev_alloc(ws, ws.d_top_rep, cap * TOP_REPS))) {
@@ -2832,10 +2842,6 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
     ws.n_bands = nb_total;
     ws.lds_cells = lds;
     if (ws.arena) {
-        ws.h_pstate_store.resize(n_paths);
-        ws.h_pstate = ws.h_pstate_store.data();
-    }
-    if (ws.arena) {
         if ((s = arena_split(ws))) return s;
     } else {
         if (!ws.d_ev_meta) {
@@ -2866,22 +2872,22 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
                 if (cls == pass) ws.h_op_order[at++] = (uint32_t)i;
             }
     }
-    // The layout's uploads: staged into one pinned host buffer at the upload
-    // block's offsets and sent with one copy (a copy from pageable memory goes
-    // through the runtime's own staging, a host round trip each).  Arena
-    // workspaces, which may not allocate, copy each section from its source.
+    // The layout's uploads: staged into one host buffer at the upload block's
+    // offsets and sent with one copy, pinned but for arena workspaces, which may
+    // not allocate such memory (a copy from pageable memory goes through the
+    // runtime's own staging, a host round trip each: five of them and two for
+    // the results took 33 of the 193 us of 384 glyph tiles).
     const void *sec_src[LAY_SECTIONS] = {ops, op_path.data(), ws.h_op_order.data(), pd.data(),
                                          band_path.data(), rblock.data(), ws.h_items.data()};
     size_t sec_len[LAY_SECTIONS];
     for (int k = 0; k < LAY_SECTIONS; ++k) sec_len[k] = sec_bytes[k];
     if (!ws.op_ordered) sec_len[2] = 0;
-    if (ws.arena) {
-        for (int k = 0; k < LAY_SECTIONS; ++k)
-            if (sec_len[k])
-                FT_HIP(hipMemcpyAsync(ws.d_lay + sec_off[k], sec_src[k], sec_len[k], hipMemcpyHostToDevice,
-                                      ws.stream));
-    } else if (lay_bytes) {
-        if (lay_bytes > ws.cap_pin) {
+    if (lay_bytes) {
+        uint8_t *stage = ws.h_pin;
+        if (ws.arena) {
+            if (lay_bytes > ws.h_stage.size()) ws.h_stage.resize(lay_bytes);
+            stage = ws.h_stage.data();
+        } else if (lay_bytes > ws.cap_pin) {
             if (ws.h_pin) (void)hipHostFree(ws.h_pin);
             ws.h_pin = nullptr;
             ws.cap_pin = 0;
@@ -2890,10 +2896,11 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
                 return FT_ENOMEM;
             }
             ws.cap_pin = lay_bytes;
+            stage = ws.h_pin;
         }
         for (int k = 0; k < LAY_SECTIONS; ++k)
-            if (sec_len[k]) memcpy(ws.h_pin + sec_off[k], sec_src[k], sec_len[k]);
-        FT_HIP(hipMemcpyAsync(ws.d_lay, ws.h_pin, lay_bytes, hipMemcpyHostToDevice, ws.stream));
+            if (sec_len[k]) memcpy(stage + sec_off[k], sec_src[k], sec_len[k]);
+        FT_HIP(hipMemcpyAsync(ws.d_lay, stage, lay_bytes, hipMemcpyHostToDevice, ws.stream));
     }
     ws.uploads_pending = true;
     return FT_OK;

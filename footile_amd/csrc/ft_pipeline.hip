@@ -1774,26 +1774,23 @@ struct SmallLds {
     union {
         struct {  // events: flatten to compaction
             I2 xy[SMALL_EVENTS];
-            uint32_t meta[SMALL_EVENTS], last[SMALL_EVENTS], kept[SMALL_EVENTS], idx[SMALL_EVENTS];
+            uint32_t meta[SMALL_EVENTS], kept[SMALL_EVENTS], idx[SMALL_EVENTS];
         } ev;
         struct {  // a stroke's flattened (x, y, width, kind) events and its last close so far
             F4 f[SMALL_EVENTS];
             uint32_t last[SMALL_EVENTS];
         } st;
-        EdgeRec edges[SMALL_EVENTS];  // after compaction
     } a;
     union {
-        uint32_t cnt_e[SMALL_ITEMS];   // (op, lane) event counts, then their exclusive scan
-        I2 pts[SMALL_EVENTS];          // after the emit
+        uint32_t cnt[SMALL_EVENTS];    // a stroke's packed counts, then their exclusive scan
+        I2 pts[SMALL_EVENTS];          // after the compaction
     } b;
-    union {
-        uint32_t cnt_c[SMALL_ITEMS];   // (op, lane) close counts, then their exclusive scan
-        uint32_t pt_run[SMALL_EVENTS];
-    } c;
+    uint32_t pt_run[SMALL_EVENTS];
     int32_t run_first[SMALL_RUNS];
     uint32_t run_close[SMALL_RUNS], run_path[SMALL_RUNS], run_start[SMALL_RUNS], run_end[SMALL_RUNS];
     uint32_t op_path[SMALL_OPS];
-    uint32_t op_item[SMALL_OPS];  // the op's first (op, lane) item
+    uint32_t op_item[SMALL_OPS];  // the curves in order, then the other ops
+    __align__(16) uint32_t op_cnt[SMALL_OPS];  // the ops' packed counts, then their prefix
     ft_path_op ops[SMALL_OPS];
     PathDev path;
     PathState ps;
@@ -1857,16 +1854,26 @@ struct SmallOps {
     ft_path_op op[SMALL_ARG_OPS];
 };
 
+constexpr uint32_t SMALL_SPLIT = 5;  // a small figure's curves take 32 lanes when the items fit
+
+// Points of a curve lane that a small figure keeps in LDS from the count to
+// the emit; a lane with more flattens again.
+constexpr uint32_t SMALL_LEAF = 2;
 // A small stroke's stroker data beside SmallLds: the pen-width marks of the
 // ops and their running maximum, the stored points, the sub-strokes, and
 // the first ITEM_PTS (transformed) outline points of every outline item,
 // which its count computes and its emit then replays.
 constexpr uint32_t ITEM_PTS = 2;
 struct SmallStrokeLds {
-    F4 spts[SMALL_EVENTS];
+    union {
+        struct {
+            F4 spts[SMALL_EVENTS];
+            SV2 item_pt[ITEM_PTS][SMALL_EVENTS];
+        };
+        F4 leaf[SMALL_LEAF * SMALL_ITEMS];  // before the stroker: small_flatten's kept points
+    };
     uint32_t lastpw[SMALL_OPS];
     uint32_t sub_start[SMALL_RUNS], sub_event[SMALL_RUNS], sub_n[SMALL_RUNS], sub_joined[SMALL_RUNS];
-    SV2 item_pt[ITEM_PTS][SMALL_EVENTS];
 };
 
 // Fill events of a small figure go to the event and run arrays in LDS.
@@ -1885,79 +1892,153 @@ __device__ inline EventSink small_fill_sink(SmallLds &S) {
     return em;
 }
 
-// The op of (op, lane) item t: the last op whose first item is at or before
-// t (every op has at least one item).
-__device__ inline uint32_t small_item_op(const uint32_t *op_item, uint32_t n_ops, uint32_t t) {
-    uint32_t lo = 0, hi = n_ops;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) / 2;
-        if (op_item[mid] <= t)
-            lo = mid;
-        else
-            hi = mid;
+template <bool STROKE>
+struct SmallLeaf {  // as the event sink stores them: Fixed points, or (x, y, width)
+    using T = I2;
+    __device__ static T of(WP q) {
+        T v;
+        v.x = fx_from_f32(q.x);
+        v.y = fx_from_f32(q.y);
+        return v;
     }
-    return lo;
-}
+    __device__ static void put(EventSink &em, T v) { em.point_fx(v); }
+};
+template <>
+struct SmallLeaf<true> {
+    using T = F4;
+    __device__ static T of(WP q) {
+        T v;
+        v.x = q.x;
+        v.y = q.y;
+        v.z = q.w;
+        v.w = 0.0f;
+        return v;
+    }
+    __device__ static void put(EventSink &em, T v) {
+        WP q;
+        q.x = v.x;
+        q.y = v.y;
+        q.w = v.z;
+        em.point(q);
+    }
+};
 
-constexpr uint32_t SMALL_SPLIT = 5;  // a small figure's curves take 32 lanes when the items fit
-
-// Stages 1-2 in one block: the (op, lane) event and close counts, their block
-// scans, and the emit through `em`.  A curve's subdivision tree is split
+// Stages 1-2 in one block: the (op, lane) event and close counts, their
+// prefix, and the emit through `em`.  A curve's subdivision tree is split
 // SMALL_SPLIT levels down over 2^SMALL_SPLIT lanes (FLAT_SPLIT if those
 // items would not fit SMALL_ITEMS), every other op takes one lane: the
 // points and their order are the same for any split.  False (in every
 // thread, nothing emitted) when flattening fails or the events or closes
 // exceed their limits.
-// A small fill keeps each curve lane's first SMALL_LEAF points in LDS
-// (leaf[k * SMALL_ITEMS + t], with the lane's leaf count in n_leaf[t]), so
-// that its emit is a copy unless the lane has more.
-constexpr uint32_t SMALL_LEAF = 2;
-
-__device__ bool small_flatten(SmallLds &S, uint32_t n_ops, uint32_t mode, const uint32_t *lastpw, EventSink em,
-                              uint32_t max_runs, uint32_t &n_events, uint32_t &n_runs, uint32_t &bad,
-                              I2 *leaf = nullptr, uint16_t *n_leaf = nullptr) {
-    const uint32_t tid = threadIdx.x;
-    static_assert(SMALL_OPS <= SBLOCK, "one op per thread");
+//
+// A thread's items are of the curves first, then of the other ops, so that an
+// item's op is one LDS read and a curve's lanes are an aligned part of a
+// wavefront: their prefix is taken in registers, and only the ops' totals (at
+// most 256) go through LDS, where one wavefront scans them.  (Items in op
+// order, found by binary search, with block scans over all of them took 8.0
+// us of a plain fill's 13 and 10 of a stroke's 23; the calls went from 33.6 to
+// 30.2 us and from 47.4 to 42.4.)
+template <bool STROKE>
+__device__ __forceinline__ bool small_flatten(SmallLds &S, uint32_t n_ops, const uint32_t *lastpw, EventSink em, uint32_t max_runs,
+                              uint32_t &n_events, uint32_t &n_runs, uint32_t &bad,
+                              typename SmallLeaf<STROKE>::T *leaf) {
+    using Leaf = SmallLeaf<STROKE>;
+    constexpr uint32_t mode = STROKE ? MODE_STROKE : MODE_FILL;
+    constexpr int UNROLL = STROKE ? 1 : SMALL_ITEMS / SBLOCK;
+    // an op's total and the prefix: events in the low 20 bits, closes above
+    // (an op's events are at most SMALL_EVENTS or the figure is not handled)
+    constexpr uint32_t EV_BITS = 20, EV_MASK = (1u << EV_BITS) - 1u;
+    static_assert(SMALL_OPS * SMALL_EVENTS <= EV_MASK && (SMALL_EVENTS << SMALL_SPLIT) <= EV_MASK && 2u * SMALL_OPS < (1u << (32 - EV_BITS)), "packed counts");
+    static_assert(SMALL_OPS == 256, "one wavefront scans the ops, four per lane");
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const uint32_t tag = tid < n_ops ? S.ops[tid].tag : TAG_CLOSE;
     const bool curve = (tag == TAG_QUAD) | (tag == TAG_CUBIC);
-    const uint32_t n_curves = (uint32_t)__syncthreads_count(curve ? 1 : 0);
-    const uint32_t sp = n_curves * ((1u << SMALL_SPLIT) - 1u) + n_ops <= SMALL_ITEMS ? SMALL_SPLIT : FLAT_SPLIT;
-    if (tid < SMALL_OPS) S.op_item[tid] = tid < n_ops ? (curve ? 1u << sp : 1u) : 0u;
+    const unsigned long long cm = __ballot(curve);
+    if (lane == 0 && wid < SMALL_OPS / 64) S.w[wid] = (uint32_t)__popcll(cm);
     __syncthreads();
-    const uint32_t n_items = small_scan<false>(S.op_item, n_ops, S.w);
-    // item t's op, lane and the op's last lane
-    auto lane_of = [&](uint32_t t, uint32_t &i, uint32_t &s, uint32_t &last) {
-        i = small_item_op(S.op_item, n_ops, t);
-        const uint32_t first = S.op_item[i];
-        const uint32_t end = i + 1 < n_ops ? S.op_item[i + 1] : n_items;
-        s = t - first;
-        last = end - first - 1;
-    };
+    uint32_t n_curves = 0, before = (uint32_t)__popcll(cm & ((1ull << lane) - 1ull));
+#pragma unroll
+    for (uint32_t w = 0; w < SMALL_OPS / 64; ++w) {
+        before += w < wid ? S.w[w] : 0u;
+        n_curves += S.w[w];
+    }
+    if (tid < n_ops) S.op_item[curve ? before : n_curves + tid - before] = tid;
+    if (tid < SMALL_OPS) S.op_cnt[tid] = 0;
+    const uint32_t sp = n_curves * ((1u << SMALL_SPLIT) - 1u) + n_ops <= SMALL_ITEMS ? SMALL_SPLIT : FLAT_SPLIT;
+    const uint32_t n_lanes = n_curves << sp, n_items = n_lanes + n_ops - n_curves;
+    __syncthreads();
+    // an item's facts for the emit: its place within the op (as an op's total),
+    // the leaves up to LEAF_MANY, and whether it emits the final close.  (A
+    // thread's two items are unrolled for a fill, 0.7 us of 30, and one after
+    // the other for a stroke, whose longer code then spills registers.)
+    constexpr uint32_t LEAF_MANY = SMALL_LEAF + 1, LEAF_AT = EV_BITS + 4, CLOSE_AT = LEAF_AT + 2;
+    static_assert(LEAF_MANY < 4, "two bits");
+    uint32_t *const facts = S.pt_run;  // (free until the compaction)
     uint32_t err = 0;
+#pragma unroll UNROLL
     for (uint32_t t = tid; t < SMALL_ITEMS; t += SBLOCK) {
+        const bool on = t < n_items, cl = t < n_lanes;
+        const uint32_t s = cl ? t & ((1u << sp) - 1u) : 0u, last = cl ? (1u << sp) - 1u : 0u;
+        const uint32_t i = on ? S.op_item[cl ? t >> sp : n_curves + (t - n_lanes)] : 0u;
         OpCount c = {0, 0, 0, 0, 0};
-        if (t < n_items) {
-            uint32_t i, s, last;
-            lane_of(t, i, s, last);
-            c = count_op(S.ops, S.op_path, &S.path, i, s, mode, lastpw, leaf ? leaf + t : nullptr, SMALL_ITEMS, sp,
-                         last, SMALL_LEAF);
+        if (on)
+            c = count_op_keep(
+                S.ops, S.op_path, &S.path, i, s, mode, lastpw,
+                [&](uint32_t k, WP q) {
+                    if (k < SMALL_LEAF) leaf[k * SMALL_ITEMS + t] = Leaf::of(q);
+                },
+                sp, last);
+        const bool many = c.ne > SMALL_EVENTS;
+        const uint32_t v = many ? 0u : c.ne | (c.nc << EV_BITS);
+        uint32_t incl = v;
+        for (uint32_t o = 1; o < (1u << sp); o <<= 1) {  // (uniform: every lane takes part)
+            const uint32_t u = (uint32_t)__shfl_up((int)incl, o, 1 << sp);
+            incl += (cl & (s >= o)) ? u : 0u;
         }
-        if (n_leaf) n_leaf[t] = (uint16_t)(c.leaves < 0xFFFFu ? c.leaves : 0xFFFFu);
-        err |= c.err;
-        S.b.cnt_e[t] = c.ne;
-        S.c.cnt_c[t] = c.nc;
+        err |= c.err | (many ? 1u : 0u);
+        if (on & (s == last)) {
+            const bool over = (incl & EV_MASK) > SMALL_EVENTS;
+            err |= over ? 1u : 0u;
+            S.op_cnt[i] = over ? 0u : incl;
+        }
+        facts[t] = (incl - v) | ((c.leaves < LEAF_MANY ? c.leaves : LEAF_MANY) << LEAF_AT) |
+                   ((c.flags & OPC_LAST_CLOSE) ? 1u << CLOSE_AT : 0u);
     }
     if (err) S.flag = 1;
     __syncthreads();
-    n_events = small_scan<false>(S.b.cnt_e, n_items, S.w);
-    n_runs = small_scan<false>(S.c.cnt_c, n_items, S.w2);
+    if (wid == 0) {
+        uint4 q = reinterpret_cast<const uint4 *>(S.op_cnt)[lane];
+        const uint32_t a1 = q.x, a2 = a1 + q.y, a3 = a2 + q.z, all = a3 + q.w;
+        const uint32_t incl = wave_incl_dpp<false>(all), pre = incl - all;
+        reinterpret_cast<uint4 *>(S.op_cnt)[lane] = make_uint4(pre, pre + a1, pre + a2, pre + a3);
+        if (lane == 63) S.w[0] = incl;
+    }
+    __syncthreads();
+    n_events = S.w[0] & EV_MASK;
+    n_runs = S.w[0] >> EV_BITS;
     if (S.flag | (n_events > SMALL_EVENTS) | (n_runs > max_runs)) return false;
-    for (uint32_t t = tid; t < n_items; t += SBLOCK) {
-        const unsigned long long off = ((unsigned long long)S.b.cnt_e[t] << 32) | S.c.cnt_c[t];
-        uint32_t i, s, last;
-        lane_of(t, i, s, last);
-        bad |= emit_op(S.ops, S.op_path, &S.path, i, s, mode, lastpw, off, em, leaf ? leaf + t : nullptr,
-                       n_leaf ? n_leaf[t] : 0u, SMALL_ITEMS, sp, last, SMALL_LEAF);
+#pragma unroll UNROLL
+    for (uint32_t t = tid; t < SMALL_ITEMS; t += SBLOCK) {
+        if (t >= n_items) continue;
+        const bool cl = t < n_lanes;
+        const uint32_t s = cl ? t & ((1u << sp) - 1u) : 0u, last = cl ? (1u << sp) - 1u : 0u;
+        const uint32_t i = S.op_item[cl ? t >> sp : n_curves + (t - n_lanes)], f = facts[t];
+        const uint32_t leaves = (f >> LEAF_AT) & 3u;
+        const uint32_t o = S.op_cnt[i] + (f & ((1u << LEAF_AT) - 1u));
+        EventSink e = em;
+        e.e = o & EV_MASK;
+        e.run = o >> EV_BITS;
+        e.p = 0;
+        if (cl & (leaves <= SMALL_LEAF)) {
+#pragma unroll
+            for (uint32_t k = 0; k < SMALL_LEAF; ++k)
+                if (k < leaves) Leaf::put(e, leaf[k * SMALL_ITEMS + t]);
+            if ((f >> CLOSE_AT) & 1u) e.close(true);
+            bad |= e.bad;
+        } else {
+            const unsigned long long off = ((unsigned long long)(o & EV_MASK) << 32) | (o >> EV_BITS);
+            bad |= emit_op(S.ops, S.op_path, &S.path, i, s, mode, lastpw, off, e, nullptr, 0u, 0, sp, last);
+        }
     }
     __syncthreads();
     return true;
@@ -1967,26 +2048,25 @@ __device__ bool small_flatten(SmallLds &S, uint32_t n_ops, uint32_t mode, const 
 // S.a.st.f to the outline's fill events and runs.  False (in every thread)
 // when the sub-strokes, outline items, events or closes exceed their limits
 // or a join fails to flatten; nothing usable is written then.
-__device__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, uint32_t n_sev, StrokeParams sp, uint32_t &n_events,
+__device__ __forceinline__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, uint32_t n_sev, StrokeParams sp, uint32_t &n_events,
                               uint32_t &n_runs, uint32_t &bad) {
     const uint32_t tid = threadIdx.x;
     // flags (k_st_flags): pushed -> stored point index, first point of a run
     // -> sub-stroke index, closes -> the last close so far
     for (uint32_t e = tid; e < n_sev; e += SBLOCK) {
         const StrokeFlags f = stroke_flags(e, S.a.st.f);
-        S.b.cnt_e[e] = f.pushed ? 1u : 0u;
-        S.c.cnt_c[e] = f.first ? 1u : 0u;
+        S.b.cnt[e] = (f.pushed ? 1u : 0u) | (f.first ? 1u << 16 : 0u);
         S.a.st.last[e] = f.is_pt ? 0u : e + 1;
     }
     __syncthreads();
-    const uint32_t n_pts = small_scan<false>(S.b.cnt_e, n_sev, S.w);  // below the 65,535 cap
-    const uint32_t n_subs = small_scan<false>(S.c.cnt_c, n_sev, S.w2);
-    (void)small_scan<true>(S.a.st.last, n_sev, S.w);
+    const uint32_t n_both = small_scan<false>(S.b.cnt, n_sev, S.w);  // both at most SMALL_EVENTS
+    const uint32_t n_pts = n_both & 0xFFFFu, n_subs = n_both >> 16;
+    (void)small_scan<true>(S.a.st.last, n_sev, S.w2);
     if (n_subs > SMALL_RUNS) return false;
     // compaction (k_st_compact)
     for (uint32_t e = tid; e < n_sev; e += SBLOCK) {
         const StrokeFlags f = stroke_flags(e, S.a.st.f);
-        const uint32_t sidx = S.b.cnt_e[e], sub = S.c.cnt_c[e];
+        const uint32_t sidx = S.b.cnt[e] & 0xFFFFu, sub = S.b.cnt[e] >> 16;
         if (f.pushed) T.spts[sidx] = S.a.st.f[e];
         if (f.first) {
             T.sub_start[sub] = sidx;
@@ -2009,7 +2089,10 @@ __device__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, uint32_t n_sev, St
     const uint32_t n_items = n_subs ? 2u * (n_pts + n_subs) + 1u : 1u;
     if (n_items > SMALL_EVENTS) return false;
     __syncthreads();
-    // outline items: line and close counts (k_st_count)
+    // outline items: line and close counts (k_st_count), events in the low 22
+    // bits and closes (at most one per sub-stroke side and the last) above
+    constexpr uint32_t NE_BITS = 22, NE_MASK = (1u << NE_BITS) - 1u, MAX_NE = SMALL_EVENTS - 1;
+    static_assert(MAX_NE * SMALL_EVENTS <= NE_MASK && 2 * SMALL_RUNS + 1 < (1u << (32 - NE_BITS)), "packed counts");
     auto sub_of = [&](uint32_t t, StrokeSub &sub, bool &fwd, uint32_t &k) {
         const uint32_t si = st_item_sub(t, T.sub_start, n_subs);
         sub.start = T.sub_start[si];
@@ -2046,24 +2129,26 @@ __device__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, uint32_t n_sev, St
                         ++nc;
                     });
         }
-        S.b.cnt_e[t] = ne;
-        S.c.cnt_c[t] = nc;
+        const bool many = ne > MAX_NE;  // (more events than a small figure takes)
+        err |= many ? 1u : 0u;
+        S.b.cnt[t] = many ? 0u : ne | (nc << NE_BITS);
     }
     if (err) S.flag = 1;
     __syncthreads();
-    n_events = small_scan<false>(S.b.cnt_e, n_items, S.w);
-    n_runs = small_scan<false>(S.c.cnt_c, n_items, S.w2);
+    const uint32_t n_total = small_scan<false>(S.b.cnt, n_items, S.w);
+    n_events = n_total & NE_MASK;
+    n_runs = n_total >> NE_BITS;
     if (S.flag | (n_events > SMALL_EVENTS) | (n_runs > SMALL_RUNS)) return false;
     // the outline's events (k_st_emit), transformed again as Plotter::fill
     // does: an item of at most ITEM_PTS points replays what its count kept
     const EventSink sink = small_fill_sink(S);
     for (uint32_t t = tid; t < n_items; t += SBLOCK) {
         EventSink em = sink;
-        em.e = S.b.cnt_e[t];
-        em.run = S.c.cnt_c[t];
+        const uint32_t c0 = S.b.cnt[t], c1 = t + 1 < n_items ? S.b.cnt[t + 1] : n_total;
+        em.e = c0 & NE_MASK;
+        em.run = c0 >> NE_BITS;
         em.p = 0;
-        const uint32_t e1 = t + 1 < n_items ? S.b.cnt_e[t + 1] : n_events;
-        const uint32_t r1 = t + 1 < n_items ? S.c.cnt_c[t + 1] : n_runs;
+        const uint32_t e1 = c1 & NE_MASK, r1 = c1 >> NE_BITS;
         const uint32_t n_cl = r1 - (uint32_t)em.run, n_pt = (e1 - (uint32_t)em.e) - n_cl;
         if (t + 1 == n_items) {
             em.close(true);
@@ -2131,13 +2216,11 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
         em.cap_runs = SMALL_EVENTS;
         em.ev_f = S.a.st.f;
         uint32_t n_sev = 0, n_scl = 0;
-        ok = small_flatten(S, n_ops, MODE_STROKE, T.lastpw, em, SMALL_EVENTS, n_sev, n_scl, bad) &&
+        ok = small_flatten<true>(S, n_ops, T.lastpw, em, SMALL_EVENTS, n_sev, n_scl, bad, T.leaf) &&
              small_stroker(S, T, n_sev, sp, n_events, n_runs, bad);
     } else {
         __shared__ I2 s_leaf[SMALL_LEAF * SMALL_ITEMS];
-        __shared__ uint16_t s_nleaf[SMALL_ITEMS];
-        ok = small_flatten(S, n_ops, MODE_FILL, nullptr, small_fill_sink(S), SMALL_RUNS, n_events, n_runs, bad,
-                           s_leaf, s_nleaf);
+        ok = small_flatten<false>(S, n_ops, nullptr, small_fill_sink(S), SMALL_RUNS, n_events, n_runs, bad, s_leaf);
     }
     if (!ok) {
         if (tid == 0) st->overflow = host->st.overflow = SMALL_NOT_HANDLED;
@@ -2151,16 +2234,18 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
     L.n_runs = n_runs;
     L.cap_points = SMALL_EVENTS;
     L.n_pairs = 0;
-    // 3. Fig ingest: pushed marks and their running maximum, then kept points
-    for (uint32_t e = tid; e < n_events; e += SBLOCK)
-        ingest_event(e, L, S.a.ev.meta, S.a.ev.xy, S.run_first, S.run_path, S.a.ev.last, bad);
-    __syncthreads();
-    (void)small_scan<true>(S.a.ev.last, n_events, S.w);
+    // 3. Fig ingest: the kept points in their local form (a closing walk too
+    // long for it leaves the figure to the full pipeline)
+    uint32_t long_walk = 0;
     for (uint32_t e = tid; e < n_events; e += SBLOCK) {
-        const uint32_t k = kept_event(e, L, S.a.ev.meta, S.a.ev.xy, S.run_first, S.run_close, S.a.ev.last, bad);
+        uint32_t first_of;
+        const uint32_t k = kept_event_local(e, L, S.a.ev.meta, S.a.ev.xy, S.run_close, KEPT_WALK, bad, long_walk,
+                                            first_of);
+        if (first_of != NO_IDX) S.run_first[first_of] = (int32_t)e;
         S.a.ev.kept[e] = k;
         S.a.ev.idx[e] = k;
     }
+    bad |= long_walk;
     __syncthreads();
     const uint32_t n_kept = small_scan<false>(S.a.ev.idx, n_events, S.w);
     // 4. the path's counts (no cap below 65,535 points) and compaction with
@@ -2182,7 +2267,7 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
     for (uint32_t e = tid; e < n_events; e += SBLOCK) {
         TopCand tc;
         compact_event(e, L, S.a.ev.meta, S.a.ev.xy, S.a.ev.kept, S.a.ev.idx, S.run_first, S.run_path, S.run_start,
-                      S.run_end, S.b.pts, S.c.pt_run, &S.ps, bad, &tc);
+                      S.run_end, S.b.pts, S.pt_run, &S.ps, bad, &tc);
         if (tc.path != NO_IDX && tc.key < kmin) kmin = tc.key;
     }
 #pragma unroll
@@ -2198,25 +2283,17 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
         S.ps.topkey = m;
     }
     __syncthreads();
-    // 5. Edge::new per stored point (the events' LDS now holds the edges)
-    EdgeRec E[SMALL_PER_THREAD];
+    // 5. Edge::new per stored point, to the edge list of the raster blocks
     uint32_t tmin = NO_IDX;
 #pragma unroll
     for (uint32_t j = 0; j < SMALL_PER_THREAD; ++j) {
         const uint32_t i = tid + j * SBLOCK;
-        E[j].flags = 0;
         if (i < n_kept) {
-            const EdgeEval r = edge_eval(i, L, S.c.pt_run, S.run_path, S.run_start, S.run_end, &S.path, S.b.pts,
+            const EdgeEval r = edge_eval(i, L, S.pt_run, S.run_path, S.run_start, S.run_end, &S.path, S.b.pts,
                                          &S.ps, bad);
-            E[j] = r.E;
+            edges[i] = r.E;
             if (r.top && r.top_local < tmin) tmin = r.top_local;
         }
-    }
-    __syncthreads();  // every event read is done: the edges take their LDS
-#pragma unroll
-    for (uint32_t j = 0; j < SMALL_PER_THREAD; ++j) {
-        const uint32_t i = tid + j * SBLOCK;
-        if (i < n_kept) S.a.edges[i] = E[j];
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -2232,7 +2309,7 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
         S.ps.topidx = m;
         uint32_t b2 = 0;
         const bool has = S.ps.topkey != NO_KEY && m != NO_IDX;
-        S.ps.fwd = has ? (path_forward(S.ps, L, S.b.pts, S.c.pt_run, S.run_start, S.run_end, b2) ? 1u : 0u) : 0u;
+        S.ps.fwd = has ? (path_forward(S.ps, L, S.b.pts, S.pt_run, S.run_start, S.run_end, b2) ? 1u : 0u) : 0u;
         if (b2) S.flag = 1;
     }
     __syncthreads();
@@ -2240,8 +2317,7 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
         if (tid == 0) st->overflow = host->st.overflow = SMALL_NOT_HANDLED;
         return;
     }
-    // 6. the edge list and the path's state for the raster blocks
-    for (uint32_t i = tid; i < n_kept; i += SBLOCK) edges[i] = S.a.edges[i];
+    // 6. the path's state for the raster blocks
     if (tid == 0) {
         ps[0] = S.ps;
         host_ps[0] = S.ps;

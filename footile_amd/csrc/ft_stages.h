@@ -255,13 +255,14 @@ enum : uint32_t { OPC_CURVE = 1u, OPC_LAST_CLOSE = 2u };
 // so that emitting the lane is a copy unless it has more leaves.
 constexpr uint32_t LEAF_CACHE = 8;
 
+// keep(k, q): a curve lane's point k, as it is counted.
 // sp / last_lane: a curve's lanes split its tree sp levels down, and the
 // op's last lane (which emits the path's final close) is last_lane; the
 // pipeline gives every op OP_LANES lanes.
-FT_INLINE OpCount count_op(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
-                              uint32_t s, uint32_t mode, const uint32_t *lastpw, I2 *cache = nullptr,
-                              size_t stride = 0, uint32_t sp = FLAT_SPLIT, uint32_t last_lane = OP_LANES - 1,
-                              uint32_t cap = LEAF_CACHE) {
+template <class Keep>
+FT_INLINE OpCount count_op_keep(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
+                                uint32_t s, uint32_t mode, const uint32_t *lastpw, Keep &&keep, uint32_t sp,
+                                uint32_t last_lane) {
     OpCount c = {0, 0, 0, 0, 0};
     const uint32_t p = op_path[i];
     if (p == NO_IDX) return c;
@@ -276,16 +277,7 @@ FT_INLINE OpCount count_op(const ft_path_op *ops, const uint32_t *op_path, const
     case TAG_CUBIC: {
         const WP pen = pen_before(ops, lastpw, i, P);
         const float sw = width_before(ops, lastpw, i, P);
-        I2 *const keep = mode == MODE_FILL ? cache : nullptr;
-        auto cnt = [&](WP q) {
-            const uint32_t k = c.leaves - 1;  // flatten counts a leaf before handing it over
-            if (keep && k < cap) {
-                I2 v;
-                v.x = fx_from_f32(q.x);
-                v.y = fx_from_f32(q.y);
-                keep[k * stride] = v;
-            }
-        };
+        auto cnt = [&](WP q) { keep(c.leaves - 1, q); };  // flatten counts a leaf before handing it over
         const uint32_t rc = o.tag == TAG_QUAD ? flatten_share(quad_of(o, pen, sw, P), P.tol_sq, s, c.leaves, cnt, sp)
                                               : flatten_share(cubic_of(o, pen, sw, P), P.tol_sq, s, c.leaves, cnt, sp);
         if (rc)
@@ -304,6 +296,23 @@ FT_INLINE OpCount count_op(const ft_path_op *ops, const uint32_t *op_path, const
         c.flags |= OPC_LAST_CLOSE;
     }
     return c;
+}
+
+FT_INLINE OpCount count_op(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
+                              uint32_t s, uint32_t mode, const uint32_t *lastpw, I2 *cache = nullptr,
+                              size_t stride = 0) {
+    I2 *const to = mode == MODE_FILL ? cache : nullptr;
+    return count_op_keep(
+        ops, op_path, paths, i, s, mode, lastpw,
+        [&](uint32_t k, WP q) {
+            if (to && k < LEAF_CACHE) {
+                I2 v;
+                v.x = fx_from_f32(q.x);
+                v.y = fx_from_f32(q.y);
+                to[k * stride] = v;
+            }
+        },
+        FLAT_SPLIT, OP_LANES - 1);
 }
 
 FT_HD inline unsigned long long pack_count(OpCount c) { return ((unsigned long long)c.ne << 32) | c.nc; }
@@ -384,12 +393,11 @@ struct EventSink {
 // before them).
 // `cache` / `cached`: the lane's points kept by count_op (point k at
 // cache[k * stride]) and their number (used in fill runs when it is at most
-// the cache's capacity `cap`).
+// the cache's capacity).
 FT_INLINE uint32_t emit_op(const ft_path_op *ops, const uint32_t *op_path, const PathDev *paths, uint32_t i,
                               uint32_t s, uint32_t mode, const uint32_t *lastpw, unsigned long long off,
                               EventSink em, const I2 *cache = nullptr, uint32_t cached = 0, size_t stride = 0,
-                              uint32_t sp = FLAT_SPLIT, uint32_t last_lane = OP_LANES - 1,
-                              uint32_t cap = LEAF_CACHE) {
+                              uint32_t sp = FLAT_SPLIT, uint32_t last_lane = OP_LANES - 1) {
     const uint32_t p = op_path[i];
     if (p == NO_IDX) return 0;
     const PathDev &P = paths[p];
@@ -413,7 +421,7 @@ FT_INLINE uint32_t emit_op(const ft_path_op *ops, const uint32_t *op_path, const
         break;
     case TAG_QUAD:
     case TAG_CUBIC: {
-        if (cache && mode == MODE_FILL && cached <= cap) {
+        if (cache && mode == MODE_FILL && cached <= LEAF_CACHE) {
             for (uint32_t k = 0; k < cached; ++k) em.point_fx(cache[k * stride]);
             break;
         }

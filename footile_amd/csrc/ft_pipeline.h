@@ -93,7 +93,7 @@ struct Workspace {
     unsigned long long *d_op_cnt = nullptr, *d_op_off = nullptr;
     unsigned long long *d_sub_off = nullptr;  // per (op, lane): offset within the op (+ leaf count)
     I2 *d_leaf = nullptr;                      // per (op, lane): its first LEAF_CACHE points (fill runs)
-    uint32_t *d_op_pw = nullptr, *d_op_lastpw = nullptr;
+    uint32_t *d_op_lastpw = nullptr;  // strokes: the last PenWidth op up to each op
     // events and everything sized by them
     size_t cap_events = 0;
     I2 *d_ev_xy = nullptr;
@@ -109,10 +109,9 @@ struct Workspace {
     U2 *d_pt_band = nullptr;  // per stored point: its edge's band range
     // stroker stages (MODE_STROKE), sized by cap_events
     size_t cap_stroke = 0;
-    unsigned long long *d_st_flags = nullptr, *d_st_off = nullptr;
-    uint32_t *d_st_last = nullptr;
+    unsigned long long *d_st_off = nullptr;
     F4 *d_spts = nullptr;
-    uint32_t *d_sub_start = nullptr, *d_sub_event = nullptr, *d_sub_n = nullptr, *d_sub_joined = nullptr;
+    uint32_t *d_sub_start = nullptr, *d_sub_event = nullptr;
     unsigned long long *d_it_cnt = nullptr, *d_it_off = nullptr;  // 4 cap_events + 1 items
     uint32_t join = 0;  // ft_join
     float miter = 4.0f, stroke_tol_sq = 0.09f;

@@ -120,10 +120,15 @@ __global__ __launch_bounds__(BLOCK) void k_clear(PathState *ps, unsigned long lo
 // ---------------------------------------------------------------------------
 // Stages 1-2: ops -> events (count, scan, emit).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) void k_pen_width_mark(const ft_path_op *ops, uint32_t n_ops, uint32_t *op_pw) {
-    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n_ops; i += gridDim.x * BLOCK)
-        op_pw[i] = ops[i].tag == TAG_PEN_WIDTH ? i + 1 : 0u;
-}
+// PenWidth ops as a scan source: the running maximum of i + 1 over them is the
+// last one up to each op.
+struct PenWidthSrc {
+    static constexpr uint32_t ITEMS = 4;
+    const ft_path_op *ops;
+    uint32_t bad;
+    __device__ void bind(const DevStatus *) {}
+    __device__ uint32_t value(uint64_t i, bool) { return ops[i].tag == TAG_PEN_WIDTH ? (uint32_t)i + 1 : 0u; }
+};
 
 constexpr unsigned long long SUB_CACHED = 1ull << 30, SUB_LAST_CLOSE = 1ull << 31;
 
@@ -221,22 +226,25 @@ __global__ __launch_bounds__(BLOCK) void k_emit(const ft_path_op *ops, const uin
     if (bad) raise_err(st, FT_EDEVICE);
 }
 
-// Flattening in one pass, for fill runs whose (op, lane) items fit one
+// Flattening in one pass, for runs whose (op, lane) items fit one
 // resident grid at one item per thread and are taken in op order: a block
-// takes the items of its look-back ticket, counts them (keeping each curve
-// lane's first LEAF_CACHE points in LDS), takes its prefix by look-back over
-// the tickets before it, and emits them (a copy from LDS unless a lane has
-// more leaves).  Writes each op's offset
+// takes the items of its look-back ticket, counts them (a fill keeping each
+// curve lane's first LEAF_CACHE points in LDS), takes its prefix by look-back
+// over the tickets before it, and emits them (a copy from LDS unless a lane
+// has more leaves; a stroke flattens again).  Writes each op's offset
 // (op_off, as the op scan does) and the run's event and close totals (as
 // k_emit does).
+template <bool STROKE>
 __global__ __launch_bounds__(BLOCK) void k_flatten(const ft_path_op *ops, const uint32_t *op_path,
-                                                   const PathDev *paths, uint32_t n_ops,
+                                                   const PathDev *paths, uint32_t n_ops, const uint32_t *lastpw,
                                                    unsigned long long *op_off, unsigned long long *lb,
                                                    EventSink sink, DevStatus *st, bool tickets) {
+    constexpr uint32_t mode = STROKE ? MODE_STROKE : MODE_FILL;
     __shared__ unsigned long long s_wave[BLOCK / 64];
     __shared__ unsigned long long s_prefix;
     __shared__ uint32_t s_tk;
-    __shared__ I2 s_leaf[LEAF_CACHE * BLOCK];  // point k of thread j at s_leaf[k * BLOCK + j]
+    __shared__ I2 s_leaf[STROKE ? 1 : LEAF_CACHE * BLOCK];  // point k of thread j at s_leaf[k * BLOCK + j]
+    I2 *const leaf = STROKE ? nullptr : s_leaf + threadIdx.x;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint64_t n_items = (uint64_t)n_ops * OP_LANES;
     // the block's items are those of its look-back ticket (or of its index)
@@ -249,7 +257,7 @@ __global__ __launch_bounds__(BLOCK) void k_flatten(const ft_path_op *ops, const 
     const bool live = t < n_items;
     const uint32_t i = live ? (uint32_t)(t >> FLAT_SPLIT) : 0u, s = (uint32_t)t & (OP_LANES - 1);
     OpCount c = {0, 0, 0, 0};
-    if (live) c = count_op(ops, op_path, paths, i, s, MODE_FILL, nullptr, s_leaf + threadIdx.x, BLOCK);
+    if (live) c = count_op(ops, op_path, paths, i, s, mode, lastpw, leaf, BLOCK);
     const unsigned long long v = live ? pack_count(c) : 0ull;
     uint32_t leaves = c.leaves;
 #pragma unroll
@@ -288,7 +296,7 @@ __global__ __launch_bounds__(BLOCK) void k_flatten(const ft_path_op *ops, const 
     // a lane whose events would pass the capacity writes nothing: the host
     // grows the buffers and runs again
     if (!live || (off >> 32) + c.ne > sink.cap_events || (uint32_t)off + c.nc > sink.cap_runs) return;
-    if (emit_op(ops, op_path, paths, i, s, MODE_FILL, nullptr, off, sink, s_leaf + threadIdx.x, c.leaves, BLOCK))
+    if (emit_op(ops, op_path, paths, i, s, mode, lastpw, off, sink, leaf, c.leaves, BLOCK))
         raise_err(st, FT_EDEVICE);
 }
 
@@ -762,16 +770,18 @@ struct DevMath {
     __device__ static float sin(float t) { return (float)::sin((double)t); }
 };
 
-__global__ __launch_bounds__(BLOCK) void k_st_flags(const F4 *ev, unsigned long long *flags, uint32_t *last,
-                                                    DevStatus *st) {
-    if (run_failed(st)) return;
-    const uint32_t n = st->n_events;
-    for (uint32_t e = blockIdx.x * BLOCK + threadIdx.x; e < n; e += gridDim.x * BLOCK) {
-        const StrokeFlags f = stroke_flags(e, ev);
-        flags[e] = ((unsigned long long)(f.pushed ? 1u : 0u) << 32) | (f.first ? 1u : 0u);
-        last[e] = f.is_pt ? 0u : e + 1;
+// The stored points and sub-strokes before each event (points in the high
+// word), computed inside their scan.
+struct StrokeFlagSrc {
+    static constexpr uint32_t ITEMS = 4;
+    const F4 *ev;
+    uint32_t bad;
+    __device__ void bind(const DevStatus *) {}
+    __device__ unsigned long long value(uint64_t i, bool) {
+        const StrokeFlags f = stroke_flags((uint32_t)i, ev);
+        return ((unsigned long long)(f.pushed ? 1u : 0u) << 32) | (f.first ? 1u : 0u);
     }
-}
+};
 
 __global__ __launch_bounds__(BLOCK) void k_st_compact(const F4 *ev, const unsigned long long *off, F4 *spts,
                                                       uint32_t *sub_start, uint32_t *sub_event, uint32_t cap,
@@ -793,41 +803,62 @@ __global__ __launch_bounds__(BLOCK) void k_st_compact(const F4 *ev, const unsign
     if (bad) raise_err(st, FT_EDEVICE);
 }
 
-// One thread per sub-stroke: point count, joined flag, and the number of
-// sub-strokes below the cap; then the outline's item count.
-__global__ __launch_bounds__(BLOCK) void k_st_subs(const F4 *ev, const uint32_t *last_close,
-                                                   const uint32_t *sub_start, const uint32_t *sub_event,
-                                                   uint32_t *sub_n, uint32_t *sub_joined, uint32_t cap,
-                                                   DevStatus *st) {
-    if (run_failed(st)) return;
-    const unsigned long long tot = st->st_total;
-    const uint32_t n_ev = st->n_events, total_subs = (uint32_t)tot;
-    const uint32_t n_kept = (uint32_t)(tot >> 32) < FT_MAX_POINTS ? (uint32_t)(tot >> 32) : FT_MAX_POINTS;
-    if (total_subs > cap) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) raise_err(st, FT_EDEVICE);
-        return;
-    }
-    for (uint32_t s = blockIdx.x * BLOCK + threadIdx.x; s < total_subs; s += gridDim.x * BLOCK) {
-        const uint32_t a = sub_start[s];
-        const bool kept = a < FT_MAX_POINTS;
-        const bool more = s + 1 < total_subs;
-        const uint32_t a1 = more ? sub_start[s + 1] : n_kept;
-        const bool last_kept = kept & (!more | (a1 >= FT_MAX_POINTS));
-        const uint32_t end = a1 < n_kept ? a1 : n_kept;
-        // closes up to the next sub-stroke's first point (or the end) apply to this one
-        const uint32_t range_end = (last_kept | !more) ? n_ev : sub_event[s + 1];
-        const uint32_t lc = last_close[range_end ? range_end - 1 : 0];
-        const bool has_close = (range_end > 0) & (lc > 0) & (lc - 1 >= sub_event[s]) & (lc - 1 < n_ev);
-        const F4 ce = ev[has_close ? lc - 1 : 0];
-        const bool joined = has_close & (ce.w == 2.0f);
-        sub_n[s] = kept & (end > a) ? end - a : 0u;
-        sub_joined[s] = joined ? 1u : 0u;
-        if (last_kept) {
-            st->st_subs = s + 1;
-            st->st_items = 2u * (n_kept + s + 1) + 1u;
+// The sub-strokes and outline items of a run, from the totals of the stored
+// points' scan and the compacted tables: what a pass over the sub-strokes and
+// a running maximum of the closes would leave behind, read where it is needed
+// (two dispatches and 9 us less of a 166 us stroke of 3,000 lines).
+struct StrokeRun {
+    const F4 *ev;
+    const uint32_t *sub_start, *sub_event;
+    uint32_t n_ev, n_subs, n_pts;  // events; sub-strokes; points stored (at most FT_MAX_POINTS)
+    uint32_t subs, items;          // sub-strokes below the cap; outline items
+    bool capped;
+};
+// tot: stored points << 32 | sub-strokes (the scan's total).
+__device__ inline StrokeRun stroke_run(unsigned long long tot, uint32_t n_ev, const F4 *ev, const uint32_t *sub_start,
+                                       const uint32_t *sub_event) {
+    const uint32_t n = (uint32_t)(tot >> 32);
+    StrokeRun r;
+    r.ev = ev;
+    r.sub_start = sub_start;
+    r.sub_event = sub_event;
+    r.n_ev = n_ev;
+    r.n_subs = (uint32_t)tot;
+    r.capped = n > FT_MAX_POINTS;
+    r.n_pts = r.capped ? FT_MAX_POINTS : n;
+    r.subs = r.n_subs;
+    if (r.capped) {  // the sub-strokes whose first point is stored
+        uint32_t lo = 0, hi = r.n_subs;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (sub_start[mid] < FT_MAX_POINTS)
+                lo = mid + 1;
+            else
+                hi = mid;
         }
+        r.subs = lo;
     }
-    if (total_subs == 0 && blockIdx.x == 0 && threadIdx.x == 0) st->st_items = 1u;  // the final close only
+    r.items = r.subs ? 2u * (r.n_pts + r.subs) + 1u : 1u;
+    return r;
+}
+// Sub-stroke s < r.subs.  It is joined if the last close up to the next
+// sub-stroke's first point, or up to the end of the events for the last one
+// stored, joins.  Before a first point that close is the event before it.  At
+// the end it is the last event or, if that is a point, the one before the last
+// run's first point.
+__device__ inline StrokeSub stroke_sub(const StrokeRun &r, uint32_t s) {
+    const bool more = s + 1 < r.subs;
+    const uint32_t s1 = more ? s + 1 : r.n_subs - 1;
+    const uint32_t a = r.sub_start[s], a1 = r.sub_start[s1], e = r.sub_event[s], e1 = r.sub_event[s1];
+    const bool ends_in_close = r.ev[r.n_ev - 1].w != 0.0f;
+    const uint32_t lc = more ? e1 : (ends_in_close ? r.n_ev : e1);  // the close, plus one
+    const bool has_close = (lc > 0) & (lc - 1 >= e) & (lc - 1 < r.n_ev);
+    const uint32_t end = more ? a1 : r.n_pts;
+    StrokeSub sub;
+    sub.start = a;
+    sub.n = end > a ? end - a : 0u;
+    sub.joined = has_close & (r.ev[has_close ? lc - 1 : 0].w == 2.0f);
+    return sub;
 }
 
 __device__ inline uint32_t st_item_sub(uint32_t t, const uint32_t *sub_start, uint32_t n_subs) {
@@ -847,39 +878,167 @@ struct StrokeParams {
     float miter, tol_sq;
 };
 
-__global__ __launch_bounds__(BLOCK) void k_st_count(const F4 *spts, const uint32_t *sub_start, const uint32_t *sub_n,
-                                                    const uint32_t *sub_joined, StrokeParams sp,
+// Item t < r.items - 1 of the outline through line and close.
+template <class Line, class Close, class Ends = NoEnds>
+__device__ __forceinline__ uint32_t outline_item(const StrokeRun &r, uint32_t t, const F4 *spts, const StrokeParams &sp,
+                                                 Line &&line, Close &&close, Ends ends = Ends()) {
+    const uint32_t si = st_item_sub(t, r.sub_start, r.subs);
+    const StrokeSub sub = stroke_sub(r, si);
+    const uint32_t local = t - 2u * (sub.start + si);
+    const bool fwd = local <= sub.n;
+    const uint32_t k = fwd ? local : local - (sub.n + 1);
+    if (!sub.n) return 0;
+    return stroke_item<DevMath>(sub, fwd, k, spts, sp.join, sp.miter, sp.tol_sq, line, close, ends);
+}
+
+// The outline in one pass, for strokes whose items fit SCAN_GRID_MAX blocks: a
+// block takes the items of its look-back ticket, builds them (keeping an
+// item's first ITEM_CACHE transformed points in LDS), takes its prefix, and
+// copies the points out (an item with more is built again).  What bounds it is
+// one round join's walk: a chain of square roots and divisions per arc point.
+// Walking it from the arc's ends for every point, once to count and once to
+// emit with a scan between, took 14 + 5 + 18 us of a 3,000-line stroke with
+// round joins; this takes 16.
+//
+// Tickets go to as many blocks as there are items for, whatever the grid.  A
+// block that finds the run failed has a part in the look-back all the same: an
+// error may be this kernel's own, and later blocks wait for its count.
+constexpr uint32_t ITEM_CACHE = 10;
+constexpr uint32_t ARC_ENDS = 5;  // levels kept, 32 points of an arc
+struct LdsEnds {
+    static constexpr uint32_t LEVELS = ARC_ENDS;
+    SV2 *at;  // the thread's column
+    __device__ void put(uint32_t lv, SV2 v) const { at[lv * BLOCK] = v; }
+    __device__ SV2 get(uint32_t lv) const { return at[lv * BLOCK]; }
+};
+__global__ __launch_bounds__(BLOCK) void k_st_outline(const F4 *spts, const F4 *ev, const uint32_t *sub_start,
+                                                      const uint32_t *sub_event, uint32_t cap, StrokeParams sp,
+                                                      const PathDev *paths, unsigned long long *lb, EventSink sink,
+                                                      DevStatus *st) {
+    __shared__ SV2 s_pt[ITEM_CACHE * BLOCK];  // point k of thread j at s_pt[k * BLOCK + j]
+    __shared__ SV2 s_ends[ARC_ENDS * BLOCK];
+    __shared__ unsigned long long s_wave[BLOCK / 64];
+    __shared__ unsigned long long s_prefix;
+    __shared__ uint32_t s_tk;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const bool fits = (uint32_t)st->st_total <= cap;  // else more sub-strokes than the table holds
+    const StrokeRun r = stroke_run(fits ? st->st_total : 0ull, (uint32_t)(st->op_total >> 32), ev, sub_start, sub_event);
+    if ((uint64_t)blockIdx.x * BLOCK >= r.items) return;  // the tickets are the other blocks'
+    if (tid == 0) {
+        s_tk = lookback_ticket(lb);
+        if (!fits) raise_err(st, FT_EDEVICE);
+    }
+    __syncthreads();
+    const uint32_t b = s_tk, t = b * BLOCK + tid;
+    const PathDev &P = paths[0];
+    uint32_t ne = 0, nc = 0, err = 0;
+    if (fits && !run_failed(st)) {
+        if (t + 1 == r.items) {
+            ne = nc = 1;  // Plotter::fill's final close
+        } else if (t < r.items) {
+            // (an item's points all come before its close, at most one)
+            err = outline_item(
+                r, t, spts, sp,
+                [&](SV2 q) {
+                    if (ne < ITEM_CACHE) {
+                        const WP w = xform(P, q.x, q.y, 0.0f);
+                        SV2 v;
+                        v.x = w.x;
+                        v.y = w.y;
+                        s_pt[ne * BLOCK + tid] = v;
+                    }
+                    ++ne;
+                },
+                [&]() {
+                    ++ne;
+                    ++nc;
+                },
+                LdsEnds{s_ends + tid});
+        }
+    }
+    if (err) raise_err(st, err);
+    const unsigned long long v = ((unsigned long long)ne << 32) | nc;
+    const unsigned long long winc = wave_incl_t<unsigned long long, false>(v);
+    if (lane == 63) s_wave[wid] = winc;
+    __syncthreads();
+    unsigned long long wpre = 0, btot = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < BLOCK / 64; ++w) {
+        wpre += w < wid ? s_wave[w] : 0ull;
+        btot += s_wave[w];
+    }
+    if (wid == 0) {
+        const unsigned long long prefix = lookback_prefix<unsigned long long, false>(lb, b, btot, st);
+        if (lane == 0) s_prefix = prefix;
+    }
+    __syncthreads();
+    const unsigned long long off = s_prefix + wpre + winc - v;
+    if (t + 1 == r.items) {  // the run's totals
+        const unsigned long long tot = off + v;
+        const uint32_t n_events = (uint32_t)(tot >> 32);
+        st->stroke_total = tot;
+        st->n_events = n_events;
+        st->n_closes = (uint32_t)tot;
+        if (n_events > sink.cap_events) {
+            atomicOr(&st->overflow, 1u);
+            st->need_events = n_events;
+        }
+    }
+    // (past the capacity nothing is written: the host grows it and runs again)
+    if ((off >> 32) + ne > sink.cap_events || (uint32_t)off + nc > sink.cap_runs) return;
+    EventSink em = sink;
+    em.e = off >> 32;
+    em.run = (uint32_t)off;
+    em.p = 0;
+    const uint32_t n_pt = ne - nc;
+    if (n_pt <= ITEM_CACHE) {
+        for (uint32_t k = 0; k < n_pt; ++k) {
+            WP w;
+            w.x = s_pt[k * BLOCK + tid].x;
+            w.y = s_pt[k * BLOCK + tid].y;
+            w.w = 0.0f;
+            em.point(w);
+        }
+        if (nc) em.close(true);
+    } else {
+        (void)outline_item(
+            r, t, spts, sp, [&](SV2 q) { em.point(xform(P, q.x, q.y, 0.0f)); }, [&]() { em.close(true); },
+            LdsEnds{s_ends + tid});
+    }
+    if (em.bad) raise_err(st, FT_EDEVICE);
+}
+
+// The general form, for longer strokes: items counted, scanned and built again.
+__global__ __launch_bounds__(BLOCK) void k_st_count(const F4 *spts, const F4 *ev, const uint32_t *sub_start,
+                                                    const uint32_t *sub_event, uint32_t cap, StrokeParams sp,
                                                     unsigned long long *cnt, DevStatus *st) {
     if (run_failed(st)) return;
-    const uint32_t n_items = st->st_items, n_subs = st->st_subs;
-    for (uint32_t t = blockIdx.x * BLOCK + threadIdx.x; t < n_items; t += gridDim.x * BLOCK) {
+    if ((uint32_t)st->st_total > cap) {  // more sub-strokes than the table holds
+        if (blockIdx.x == 0 && threadIdx.x == 0) raise_err(st, FT_EDEVICE);
+        return;
+    }
+    const StrokeRun r = stroke_run(st->st_total, st->n_events, ev, sub_start, sub_event);
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->st_items = r.items;
+    for (uint32_t t = blockIdx.x * BLOCK + threadIdx.x; t < r.items; t += gridDim.x * BLOCK) {
         uint32_t ne = 0, nc = 0, err = 0;
-        if (t + 1 == n_items) {
+        if (t + 1 == r.items)
             ne = nc = 1;  // Plotter::fill's final close
-        } else if (n_subs) {
-            const uint32_t si = st_item_sub(t, sub_start, n_subs);
-            StrokeSub sub;
-            sub.start = sub_start[si];
-            sub.n = sub_n[si];
-            sub.joined = sub_joined[si] != 0;
-            const uint32_t local = t - 2u * (sub.start + si);
-            const bool fwd = local <= sub.n;
-            const uint32_t k = fwd ? local : local - (sub.n + 1);
-            if (sub.n)
-                err = stroke_item<DevMath>(
-                    sub, fwd, k, spts, sp.join, sp.miter, sp.tol_sq, [&](SV2) { ++ne; },
-                    [&]() {
-                        ++ne;
-                        ++nc;
-                    });
-        }
+        else
+            err = outline_item(
+                r, t, spts, sp, [&](SV2) { ++ne; },
+                [&]() {
+                    ++ne;
+                    ++nc;
+                });
         if (err) raise_err(st, err);
         cnt[t] = ((unsigned long long)ne << 32) | nc;
     }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_st_emit(const F4 *spts, const uint32_t *sub_start, const uint32_t *sub_n,
-                                                   const uint32_t *sub_joined, StrokeParams sp,
+// (The flattened events' count is read from op_total: n_events becomes the
+// outline's here.)
+__global__ __launch_bounds__(BLOCK) void k_st_emit(const F4 *spts, const F4 *ev, const uint32_t *sub_start,
+                                                   const uint32_t *sub_event, StrokeParams sp,
                                                    const unsigned long long *off, const PathDev *paths,
                                                    EventSink sink, DevStatus *st) {
     if (run_failed(st)) return;
@@ -894,30 +1053,19 @@ __global__ __launch_bounds__(BLOCK) void k_st_emit(const F4 *spts, const uint32_
         }
     }
     if (n_events > sink.cap_events) return;
-    const uint32_t n_items = st->st_items, n_subs = st->st_subs;
+    const StrokeRun r = stroke_run(st->st_total, (uint32_t)(st->op_total >> 32), ev, sub_start, sub_event);
     const PathDev &P = paths[0];
     uint32_t bad = 0;
-    for (uint32_t t = blockIdx.x * BLOCK + threadIdx.x; t < n_items; t += gridDim.x * BLOCK) {
+    for (uint32_t t = blockIdx.x * BLOCK + threadIdx.x; t < r.items; t += gridDim.x * BLOCK) {
         EventSink em = sink;
         em.e = off[t] >> 32;
         em.run = (uint32_t)off[t];
         em.p = 0;
-        if (t + 1 == n_items) {
+        if (t + 1 == r.items)
             em.close(true);
-        } else if (n_subs) {
-            const uint32_t si = st_item_sub(t, sub_start, n_subs);
-            StrokeSub sub;
-            sub.start = sub_start[si];
-            sub.n = sub_n[si];
-            sub.joined = sub_joined[si] != 0;
-            const uint32_t local = t - 2u * (sub.start + si);
-            const bool fwd = local <= sub.n;
-            const uint32_t k = fwd ? local : local - (sub.n + 1);
-            if (sub.n)
-                stroke_item<DevMath>(
-                    sub, fwd, k, spts, sp.join, sp.miter, sp.tol_sq,
-                    [&](SV2 q) { em.point(xform(P, q.x, q.y, 0.0f)); }, [&]() { em.close(true); });
-        }
+        else
+            (void)outline_item(
+                r, t, spts, sp, [&](SV2 q) { em.point(xform(P, q.x, q.y, 0.0f)); }, [&]() { em.close(true); });
         bad |= em.bad;
     }
     if (bad) raise_err(st, FT_EDEVICE);
@@ -1776,9 +1924,8 @@ struct SmallLds {
             I2 xy[SMALL_EVENTS];
             uint32_t meta[SMALL_EVENTS], kept[SMALL_EVENTS], idx[SMALL_EVENTS];
         } ev;
-        struct {  // a stroke's flattened (x, y, width, kind) events and its last close so far
+        struct {  // a stroke's flattened (x, y, width, kind) events
             F4 f[SMALL_EVENTS];
-            uint32_t last[SMALL_EVENTS];
         } st;
     } a;
     union {
@@ -2051,17 +2198,15 @@ __device__ __forceinline__ bool small_flatten(SmallLds &S, uint32_t n_ops, const
 __device__ __forceinline__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, uint32_t n_sev, StrokeParams sp, uint32_t &n_events,
                               uint32_t &n_runs, uint32_t &bad) {
     const uint32_t tid = threadIdx.x;
-    // flags (k_st_flags): pushed -> stored point index, first point of a run
+    // flags (stroke_flags): pushed -> stored point index, first point of a run
     // -> sub-stroke index, closes -> the last close so far
     for (uint32_t e = tid; e < n_sev; e += SBLOCK) {
         const StrokeFlags f = stroke_flags(e, S.a.st.f);
         S.b.cnt[e] = (f.pushed ? 1u : 0u) | (f.first ? 1u << 16 : 0u);
-        S.a.st.last[e] = f.is_pt ? 0u : e + 1;
     }
     __syncthreads();
     const uint32_t n_both = small_scan<false>(S.b.cnt, n_sev, S.w);  // both at most SMALL_EVENTS
     const uint32_t n_pts = n_both & 0xFFFFu, n_subs = n_both >> 16;
-    (void)small_scan<true>(S.a.st.last, n_sev, S.w2);
     if (n_subs > SMALL_RUNS) return false;
     // compaction (k_st_compact)
     for (uint32_t e = tid; e < n_sev; e += SBLOCK) {
@@ -2074,17 +2219,17 @@ __device__ __forceinline__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, ui
         }
     }
     __syncthreads();
-    // sub-strokes (k_st_subs; every point is kept)
+    // sub-strokes (as stroke_sub; every point is kept)
     for (uint32_t s = tid; s < n_subs; s += SBLOCK) {
         const uint32_t a = T.sub_start[s];
         const bool more = s + 1 < n_subs;
         const uint32_t end = more ? T.sub_start[s + 1] : n_pts;
         const uint32_t range_end = more ? T.sub_event[s + 1] : n_sev;
-        const uint32_t lc = S.a.st.last[range_end ? range_end - 1 : 0];
-        const bool has_close = (range_end > 0) & (lc > 0) & (lc - 1 >= T.sub_event[s]) & (lc - 1 < n_sev);
-        const F4 ce = S.a.st.f[has_close ? lc - 1 : 0];
+        // the last close of the sub-stroke, if any, is its range's last event
+        // (see stroke_sub)
+        const F4 ce = S.a.st.f[range_end ? range_end - 1 : 0];
         T.sub_n[s] = end > a ? end - a : 0u;
-        T.sub_joined[s] = (has_close & (ce.w == 2.0f)) ? 1u : 0u;
+        T.sub_joined[s] = ce.w == 2.0f ? 1u : 0u;
     }
     const uint32_t n_items = n_subs ? 2u * (n_pts + n_subs) + 1u : 1u;
     if (n_items > SMALL_EVENTS) return false;
@@ -2444,7 +2589,10 @@ static ft_status dev_alloc(Workspace &ws, T *&ptr, size_t n) {
 // its occupancy per compute unit, at most four, times the CUs.
 static ft_status flatten_resident(Workspace &ws) {
     int per_cu = 0, cus = 0;
-    FT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_flatten, BLOCK, 0));
+    int stroke = 0;
+    FT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_flatten<false>, BLOCK, 0));
+    FT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&stroke, k_flatten<true>, BLOCK, 0));
+    per_cu = std::min(per_cu, stroke);
     FT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ws.device));
     const uint32_t g = (uint32_t)((cus > 0 ? cus : 0) * (per_cu < 4 ? (per_cu > 0 ? per_cu : 0) : 4));
     ws.flat_resident = g < SCAN_GRID_MAX ? g : SCAN_GRID_MAX;
@@ -2514,10 +2662,9 @@ void ws_free(Workspace &ws) {
     }
     // (the layout's upload pointers point into d_lay, the status and path
     // states into d_sp)
-    void *bufs[] = {ws.d_lay, ws.d_op_cnt, ws.d_op_off, ws.d_sub_off, ws.d_leaf, ws.d_op_pw, ws.d_op_lastpw,
+    void *bufs[] = {ws.d_lay, ws.d_op_cnt, ws.d_op_off, ws.d_sub_off, ws.d_leaf, ws.d_op_lastpw,
                     ws.d_ev_xy, ws.d_ev_f, ws.d_ev_meta, ws.d_ev_kept, ws.d_ev_idx, ws.d_ev_last,
-                    ws.d_st_flags, ws.d_st_off, ws.d_st_last, ws.d_spts, ws.d_sub_start, ws.d_sub_event, ws.d_sub_n,
-                    ws.d_sub_joined, ws.d_it_cnt, ws.d_it_off,
+                    ws.d_st_off, ws.d_spts, ws.d_sub_start, ws.d_sub_event, ws.d_it_cnt, ws.d_it_off,
                     ws.d_run_first, ws.d_run_close, ws.d_run_path, ws.d_run_start, ws.d_run_end, ws.d_pts,
                     ws.d_pt_run, ws.d_edges, ws.d_pt_band, ws.d_band_cnt, ws.d_band_off, ws.d_band_cur, ws.d_band_list,
                     ws.d_scan_state, ws.d_top_rep, ws.d_stats, ws.d_sp};
@@ -2595,14 +2742,12 @@ static ft_status ensure_event_capacity(Workspace &ws, size_t need) {
 }
 
 static ft_status ensure_stroke_capacity(Workspace &ws) {
-    if (ws.cap_stroke == ws.cap_events && ws.d_st_flags) return FT_OK;
+    if (ws.cap_stroke == ws.cap_events && ws.d_st_off) return FT_OK;
     const size_t cap = ws.cap_events, items = 4 * cap + 1;
     ft_status s;
-    if ((s = dev_alloc(ws, ws.d_st_flags, cap)) || (s = dev_alloc(ws, ws.d_st_off, cap)) ||
-        (s = dev_alloc(ws, ws.d_st_last, cap)) || (s = dev_alloc(ws, ws.d_spts, cap)) || (s = dev_alloc(ws, ws.d_sub_start, cap)) ||
-        (s = dev_alloc(ws, ws.d_sub_event, cap)) || (s = dev_alloc(ws, ws.d_sub_n, cap)) ||
-        (s = dev_alloc(ws, ws.d_sub_joined, cap)) || (s = dev_alloc(ws, ws.d_it_cnt, items)) ||
-        (s = dev_alloc(ws, ws.d_it_off, items))) {
+    if ((s = dev_alloc(ws, ws.d_st_off, cap)) || (s = dev_alloc(ws, ws.d_spts, cap)) ||
+        (s = dev_alloc(ws, ws.d_sub_start, cap)) || (s = dev_alloc(ws, ws.d_sub_event, cap)) ||
+        (s = dev_alloc(ws, ws.d_it_cnt, items)) || (s = dev_alloc(ws, ws.d_it_off, items))) {
         ws.cap_stroke = 0;
         return s;
     }
@@ -2650,11 +2795,10 @@ static void arena_rewind(Workspace &ws) {
     void **ptrs[] = {(void **)&ws.d_lay, (void **)&ws.d_ops, (void **)&ws.d_op_path, (void **)&ws.d_op_order,
                      (void **)&ws.d_paths,
                      (void **)&ws.d_band_path, (void **)&ws.d_op_cnt, (void **)&ws.d_op_off, (void **)&ws.d_sub_off,
-                     (void **)&ws.d_leaf, (void **)&ws.d_op_pw, (void **)&ws.d_op_lastpw, (void **)&ws.d_ev_xy,
+                     (void **)&ws.d_leaf, (void **)&ws.d_op_lastpw, (void **)&ws.d_ev_xy,
                      (void **)&ws.d_ev_f, (void **)&ws.d_ev_meta, (void **)&ws.d_ev_kept, (void **)&ws.d_ev_idx,
-                     (void **)&ws.d_ev_last, (void **)&ws.d_st_flags, (void **)&ws.d_st_off, (void **)&ws.d_st_last,
-                     (void **)&ws.d_spts, (void **)&ws.d_sub_start, (void **)&ws.d_sub_event, (void **)&ws.d_sub_n,
-                     (void **)&ws.d_sub_joined, (void **)&ws.d_it_cnt, (void **)&ws.d_it_off,
+                     (void **)&ws.d_ev_last, (void **)&ws.d_st_off, (void **)&ws.d_spts, (void **)&ws.d_sub_start,
+                     (void **)&ws.d_sub_event, (void **)&ws.d_it_cnt, (void **)&ws.d_it_off,
                      (void **)&ws.d_run_first, (void **)&ws.d_run_close, (void **)&ws.d_run_path,
                      (void **)&ws.d_rblock, (void **)&ws.d_run_start, (void **)&ws.d_run_end, (void **)&ws.d_pts,
                      (void **)&ws.d_pt_run, (void **)&ws.d_edges, (void **)&ws.d_pt_band, (void **)&ws.d_band_cnt,
@@ -2851,7 +2995,7 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
     if (n_ops > ws.cap_ops || !ws.d_op_cnt) {  // per-op scratch
         ws.cap_ops = n_ops ? n_ops : 1;
         if ((s = dev_alloc(ws, ws.d_op_cnt, ws.cap_ops)) ||
-            (s = dev_alloc(ws, ws.d_op_off, ws.cap_ops)) || (s = dev_alloc(ws, ws.d_op_pw, ws.cap_ops)) ||
+            (s = dev_alloc(ws, ws.d_op_off, ws.cap_ops)) ||
             (s = dev_alloc(ws, ws.d_sub_off, ws.cap_ops * OP_LANES)) ||
             (s = dev_alloc(ws, ws.d_leaf, ws.cap_ops * OP_LANES * LEAF_CACHE)) ||
             (s = dev_alloc(ws, ws.d_op_lastpw, ws.cap_ops))) {
@@ -3110,9 +3254,9 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
                           keep_failed ? 1u : 0u, host_err);
     const uint32_t *lastpw = nullptr;
     if (mode != MODE_FILL && n_ops) {
-        k_pen_width_mark<<<grid_for(n_ops), BLOCK, 0, s>>>(ws.d_ops, n_ops, ws.d_op_pw);
-        scan_launch<uint32_t, true>(s, ws.scan_resident, ws.d_op_pw, ws.d_op_lastpw, nullptr, n_ops, n_ops,
-                                    lb + 10 * tiles, nullptr, st, false, false, ws.tickets);
+        const PenWidthSrc pw{ws.d_ops, 0u};
+        scan_launch_src<uint32_t, true>(s, ws.scan_resident, pw, ws.d_op_lastpw, nullptr, n_ops, n_ops,
+                                        lb + 10 * tiles, nullptr, st, false, false, ws.tickets);
         lastpw = ws.d_op_lastpw;
     }
     if (n_ops) {
@@ -3131,9 +3275,10 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
         em.run_start = ws.d_run_start;
         em.run_end = ws.d_run_end;
         const size_t n_items = (size_t)n_ops * OP_LANES;
-        if (mode == MODE_FILL && !order && flatten_in_one_pass(ws, n_ops)) {
-            k_flatten<<<(uint32_t)((n_items + BLOCK - 1) / BLOCK), BLOCK, 0, s>>>(
-                ws.d_ops, ws.d_op_path, ws.d_paths, n_ops, ws.d_op_off, lb, em, st, ws.tickets);
+        if ((mode == MODE_FILL || mode == MODE_STROKE) && !order && flatten_in_one_pass(ws, n_ops)) {
+            (mode == MODE_STROKE ? k_flatten<true> : k_flatten<false>)<<<(uint32_t)((n_items + BLOCK - 1) / BLOCK), BLOCK,
+                                                                        0, s>>>(
+                ws.d_ops, ws.d_op_path, ws.d_paths, n_ops, lastpw, ws.d_op_off, lb, em, st, ws.tickets);
         } else {
             k_count<<<grid_for(n_items), BLOCK, 0, s>>>(ws.d_ops, ws.d_op_path, ws.d_paths, n_ops, mode, lastpw, order,
                                                         ws.d_op_cnt, ws.d_sub_off, leaf, ws.cap_ops * OP_LANES, st);
@@ -3151,19 +3296,10 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
         sp.join = ws.join;
         sp.miter = ws.miter;
         sp.tol_sq = ws.n_paths ? ws.stroke_tol_sq : 0.0f;
-        k_st_flags<<<ge, BLOCK, 0, s>>>(ws.d_ev_f, ws.d_st_flags, ws.d_st_last, st);
-        scan_launch<unsigned long long, false>(s, ws.scan_resident, ws.d_st_flags, ws.d_st_off, &st->n_events, 0, cap,
-                                               lb + 12 * tiles, &st->st_total, st, true, false, ws.tickets);
-        scan_launch<uint32_t, true>(s, ws.scan_resident, ws.d_st_last, ws.d_st_last, &st->n_events, 0, cap,
-                                    lb + 14 * tiles, nullptr, st, true, true, ws.tickets);
+        const StrokeFlagSrc flags{ws.d_ev_f, 0u};
+        scan_launch_src<unsigned long long, false>(s, ws.scan_resident, flags, ws.d_st_off, &st->n_events, 0, cap,
+                                                   lb + 12 * tiles, &st->st_total, st, true, false, ws.tickets);
         k_st_compact<<<ge, BLOCK, 0, s>>>(ws.d_ev_f, ws.d_st_off, ws.d_spts, ws.d_sub_start, ws.d_sub_event, cap, st);
-        k_st_subs<<<ge, BLOCK, 0, s>>>(ws.d_ev_f, ws.d_st_last, ws.d_sub_start, ws.d_sub_event, ws.d_sub_n,
-                                       ws.d_sub_joined, cap, st);
-        k_st_count<<<grid_for(cap_items), BLOCK, 0, s>>>(ws.d_spts, ws.d_sub_start, ws.d_sub_n, ws.d_sub_joined, sp,
-                                                         ws.d_it_cnt, st);
-        scan_launch<unsigned long long, false>(s, ws.scan_resident, ws.d_it_cnt, ws.d_it_off, &st->st_items, 0,
-                                               (uint32_t)cap_items, lb + 16 * tiles, &st->stroke_total, st, true,
-                                               false, ws.tickets);
         EventSink em{};
         em.cap_events = ws.cap_events;
         em.cap_runs = cap;
@@ -3176,8 +3312,20 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
         em.run_path = ws.d_run_path;
         em.run_start = ws.d_run_start;
         em.run_end = ws.d_run_end;
-        k_st_emit<<<grid_for(cap_items), BLOCK, 0, s>>>(ws.d_spts, ws.d_sub_start, ws.d_sub_n, ws.d_sub_joined, sp,
-                                                        ws.d_it_off, ws.d_paths, em, st);
+        const size_t outline_blocks = (cap_items + BLOCK - 1) / BLOCK;
+        if (outline_blocks <= SCAN_GRID_MAX) {
+            k_st_outline<<<(uint32_t)outline_blocks, BLOCK, 0, s>>>(ws.d_spts, ws.d_ev_f, ws.d_sub_start,
+                                                                    ws.d_sub_event, cap, sp, ws.d_paths,
+                                                                    lb + 16 * tiles, em, st);
+        } else {
+            k_st_count<<<grid_for(cap_items), BLOCK, 0, s>>>(ws.d_spts, ws.d_ev_f, ws.d_sub_start, ws.d_sub_event,
+                                                             cap, sp, ws.d_it_cnt, st);
+            scan_launch<unsigned long long, false>(s, ws.scan_resident, ws.d_it_cnt, ws.d_it_off, &st->st_items, 0,
+                                                   (uint32_t)cap_items, lb + 16 * tiles, &st->stroke_total, st, true,
+                                                   false, ws.tickets);
+            k_st_emit<<<grid_for(cap_items), BLOCK, 0, s>>>(ws.d_spts, ws.d_ev_f, ws.d_sub_start, ws.d_sub_event, sp,
+                                                            ws.d_it_off, ws.d_paths, em, st);
+        }
     }
     if (mode == MODE_FILL || mode == MODE_STROKE) {
         const uint32_t ge = grid_for(ws.cap_events);

@@ -140,8 +140,16 @@ FT_HD inline Offset stroke_offset(F4 p0, F4 p1) {
 // order: leaf = the node's end point; a node (a, b) splits at the point c on
 // the circle of radius width/2 around p.  Returns 0, or FT_ERANGE past depth
 // FT_FLATTEN_MAX_DEPTH or FT_FLATTEN_MAX_LEAVES leaves.
-template <class Emit>
-FT_HD uint32_t stroke_arc(F4 p, SV2 a0, SV2 b0, float tol_sq, uint32_t &leaves, Emit &&emit) {
+// A leaf's successor starts where the leaf ends and ends where its ancestor's
+// right half does: `ends` keeps that end for the first Ends::LEVELS levels;
+// below them (or with NoEnds) the walk derives the node from the root again.
+struct NoEnds {
+    static constexpr uint32_t LEVELS = 0;
+    FT_HD void put(uint32_t, SV2) const {}
+    FT_HD SV2 get(uint32_t) const { return SV2{0.0f, 0.0f}; }
+};
+template <class Ends, class Emit>
+FT_HD uint32_t stroke_arc(F4 p, SV2 a0, SV2 b0, float tol_sq, uint32_t &leaves, Emit &&emit, Ends ends) {
     const float h = p.z / 2.0f;
     SV2 a = a0, b = b0;
     uint32_t depth = 0, bits = 0;
@@ -165,6 +173,11 @@ FT_HD uint32_t stroke_arc(F4 p, SV2 a0, SV2 b0, float tol_sq, uint32_t &leaves, 
             }
             if (depth == 0) return 0;
             bits |= 1u;
+            if (depth <= Ends::LEVELS) {
+                a = b;
+                b = ends.get(depth - 1);
+                continue;
+            }
             a = a0;
             b = b0;
             for (int lv = (int)depth - 1; lv >= 0; --lv) {
@@ -176,6 +189,7 @@ FT_HD uint32_t stroke_arc(F4 p, SV2 a0, SV2 b0, float tol_sq, uint32_t &leaves, 
             }
         } else {
             if (depth >= FT_FLATTEN_MAX_DEPTH) return FT_ERANGE;
+            if (depth < Ends::LEVELS) ends.put(depth, b);
             b = c;
             bits <<= 1;
             ++depth;
@@ -185,9 +199,9 @@ FT_HD uint32_t stroke_arc(F4 p, SV2 a0, SV2 b0, float tol_sq, uint32_t &leaves, 
 
 // Ops of Stroke::join (stroker.rs:330-396) at p between the offset segments
 // (a0, a1) and (b0, b1), through `line(x, y)`.
-template <class M, class Line>
+template <class M, class Line, class Ends = NoEnds>
 FT_HD uint32_t stroke_join(uint32_t join, float miter, float tol_sq, F4 p, SV2 a0, SV2 a1, SV2 b0, SV2 b1,
-                           uint32_t &leaves, Line &&line) {
+                           uint32_t &leaves, Line &&line, Ends ends = Ends()) {
     if (join == FT_JOIN_MITER) {
         if (miter > 0.0f) {
             const float sm_min = 1.0f / miter;
@@ -217,16 +231,16 @@ FT_HD uint32_t stroke_join(uint32_t join, float miter, float tol_sq, F4 p, SV2 a
         return 0;
     }
     line(a1);
-    return stroke_arc(p, a1, b0, tol_sq, leaves, line);
+    return stroke_arc(p, a1, b0, tol_sq, leaves, line, ends);
 }
 
 // Item t of the outline: side `fwd` of sub-stroke s, segment k (k <= s.n).
 // Calls line(SV2) / close() in output order; returns 0 or FT_ERANGE.
 // Items are laid out per sub-stroke: (n + 1) forward slots, then (n + 1)
 // reverse slots, so item order is output order.
-template <class M, class Line, class Close>
+template <class M, class Line, class Close, class Ends = NoEnds>
 FT_HD uint32_t stroke_item(const StrokeSub &s, bool fwd, uint32_t k, const F4 *pts, uint32_t join, float miter,
-                           float tol_sq, Line &&line, Close &&close) {
+                           float tol_sq, Line &&line, Close &&close, Ends ends = Ends()) {
     const uint32_t len = stroke_sub_len(s);
     if (k >= len) return 0;
     const uint32_t v0 = stroke_vertex(s, fwd, k), v1 = stroke_vertex(s, fwd, k + 1);
@@ -238,7 +252,7 @@ FT_HD uint32_t stroke_item(const StrokeSub &s, bool fwd, uint32_t k, const F4 *p
     } else {
         const uint32_t u0 = stroke_vertex(s, fwd, k - 1);
         const Offset prev = stroke_offset(pts[u0], p0);
-        err = stroke_join<M>(join, miter, tol_sq, p0, prev.r0, prev.r1, cur.r0, cur.r1, leaves, line);
+        err = stroke_join<M>(join, miter, tol_sq, p0, prev.r0, prev.r1, cur.r0, cur.r1, leaves, line, ends);
     }
     if (k + 1 == len) {
         if (!s.joined) line(cur.r1);

@@ -81,7 +81,7 @@ struct DevStatus {
     unsigned long long op_total;      // packed (events << 32 | closes) of all ops
     unsigned long long st_total;      // stroker: points stored << 32 | sub-strokes, before the cap
     unsigned long long stroke_total;  // stroker outline: events << 32 | closes
-    uint32_t st_subs, st_items;       // sub-strokes kept; outline items
+    uint32_t st_items, pad0;          // stroker: outline items (general form)
     uint32_t spin_fail;
     uint32_t pad;
     uint32_t *host_err;  // a pinned host word that also receives `err` when it is raised (null: none)

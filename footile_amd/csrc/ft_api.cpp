@@ -115,7 +115,7 @@ ft_status plotter_fill_ops(ft_plotter *p, ft_fill_rule rule, const ft_path_op *o
         p->last_stored = stored;
         return FT_OK;
     }
-    s = ft::ws_set_batch(p->ws, ops, n, &d, 1);
+    s = ft::ws_set_batch(p->ws, ops, n, &d, 1, 0, true);
     if (s) return s;
     s = ft::ws_run(p->ws, ft::MODE_FILL, true);
     if (s) return s;
@@ -227,7 +227,7 @@ ft_status ft_plotter_stroke(ft_plotter *p, const ft_path_op *ops, size_t n, cons
         p->last_offered = offered;
         p->last_stored = stored;
     } else {
-        s = ft::ws_set_batch(p->ws, ops, n, &d, 1, ft::PATH_WHOLE);
+        s = ft::ws_set_batch(p->ws, ops, n, &d, 1, ft::PATH_WHOLE, true);
         if (s) return s;
         s = ft::ws_run(p->ws, ft::MODE_STROKE, true);
         if (s) return s;
@@ -317,7 +317,7 @@ ft_status ft_fig_fill(ft_fill_rule rule, const float *xy, const uint8_t *close_a
         d.tolerance = 0.3f;
         d.pen_width = 1.0f;
         // raw points: Fig::add_point receives the caller's f32 values
-        s = ft::ws_set_batch(ws, ops.data(), ops.size(), &d, 1, ft::PATH_RAW);
+        s = ft::ws_set_batch(ws, ops.data(), ops.size(), &d, 1, ft::PATH_RAW, true);
         if (!s) s = ft::ws_run(ws, ft::MODE_FILL, false);
         if (!s && bytes && hipMemcpy(pixels, d_px, bytes, hipMemcpyDeviceToHost) != hipSuccess) s = FT_EDEVICE;
     }

@@ -67,6 +67,7 @@ struct Workspace {
     uint8_t *h_pin = nullptr;      // pinned staging of the layout's uploads
     std::vector<uint8_t> h_stage;  // the same in arena mode, in plain memory
     size_t cap_pin = 0;
+    size_t upload_owed = 0;        // bytes of it that the next run's first kernel copies
     bool op_ordered = false;
     // the kept flags take the ingest pass (pushed marks and their running
     // maximum) instead of their local form: set for the rest of a layout
@@ -183,9 +184,11 @@ ft_status ws_reserve_like(Workspace &dst, const Workspace &src);
 ft_status ws_init_arena(Workspace &ws, void *arena, size_t bytes, hipStream_t stream);
 void ws_free(Workspace &ws);
 // Upload a batch layout: ops + path descriptors (host arrays).
-// extra_flags (PATH_RAW, ...) are or-ed into every path's flags.
+// extra_flags (PATH_RAW, ...) are or-ed into every path's flags.  run_next: a
+// run on the workspace's stream is the next thing that happens to it, so a
+// small layout's upload may be left to its first kernel.
 ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const ft_fill_desc *paths,
-                       size_t n_paths, uint32_t extra_flags = 0);
+                       size_t n_paths, uint32_t extra_flags = 0, bool run_next = false);
 // Re-upload only the ops (same count and layout) -- for a plotter reusing ws.
 ft_status ws_upload_ops(Workspace &ws, const ft_path_op *ops, size_t n_ops);
 // Enqueue a run (MODE_FILL: the fills; MODE_STROKE: the strokes, with the

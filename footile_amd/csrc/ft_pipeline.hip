@@ -78,12 +78,21 @@ __device__ inline void block_reduce_keyed(bool has, uint32_t key, T v, T identit
 }
 
 // ---------------------------------------------------------------------------
-// Stage 0: clear per-run state (a kernel, not hipMemsetAsync: graph-safe).
+// Stage 0: clear per-run state (a kernel, not hipMemsetAsync: graph-safe) and,
+// for a layout that has not been uploaded, copy it from its pinned staging: a
+// copy by the runtime in front of the first kernel costs 14 us more (a plotter
+// fill of 1,000 lines takes 60 us, 74 with it).
 // ---------------------------------------------------------------------------
+struct Upload {
+    const uint4 *src;  // pinned host memory
+    uint4 *dst;
+    uint32_t n;        // 16-byte words
+};
 __global__ __launch_bounds__(BLOCK) void k_clear(PathState *ps, unsigned long long *top_rep, uint32_t n_paths,
                                                  uint32_t *band_cnt, uint32_t *band_cur, uint32_t n_slots,
                                                  unsigned long long *lb, uint32_t n_lb, DevStatus *st,
-                                                 uint32_t keep_failed, uint32_t *host_err) {
+                                                 uint32_t keep_failed, uint32_t *host_err, Upload up) {
+    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < up.n; i += gridDim.x * BLOCK) up.dst[i] = up.src[i];
     uint32_t n = n_paths * TOP_REPS > n_slots ? n_paths * TOP_REPS : n_slots;
     n = n > n_lb ? n : n_lb;
     for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
@@ -437,8 +446,39 @@ __global__ __launch_bounds__(BLOCK) void k_kept_local(Limits L0, const uint32_t 
     if (bad) raise_err(st, FT_EDEVICE);
 }
 
-// One wavefront per path; the cap point is found by a 64-way search (each
-// round probes 64 events at once), a few round trips for any path length.
+// The cap point of a path whose points reach the cap, and whether its re-pop
+// drops it, by one wavefront: a 64-way search (each round probes 64 events at
+// once), a few round trips for any path length.
+__device__ inline uint32_t cap_search(const CapSpan &c, const Limits &L, const uint32_t *ev_meta, const I2 *ev_xy,
+                                      const uint32_t *ev_kept, const uint32_t *ev_idx, const int32_t *run_first,
+                                      uint32_t &bad) {
+    const uint32_t lane = threadIdx.x & 63;
+    // cap_after is false below lo and true from hi on (hi = ee: none)
+    uint32_t lo = c.eb, hi = c.ee;
+    while (hi - lo > 64) {
+        const uint32_t step = (hi - lo + 63) / 64;
+        uint32_t m = lo + (lane + 1) * step - 1;
+        m = m < hi ? m : hi - 1;
+        const unsigned long long t = __ballot(cap_after(m, c, ev_kept, ev_idx));
+        if (t) {
+            const int f = __ffsll((long long)t) - 1;
+            const uint32_t mf = __shfl(m, f, 64), mp = __shfl(m, f > 0 ? f - 1 : 0, 64);
+            hi = mf;
+            lo = f > 0 ? mp + 1 : lo;
+        } else {
+            lo = hi;
+        }
+    }
+    const uint32_t m = lo + lane;
+    const unsigned long long t = __ballot((m < hi) && cap_after(m < hi ? m : lo, c, ev_kept, ev_idx));
+    const uint32_t ea = t ? lo + (uint32_t)(__ffsll((long long)t) - 1) : hi;
+    bad |= ea < c.ee ? 0u : 1u;
+    uint32_t repop = 0;
+    if (lane == 0 && ea < c.ee) repop = cap_repop(ea, c, L, ev_meta, ev_xy, run_first);
+    return repop;  // (lane 0's)
+}
+
+// One wavefront per path.
 __global__ __launch_bounds__(BLOCK) void k_cap(Limits L0, const PathDev *paths, const unsigned long long *op_off,
                                                const uint32_t *ev_meta, const I2 *ev_xy, const uint32_t *ev_kept,
                                                const uint32_t *ev_idx, const int32_t *run_first, PathState *ps,
@@ -450,30 +490,7 @@ __global__ __launch_bounds__(BLOCK) void k_cap(Limits L0, const PathDev *paths, 
     uint32_t bad = 0;
     for (uint32_t p = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6); p < L.n_paths; p += waves) {
         const CapSpan c = cap_span(p, L, paths, op_off, ev_kept, ev_idx, bad);
-        uint32_t repop = 0;
-        if (c.over) {
-            // cap_after is false below lo and true from hi on (hi = ee: none)
-            uint32_t lo = c.eb, hi = c.ee;
-            while (hi - lo > 64) {
-                const uint32_t step = (hi - lo + 63) / 64;
-                uint32_t m = lo + (lane + 1) * step - 1;
-                m = m < hi ? m : hi - 1;
-                const unsigned long long t = __ballot(cap_after(m, c, ev_kept, ev_idx));
-                if (t) {
-                    const int f = __ffsll((long long)t) - 1;
-                    const uint32_t mf = __shfl(m, f, 64), mp = __shfl(m, f > 0 ? f - 1 : 0, 64);
-                    hi = mf;
-                    lo = f > 0 ? mp + 1 : lo;
-                } else {
-                    lo = hi;
-                }
-            }
-            const uint32_t m = lo + lane;
-            const unsigned long long t = __ballot((m < hi) && cap_after(m < hi ? m : lo, c, ev_kept, ev_idx));
-            const uint32_t ea = t ? lo + (uint32_t)(__ffsll((long long)t) - 1) : hi;
-            bad |= ea < c.ee ? 0u : 1u;
-            if (lane == 0 && ea < c.ee) repop = cap_repop(ea, c, L, ev_meta, ev_xy, run_first);
-        }
+        const uint32_t repop = c.over ? cap_search(c, L, ev_meta, ev_xy, ev_kept, ev_idx, run_first, bad) : 0u;
         if (lane == 0) cap_store(p, c, repop, ps);
     }
     if (bad) raise_err(st, FT_EDEVICE);
@@ -485,6 +502,11 @@ __global__ __launch_bounds__(BLOCK) void k_cap(Limits L0, const PathDev *paths, 
 // path's TOP_REPS partial minima (block b into b mod TOP_REPS), so that a
 // batch of few paths does not queue every block's atomic on one address;
 // k_edges then folds the partials into PathState::topkey.
+//
+// ONE: the batch is one path, whose span is the whole run: its state needs no
+// per-path search of the events, and every block makes it for itself (a launch
+// of k_cap and its gap less, 4 of 89 us of a 1,500-segment plotter call).
+template <bool ONE>
 __global__ __launch_bounds__(BLOCK) void k_compact(Limits L0, const uint32_t *ev_meta, const I2 *ev_xy,
                                                    const uint32_t *ev_kept, const uint32_t *ev_idx,
                                                    const int32_t *run_first, const uint32_t *run_path,
@@ -493,6 +515,28 @@ __global__ __launch_bounds__(BLOCK) void k_compact(Limits L0, const uint32_t *ev
     if (run_failed(st)) return;
     const Limits L = run_limits(st, L0.n_ops, L0.n_paths, L0.n_bands, L0.cap_points);
     uint32_t bad = 0;
+    __shared__ PathState s_ps;
+    if constexpr (ONE) {
+        if (threadIdx.x < 64) {
+            CapSpan c;
+            c.eb = c.base = 0;
+            c.ee = L.n_events;
+            c.offered = L.n_events - L.n_runs;
+            c.stored = st->n_kept;
+            c.over = c.stored >= FT_MAX_POINTS;
+            const uint32_t repop = c.over ? cap_search(c, L, ev_meta, ev_xy, ev_kept, ev_idx, run_first, bad) : 0u;
+            if (threadIdx.x == 0) {
+                PathState s;
+                s.topkey = NO_KEY;
+                s.topidx = NO_IDX;
+                s.n_edges = s.fwd = 0;
+                cap_store(0, c, repop, &s);
+                s_ps = s;
+                if (blockIdx.x == 0) ps[0] = s;
+            }
+        }
+        __syncthreads();
+    }
     for (uint32_t base = blockIdx.x * BLOCK; base < L.n_events; base += gridDim.x * BLOCK) {
         const uint32_t e = base + threadIdx.x;
         TopCand c;
@@ -500,7 +544,7 @@ __global__ __launch_bounds__(BLOCK) void k_compact(Limits L0, const uint32_t *ev
         c.key = NO_KEY;
         if (e < L.n_events)
             compact_event(e, L, ev_meta, ev_xy, ev_kept, ev_idx, run_first, run_path, run_start, run_end, pts,
-                          pt_run, ps, bad, &c);
+                          pt_run, ONE ? &s_ps : ps, bad, &c);
         block_reduce_keyed<unsigned long long>(
             c.path != NO_IDX, c.path, c.key, NO_KEY,
             [](unsigned long long a, unsigned long long b) { return a < b ? a : b; },
@@ -591,13 +635,23 @@ __device__ inline uint32_t bin_window_counts(const bool *on, const uint32_t *g0,
 
 // One thread per stored point [0, n_kept): Edge::new, the point's band
 // record for k_bin, and the pairs per (band, replica).
-template <int BIN_ITEMS>
+//
+// With SCAN (at most BAND_SCAN_MAX counters) the block that finishes last also
+// makes the counters' list offsets: a scan kernel of one block and its gap
+// less.  Its reads are agent-scope atomics, as the counters' adds are, and each
+// block's adds are done (vmcnt) before it counts itself finished: no fence, so
+// no write-back of the caches.  No block waits on another.
+constexpr uint32_t BAND_SCAN_ITEMS = 16, BAND_SCAN_MAX = BAND_SCAN_ITEMS * BLOCK;
+template <int BIN_ITEMS, bool SCAN>
 __global__ __launch_bounds__(BLOCK) void k_edges(Limits L0, uint32_t band_shift, const uint32_t *pt_run,
                                                  const uint32_t *run_path, const uint32_t *run_start,
                                                  const uint32_t *run_end, const PathDev *paths, const I2 *pts,
-                                                 EdgeRec *edges, U2 *pt_band, uint32_t *band_cnt, PathState *ps,
+                                                 EdgeRec *edges, U2 *pt_band, uint32_t *band_cnt, uint32_t *band_off,
+                                                 unsigned long long *done, PathState *ps,
                                                  const unsigned long long *top_rep, DevStatus *st) {
     __shared__ __align__(16) uint32_t s_h[BIN_WINDOW];
+    __shared__ uint32_t s_t[SCAN ? BLOCK * (BAND_SCAN_ITEMS + 1) : 1];  // the counters, one padded row per thread
+    __shared__ uint32_t s_last;
     __shared__ uint32_t s_w[BLOCK / 64];
     if (run_failed(st)) return;
     const Limits L = run_limits(st, L0.n_ops, L0.n_paths, L0.n_bands, L0.cap_points);
@@ -643,6 +697,52 @@ __global__ __launch_bounds__(BLOCK) void k_edges(Limits L0, uint32_t band_shift,
         __syncthreads();
     }
     if (bad) raise_err(st, FT_EDEVICE);
+    if constexpr (SCAN) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) s_last = atomicAdd(done, 1ull) == gridDim.x - 1 ? 1u : 0u;
+        __syncthreads();
+        if (!s_last) return;
+        constexpr uint32_t ROW = BAND_SCAN_ITEMS + 1;
+        const uint32_t n_slots = L.n_bands << band_shift, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+        uint32_t v[BAND_SCAN_ITEMS];
+#pragma unroll
+        for (uint32_t j = 0; j < BAND_SCAN_ITEMS; ++j) {
+            const uint32_t k = j * BLOCK + tid;
+            v[j] = k < n_slots ? __hip_atomic_load(&band_cnt[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < BAND_SCAN_ITEMS; ++j) {
+            const uint32_t k = j * BLOCK + tid;
+            s_t[(k / BAND_SCAN_ITEMS) * ROW + k % BAND_SCAN_ITEMS] = v[j];
+        }
+        __syncthreads();
+        uint32_t run = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < BAND_SCAN_ITEMS; ++j) {
+            const uint32_t x = s_t[tid * ROW + j];
+            v[j] = run;
+            run += x;
+        }
+        const uint32_t incl = wave_incl_dpp<false>(run);
+        if (lane == 63) s_w[wid] = incl;
+        __syncthreads();
+        uint32_t pre = incl - run, all = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < BLOCK / 64; ++w) {
+            pre += w < wid ? s_w[w] : 0u;
+            all += s_w[w];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < BAND_SCAN_ITEMS; ++j) s_t[tid * ROW + j] = pre + v[j];
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < BAND_SCAN_ITEMS; ++j) {
+            const uint32_t k = j * BLOCK + tid;
+            if (k < n_slots) band_off[k] = s_t[(k / BAND_SCAN_ITEMS) * ROW + k % BAND_SCAN_ITEMS];
+        }
+        if (tid == 0) st->n_pairs = all;
+    }
 }
 
 // Scatters each point's pairs into the band lists: one atomic per nonzero
@@ -2322,7 +2422,7 @@ __device__ __forceinline__ bool small_stroker(SmallLds &S, SmallStrokeLds &T, ui
     return true;
 }
 
-// ops: the figure's ops in device memory, or null when `inl` carries them.
+// ops: the figure's ops in pinned host memory, or null when `inl` carries them.
 // STROKE: Plotter::stroke (flatten with widths, the stroker, then the
 // outline's fill); else Plotter::fill.
 template <bool STROKE>
@@ -2341,7 +2441,13 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
     }
     const uint32_t n_in = n_ops < SMALL_OPS ? n_ops : SMALL_OPS;
     for (uint32_t i = tid; i < SMALL_OPS; i += SBLOCK) S.op_path[i] = 0;
-    for (uint32_t i = tid; i < n_in; i += SBLOCK) S.ops[i] = ops ? ops[i] : inl.op[i < SMALL_ARG_OPS ? i : 0];
+    {  // word by word: whole lines over the bus
+        constexpr uint32_t WORDS = sizeof(ft_path_op) / 4;
+        const uint32_t n_w = (ops || n_in <= SMALL_ARG_OPS ? n_in : SMALL_ARG_OPS) * WORDS;
+        const uint32_t *const src = ops ? reinterpret_cast<const uint32_t *>(ops) : reinterpret_cast<const uint32_t *>(inl.op);
+        uint32_t *const dst = reinterpret_cast<uint32_t *>(S.ops);
+        for (uint32_t i = tid; i < n_w; i += SBLOCK) dst[i] = src[i];
+    }
     __syncthreads();
     // 1-2. flatten (and for a stroke, the stroker) into the fill events in LDS
     uint32_t n_events = 0, n_runs = 0, bad = 0;
@@ -2879,8 +2985,14 @@ static uint32_t tile_grid_for(const Workspace &ws, int f, uint32_t cells) {
     return (uint32_t)std::min<uint64_t>(g, ws.it_count[f]);
 }
 
+// Layouts up to this size go up in the first kernel of the run that follows:
+// plotter fills of 16,000 lines (0.6 MB) take 108 us so and 125 with the
+// runtime's copy, of 32,000 156 and 174, of 64,000 (2.4 MB) 324 and 319.
+constexpr size_t UPLOAD_IN_CLEAR = 1u << 20;
+
 ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const ft_fill_desc *paths,
-                       size_t n_paths, uint32_t extra_flags) {
+                       size_t n_paths, uint32_t extra_flags, bool run_next) {
+    ws.upload_owed = 0;
     if (n_ops >= 0x7FFFFFFFu || n_paths >= 0x7FFFFFFFu) return FT_EINVAL;
     graph_drop(ws);
     ws.ingest_pass = false;
@@ -3120,7 +3232,11 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
         }
         for (int k = 0; k < LAY_SECTIONS; ++k)
             if (sec_len[k]) memcpy(stage + sec_off[k], sec_src[k], sec_len[k]);
-        FT_HIP(hipMemcpyAsync(ws.d_lay, stage, lay_bytes, hipMemcpyHostToDevice, ws.stream));
+        // (lay_bytes is a multiple of 256)
+        if (run_next && !ws.arena && lay_bytes <= UPLOAD_IN_CLEAR)
+            ws.upload_owed = lay_bytes;
+        else
+            FT_HIP(hipMemcpyAsync(ws.d_lay, stage, lay_bytes, hipMemcpyHostToDevice, ws.stream));
     }
     ws.uploads_pending = true;
     return FT_OK;
@@ -3248,10 +3364,13 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
     // no marker packet stalls the stream between kernels.
     const size_t n_slots = ws.n_bands << ws.band_shift;
     uint32_t *const host_err = report ? &report->late_err : nullptr;
+    Upload up{reinterpret_cast<const uint4 *>(ws.h_pin), reinterpret_cast<uint4 *>(ws.d_lay),
+              (uint32_t)(ws.upload_owed / sizeof(uint4))};
+    ws.upload_owed = 0;
     hipExtLaunchKernelGGL(k_clear, dim3(grid_for(std::max(std::max(ws.n_paths * TOP_REPS, n_slots), (size_t)n_lb))),
                           dim3(BLOCK), 0, s, ev ? ev[0] : nullptr, nullptr, 0, ws.d_pstate, ws.d_top_rep,
                           (uint32_t)ws.n_paths, ws.d_band_cnt, ws.d_band_cur, (uint32_t)n_slots, lb, n_lb, st,
-                          keep_failed ? 1u : 0u, host_err);
+                          keep_failed ? 1u : 0u, host_err, up);
     const uint32_t *lastpw = nullptr;
     if (mode != MODE_FILL && n_ops) {
         const PenWidthSrc pw{ws.d_ops, 0u};
@@ -3380,20 +3499,24 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
                                              (uint32_t)ws.cap_events, lb + 2 * tiles, &st->n_kept, st, true, false, ws.tickets);
             }
         }
-        k_cap<<<grid_for(ws.n_paths * 64), BLOCK, 0, s>>>(L0, ws.d_paths, ws.d_op_off, ws.d_ev_meta, ws.d_ev_xy,
-                                                     ws.d_ev_kept, ws.d_ev_idx, ws.d_run_first, ws.d_pstate, st);
-        k_compact<<<ge, BLOCK, 0, s>>>(L0, ws.d_ev_meta, ws.d_ev_xy, ws.d_ev_kept, ws.d_ev_idx, ws.d_run_first,
+        const bool one = ws.n_paths == 1;
+        if (!one)
+            k_cap<<<grid_for(ws.n_paths * 64), BLOCK, 0, s>>>(L0, ws.d_paths, ws.d_op_off, ws.d_ev_meta, ws.d_ev_xy,
+                                                         ws.d_ev_kept, ws.d_ev_idx, ws.d_run_first, ws.d_pstate, st);
+        (one ? k_compact<true> : k_compact<false>)<<<ge, BLOCK, 0, s>>>(L0, ws.d_ev_meta, ws.d_ev_xy, ws.d_ev_kept, ws.d_ev_idx, ws.d_run_first,
                                        ws.d_run_path, ws.d_run_start, ws.d_run_end, ws.d_pts, ws.d_pt_run, ws.d_pstate,
                                        top_rep, st);
         const bool wide = ws.cap_events >= BIN_WIDE_MIN;
-        (wide ? k_edges<4> : k_edges<1>)<<<ge, BLOCK, 0, s>>>(
+        const bool scan_in_edges = !wide && ws.n_bands && n_slots <= BAND_SCAN_MAX;
+        (wide ? k_edges<4, false> : (scan_in_edges ? k_edges<1, true> : k_edges<1, false>))<<<ge, BLOCK, 0, s>>>(
             L0, ws.band_shift, ws.d_pt_run, ws.d_run_path, ws.d_run_start, ws.d_run_end, ws.d_paths, ws.d_pts,
-            ws.d_edges, ws.d_pt_band, ws.d_band_cnt, ws.d_pstate, top_rep, st);
+            ws.d_edges, ws.d_pt_band, ws.d_band_cnt, ws.d_band_off, lb + 4 * tiles, ws.d_pstate, top_rep, st);
         if (ws.n_bands) {
             // pairs per (band, replica) -> list segment offsets and the pair total
             const uint32_t n_slots = (uint32_t)(ws.n_bands << ws.band_shift);
-            scan_launch<uint32_t, false>(s, ws.scan_resident, ws.d_band_cnt, ws.d_band_off, nullptr, n_slots, n_slots,
-                                         lb + 4 * tiles, &st->n_pairs, st, true, false, ws.tickets);
+            if (!scan_in_edges)
+                scan_launch<uint32_t, false>(s, ws.scan_resident, ws.d_band_cnt, ws.d_band_off, nullptr, n_slots,
+                                             n_slots, lb + 4 * tiles, &st->n_pairs, st, true, false, ws.tickets);
             (wide ? k_bin<4> : k_bin<1>)<<<ge, BLOCK, 0, s>>>(
                 L0, ws.band_shift, ws.d_pt_band, ws.d_band_off, ws.d_band_cur, ws.d_band_list, ws.cap_pairs, ws.d_pts,
                 ws.d_pt_run, ws.d_run_start, ws.d_run_end, ws.d_pstate, st);
@@ -3589,21 +3712,14 @@ ft_status ws_small_fill(Workspace &ws, const ft_path_op *ops, size_t n_ops, cons
     ft_status s;
     if (!ws.d_edges || ws.cap_events < SMALL_EVENTS)
         if ((s = ensure_event_capacity(ws, SMALL_EVENTS))) return s;
-    // the ops: inside the launch when they fit, else through the pinned
-    // staging into the upload block
+    // the ops: inside the launch when they fit, else in the pinned staging,
+    // which the kernel reads (once) over the bus
     SmallOps inl;  // the launch copies its arguments
     const ft_path_op *d_ops = nullptr;
     const size_t bytes = n_ops * sizeof(ft_path_op);
     if (n_ops <= SMALL_ARG_OPS) {
         memcpy(inl.op, ops, bytes);
     } else {
-        if (bytes > ws.cap_lay || !ws.d_lay) {
-            if ((s = dev_alloc(ws, ws.d_lay, bytes + 256))) {
-                ws.cap_lay = 0;
-                return s;
-            }
-            ws.cap_lay = bytes + 256;
-        }
         if (bytes > ws.cap_pin) {
             if (ws.h_pin) (void)hipHostFree(ws.h_pin);
             ws.h_pin = nullptr;
@@ -3615,8 +3731,7 @@ ft_status ws_small_fill(Workspace &ws, const ft_path_op *ops, size_t n_ops, cons
             ws.cap_pin = bytes;
         }
         memcpy(ws.h_pin, ops, bytes);
-        d_ops = reinterpret_cast<const ft_path_op *>(ws.d_lay);
-        FT_HIP(hipMemcpyAsync(ws.d_lay, ws.h_pin, bytes, hipMemcpyHostToDevice, ws.stream));
+        d_ops = reinterpret_cast<const ft_path_op *>(ws.h_pin);
     }
     // the layout's pointers into the upload block are stale from here on: the
     // next full-pipeline call lays the batch out again

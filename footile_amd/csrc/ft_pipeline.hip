@@ -638,10 +638,12 @@ __device__ inline uint32_t bin_window_counts(const bool *on, const uint32_t *g0,
 //
 // With SCAN (at most BAND_SCAN_MAX counters) the block that finishes last also
 // makes the counters' list offsets: a scan kernel of one block and its gap
-// less.  Its reads are agent-scope atomics, as the counters' adds are, and each
+// less.  To BAND_SCAN_GRID blocks, whose adds to one word go by quickly (98
+// blocks: 7.3 us, 5.4 without the scan, which takes 4.7 alone; 1,255 blocks:
+// 21.7 and 8.3, and 6.0).  Its reads are agent-scope atomics, as the counters' adds are, and each
 // block's adds are done (vmcnt) before it counts itself finished: no fence, so
 // no write-back of the caches.  No block waits on another.
-constexpr uint32_t BAND_SCAN_ITEMS = 16, BAND_SCAN_MAX = BAND_SCAN_ITEMS * BLOCK;
+constexpr uint32_t BAND_SCAN_ITEMS = 16, BAND_SCAN_MAX = BAND_SCAN_ITEMS * BLOCK, BAND_SCAN_GRID = 256;
 template <int BIN_ITEMS, bool SCAN>
 __global__ __launch_bounds__(BLOCK) void k_edges(Limits L0, uint32_t band_shift, const uint32_t *pt_run,
                                                  const uint32_t *run_path, const uint32_t *run_start,
@@ -3129,9 +3131,12 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
     }
     size_t nb_total = band_path.size();
     // replicas per band counter: enough that the slots spread over about
-    // BAND_SLOTS_MIN counters, at most 2^BAND_SHIFT_MAX
+    // BAND_SLOTS_MIN counters, at most 2^BAND_SHIFT_MAX; where k_edges' last
+    // block scans them, at most BAND_SCAN_MAX
     uint32_t shift = 0;
     while (shift < BAND_SHIFT_MAX && (nb_total << shift) < BAND_SLOTS_MIN) ++shift;
+    if (!ws.arena && 16 * n_ops <= (size_t)BAND_SCAN_GRID * BLOCK && nb_total <= BAND_SCAN_MAX)
+        while (shift > 0 && (nb_total << shift) > BAND_SCAN_MAX) --shift;
     if ((nb_total << shift) >= 0x7FFFFFFFu) return FT_ENOTSUP;
     const size_t n_slots = nb_total << shift;
     if (n_slots > ws.cap_band_slots || !ws.d_band_cnt) {
@@ -3447,7 +3452,9 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
         }
     }
     if (mode == MODE_FILL || mode == MODE_STROKE) {
-        const uint32_t ge = grid_for(ws.cap_events);
+        // (an arena's capacity is whatever its bytes hold: the grid-stride
+        // kernels take a grid for the events a first layout expects instead)
+        const uint32_t ge = grid_for(ws.arena ? std::min(ws.cap_events, 16 * n_ops + (size_t)1024) : ws.cap_events);
         Limits L0{};
         L0.n_ops = n_ops;
         L0.n_paths = (uint32_t)ws.n_paths;
@@ -3507,7 +3514,7 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
                                        ws.d_run_path, ws.d_run_start, ws.d_run_end, ws.d_pts, ws.d_pt_run, ws.d_pstate,
                                        top_rep, st);
         const bool wide = ws.cap_events >= BIN_WIDE_MIN;
-        const bool scan_in_edges = !wide && ws.n_bands && n_slots <= BAND_SCAN_MAX;
+        const bool scan_in_edges = !wide && ws.n_bands && n_slots <= BAND_SCAN_MAX && ge <= BAND_SCAN_GRID;
         (wide ? k_edges<4, false> : (scan_in_edges ? k_edges<1, true> : k_edges<1, false>))<<<ge, BLOCK, 0, s>>>(
             L0, ws.band_shift, ws.d_pt_run, ws.d_run_path, ws.d_run_start, ws.d_run_end, ws.d_paths, ws.d_pts,
             ws.d_edges, ws.d_pt_band, ws.d_band_cnt, ws.d_band_off, lb + 4 * tiles, ws.d_pstate, top_rep, st);

@@ -267,11 +267,15 @@ __global__ __launch_bounds__(BLOCK) void k_scan(Src src, T *out, const uint32_t 
     __shared__ T s_prefix;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint32_t tid = threadIdx.x;
-    if (tid == 0) {  // status, length and the block's ticket in one round trip
+    if (tid == 0) {
         const uint32_t e = st->err, o = st->overflow;
         const uint32_t nn = n_dev ? *n_dev : n_host;
-        s_tk = tickets ? lookback_ticket(lb) : blockIdx.x;
-        s_fail = (check_failed & ((e | o) != 0u)) ? 1u : 0u;
+        // (tickets go to the blocks there are items for: the grid may be sized
+        // for many more, whose atomics on one word would hold these up)
+        const uint64_t nc = nn < n_cap ? nn : n_cap;
+        const bool on = (uint64_t)blockIdx.x * tiles_per_block * TILE < nc;
+        s_tk = tickets & on ? lookback_ticket(lb) : blockIdx.x;
+        s_fail = (check_failed & ((e | o) != 0u)) | !on ? 1u : 0u;
         s_n = nn;
     }
     __syncthreads();

@@ -236,7 +236,7 @@ __device__ inline T lookback_prefix(unsigned long long *lb, uint32_t b, T btot, 
 
 // Items of a scan read from an array.  A scan's source gives item i's value;
 // `first` is true on the one visit of pass 1, where a source may also store
-// per-item side outputs.  bind() runs after the status check; `bad` set by a
+// per-item side outputs.  bind() runs before the status check; `bad` set by a
 // source raises FT_EDEVICE.
 template <typename T>
 struct ArraySrc {
@@ -267,6 +267,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan(Src src, T *out, const uint32_t 
     __shared__ T s_prefix;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint32_t tid = threadIdx.x;
+    src.bind(st);  // (in flight with the reads below)
     if (tid == 0) {
         const uint32_t e = st->err, o = st->overflow;
         const uint32_t nn = n_dev ? *n_dev : n_host;
@@ -275,12 +276,17 @@ __global__ __launch_bounds__(BLOCK) void k_scan(Src src, T *out, const uint32_t 
         const uint64_t nc = nn < n_cap ? nn : n_cap;
         const bool on = (uint64_t)blockIdx.x * tiles_per_block * TILE < nc;
         s_tk = tickets & on ? lookback_ticket(lb) : blockIdx.x;
-        s_fail = (check_failed & ((e | o) != 0u)) | !on ? 1u : 0u;
+        // A failed run's block leaves no items, but says so: the error may be
+        // another block's of this very scan, and later blocks wait for this
+        // one's count.
+        const bool fail = check_failed & ((e | o) != 0u);
+        if (fail & on)
+            __hip_atomic_store(&lb[2 * (size_t)s_tk + 2], LB_READY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_fail = fail | !on ? 1u : 0u;
         s_n = nn;
     }
     __syncthreads();
     if (s_fail) return;
-    src.bind(st);
     const uint32_t b = s_tk;
     const uint64_t n = s_n < n_cap ? s_n : n_cap;
     const uint64_t n_tiles = (n + TILE - 1) / TILE;

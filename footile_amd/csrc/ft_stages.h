@@ -456,6 +456,7 @@ struct Limits {
     uint32_t n_runs;      // runs (= closes) of this run
     uint32_t cap_points;  // capacity of the point / edge arrays
     uint32_t n_pairs;     // (edge, band) pairs of this run
+    uint32_t n_kept;      // points kept, before the caps
 };
 
 FT_HD inline bool i2_eq(I2 a, I2 b) { return (a.x == b.x) & (a.y == b.y); }

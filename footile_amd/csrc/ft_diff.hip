@@ -10,8 +10,8 @@
 //                paths, 16 per round, from integer LDS cells and a prefix sum,
 //                composite, the canvas and (in a step) its value before every
 //                round, which the backward starts from
-//   k_loss, k_loss_sum   L2 against a target: d loss / d canvas and the loss,
-//                summed on the device in a fixed order
+//   k_loss       L2 against a target: d loss / d canvas and the loss, summed on
+//                the device in a fixed order
 //   k_backward   the rounds last to first: coverage again, d loss / d alpha
 //                per pixel and path, the colours' gradients summed over the
 //                tile, and one lane per edge piece gathering its gradient from
@@ -798,25 +798,77 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
     if (canvas && in) canvas[((uint64_t)im * S.H + Y) * S.W + X] = C;
 }
 
-// loss partials per block (sum of squared differences); grad = 2 (C - T) / N.
+// The loss, and grad = 2 (C - T) / N: a sum of squared differences per block,
+// and their sum in a fixed order by the block that finishes last, so that a
+// step and a separate ft_diff_loss of the same canvas give the same value.
+// VEC floats per load (4 where every pointer is aligned for it).  LOSS_GRID
+// blocks, one per CU with LOSS_UNROLL loads of each kind in flight: their adds
+// to the one counter go by quickly.  (1,024 blocks of single floats and a
+// second kernel for the sum: 5.1 + 5.2 us for 512x512, 55 + 5 for 64 images of
+// 256x256; now 7.4 and 48.)
+constexpr uint32_t LOSS_GRID = 256;
+constexpr int LOSS_UNROLL = 4;
+template <int VEC>
 __global__ __launch_bounds__(BLOCK) void k_loss(const float *canvas, const float *target, float *grad, uint64_t n,
-                                                double *partial) {
+                                                unsigned long long *partial, uint32_t *done, double *loss) {
     __shared__ double s_w[BLOCK / 64];
+    __shared__ uint32_t s_last;
+    struct __align__(4 * VEC) Vec {
+        float v[VEC];
+    };
+    const Vec *const vc = reinterpret_cast<const Vec *>(canvas), *const vt = reinterpret_cast<const Vec *>(target);
+    Vec *const vg = reinterpret_cast<Vec *>(grad);
+    const uint64_t nv = n / VEC, stride = (uint64_t)LOSS_GRID * BLOCK;  // (n is a multiple of 4)
     double acc = 0.0;
     const float scale = (float)(2.0 / (double)n);
-    for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * BLOCK) {
-        const float r = canvas[i] - target[i];
-        acc += (double)r * (double)r;
-        if (grad) grad[i] = scale * r;
-    }
+    for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < nv; i += LOSS_UNROLL * stride) {
+        Vec c[LOSS_UNROLL], t[LOSS_UNROLL];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
+        for (int u = 0; u < LOSS_UNROLL; ++u) {
+            const uint64_t k = i + u * stride;
+            if (k < nv) {
+                c[u] = vc[k];
+                t[u] = vt[k];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < LOSS_UNROLL; ++u) {
+            const uint64_t k = i + u * stride;
+            if (k >= nv) continue;
+            Vec g;
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) {
+                const float r = c[u].v[x] - t[u].v[x];
+                acc += (double)r * (double)r;
+                g.v[x] = scale * r;
+            }
+            if (grad) vg[k] = g;
+        }
+    }
+    auto block_sum = [&](double v) {  // (thread 0's)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = v;
+        __syncthreads();
         double t = 0.0;
         for (int w = 0; w < BLOCK / 64; ++w) t += s_w[w];
-        partial[blockIdx.x] = t;
+        return t;
+    };
+    const double mine = block_sum(acc);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&partial[blockIdx.x], __builtin_bit_cast(unsigned long long, mine), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        s_last = atomicAdd(done, 1u) == LOSS_GRID - 1 ? 1u : 0u;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    static_assert(LOSS_GRID == BLOCK, "one partial per thread");
+    const unsigned long long p = __hip_atomic_load(&partial[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double all = block_sum(__builtin_bit_cast(double, p));
+    if (threadIdx.x == 0) {
+        *loss = all;
+        *done = 0;  // for the next run
     }
 }
 
@@ -1054,23 +1106,6 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
     if (bad) raise_err(st, FT_EDEVICE);
 }
 
-// The loss partials summed in a fixed order by one block: the same value for
-// a step and for a separate ft_diff_loss of the same canvas.
-__global__ __launch_bounds__(BLOCK) void k_loss_sum(const double *partial, uint32_t n, double *out) {
-    __shared__ double s_w[BLOCK / 64];
-    double acc = 0.0;
-    for (uint32_t i = threadIdx.x; i < n; i += BLOCK) acc += partial[i];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int w = 0; w < BLOCK / 64; ++w) t += s_w[w];
-        out[0] = t;
-    }
-}
-
 // The edge gradients of a path's edge e, with the y gradients completed by
 // the slope's share: (x, y) of its first vertex, (x, y) of its second.
 __device__ __forceinline__ float4 edge_grad(const DScene &S, const float4 *gedge, uint32_t vb, uint32_t V,
@@ -1082,50 +1117,59 @@ __device__ __forceinline__ float4 edge_grad(const DScene &S, const float4 *gedge
     return make_float4(g.x, g.x != 0.0f ? fmaf(-sl, g.x, g.z) : g.z, g.y, g.y != 0.0f ? fmaf(-sl, g.y, g.w) : g.w);
 }
 
-// Control point gradients from edge gradients (one thread per point): the sum
-// over the point's cubics' vertices of their Bernstein weights times the
-// vertex's gradient, which is its two edges' shares.
-// One block also reports the run's status, every other kernel of the run
-// being done.
+// Control point gradients from edge gradients: the sum over the point's
+// cubics' vertices of their Bernstein weights times the vertex's gradient,
+// which is its two edges' shares.  DSEG lanes per point, one per vertex of a
+// cubic; a vertex's second edge is its neighbour's first.  (One thread per
+// point walked its 16 or 32 vertices one after another, a chain of loads and
+// divisions: 7.0 us for 200x120, 8.8 for 512x512 and 60 for 64 images, now
+// 4.0, 4.2 and 63.)  One block also reports the run's status, every other kernel of the
+// run being done.
 __global__ __launch_bounds__(BLOCK) void k_point_grad(DScene S, const float4 *gedge, float2 *gpts, uint32_t n_pts,
                                                       const uint32_t *pt_path, const DevStatus *st,
                                                       HostStatus *report) {
+    static_assert(DSEG == 16, "a point's lanes are one DPP row");
     if (blockIdx.x == 0) report_status(report, st, nullptr, nullptr, 0);
-    for (uint32_t m = blockIdx.x * BLOCK + threadIdx.x; m < n_pts; m += gridDim.x * BLOCK) {
-        const uint32_t k = pt_path[m];
-        const uint32_t local = m - S.pt_off[k];
+    const uint32_t q = threadIdx.x % DSEG;  // vertex q + 1 of the cubic
+    constexpr uint32_t PTS = BLOCK / DSEG;
+    for (uint32_t mb = blockIdx.x * PTS; mb < n_pts; mb += gridDim.x * PTS) {
+        const uint32_t m = mb + threadIdx.x / DSEG;
+        const bool on = m < n_pts;
+        const uint32_t k = pt_path[on ? m : 0u];
+        const uint32_t local = on ? m - S.pt_off[k] : 0u;
         const uint32_t n_cub = (S.pt_off[k + 1] - S.pt_off[k] - 1) / 3;
         const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
         float2 acc = make_float2(0.0f, 0.0f);
-        if (local == 0) {
+        if (local == 0 && q == 0) {
             const float4 g = edge_grad(S, gedge, vb, V, 0), l = edge_grad(S, gedge, vb, V, V - 1);
             acc = make_float2(g.x + l.z, g.y + l.w);
         }
         // the point is control r of cubic c (and control 0 of cubic c + 1 when r == 3)
+#pragma unroll
         for (int pass = 0; pass < 2; ++pass) {
-            uint32_t c, r;
-            if (pass == 0) {
-                if (local == 0) continue;
-                c = (local - 1) / 3;
-                r = (local - 1) % 3 + 1;
-            } else {
-                if (local % 3 != 0) continue;
-                c = local / 3;
-                r = 0;
-                if (c >= n_cub) continue;
+            const bool has = pass == 0 ? local != 0 : (local % 3 == 0) & (local / 3 < n_cub);
+            const uint32_t c = pass == 0 ? (local ? (local - 1) / 3 : 0u) : (has ? local / 3 : 0u);
+            const uint32_t r = pass == 0 ? (local ? (local - 1) % 3 + 1 : 0u) : 0u;
+            if (pass == 1 && !__any(has)) continue;
+            const float4 in = edge_grad(S, gedge, vb, V, c * DSEG + q);  // the edge into vertex c * DSEG + q + 1
+            // and the one out of it: the next lane's, the last lane's its own
+            float2 out = make_float2(__shfl_down(in.x, 1, DSEG), __shfl_down(in.y, 1, DSEG));
+            if (q == DSEG - 1) {
+                const float4 e = edge_grad(S, gedge, vb, V, (c + 1) * DSEG);
+                out = make_float2(e.x, e.y);
             }
-            float4 in = edge_grad(S, gedge, vb, V, c * DSEG);  // the edge into vertex c * DSEG + 1
-#pragma unroll 4
-            for (int j = 1; j <= DSEG; ++j) {
-                const float4 out = edge_grad(S, gedge, vb, V, c * DSEG + (uint32_t)j);
-                float w[4];
-                bern(j, w);
-                acc.x += w[r] * (in.z + out.x);
-                acc.y += w[r] * (in.w + out.y);
-                in = out;
-            }
+            float w[4];
+            bern((int)q + 1, w);
+            const float wr = r == 0 ? w[0] : (r == 1 ? w[1] : (r == 2 ? w[2] : w[3]));
+            acc.x += has ? wr * (in.z + out.x) : 0.0f;
+            acc.y += has ? wr * (in.w + out.y) : 0.0f;
         }
-        gpts[m] = acc;
+#pragma unroll
+        for (int o = DSEG / 2; o > 0; o >>= 1) {
+            acc.x += __shfl_xor(acc.x, o, DSEG);
+            acc.y += __shfl_xor(acc.y, o, DSEG);
+        }
+        if (on & (q == 0)) gpts[m] = acc;
     }
 }
 
@@ -1155,16 +1199,15 @@ struct ft_diff {
     float4 *d_ck = nullptr;
     uint32_t ck_pitch = 0;  // checkpoint pixels per row
     uint64_t ck_stride = 0;  // and per checkpoint
-    double *d_partial = nullptr;  // [LOSS_GRID] loss partials
-    double *h_loss = nullptr;     // pinned: the summed loss, written by k_loss_sum
+    unsigned long long *d_partial = nullptr;  // [LOSS_GRID] loss partials (doubles)
+    uint32_t *d_done = nullptr;   // blocks of k_loss done: 0 between its runs
+    double *h_loss = nullptr;     // pinned: the summed loss, written by k_loss
     DevStatus *d_status = nullptr;
     HostStatus *h_status = nullptr;  // pinned: written by a run's last kernel
     bool clean = false;  // d_lb and d_status are as k_clear_run leaves them
 };
 
 namespace {
-
-constexpr uint32_t LOSS_GRID = 1024;
 
 #define FD_HIP(call)                                 \
     do {                                             \
@@ -1303,10 +1346,12 @@ ft_status run_forward(ft_diff *d, const float *points, const float *colours, flo
     return FT_ENOMEM;
 }
 
-// Enqueues the loss partials and their fixed-order sum (to h_loss).
+// Enqueues the loss (to h_loss) and its gradient.
 ft_status launch_loss(ft_diff *d, const float *canvas, const float *target, float *grad) {
-    k_loss<<<LOSS_GRID, BLOCK, 0, d->stream>>>(canvas, target, grad, d->canvas_floats, d->d_partial);
-    k_loss_sum<<<1, BLOCK, 0, d->stream>>>(d->d_partial, LOSS_GRID, d->h_loss);
+    const uintptr_t low = reinterpret_cast<uintptr_t>(canvas) | reinterpret_cast<uintptr_t>(target) |
+                          reinterpret_cast<uintptr_t>(grad);
+    (low & 15u ? k_loss<1> : k_loss<4>)<<<LOSS_GRID, BLOCK, 0, d->stream>>>(canvas, target, grad, d->canvas_floats,
+                                                                           d->d_partial, d->d_done, d->h_loss);
     FD_HIP(hipGetLastError());
     return FT_OK;
 }
@@ -1330,7 +1375,8 @@ ft_status launch_backward(ft_diff *d, const float *colours, const float *grad_ca
     k_backward<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
         S, reinterpret_cast<const float4 *>(colours), reinterpret_cast<const float4 *>(grad_canvas), d->d_ck,
         d->ck_pitch, d->ck_stride, d->d_gedge, grad_colours, d->d_status);
-    k_point_grad<<<grid_of(d->n_pts), BLOCK, 0, d->stream>>>(S, d->d_gedge, reinterpret_cast<float2 *>(grad_points),
+    k_point_grad<<<grid_of((uint64_t)d->n_pts * DSEG), BLOCK, 0, d->stream>>>(
+        S, d->d_gedge, reinterpret_cast<float2 *>(grad_points),
                                                              d->n_pts, d->d_pt_path, d->d_status, d->h_status);
     FD_HIP(hipGetLastError());
     return FT_OK;
@@ -1432,8 +1478,10 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
              (st = dalloc(d->d_cell_off, cells)) || (st = dalloc(d->d_cell_cur, cells)) ||
              (st = dalloc(d->d_cell_edge, d->cap_pairs)) || (st = dalloc(d->d_lb, std::max<size_t>(4 * d->cap_tiles, lookback_words(GEOM_BLOCKS)))) ||
              (st = dalloc(d->d_ck, n_ck * d->ck_stride)) || (st = dalloc(d->d_partial, LOSS_GRID)) ||
-             (st = dalloc(d->d_status, 1)))
+             (st = dalloc(d->d_status, 1)) || (st = dalloc(d->d_done, 1)))
         ;
+    else if (hipMemset(d->d_done, 0, sizeof(uint32_t)) != hipSuccess)
+        st = FT_EDEVICE;
     else if (hipHostMalloc(reinterpret_cast<void **>(&d->h_loss), sizeof(double), hipHostMallocCoherent) !=
                  hipSuccess ||
              hipHostMalloc(reinterpret_cast<void **>(&d->h_status), sizeof(HostStatus), hipHostMallocCoherent) !=
@@ -1461,7 +1509,7 @@ void ft_diff_free(ft_diff *d) {
     if (!d) return;
     void *bufs[] = {d->d_pt_off,   d->d_vtx_off,  d->d_vtx_path, d->d_pt_path,   d->d_img_first, d->d_vtx,
                     d->d_gedge,     d->d_cell_cnt, d->d_cell_off, d->d_cell_cur,  d->d_cell_edge, d->d_lb,
-                    d->d_ck,       d->d_partial,  d->d_status};
+                    d->d_ck,       d->d_partial,  d->d_status,   d->d_done};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (d->h_loss) (void)hipHostFree(d->h_loss);

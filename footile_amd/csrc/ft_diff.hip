@@ -938,7 +938,7 @@ __device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, floa
 // columns right of it from the prefix sums.  (Evaluating each piece on all 64
 // pixels of every wavefront it touches and reducing the three sums over the
 // wavefront took 18.4 ms for 64 images of 256x256 with 17,500 paths; this
-// form takes 3.8 ms, and 252 us instead of 869 for one 512x512 image of 256
+// form takes 3.6 ms, and 252 us instead of 869 for one 512x512 image of 256
 // paths.  Adding four vertex gradients per piece instead of EdgeGrad's two and
 // its ends took 4.5 ms and 332 us.)  Four wavefronts per SIMD are asked for: without, the kernel takes
 // 156 VGPRs, a CU holds three blocks, and the 1,024 blocks of a 512x512 image
@@ -991,16 +991,18 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
             float A[SEG];
             round_cover<false>(S, R, s, cur, piece_of(cv.p, cv.q, (int)Y), (int)Y, xb0, s_cells, pitch, A, bad);
             const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
-            float q[SEG], d[SEG];  // f . canvas under path j, and f . c_j - c_j.w q_j
+            float q[SEG];  // f . canvas under path j
+            // f . c_j - c_j.w q_j, made again in the second pass: kept beside q it
+            // spilled 16 more registers (3.77 ms instead of 3.57 for 64 images)
+            auto d_of = [&](const float4 &c, float qj) {
+                return fmaf(-c.w, qj, fmaf(f.w, c.w, fmaf(f.z, c.z, fmaf(f.y, c.y, f.x * c.x))));
+            };
             float qr = fmaf(f.w, C.w, fmaf(f.z, C.z, fmaf(f.y, C.y, f.x * C.x)));
 #pragma unroll
             for (uint32_t j = 0; j < SEG; ++j) {
                 const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
-                const float fc = fmaf(f.w, c.w, fmaf(f.z, c.z, fmaf(f.y, c.y, f.x * c.x)));
-                const float al = alpha_cover(A[j]);
                 q[j] = qr;
-                d[j] = fmaf(-c.w, qr, fc);
-                qr = fmaf(al, d[j], qr);  // = al f . c_j + (1 - c_j.w al) q_j
+                qr = fmaf(alpha_cover(A[j]), d_of(c, qr), qr);  // = al f . c_j + (1 - c_j.w al) q_j
             }
             float z[SEG / 2];
             const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0, b1 = (lane & 2) != 0, b0 = (lane & 1) != 0;
@@ -1010,16 +1012,16 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
 #pragma unroll
                 for (uint32_t h = 2; h-- > 0;) {
                     const uint32_t j = 2 * jp + h;
-                    const float cw = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u).w;
+                    const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
                     const float al = alpha_cover(A[j]);
-                    const float dal = T * d[j], V = T * al;
+                    const float dal = T * d_of(c, q[j]), V = T * al;
                     const bool part = (fabsf(A[j]) < 1.0f) & (A[j] != 0.0f);
                     const float dA = part ? (A[j] > 0.0f ? dal : -dal) : 0.0f;
                     r[h][0] = V * f.x;
                     r[h][1] = V * f.y;
                     r[h][2] = V * f.z;
                     r[h][3] = V * (f.w - q[j]);
-                    T *= fmaf(-cw, al, 1.0f);
+                    T *= fmaf(-c.w, al, 1.0f);
                     s_dA[j * pitch + tid] = dA;
                     s_pre[j * pitch + tid] = wave_incl_f32(dA);
                 }

@@ -423,7 +423,7 @@ __global__ __launch_bounds__(BLOCK) void k_fill_cells(DScene S, DevStatus *st) {
 // prefix sum then gives every pixel's coverage.  (Evaluating every piece that
 // touches a wavefront's columns on all of its pixels took 3.84 ms for 64
 // images of 256x256 with 17,500 paths, most of it on pixels outside the
-// ramp; this form takes 1.27 ms, and 91 us instead of 297 for one 512x512
+// ramp; this form takes 1.13 ms, and 83 us instead of 297 for one 512x512
 // image of 256 paths.  What is left is VALU work: per path and pixel about 9
 // instructions of prefix sum and 9 of composite.)
 //
@@ -643,11 +643,12 @@ __device__ __forceinline__ void scatter_piece(T *cells, uint32_t row_at, const R
 // time) and any further ones.  cells: SEG rows of pitch `pitch`, zero on
 // entry; with ZERO zero again on exit, behind a barrier, else the caller's to
 // use: each thread has read its own column.  Every thread calls it.
-template <bool ZERO>
+template <bool ZERO, uint32_t TW>
 __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t s, const PieceRef &ref,
                                             const Piece &first, int Y, float xb0, int *cells,
-                                            uint32_t pitch, float A[SEG], uint32_t &bad) {
-    const int tid = threadIdx.x, tw = (int)blockDim.x;
+                                            float A[SEG], uint32_t &bad) {
+    const int tid = threadIdx.x, tw = TW ? (int)TW : (int)blockDim.x;
+    const uint32_t pitch = (uint32_t)tw + 1;
     const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];
     const uint32_t heavy = R.marks[s] >> 16;
 #pragma unroll
@@ -741,6 +742,12 @@ __device__ __forceinline__ float4 round_colour(const float4 *__restrict__ colour
 // every round but the first, at slot (image row) * ck_pitch + X; canvas may
 // be null.  One block also clears the n_lb look-back words of the geometry
 // (done by now) for the next run and, with `report`, reports the status.
+//
+// TW: the tile's width where it is TILE_MAX (any wider than 192 pixels), else
+// 0 and the block's.  As a constant it makes the LDS rows' addresses offsets of
+// one register instead of sixteen (here 1.17 -> 1.13 ms for 64 images of
+// 256x256, 86 -> 83 us for 512x512; k_backward 3.57 -> 3.19 ms).
+template <uint32_t TW>
 __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 *__restrict__ colours,
                                                       float4 *__restrict__ canvas, float4 *__restrict__ ck,
                                                       uint32_t ck_pitch, uint64_t ck_stride, DevStatus *st,
@@ -753,7 +760,7 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
         for (uint32_t i = threadIdx.x; i < n_lb; i += blockDim.x) lb[i] = 0;
     }
     if (run_failed(st)) return;
-    const uint32_t tw = blockDim.x, pitch = tw + 1;
+    const uint32_t tw = TW ? TW : blockDim.x, pitch = tw + 1;
     const uint32_t X = blockIdx.x * tw + threadIdx.x, Y = blockIdx.y, im = blockIdx.z;
     const float xb0 = (float)(blockIdx.x * tw);
     const uint32_t k0 = S.img_first[im], np = S.img_first[im + 1] - k0;
@@ -781,7 +788,7 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
                 if (s + 2 < rounds) nref = piece_ref(S, R, s + 2, R.pb[(s + 2) * SEG] + threadIdx.x);
             }
             float A[SEG];
-            round_cover<true>(S, R, s, cur, first, (int)Y, xb0, s_cells, pitch, A, bad);
+            round_cover<true, TW>(S, R, s, cur, first, (int)Y, xb0, s_cells, A, bad);
             const uint32_t j0 = ja + s * SEG;
             const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
             if (ck && j0 && in) ck[(uint64_t)(j0 / SEG) * ck_stride + slot] = C;
@@ -938,11 +945,12 @@ __device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, floa
 // columns right of it from the prefix sums.  (Evaluating each piece on all 64
 // pixels of every wavefront it touches and reducing the three sums over the
 // wavefront took 18.4 ms for 64 images of 256x256 with 17,500 paths; this
-// form takes 3.6 ms, and 252 us instead of 869 for one 512x512 image of 256
+// form takes 3.0 ms, and 240 us instead of 869 for one 512x512 image of 256
 // paths.  Adding four vertex gradients per piece instead of EdgeGrad's two and
 // its ends took 4.5 ms and 332 us.)  Four wavefronts per SIMD are asked for: without, the kernel takes
 // 156 VGPRs, a CU holds three blocks, and the 1,024 blocks of a 512x512 image
 // run in two passes (370 us).
+template <uint32_t TW>
 __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4 *__restrict__ colours,
                                                        const float4 *__restrict__ grad_canvas,
                                                        const float4 *__restrict__ ck, uint32_t ck_pitch,
@@ -952,7 +960,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
     __shared__ RowLds R;
     __shared__ float s_gc[64];  // the round's colour gradients, in sum-tree order
     if (run_failed(st)) return;
-    const uint32_t tw = blockDim.x, pitch = tw + 1;
+    const uint32_t tw = TW ? TW : blockDim.x, pitch = tw + 1;
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t X = blockIdx.x * tw + threadIdx.x, Y = blockIdx.y, im = blockIdx.z;
     const float xb0 = (float)(blockIdx.x * tw);
@@ -989,7 +997,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                 if (s > 1) nref = piece_ref(S, R, s - 2, R.pb[(s - 2) * SEG] + threadIdx.x);
             }
             float A[SEG];
-            round_cover<false>(S, R, s, cur, piece_of(cv.p, cv.q, (int)Y), (int)Y, xb0, s_cells, pitch, A, bad);
+            round_cover<false, TW>(S, R, s, cur, piece_of(cv.p, cv.q, (int)Y), (int)Y, xb0, s_cells, A, bad);
             const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
             float q[SEG];  // f . canvas under path j
             // f . c_j - c_j.w q_j, made again in the second pass: kept beside q it
@@ -1013,6 +1021,8 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                 for (uint32_t h = 2; h-- > 0;) {
                     const uint32_t j = 2 * jp + h;
                     const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
+                    // (else the first pass's alpha and d stay in registers: 3.19 ms, 3.03 so)
+                    asm("" : "+v"(A[j]), "+v"(q[j]));
                     const float al = alpha_cover(A[j]);
                     const float dal = T * d_of(c, q[j]), V = T * al;
                     const bool part = (fabsf(A[j]) < 1.0f) & (A[j] != 0.0f);
@@ -1328,7 +1338,7 @@ ft_status launch_forward(ft_diff *d, const float *colours, float *canvas, bool k
     const uint32_t blocks = geometry_blocks(d);
     const uint32_t tw = tile_width(d);
     const size_t lds = (size_t)SEG * (tw + 1) * sizeof(int);
-    k_forward<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
+    (tw == TILE_MAX ? k_forward<TILE_MAX> : k_forward<0>)<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
         scene_of(d), reinterpret_cast<const float4 *>(colours), reinterpret_cast<float4 *>(canvas),
         keep ? d->d_ck : nullptr, d->ck_pitch, d->ck_stride, d->d_status, d->d_lb,
         blocks ? (uint32_t)lookback_words(blocks) : 0u, last ? d->h_status : nullptr);
@@ -1374,7 +1384,7 @@ ft_status launch_backward(ft_diff *d, const float *colours, const float *grad_ca
     DScene S = scene_of(d);
     const uint32_t tw = tile_width(d);
     const size_t lds = 2 * (size_t)SEG * (tw + 1) * sizeof(float);
-    k_backward<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
+    (tw == TILE_MAX ? k_backward<TILE_MAX> : k_backward<0>)<<<dim3(tiles_of(d), d->H, d->n_images), tw, lds, d->stream>>>(
         S, reinterpret_cast<const float4 *>(colours), reinterpret_cast<const float4 *>(grad_canvas), d->d_ck,
         d->ck_pitch, d->ck_stride, d->d_gedge, grad_colours, d->d_status);
     k_point_grad<<<grid_of((uint64_t)d->n_pts * DSEG), BLOCK, 0, d->stream>>>(

@@ -141,7 +141,7 @@ struct Workspace {
     std::vector<uint64_t> h_sp_store;  // h_status and h_pstate in arena mode
     bool pstate_copied = false;  // the status copy since the last launch included the path states
     bool status_owed = false;    // eager launches left their status on the device: ws_finish copies it
-    bool status_reported = false;  // the last eager launch's raster writes it to h_status itself
+    bool status_reported = false;  // the last eager launch writes it to h_status itself
     bool edges_counted = false;  // PathState::n_edges holds the last run's counts
     // band / LDS geometry of the next ws_set_batch: `tuning` as it stands when
     // `tuned` (ft_batch_set_tuning), else default_tuning's per path

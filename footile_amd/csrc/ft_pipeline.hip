@@ -769,17 +769,29 @@ __global__ __launch_bounds__(BLOCK) void k_bin(Limits L0, uint32_t band_shift, c
                                                const uint32_t *band_off, uint32_t *band_cur, uint32_t *band_list,
                                                uint64_t cap_pairs, const I2 *pts, const uint32_t *pt_run,
                                                const uint32_t *run_start, const uint32_t *run_end, PathState *ps,
-                                               DevStatus *st) {
+                                               DevStatus *st, HostStatus *report, PathState *report_ps) {
     __shared__ __align__(16) uint32_t s_h[BIN_WINDOW];
     __shared__ __align__(16) uint32_t s_base[BIN_WINDOW];
     __shared__ uint32_t s_w[BLOCK / 64];
+    // This kernel, the last before the raster, reports the run (not the raster
+    // itself, whose uniform reads a store in front of them makes vector loads);
+    // an error of the raster's reaches the host as a late one.
+    const bool reports = report && blockIdx.x == 0;
     Limits L = L0;
-    if (!run_begin(st, L)) return;
+    const bool fine = run_begin(st, L);
     const uint32_t n_pairs = L.n_pairs;
-    if (n_pairs > cap_pairs) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (!fine | (n_pairs > cap_pairs)) {
+        if (fine && blockIdx.x == 0 && threadIdx.x == 0) {
             atomicOr(&st->overflow, 2u);
             st->need_pairs = n_pairs;
+        }
+        if (reports) {
+            __syncthreads();
+            report_status(report, st, report_ps, ps, L0.n_paths);
+            if (fine && threadIdx.x == 0) {  // (the words just written, whatever copy of them the block read)
+                report->st.overflow = 2u;
+                report->st.need_pairs = n_pairs;
+            }
         }
         return;
     }
@@ -853,6 +865,7 @@ __global__ __launch_bounds__(BLOCK) void k_bin(Limits L0, uint32_t band_shift, c
         __syncthreads();
     }
     if (bad) raise_err(st, FT_EDEVICE);
+    if (reports) report_status(report, st, report_ps, ps, L0.n_paths);
 }
 
 // Edges per path over the stored points (reported on request, not needed by
@@ -1607,7 +1620,7 @@ template <int FMT, class Src, bool SPLIT = false>
 __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, const PathState &S, int fwd,
                                              uint32_t y0, uint32_t y1, Src src, uint32_t cnt, bool list_ok,
                                              const EdgeRec *edges, uint4 *s_dyn, uint32_t *s_segsum,
-                                             DevStatus *st, uint32_t &n_pairs_acc, uint32_t &n_adds_acc) {
+                                             bool &bad, uint32_t &n_pairs_acc, uint32_t &n_adds_acc) {
     constexpr bool HAS_LUT = FMT != FMT_MATTE8;
     constexpr uint32_t CR = cell_round<FMT>();
     uint4 *const lut = s_dyn;
@@ -1620,7 +1633,7 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
     const int64_t first = !has_pts ? (int64_t)H : (top_row > 0 ? top_row : 0);
     constexpr uint32_t fmt = FMT;
     if (P.fmt != fmt) {  // the block table groups paths by format
-        if (threadIdx.x == 0) raise_err(st, FT_EDEVICE);
+        bad = true;
         return;
     }
     const uint32_t bpp = fmt == FMT_RGBA8P ? 4 : (fmt == FMT_GRAYA8P ? 2 : 1);
@@ -1666,7 +1679,7 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
     // the group's rows in 32 bits: an edge's rows are within +-2^16, so a
     // raster row past 2^31 - 1 has none either way
     const int32_t g0 = ry0 < 0x7FFFFFFFu ? (int32_t)ry0 : 0x7FFFFFFF, g1 = y1 < 0x7FFFFFFFu ? (int32_t)y1 : 0x7FFFFFFF;
-    if (!list_ok && threadIdx.x == 0) raise_err(st, FT_EDEVICE);
+    bad |= !list_ok;
     // Cell pass, taller groups: the block takes CR list entries at a time; their
     // (edge, row) pairs are laid out by a scan of the rows per edge and spread
     // evenly over the threads (each finds its pair's edge by binary search in
@@ -1687,7 +1700,7 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
             for (uint32_t k = threadIdx.x; k < kn; k += BLOCK) {
                 const uint32_t ei = src(k0 + k);
                 const bool in = ei < L.cap_points;
-                if (!in) raise_err(st, FT_EDEVICE);
+                bad |= !in;
                 const EdgeRec E = edges[in ? ei : 0u];
                 const int32_t a = fx_int(E.y_upper) - shift, b = fx_int(E.y_lower) - shift;
                 if (in & ((E.flags & 1u) != 0) & (a < g1) & (b >= g0))
@@ -1740,7 +1753,7 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
         EdgeRec E[EB];
 #pragma unroll
         for (int j = 0; j < EB; ++j) {
-            if (ok[j] & (ei[j] >= L.cap_points)) raise_err(st, FT_EDEVICE);
+            bad |= ok[j] & (ei[j] >= L.cap_points);
             ok[j] = ok[j] & (ei[j] < L.cap_points);
             E[j] = edges[ok[j] ? ei[j] : 0u];
             ok[j] = ok[j] & ((E[j].flags & 1u) != 0);  // a point without an edge (path edge lists)
@@ -1769,7 +1782,7 @@ __device__ __forceinline__ void raster_group(const Limits &L, const PathDev &P, 
         const uint32_t k = k0 + threadIdx.x;
         bool okk = (threadIdx.x < CR) & (k < cnt);
         const uint32_t ei = src(okk ? k : 0u);
-        if (okk & (ei >= L.cap_points)) raise_err(st, FT_EDEVICE);
+        bad |= okk & (ei >= L.cap_points);
         okk = okk & (ei < L.cap_points);
         const EdgeRec E = edges[okk ? ei : 0u];
         okk = okk & ((E.flags & 1u) != 0);  // a point without an edge (path edge lists)
@@ -1919,15 +1932,14 @@ __global__ __launch_bounds__(BLOCK) void k_raster(Limits L0, const PathDev *path
                                                   uint32_t first_block, uint32_t band_shift,
                                                   const uint32_t *band_off, const uint32_t *band_list,
                                                   const EdgeRec *edges, const PathState *ps, DevStatus *st,
-                                                  unsigned long long *stats, HostStatus *report, PathState *report_ps) {
+                                                  unsigned long long *stats) {
     extern __shared__ uint4 s_dyn[];
     __shared__ uint32_t s_segsum[BLOCK / 64];
     __shared__ uint32_t s_stat[2 * BLOCK / 64];
-    // (blocks are ordered largest first: the last one has time to report)
-    if (report && blockIdx.x == gridDim.x - 1) report_status(report, st, report_ps, ps, L0.n_paths);
-    const uint4 rb = rblock[first_block + blockIdx.x];  // (in flight with the status)
-    Limits L = L0;
-    if (!run_begin(st, L)) return;
+    // (not run_begin: with it the two 4096x4096 fills take 59.4 us, 55.7 so)
+    if (run_failed(st)) return;
+    const Limits L = run_limits(st, L0.n_ops, L0.n_paths, L0.n_bands, L0.cap_points);
+    const uint4 rb = rblock[first_block + blockIdx.x];
     const uint32_t gb = rb.x, p = rb.z;
     if ((gb >= L.n_bands) | (p >= L.n_paths)) {
         if (threadIdx.x == 0) raise_err(st, FT_EDEVICE);
@@ -1943,14 +1955,18 @@ __global__ __launch_bounds__(BLOCK) void k_raster(Limits L0, const PathDev *path
     const uint32_t b1 = b0 + R < H ? b0 + R : H;
     const uint32_t y0 = b0 + rb.y * G;
     const uint32_t y1 = y0 + G < b1 ? y0 + G : b1;
+    bool bad = false;  // an index past its array
     uint32_t n_pairs = 0, n_adds = 0;
     if (y0 < y1) {
         const PathState S = ps[p];
         const bool list_ok = (off <= end) & (end <= L.n_pairs);
         raster_group<FMT>(L, P, S, (int)S.fwd, y0, y1, BandListSrc{band_list, off},
-                              list_ok ? end - off : 0u, list_ok, edges, s_dyn, s_segsum, st, n_pairs, n_adds);
+                              list_ok ? end - off : 0u, list_ok, edges, s_dyn, s_segsum, bad, n_pairs, n_adds);
     }
     block_stats(n_pairs, n_adds, stats, first_block + blockIdx.x, s_stat);
+    // (at the end: a raise within the raster's loops, two more stores that are
+    // never reached, made two 4096x4096 Rgba8p fills take 1 us longer)
+    if (bad) raise_err(st, FT_EDEVICE);
 }
 
 // The atlas tile scheduler: a persistent grid over the work items (path,
@@ -1974,6 +1990,7 @@ __global__ __launch_bounds__(BLOCK) void k_tiles(Limits L0, const PathDev *paths
     Limits L = L0;
     if (!run_begin(st, L)) return;
     uint32_t n_pairs = 0, n_adds = 0;
+    bool bad_index = false;
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
         if (threadIdx.x == 0) s_fwd = 0;
         const uint2 w = items[first_item + it];
@@ -1997,11 +2014,12 @@ __global__ __launch_bounds__(BLOCK) void k_tiles(Limits L0, const PathDev *paths
         __syncthreads();  // s_fwd
         if (y0 < y1)
             raster_group<FMT>(L, P, S, (int)s_fwd, y0, y1, PathEdgeSrc{S.pt_base},
-                                  (has_pts && list_ok) ? S.stored : 0u, list_ok, edges, s_dyn, s_segsum, st,
+                                  (has_pts && list_ok) ? S.stored : 0u, list_ok, edges, s_dyn, s_segsum, bad_index,
                                   n_pairs, n_adds);
         __syncthreads();  // the next item reuses the LDS and s_fwd
     }
     block_stats(n_pairs, n_adds, stats, stats_slot + blockIdx.x, s_stat);
+    if (bad_index) raise_err(st, FT_EDEVICE);
 }
 
 // ---------------------------------------------------------------------------
@@ -2613,10 +2631,12 @@ __global__ __launch_bounds__(BLOCK) void k_small_raster(PathDev P, const EdgeRec
     const uint32_t y1 = y0 + G < P.height ? y0 + G : P.height;
     const bool has_pts = S.topkey != NO_KEY && S.topidx != NO_IDX && n_kept <= SMALL_EVENTS;
     uint32_t n_pairs = 0, n_adds = 0;
+    bool bad = false;
     if (y0 < y1)
         raster_group<FMT, PathEdgeSrc, true>(L, P, S, (int)S.fwd, y0, y1, PathEdgeSrc{0u},
-                                                    has_pts ? n_kept : 0u, true, edges, s_dyn, s_segsum, st, n_pairs,
+                                                    has_pts ? n_kept : 0u, true, edges, s_dyn, s_segsum, bad, n_pairs,
                                                     n_adds);
+    if (bad) raise_err(st, FT_EDEVICE);
 }
 
 // ---------------------------------------------------------------------------
@@ -3266,20 +3286,16 @@ static inline uint32_t grid_for(size_t n) {
 static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool with_pstate, bool copy_status,
                             bool keep_failed, HostStatus *report);
 
-// Whether a run's raster kernel reports the status and the path states: its
-// blocks must not be several kernels' (one pixel format, no tile scheduler),
-// and the report is one block's stores over the bus, so the path states are
-// few: REPORT_PATHS of 40 bytes each (a copy costs the same from one path to
-// some hundreds).
+// Whether a run reports the status and the path states itself (k_bin): it has
+// bands and no tile scheduler, whose kernels come without k_bin, and the report
+// is one block's stores over the bus, so the path states are few: REPORT_PATHS
+// of 40 bytes each (a copy costs the same from one path to some hundreds).
 constexpr size_t REPORT_PATHS = 16;
 static bool reports_itself(const Workspace &ws, uint32_t mode) {
     if (ws.arena || ws.fstream || !ws.d_sp || (mode != MODE_FILL && mode != MODE_STROKE)) return false;
-    int kernels = 0;
-    for (int f = 0; f < 3; ++f) {
-        if (ws.n_bands && ws.rb_count[f]) ++kernels;
+    for (int f = 0; f < 3; ++f)
         if (ws.it_count[f]) return false;
-    }
-    return kernels == 1 && ws.n_paths && ws.n_paths <= REPORT_PATHS;
+    return ws.n_bands && ws.n_paths && ws.n_paths <= REPORT_PATHS;
 }
 
 // Enqueue one run.  In graph mode a fill run is captured once into a HIP
@@ -3288,6 +3304,7 @@ static bool reports_itself(const Workspace &ws, uint32_t mode) {
 ft_status ws_launch(Workspace &ws, uint32_t mode) {
     ws.edges_counted = false;
     ws.pstate_copied = false;
+    ws.status_reported = false;
     // block-index look-back: take turns with the other workspaces' runs
     std::unique_lock<std::mutex> turn;
     if (!ws.tickets && !ws.fstream) {
@@ -3309,9 +3326,8 @@ ft_status ws_launch(Workspace &ws, uint32_t mode) {
     if (!(ws.graph && mode == MODE_FILL) || ws.fstream) {
         // An eager run leaves its status (and path states) on the device:
         // ws_finish copies them once for all the launches before it, and a
-        // failed launch stays failed until then (keep_failed).  Where the
-        // raster is one kernel over few paths on the workspace's one stream,
-        // that kernel reports them itself (k_raster, report_status).
+        // failed launch stays failed until then (keep_failed).  A run of few
+        // paths on the workspace's one stream reports them itself.
         const bool keep = ws.status_owed;
         HostStatus *const report = reports_itself(ws, mode) ? reinterpret_cast<HostStatus *>(ws.h_status) : nullptr;
         const ft_status st = ws_enqueue(ws, mode, ev, false, false, keep, report);
@@ -3536,7 +3552,7 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
                                              n_slots, lb + 4 * tiles, &st->n_pairs, st, true, false, ws.tickets);
             (wide ? k_bin<4> : k_bin<1>)<<<ge, BLOCK, 0, s>>>(
                 L0, ws.band_shift, ws.d_pt_band, ws.d_band_off, ws.d_band_cur, ws.d_band_list, ws.cap_pairs, ws.d_pts,
-                ws.d_pt_run, ws.d_run_start, ws.d_run_end, ws.d_pstate, st);
+                ws.d_pt_run, ws.d_run_start, ws.d_run_end, ws.d_pstate, st, report, ws.h_pstate);
         }
         // The raster kernels: one per pixel format with band blocks, then the
         // tile scheduler per format with tile-mode items; the timing events
@@ -3582,18 +3598,17 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
             if (f == FT_MATTE8)
                 hipExtLaunchKernelGGL(k_raster<FMT_MATTE8>, grid, dim3(BLOCK), lds, s, e0, e1, 0, L0,
                                       ws.d_paths, ws.d_rblock, ws.rb_first[f], ws.band_shift, ws.d_band_off,
-                                      ws.d_band_list, ws.d_edges, ws.d_pstate, st, stats, report,
-                                      ws.h_pstate);
+                                      ws.d_band_list, ws.d_edges, ws.d_pstate, st, stats);
             else if (f == FT_RGBA8P)
                 hipExtLaunchKernelGGL(k_raster<FMT_RGBA8P>, grid,
                                       dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_rblock, ws.rb_first[f],
                                       ws.band_shift, ws.d_band_off, ws.d_band_list, ws.d_edges, ws.d_pstate, st,
-                                      stats, report, ws.h_pstate);
+                                      stats);
             else
                 hipExtLaunchKernelGGL(k_raster<FMT_GRAYA8P>, grid,
                                       dim3(BLOCK), lds, s, e0, e1, 0, L0, ws.d_paths, ws.d_rblock, ws.rb_first[f],
                                       ws.band_shift, ws.d_band_off, ws.d_band_list, ws.d_edges, ws.d_pstate, st,
-                                      stats, report, ws.h_pstate);
+                                      stats);
         }
         if (ev && n_rl == 0) {
             FT_HIP(hipEventRecord(ev[1], s));
@@ -3621,7 +3636,7 @@ static uint32_t take_late_err(Workspace &ws) {
 
 ft_status ws_finish(Workspace &ws, bool read_pstate) {
     const bool reported = ws.status_owed && ws.status_reported;
-    if (reported) {  // the last launch's raster wrote both to the host block
+    if (reported) {  // the last launch wrote both to the host block
         ws.pstate_copied = true;
         ws.status_owed = ws.status_reported = false;
     } else if (ws.status_owed) {  // the eager launches' status, with the path states when they share its block

@@ -57,7 +57,10 @@ struct DevAtom {
 
 __device__ inline void raise_err(DevStatus *st, uint32_t code) {
     atomicCAS(&st->err, 0u, code);
-    uint32_t *const h = st->host_err;
+    // (a global store: a flat one, through the generic pointer, makes the waits
+    // around it wait for the LDS too)
+    typedef __attribute__((address_space(1))) uint32_t gword;
+    gword *const h = (gword *)st->host_err;
     if (h) __hip_atomic_store(h, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

@@ -903,14 +903,22 @@ __device__ __forceinline__ float sum_dpp(float a, float b, bool hi) {
     return (hi ? b : a) + __builtin_bit_cast(float, got);
 }
 
-// Inclusive prefix sum over the 64 lanes.
-__device__ __forceinline__ float wave_incl_f32(float v) {
-    v = dpp_add<0x111, 0xf>(v);
-    v = dpp_add<0x112, 0xf>(v);
-    v = dpp_add<0x114, 0xf>(v);
-    v = dpp_add<0x118, 0xf>(v);
-    v = dpp_add<0x142, 0xa>(v);
-    return dpp_add<0x143, 0xc>(v);
+// Suffix sums within rows of 16 lanes (row_shl 1, 2, 4, 8): lane i's is the
+// sum of lanes i .. i | 15.
+__device__ __forceinline__ float row_suffix(float v) {
+    v = dpp_add<0x101, 0xf>(v);
+    v = dpp_add<0x102, 0xf>(v);
+    v = dpp_add<0x104, 0xf>(v);
+    return dpp_add<0x108, 0xf>(v);
+}
+
+// The sum of dA over the columns [t, 64) of a chunk from its 64 row suffixes.
+// Only columns at or right of t are added, so a sum whose terms are zero is
+// zero and a large (or unbounded) dA left of t does not touch it: as the
+// difference of two prefix sums of the chunk it kept their rounding.
+__device__ __forceinline__ float chunk_right(const float *suf, int t) {
+    const float r1 = suf[16], r2 = suf[32], r3 = suf[48];
+    return ((suf[t] + (t < 16 ? r1 : 0.0f)) + (t < 32 ? r2 : 0.0f)) + (t < 48 ? r3 : 0.0f);
 }
 
 // A piece's S1 = sum dA M, S2 = sum dA dM/dx_lo, S3 = sum dA dM/dx_hi terms
@@ -940,9 +948,9 @@ __device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, floa
 // the round; T runs backward.  So a path costs a pixel about 20 operations
 // beside its coverage, where re-compositing four channels cost twice that.
 //
-// The paths' dA and its prefix sums per 64-column chunk go to LDS, and one
-// thread per piece gathers its sums: the ramp's columns one by one, and all
-// columns right of it from the prefix sums.  (Evaluating each piece on all 64
+// The paths' dA and its suffix sums per 16 columns go to LDS, and one thread
+// per piece gathers its sums: the ramp's columns one by one, and all columns
+// right of it from the suffix sums (chunk_right).  (Evaluating each piece on all 64
 // pixels of every wavefront it touches and reducing the three sums over the
 // wavefront took 18.4 ms for 64 images of 256x256 with 17,500 paths; this
 // form takes 3.0 ms, and 240 us instead of 869 for one 512x512 image of 256
@@ -956,7 +964,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                                                        const float4 *__restrict__ ck, uint32_t ck_pitch,
                                                        uint64_t ck_stride, float4 *__restrict__ gedge,
                                                        float *__restrict__ gcol, DevStatus *st) {
-    extern __shared__ __align__(16) int s_cells[];  // cells, then the prefix sums of dA; then dA
+    extern __shared__ __align__(16) int s_cells[];  // cells, then the suffix sums of dA; then dA
     __shared__ RowLds R;
     __shared__ float s_gc[64];  // the round's colour gradients, in sum-tree order
     if (run_failed(st)) return;
@@ -967,8 +975,8 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
     const uint32_t k0 = S.img_first[im], np = S.img_first[im + 1] - k0;
     const uint64_t slot = ((uint64_t)im * S.H + Y) * ck_pitch + X;
     const bool in = X < S.W;
-    float *const s_pre = reinterpret_cast<float *>(s_cells);
-    float *const s_dA = s_pre + SEG * pitch;
+    float *const s_suf = reinterpret_cast<float *>(s_cells);
+    float *const s_dA = s_suf + SEG * pitch;
     uint32_t bad = 0;
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const float4 f = in ? grad_canvas[((uint64_t)im * S.H + Y) * S.W + X] : zero;
@@ -1033,7 +1041,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                     r[h][3] = V * (f.w - q[j]);
                     T *= fmaf(-c.w, al, 1.0f);
                     s_dA[j * pitch + tid] = dA;
-                    s_pre[j * pitch + tid] = wave_incl_f32(dA);
+                    s_suf[j * pitch + tid] = row_suffix(dA);
                 }
                 const float x0 = sum2(r[0][0], r[1][0]), x1 = sum2(r[0][1], r[1][1]);
                 const float x2 = sum2(r[0][2], r[1][2]), x3 = sum2(r[0][3], r[1][3]);
@@ -1096,8 +1104,8 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                 }
                 if (m.live) {  // the columns right of the ramp
                     const int t = m.c1 > m.c0 ? m.c1 : m.c0;
-                    if (t < (int)tw) S1 += s_pre[at + (t | 63)] - ((t & 63) ? s_pre[at + t - 1] : 0.0f);
-                    for (int c = (t | 63) + 64; c < (int)tw; c += 64) S1 += s_pre[at + c];
+                    if (t < (int)tw) S1 += chunk_right(s_suf + at + (t & ~63), t & 63);
+                    for (int c = (t | 63) + 1; c < (int)tw; c += 64) S1 += chunk_right(s_suf + at + c, 0);
                     if ((S1 != 0.0f) | (S2 != 0.0f) | (S3 != 0.0f)) {
                         const bool flip = pc.xa < pc.xb;  // S2 goes with the larger x
                         const EdgeGrad g =

@@ -1,0 +1,62 @@
+"""Gradients of the differentiable fill that large ones beside them must not
+touch, component by component against FP64."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _line_cubics(corners):
+    """Control points of a path along straight lines through `corners`."""
+    c = np.asarray(corners, np.float64)
+    out = [c[:1]]
+    for a, b in zip(c[:-1], c[1:]):
+        out.append(np.stack([a + (b - a) / 4.0, a + (b - a) * 0.75, b]))
+    return np.concatenate(out)
+
+
+def _grads(w, h, cubics, points, colours, cotangent):
+    """d points, d colours on the GPU and in FP64."""
+    from footile_amd.diff import DiffRenderer, device_array
+    from footile_amd.plotter import DeviceBuffer
+    from oracle import pydiff as pd
+    image, cubics = np.zeros(len(cubics), np.uint32), np.asarray(cubics, np.uint32)
+    points, colours = points.astype(np.float32), np.asarray(colours, np.float32)
+    r = DiffRenderer(1, w, h, image, cubics)
+    gp, gc = DeviceBuffer(8 * r.n_points), DeviceBuffer(16 * r.n_paths)
+    r.backward(device_array(points), device_array(colours), device_array(cotangent), gp, gc)
+    _, want_gp, want_gc = pd.Scene(1, w, h, image, cubics).backward(points, colours, grad_canvas=cotangent)
+    return (gp.download(dtype=np.float32).reshape(-1, 2), gc.download(dtype=np.float32).reshape(-1, 4), want_gp,
+            want_gc)
+
+
+@pytest.mark.parametrize("size", [1.0e6, np.inf])
+# the second figure's left side: right after the first's, at either side of a
+# row of 16 and of a chunk of 64 columns, in a later chunk and a later tile
+@pytest.mark.parametrize("left", [9, 15, 16, 31, 47, 48, 62, 63, 64, 100, 127, 200, 255, 256, 300])
+def test_large_cotangent_left_of_an_edge(oracle, size, left):
+    """One path of two figures, joined by horizontal edges (which have no
+    pieces).  A large cotangent on a pixel of the first figure's left side, in
+    the row of the second figure's top corners, whose y gradients no edge
+    beside them cancels; cotangents of 1 in every pixel the second figure
+    crosses.  The gradients of the second figure's points are sums of at most
+    10 rows of 12 pixels, each of order 1: 1e-5 of the largest, with vertex
+    rounding (2^-24 of coordinates up to 320, 2e-5 of a pixel) on top.  FP64
+    takes the large pixel as 0: it lies left of them all."""
+    w, h = 320, 20
+    a, b = left + 0.375, left + 9.75
+    corners = [(4.5, 2.0), (4.25, 17.0), (7.5, 17.0), (a + 1.0, 17.0), (b, 17.0), (b - 1.0, 8.25), (a, 8.25),
+               (a + 1.0, 17.0), (7.5, 17.0), (7.25, 2.0), (4.5, 2.0)]
+    pts = _line_cubics(corners)
+    cubics, colours = [len(corners) - 1], [[0.3, 0.2, 0.1, 0.5]]
+    cot = np.zeros((1, h, w, 4), np.float32)
+    cot[0, 8:17, left:left + 11] = 1.0
+    _, _, want, _ = _grads(w, h, cubics, pts, colours, cot)
+    cot[0, 8, 4] = size
+    with np.errstate(invalid="ignore"):
+        gp, _, _, _ = _grads(w, h, cubics, pts, colours, cot)
+    # the points of the second figure's cubics: its bottom, right side, top and left side
+    own = np.arange(3 * 3 + 1, 3 * 7)
+    assert np.isfinite(gp[own]).all()
+    assert np.abs(want[own]).max() > 1.0
+    assert np.abs(gp[own] - want[own]).max() < 1e-4 * np.abs(want[own]).max()

@@ -429,11 +429,17 @@ __global__ __launch_bounds__(BLOCK) void k_fill_cells(DScene S, DevStatus *st) {
 //
 // Cells are integers in units of 2^-26 (an i32 add): the sum does not depend
 // on the order of the pieces, so the same inputs give the same canvas
-// whichever kernel computes it, and each column's value is rounded once, at
-// 2^-27, where a float sum rounds at every piece.  (At 2^-24 a pixel that an
-// edge covers by less than 2^-25 lost its gradient: 8.2e-6 from FP64 on a
-// 512x512 scene whose gradients are 4.4e-6 off otherwise.)  i32 holds
-// |A| < 32; a (path, row) with more than HEAVY pieces takes 64-bit cells.
+// whichever kernel computes it, and a column of n pieces is within n 2^-27 of
+// its products' sum.  i32 holds |A| < 32; a (path, row) with more than HEAVY
+// pieces takes 64-bit cells of 2^-38.
+//
+// A pixel has a gradient only where its coverage is not 0, so a column that a
+// ramp touches by less than 2^-27 would lose it (the tip of a figure that
+// reaches 1e-4 into a pixel has a gradient of 1e-4 there).  A path of which a
+// ramp column is nonzero and under TINY therefore takes 64-bit cells too, of
+// 2^-56: about one round of paths in 30 has one.  (At cells of 2^-24 for all,
+// without this, gradients of a 512x512 scene were 8.2e-6 from FP64 instead of
+// 4.4e-6.)
 //
 // Every 64-column chunk of a row stands alone: a piece left of a chunk adds
 // its whole signed height to the chunk's first cell, so no carry passes
@@ -447,14 +453,18 @@ constexpr uint32_t TILE_MAX = 256;
 constexpr uint32_t ROW_PATHS = 256;  // paths whose cell counts are staged at once
 constexpr uint32_t HEAVY = 31;       // pieces of one path in one row past which cells are 64-bit
 constexpr int RAMP_LANE = 8;         // ramps of at most this many columns are walked by one lane
-constexpr float CELL_ONE = 67108864.0f;  // 2^26
+constexpr float CELL_ONE = 0x1p26f;
+constexpr float HEAVY_ONE = 0x1p38f;     // at most 2^24 pieces: |A| < 2^24
+constexpr float FINE_ONE = 0x1p56f;      // at most HEAVY pieces: |A| < 32
+constexpr float TINY = 0x1p4f;           // of CELL_ONE: a share of 2^-22
 
 struct RowLds {
     __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of the staged paths' piece counts, then the total
     uint32_t dl[ROW_PATHS];                    // list position of a path's piece e: dl + e
     uint32_t vb[ROW_PATHS + 1];                // first vertices
     uint32_t marks[ROW_PATHS / SEG];           // per round: bit j, path j has pieces; bit 16 + j, it is heavy
-    uint32_t poison[2];                        // per round parity: bit j, path j has a piece that is no number here
+    uint32_t poison[2];                        // per round parity: bit j, path j has a piece that is no number
+                                               // here; bit 16 + j, one of a TINY share
 };
 
 // Counts and list offsets of row Y for the n <= ROW_PATHS paths from global
@@ -578,9 +588,17 @@ __device__ __forceinline__ float ramp_cover(const Ramp &m, float X1) {
     return ramp_mean(m, X1, a, b);
 }
 
+// v: a share in cell units, |v| at most a cell's one.
 template <typename T>
-__device__ __forceinline__ T cell_of(float zs, float M) {
-    return (T)__float2int_rn(zs * M);  // |zs * M| <= 2^26
+__device__ __forceinline__ T cell_of(float v) {
+    if constexpr (sizeof(T) == 8)
+        return __float2ll_rn(v);
+    else
+        return __float2int_rn(v);
+}
+// 0 < |v| < TINY
+__device__ __forceinline__ bool tiny_share(float v) {
+    return (__builtin_bit_cast(uint32_t, v) & 0x7FFFFFFFu) - 1u < __builtin_bit_cast(uint32_t, TINY) - 1u;
 }
 template <typename T>
 __device__ __forceinline__ void cell_add(T *c, T v) {
@@ -591,18 +609,23 @@ __device__ __forceinline__ void cell_add(T *c, T v) {
 }
 
 // Adds one piece per lane to its path's row of cells (row; the wavefront's
-// lanes all call it, those without a piece with m.live false).  A ramp of
-// more than RAMP_LANE columns is evaluated by the whole wavefront, one column
-// per lane, so that one long near-horizontal piece does not hold up 63 lanes.
+// lanes all call it, those without a piece with m.live false), in units of
+// 1 / one.  A ramp of more than RAMP_LANE columns is evaluated by the whole
+// wavefront, one column per lane, so that one long near-horizontal piece does
+// not hold up 63 lanes.  Returns whether a ramp column of the piece has a TINY
+// share.
 template <typename T>
-__device__ __forceinline__ void scatter_piece(T *cells, uint32_t row_at, const Ramp &m, float xb0, int tw) {
-    const float zs = m.z * CELL_ONE;
+__device__ __forceinline__ bool scatter_piece(T *cells, uint32_t row_at, const Ramp &m, float xb0, int tw, float one) {
+    const float zs = m.z * one;
     const int n = m.c1 - m.c0;
     const bool wide = m.live & (n > RAMP_LANE);
+    bool tiny = false;
     T prev = 0;
     if (m.live & !wide) {
         for (int c = m.c0; c < m.c1; ++c) {
-            const T q = cell_of<T>(zs, ramp_cover(m, xb0 + (float)(c + 1)));
+            const float v = zs * ramp_cover(m, xb0 + (float)(c + 1));
+            const T q = cell_of<T>(v);
+            tiny |= tiny_share(v);
             cell_add(&cells[row_at + c], q - ((c & 63) ? prev : (T)0));
             prev = q;
         }
@@ -623,19 +646,24 @@ __device__ __forceinline__ void scatter_piece(T *cells, uint32_t row_at, const R
         const int w0 = __builtin_amdgcn_readlane(m.c0, l), w1 = __builtin_amdgcn_readlane(m.c1, l);
         const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)row_at, l);
         const int lane = threadIdx.x & 63;
+        bool any = false;
         for (int c = w0 + lane; c < w1; c += 64) {
-            const T q = cell_of<T>(wz, ramp_cover(w, xb0 + (float)(c + 1)));
-            const T b = ((c > w0) & ((c & 63) != 0)) ? cell_of<T>(wz, ramp_cover(w, xb0 + (float)c)) : (T)0;
+            const float v = wz * ramp_cover(w, xb0 + (float)(c + 1));
+            const T q = cell_of<T>(v);
+            const T b = ((c > w0) & ((c & 63) != 0)) ? cell_of<T>(wz * ramp_cover(w, xb0 + (float)c)) : (T)0;
+            any |= tiny_share(v);
             cell_add(&cells[at + c], q - b);
         }
+        tiny |= (lane == l) & (__ballot(any) != 0ull);
     }
-    if (!m.live) return;
-    if (wide) prev = cell_of<T>(zs, ramp_cover(m, xb0 + (float)m.c1));  // the last ramp column's value
+    if (!m.live) return false;
+    if (wide) prev = cell_of<T>(zs * ramp_cover(m, xb0 + (float)m.c1));  // the last ramp column's value
     // from the column after the ramp on: whole
-    const T whole = cell_of<T>(zs, 1.0f);
+    const T whole = cell_of<T>(zs);
     const int t = m.c1 > m.c0 ? m.c1 : m.c0;
     if (t < tw) cell_add(&cells[row_at + t], whole - ((t & 63) ? prev : (T)0));
     for (int c = (t | 63) + 1; c < tw; c += 64) cell_add(&cells[row_at + c], whole);
+    return tiny;
 }
 
 // Coverage A[j] of round s's paths at this thread's pixel, from the first
@@ -651,35 +679,6 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
     const uint32_t pitch = (uint32_t)tw + 1;
     const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];
     const uint32_t heavy = R.marks[s] >> 16;
-#pragma unroll
-    for (uint32_t j = 0; j < SEG; ++j) A[j] = 0.0f;
-    if (heavy) {  // (uniform) one heavy path at a time, in 64-bit cells over the same LDS
-        long long *c64 = reinterpret_cast<long long *>(cells);
-        for (uint32_t j = 0; j < SEG; ++j) {
-            if (!((heavy >> j) & 1u)) continue;
-            c64[tid] = 0;
-            __syncthreads();
-            const uint32_t e0 = R.pb[s * SEG + j], e1 = R.pb[s * SEG + j + 1];
-            for (uint32_t eb = e0; eb < e1; eb += (uint32_t)tw) {  // whole blocks: scatter_piece is collective
-                const uint32_t e = eb + (uint32_t)tid;
-                PieceRef r = piece_ref(S, R, s, e < e1 ? e : NO_IDX);
-                const PieceVtx u = piece_vtx(S, R, s, r, bad);
-                Piece pc = piece_of(u.p, u.q, Y);
-                pc.live &= r.j != NO_IDX;
-                const Ramp m = ramp_of(pc, xb0, tw);
-                if (m.nan) atomicOr(&R.poison[s & 1], 1u << j);
-                scatter_piece<long long>(c64, 0u, m, xb0, tw);
-            }
-            __syncthreads();
-            const long long sum = (long long)wave_incl_t<unsigned long long, false>((unsigned long long)c64[tid]);
-            const float a = (float)sum * (1.0f / CELL_ONE);
-#pragma unroll
-            for (uint32_t k = 0; k < SEG; ++k) A[k] = k == j ? a : A[k];
-            __syncthreads();
-        }
-        c64[tid] = 0;
-        __syncthreads();
-    }
     for (uint32_t eb = base; eb < end; eb += (uint32_t)tw) {
         if (eb + ((uint32_t)tid & ~63u) >= end) break;  // no piece for this wavefront
         PieceRef r = ref;
@@ -693,8 +692,8 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
         const uint32_t j = r.j != NO_IDX ? r.j : 0u;
         pc.live &= ((heavy >> j) & 1u) == 0u;
         const Ramp m = ramp_of(pc, xb0, tw);
-        if (m.nan) atomicOr(&R.poison[s & 1], 1u << j);
-        scatter_piece<int>(cells, j * pitch, m, xb0, tw);
+        const bool tiny = scatter_piece<int>(cells, j * pitch, m, xb0, tw, CELL_ONE);
+        if (m.nan | tiny) atomicOr(&R.poison[s & 1], (m.nan ? 1u : 0x10000u) << j);
     }
     __syncthreads();
     uint32_t c[SEG];
@@ -703,20 +702,42 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
         c[j] = (uint32_t)cells[j * pitch + tid];
         if (ZERO) cells[j * pitch + tid] = 0;
     }
-    const uint32_t poison = R.poison[s & 1];
-    if (tid == 0) R.poison[(s + 1) & 1] = 0;
-    float light[SEG];
 #pragma unroll
-    for (uint32_t j = 0; j < SEG; ++j) light[j] = (float)(int)wave_incl_dpp<false>(c[j]) * (1.0f / CELL_ONE);
-    if (heavy) {
+    for (uint32_t j = 0; j < SEG; ++j) A[j] = (float)(int)wave_incl_dpp<false>(c[j]) * (1.0f / CELL_ONE);
+    uint32_t poison = R.poison[s & 1];
+    const uint32_t wide = heavy | (poison >> 16);
+    if (wide) {  // (uniform) one path at a time, in 64-bit cells over the same LDS
+        long long *c64 = reinterpret_cast<long long *>(cells);
+        for (uint32_t j = 0; j < SEG; ++j) {
+            if (!((wide >> j) & 1u)) continue;
+            const float one = ((heavy >> j) & 1u) ? HEAVY_ONE : FINE_ONE;
+            __syncthreads();  // the cells, or the path before's, are read
+            c64[tid] = 0;
+            __syncthreads();
+            const uint32_t e0 = R.pb[s * SEG + j], e1 = R.pb[s * SEG + j + 1];
+            for (uint32_t eb = e0; eb < e1; eb += (uint32_t)tw) {  // whole blocks: scatter_piece is collective
+                const uint32_t e = eb + (uint32_t)tid;
+                PieceRef r = piece_ref(S, R, s, e < e1 ? e : NO_IDX);
+                const PieceVtx u = piece_vtx(S, R, s, r, bad);
+                Piece pc = piece_of(u.p, u.q, Y);
+                pc.live &= r.j != NO_IDX;
+                const Ramp m = ramp_of(pc, xb0, tw);
+                if (m.nan) atomicOr(&R.poison[s & 1], 1u << j);
+                (void)scatter_piece<long long>(c64, 0u, m, xb0, tw, one);
+            }
+            __syncthreads();
+            const long long sum = (long long)wave_incl_t<unsigned long long, false>((unsigned long long)c64[tid]);
+            const float a = (float)sum / one;
 #pragma unroll
-        for (uint32_t j = 0; j < SEG; ++j) A[j] = ((heavy >> j) & 1u) ? A[j] : light[j];
-    } else {
-#pragma unroll
-        for (uint32_t j = 0; j < SEG; ++j) A[j] = light[j];
+            for (uint32_t k = 0; k < SEG; ++k) A[k] = k == j ? a : A[k];
+        }
+        __syncthreads();
+        if (ZERO) c64[tid] = 0;
+        poison = R.poison[s & 1];
     }
+    if (tid == 0) R.poison[(s + 1) & 1] = 0;
     // a piece without an x takes its path's whole row (coverage past 1, and so no gradient)
-    if (poison) {
+    if (poison & 0xFFFFu) {
 #pragma unroll
         for (uint32_t j = 0; j < SEG; ++j) A[j] = ((poison >> j) & 1u) ? 2.0f : A[j];
     }

@@ -60,3 +60,28 @@ def test_large_cotangent_left_of_an_edge(oracle, size, left):
     assert np.isfinite(gp[own]).all()
     assert np.abs(want[own]).max() > 1.0
     assert np.abs(gp[own] - want[own]).max() < 1e-4 * np.abs(want[own]).max()
+
+
+@pytest.mark.parametrize("x0", [8, 64, 256])  # inside a chunk, at a chunk's and a tile's border
+@pytest.mark.parametrize("eps", [2.0 ** -10, 2.0 ** -13, 2.0 ** -14])
+@pytest.mark.parametrize("flip", [False, True])
+def test_sliver_of_a_pixel_keeps_its_gradient(oracle, x0, eps, flip):
+    """A tip that reaches `eps` into the pixel left of column x0 and covers
+    0.21 eps^2 of it, down to 7.8e-10 (each of the tip's two edges half of
+    that), at either orientation, between a path below and one above it: the
+    pixel's value and the gradients of its cotangent, component by component.
+    The tip's x is off by at most 2^-21 below column 8 and by less of the
+    spacing of float32 right of that (2^-7 of the smallest eps), the coverage
+    by twice that: 3 %."""
+    w, h = 300, 9
+    corners = [(x0 - eps, 4.5), (x0 + 6.0, 5.75), (x0 + 6.0, 3.25), (x0 - eps, 4.5)]
+    box = [(x0 - 4.0, 1.5), (x0 - 4.0, 7.5), (x0 + 9.0, 7.5), (x0 + 9.0, 1.5), (x0 - 4.0, 1.5)]
+    pts = np.concatenate([_line_cubics(box), _line_cubics(corners[::-1] if flip else corners), _line_cubics(box)])
+    cubics, colours = [4, 3, 4], [[0.1, 0.3, 0.2, 0.4], [0.3, 0.2, 0.1, 0.5], [0.2, 0.1, 0.3, 0.6]]
+    cot = np.zeros((1, h, w, 4), np.float32)
+    cot[0, 4, x0 - 1] = [1.0, 0.5, -0.25, 0.75]
+    gp, gc, want_gp, want_gc = _grads(w, h, cubics, pts, colours, cot)
+    own = slice(13, 23)
+    assert np.abs(want_gp[own]).max() > 0.01 * eps
+    assert np.abs(gp[own] - want_gp[own]).max() < 0.03 * np.abs(want_gp[own]).max()
+    assert np.abs(gc[1] - want_gc[1]).max() < 0.03 * np.abs(want_gc[1]).max()

@@ -173,8 +173,7 @@ __global__ __launch_bounds__(BLOCK) void k_vertices(DScene S, const float2 *poin
 __global__ __launch_bounds__(BLOCK) void k_clear_run(unsigned long long *lb, uint32_t n_lb, DevStatus *st,
                                                      uint32_t *host_err) {
     for (uint32_t i = threadIdx.x; i < n_lb; i += BLOCK) lb[i] = 0;
-    if (threadIdx.x < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
-    if (threadIdx.x == 0) st->host_err = host_err;  // (one wavefront: after the words above)
+    status_begin(st, threadIdx.x, host_err);
 }
 
 // Rows [r0, r1] an edge overlaps within [0, H); false when none.
@@ -214,8 +213,7 @@ __global__ __launch_bounds__(BLOCK) void k_clear_cells(DScene S, float4 *gedge, 
         if (gedge && i < S.n_vtx) gedge[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (gcol && i < 4 * S.n_paths) gcol[i] = 0.0f;
     }
-    if (blockIdx.x == 0 && threadIdx.x < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->host_err = host_err;  // (one wavefront: after the words above)
+    if (blockIdx.x == 0) status_begin(st, threadIdx.x, host_err);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_rows(DScene S, DevStatus *st) {

@@ -118,11 +118,15 @@ __global__ __launch_bounds__(BLOCK) void k_clear(PathState *ps, unsigned long lo
     // The status (one wavefront's words): with keep_failed, a failed earlier
     // launch whose status the host has not read yet stays failed, so this
     // launch's kernels skip their work and the failure reaches the next read.
-    static_assert(sizeof(DevStatus) / 4 <= 64, "the status is one wavefront's words");
-    if (blockIdx.x == 0 && threadIdx.x < sizeof(DevStatus) / 4) {
-        const bool failed = (keep_failed != 0u) & ((st->err | st->overflow) != 0u);
-        if (!failed) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0;
-        if (threadIdx.x == 0) st->host_err = host_err;  // (one wavefront: after the words above)
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        // (each lane reads its own word before any is cleared: err is word 0, overflow word 1)
+        static_assert(offsetof(DevStatus, err) == 0 && offsetof(DevStatus, overflow) == 4, "lanes 0 and 1");
+        const bool set = (threadIdx.x < 2) && reinterpret_cast<const uint32_t *>(st)[threadIdx.x] != 0u;
+        const bool failed = (keep_failed != 0u) & (__ballot(set) != 0ull);
+        if (!failed)
+            status_begin(st, threadIdx.x, host_err);
+        else if (threadIdx.x == 0)
+            st->host_err = host_err;
     }
 }
 
@@ -2464,9 +2468,8 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
                                                         DevStatus *st, HostStatus *host, PathState *host_ps) {
     __shared__ SmallLds S;
     const uint32_t tid = threadIdx.x;
-    if (tid < sizeof(DevStatus) / 4) reinterpret_cast<uint32_t *>(st)[tid] = 0;
+    status_begin(st, tid, &host->late_err);
     if (tid == 0) {
-        st->host_err = &host->late_err;  // (one wavefront: after the words above)
         host->st.err = 0;
         host->st.overflow = 0;
         S.path = P;

@@ -4,9 +4,11 @@
 // the bounds-checked host build of the stage code (tests/cpu_mirror).
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/footile_hip.h"
+#include "ft_device.h"
 
 namespace ft {
 
@@ -86,6 +88,21 @@ struct DevStatus {
     uint32_t pad;
     uint32_t *host_err;  // a pinned host word that also receives `err` when it is raised (null: none)
 };
+
+// A run's start: the status zero but for host_err.  Lane `i` of one wavefront
+// (of STATUS_LANES or more) writes its own word and no other lane's: zeroing
+// every word and storing the pointer over two of them from another lane would
+// leave it to the compiler which of the two stores lasts, and a run that
+// reports itself would lose a raster's error with the pointer.
+constexpr uint32_t STATUS_LANES = (uint32_t)(offsetof(DevStatus, host_err) / sizeof(uint32_t)) + 1;
+static_assert(sizeof(DevStatus) == offsetof(DevStatus, host_err) + sizeof(uint32_t *) && STATUS_LANES <= 64,
+              "host_err is the last member");
+FT_HD inline void status_begin(DevStatus *st, uint32_t i, uint32_t *host_err) {
+    if (i + 1 < STATUS_LANES)
+        reinterpret_cast<uint32_t *>(st)[i] = 0;
+    else if (i + 1 == STATUS_LANES)
+        st->host_err = host_err;
+}
 
 struct EdgeRec {
     int32_t y_upper, y_lower, x_bot0, inv, step;

@@ -456,49 +456,70 @@ constexpr float HEAVY_ONE = 0x1p38f;     // at most 2^24 pieces: |A| < 2^24
 constexpr float FINE_ONE = 0x1p56f;      // at most HEAVY pieces: |A| < 32
 constexpr float TINY = 0x1p4f;           // of CELL_ONE: a share of 2^-22
 
+// The paths of a staging round that have pieces in the row, in path order:
+// only they are rounded up to SEG and walked.  (A path without pieces leaves
+// the row's canvas as it is.  With all paths walked, a scene of small figures
+// paid for every figure in every row: 1,024 of 24 pixels in 512x512 took 271
+// us a forward and 790 a step, now 73 and 146; 256 paths across the image 113
+// and 349, now 109 and 333.)
 struct RowLds {
-    __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of the staged paths' piece counts, then the total
+    __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of their piece counts, then the total
+    __align__(16) uint8_t path[ROW_PATHS];     // their index among the staged paths; 0 past the last
     uint32_t dl[ROW_PATHS];                    // list position of a path's piece e: dl + e
-    uint32_t vb[ROW_PATHS + 1];                // first vertices
-    uint32_t marks[ROW_PATHS / SEG];           // per round: bit j, path j has pieces; bit 16 + j, it is heavy
+    uint32_t vb[ROW_PATHS], vn[ROW_PATHS];     // first vertex and number of vertices
+    uint32_t heavy[ROW_PATHS / SEG];           // per round: bit j, its path j has more than HEAVY pieces
     uint32_t poison[2];                        // per round parity: bit j, path j has a piece that is no number
                                                // here; bit 16 + j, one of a TINY share
+    uint32_t n;                                // how many
 };
 
-// Counts and list offsets of row Y for the n <= ROW_PATHS paths from global
-// path kbase.  Every thread calls it, between barriers of the caller.
+// Row Y of the n <= ROW_PATHS paths from global path kbase.  Every thread
+// calls it, between barriers of the caller.
 __device__ void stage_row(const DScene &S, uint32_t kbase, uint32_t n, int Y, RowLds &R) {
     const uint32_t lane = threadIdx.x;
-    if (lane < 64) {
-        uint32_t c[4], o[4], sum = 0, nib = 0;
+    if (lane >= 64) return;
+    uint32_t c[4], o[4], v[5], sum = 0, live = 0;
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            const uint32_t p = 4 * lane + i;
-            const uint64_t cell = (uint64_t)(kbase + (p < n ? p : 0u)) * S.H + (uint32_t)Y;
-            c[i] = p < n ? S.cell_cnt[cell] : 0u;
-            o[i] = S.cell_off[cell];
-        }
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t p = 4 * lane + i;
+        const uint64_t cell = (uint64_t)(kbase + (p < n ? p : 0u)) * S.H + (uint32_t)Y;
+        c[i] = p < n ? S.cell_cnt[cell] : 0u;
+        o[i] = S.cell_off[cell];
+    }
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            sum += c[i];
-            nib |= ((c[i] ? 1u : 0u) | (c[i] > HEAVY ? 0x10000u : 0u)) << i;
-        }
-        const uint32_t incl = wave_incl_dpp<false>(sum);
-        uint32_t pre = incl - sum;
+    for (uint32_t i = 0; i < 5; ++i) v[i] = S.vtx_off[kbase + (4 * lane + i < n ? 4 * lane + i : n)];
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            R.pb[4 * lane + i] = pre;
-            R.dl[4 * lane + i] = o[i] - pre;
+    for (uint32_t i = 0; i < 4; ++i) {
+        sum += c[i];
+        live += c[i] ? 1u : 0u;
+    }
+    const uint32_t incl = wave_incl_dpp<false>(sum), rank1 = wave_incl_dpp<false>(live);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    const uint32_t n_live = (uint32_t)__builtin_amdgcn_readlane((int)rank1, 63);
+    uint32_t pre = incl - sum, rank = rank1 - live;
+    if (lane < ROW_PATHS / SEG) R.heavy[lane] = 0;
+    if (lane < 2) R.poison[lane] = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        if (c[i]) {
+            R.pb[rank] = pre;
+            R.path[rank] = (uint8_t)(4 * lane + i);
+            R.dl[rank] = o[i] - pre;
+            R.vb[rank] = v[i];
+            R.vn[rank] = v[i + 1] - v[i];
+            if (c[i] > HEAVY) atomicOr(&R.heavy[rank / SEG], 1u << (rank % SEG));
+            ++rank;
             pre += c[i];
         }
-        if (lane == 63) R.pb[ROW_PATHS] = incl;
-        uint32_t h = nib << (4 * (lane & 3));
-        h |= (uint32_t)__shfl_xor((int)h, 1, 64);
-        h |= (uint32_t)__shfl_xor((int)h, 2, 64);
-        if ((lane & 3) == 0) R.marks[lane >> 2] = h;
-        if (lane < 2) R.poison[lane] = 0;
+        if (4 * lane + i >= n_live) {
+            R.pb[4 * lane + i] = total;
+            R.path[4 * lane + i] = 0;
+        }
     }
-    for (uint32_t p = threadIdx.x; p <= n; p += blockDim.x) R.vb[p] = S.vtx_off[kbase + p];
+    if (lane == 63) {
+        R.pb[ROW_PATHS] = total;
+        R.n = n_live;
+    }
 }
 
 // Piece e of round s (staged paths [s * SEG, s * SEG + SEG)).
@@ -533,7 +554,7 @@ struct PieceVtx {
 __device__ __forceinline__ PieceVtx piece_vtx(const DScene &S, const RowLds &R, uint32_t s, const PieceRef &r,
                                               uint32_t &bad) {
     const uint32_t t = s * SEG + (r.j != NO_IDX ? r.j : 0u);
-    const uint32_t vb = R.vb[t], V = R.vb[t + 1] - vb;
+    const uint32_t vb = R.vb[t], V = R.vn[t];
     bad |= r.edge < V ? 0u : 1u;
     const uint32_t e = r.edge < V ? r.edge : 0u;
     PieceVtx v;
@@ -676,7 +697,7 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
     const int tid = threadIdx.x, tw = TW ? (int)TW : (int)blockDim.x;
     const uint32_t pitch = (uint32_t)tw + 1;
     const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];
-    const uint32_t heavy = R.marks[s] >> 16;
+    const uint32_t heavy = R.heavy[s];
     for (uint32_t eb = base; eb < end; eb += (uint32_t)tw) {
         if (eb + ((uint32_t)tid & ~63u) >= end) break;  // no piece for this wavefront
         PieceRef r = ref;
@@ -744,22 +765,40 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
 
 __device__ __forceinline__ float alpha_cover(float A) { return __builtin_amdgcn_fmed3f(fabsf(A), 0.0f, 1.0f); }
 
-// Colour of the image's path j, or zero where `on` is 0 (a path without
-// pieces in the row does not touch it, whatever its colour).  Uniform: scalar
-// loads, and no branch between a round's paths.
-__device__ __forceinline__ float4 round_colour(const float4 *__restrict__ colours, uint32_t k0, uint32_t np,
-                                               uint32_t j, uint32_t on) {
-    const float4 c = colours[k0 + (j < np ? j : np - 1)];
-    const uint32_t m = 0u - on;
+// The paths of round s: their number, and their index among the staged paths
+// (path j's: byte j), uniform.
+struct RoundPaths {
+    uint32_t n, w[SEG / 4];
+    __device__ __forceinline__ uint32_t at(uint32_t j) const { return (w[j / 4] >> (8 * (j % 4))) & 0xFFu; }
+};
+__device__ __forceinline__ RoundPaths round_paths(const RowLds &R, uint32_t s, uint32_t n_live) {
+    static_assert(SEG == 16, "one 16-byte read");
+    const uint4 q = *reinterpret_cast<const uint4 *>(&R.path[s * SEG]);
+    RoundPaths r;
+    r.n = n_live - s * SEG < SEG ? n_live - s * SEG : SEG;
+    r.w[0] = (uint32_t)__builtin_amdgcn_readfirstlane((int)q.x);
+    r.w[1] = (uint32_t)__builtin_amdgcn_readfirstlane((int)q.y);
+    r.w[2] = (uint32_t)__builtin_amdgcn_readfirstlane((int)q.z);
+    r.w[3] = (uint32_t)__builtin_amdgcn_readfirstlane((int)q.w);
+    return r;
+}
+
+// Colour of the round's path j, or zero past its last one (staged: the
+// colours of the staged paths).  Uniform: scalar loads, and no branch between
+// a round's paths.
+__device__ __forceinline__ float4 round_colour(const float4 *__restrict__ staged, const RoundPaths &rp, uint32_t j) {
+    const float4 c = staged[rp.at(j)];
+    const uint32_t m = j < rp.n ? 0xFFFFFFFFu : 0u;
     auto sel = [m](float v) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & m); };
     return make_float4(sel(c.x), sel(c.y), sel(c.z), sel(c.w));
 }
 
-// The canvas of one tile of one row: the image's paths composited over
-// transparent pixels, SEG at a time, with the next round's pieces loaded
-// while a round is composited.  With ck it also leaves the canvas before
-// every round but the first, at slot (image row) * ck_pitch + X; canvas may
-// be null.  One block also clears the n_lb look-back words of the geometry
+// The canvas of one tile of one row: the image's paths with pieces there
+// composited over transparent pixels, SEG at a time, with the next round's
+// pieces loaded while a round is composited.  With ck it also leaves the
+// canvas before every round but the image's first, as checkpoint (staged
+// paths before it) / SEG + round, at slot (image row) * ck_pitch + X; canvas
+// may be null.  One block also clears the n_lb look-back words of the geometry
 // (done by now) for the next run and, with `report`, reports the status.
 //
 // TW: the tile's width where it is TILE_MAX (any wider than 192 pixels), else
@@ -790,10 +829,12 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
     for (uint32_t i = threadIdx.x; i < SEG * pitch; i += tw) s_cells[i] = 0;
     for (uint32_t ja = 0; ja < np; ja += ROW_PATHS) {
         const uint32_t n = np - ja < ROW_PATHS ? np - ja : ROW_PATHS;
-        const uint32_t rounds = (n + SEG - 1) / SEG;
         __syncthreads();  // the previous paths' staging is no longer read
         stage_row(S, k0 + ja, n, (int)Y, R);
         __syncthreads();
+        const uint32_t n_live = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.n), rounds = (n_live + SEG - 1) / SEG;
+        if (!rounds) continue;
+        const float4 *const staged = colours + k0 + ja;
         PieceRef ref = piece_ref(S, R, 0, R.pb[0] + threadIdx.x);
         PieceVtx v = piece_vtx(S, R, 0, ref, bad);
         PieceRef nref = ref;
@@ -809,11 +850,11 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
             float A[SEG];
             round_cover<true, TW>(S, R, s, cur, first, (int)Y, xb0, s_cells, A, bad);
             const uint32_t j0 = ja + s * SEG;
-            const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
+            const RoundPaths rp = round_paths(R, s, n_live);
             if (ck && j0 && in) ck[(uint64_t)(j0 / SEG) * ck_stride + slot] = C;
 #pragma unroll
             for (uint32_t j = 0; j < SEG; ++j) {
-                const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
+                const float4 c = round_colour(staged, rp, j);
                 const float al = alpha_cover(A[j]), keep = fmaf(-c.w, al, 1.0f);
                 C = make_float4(fmaf(C.x, keep, c.x * al), fmaf(C.y, keep, c.y * al), fmaf(C.z, keep, c.z * al),
                                 fmaf(C.w, keep, c.w * al));
@@ -1005,10 +1046,12 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
     for (uint32_t chunk = (np + ROW_PATHS - 1) / ROW_PATHS; chunk-- > 0;) {
         const uint32_t ja = chunk * ROW_PATHS;
         const uint32_t n = np - ja < ROW_PATHS ? np - ja : ROW_PATHS;
-        const uint32_t rounds = (n + SEG - 1) / SEG;
         __syncthreads();  // the previous paths' staging is no longer read
         stage_row(S, k0 + ja, n, (int)Y, R);
         __syncthreads();
+        const uint32_t n_live = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.n), rounds = (n_live + SEG - 1) / SEG;
+        if (!rounds) continue;
+        const float4 *const staged = colours + k0 + ja;
         PieceRef ref = piece_ref(S, R, rounds - 1, R.pb[(rounds - 1) * SEG] + threadIdx.x);
         PieceVtx v = piece_vtx(S, R, rounds - 1, ref, bad);
         PieceRef nref = ref;
@@ -1025,7 +1068,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
             }
             float A[SEG];
             round_cover<false, TW>(S, R, s, cur, piece_of(cv.p, cv.q, (int)Y), (int)Y, xb0, s_cells, A, bad);
-            const uint32_t some = (uint32_t)__builtin_amdgcn_readfirstlane((int)R.marks[s]);
+            const RoundPaths rp = round_paths(R, s, n_live);
             float q[SEG];  // f . canvas under path j
             // f . c_j - c_j.w q_j, made again in the second pass: kept beside q it
             // spilled 16 more registers (3.77 ms instead of 3.57 for 64 images)
@@ -1035,7 +1078,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
             float qr = fmaf(f.w, C.w, fmaf(f.z, C.z, fmaf(f.y, C.y, f.x * C.x)));
 #pragma unroll
             for (uint32_t j = 0; j < SEG; ++j) {
-                const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
+                const float4 c = round_colour(staged, rp, j);
                 q[j] = qr;
                 qr = fmaf(alpha_cover(A[j]), d_of(c, qr), qr);  // = al f . c_j + (1 - c_j.w al) q_j
             }
@@ -1047,7 +1090,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
 #pragma unroll
                 for (uint32_t h = 2; h-- > 0;) {
                     const uint32_t j = 2 * jp + h;
-                    const float4 c = round_colour(colours, k0, np, j0 + j, (some >> j) & 1u);
+                    const float4 c = round_colour(staged, rp, j);
                     // (else the first pass's alpha and d stay in registers: 3.19 ms, 3.03 so)
                     asm("" : "+v"(A[j]), "+v"(q[j]));
                     const float al = alpha_cover(A[j]);
@@ -1079,7 +1122,8 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                 const uint32_t j = 2 * (4 * (tid & 1) + (tid & 2) + ((tid >> 2) & 1)) + (tid >> 5);
                 const uint32_t ch = ((tid >> 2) & 2) + ((tid >> 4) & 1);
                 s_gc[tid] = 0.0f;
-                if (g != 0.0f && j0 + j < np) atomicAdd(&gcol[4 * (uint64_t)(k0 + j0 + j) + ch], g);
+                if (g != 0.0f && j < rp.n)
+                    atomicAdd(&gcol[4 * (uint64_t)(k0 + ja + R.path[s * SEG + j]) + ch], g);
             }
             // the pieces' gradients
             const uint32_t base = R.pb[s * SEG], end = R.pb[(s + 1) * SEG];

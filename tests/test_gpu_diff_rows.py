@@ -1,0 +1,74 @@
+"""Scenes of many small figures: a row's rounds hold only the paths that have
+pieces in it.  Against the FP64 oracle with test_gpu_diff_cells' bounds, at
+the sizes where the rounds (16 paths) and the staging (256 paths) can go
+wrong, and against the cost of the same figures without the others."""
+import time
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_diff_cells import _check, _scene
+
+pytestmark = pytest.mark.gpu
+
+
+def _local(h, size, rows=None):
+    """Points of figures of about `size` pixels; with rows, figure k lies around row rows(k)."""
+    def points(g, n):
+        per = 1 + 3 * 2  # two cubics a path
+        k = n // per
+        c = g.uniform(size, [60.0, h - size], (k, 1, 2))
+        if rows is not None:
+            c[:, 0, 1] = [rows(i) for i in range(k)]
+        return (c + g.uniform(-size / 2, size / 2, (k, per, 2))).reshape(-1, 2)
+    return points
+
+
+@pytest.mark.parametrize("paths,images", [(40, 1), (255, 1), (257, 2), (530, 1)])
+def test_small_figures(oracle, paths, images):
+    _check(_scene(paths, 64, 48, paths, 2, images, points=_local(48, 5.0)))
+
+
+@pytest.mark.parametrize("live", [1, 15, 16, 17, 32, 33])
+@pytest.mark.parametrize("stride", [1, 7, 9])  # every stride-th path crosses row 6, the others lie below: 1 to 2 stagings
+def test_rounds_of_a_row(oracle, live, stride):
+    """`live` paths of all in row 6, spread over the others."""
+    def rows(k):
+        return 6.5 if k % stride == 0 and k // stride < live else 24.5
+    _check(_scene(live + stride, 70, 32, max(live * stride, 20) + 3, 2, points=_local(32, 4.0, rows)))
+
+
+def test_heavy_and_light_paths_among_empty_ones(oracle):
+    """Paths of many pieces in some rows (64-bit cells) between paths without any."""
+    sc = _scene(31, 48, 40, 300, 2, points=_local(40, 6.0))
+    cubics = sc.path_cubics.copy()
+    cubics[[5, 140, 299]] = 130
+    g = np.random.default_rng(32)
+    n = 1 + 3 * cubics.astype(np.int64)
+    c = np.repeat(g.uniform(4.0, [44.0, 36.0], (300, 2)), n, axis=0)
+    sc.path_cubics = cubics
+    sc.points = (c + g.uniform(-3.0, 3.0, (int(n.sum()), 2))).astype(np.float32)
+    _check(sc, pieces=600)
+
+
+def _median_forward(sc):
+    from footile_amd.diff import DiffRenderer, device_array
+    r = DiffRenderer.for_scene(sc)
+    p, c, canvas = device_array(sc.points), device_array(sc.colours), r.new_canvas()
+    times = []
+    for k in range(40):
+        a = time.perf_counter()
+        r.forward(p, c, canvas)
+        if k >= 10:
+            times.append(time.perf_counter() - a)
+    return float(np.median(times))
+
+
+def test_paths_without_pieces_cost_little():
+    """16 figures across a 512x512 image, alone and before 1,008 paths outside
+    it: a row's work is that of its own paths.  (Walking all of them took 6
+    times as long; staging their counts takes a tenth.)"""
+    few = _scene(41, 512, 512, 16, 2)
+    more = _scene(41, 512, 512, 1024, 2, points=lambda g, n: g.uniform(600.0, 700.0, (n, 2)))
+    more.points[:len(few.points)] = few.points
+    assert _median_forward(more) < 2.5 * _median_forward(few)

@@ -2080,7 +2080,7 @@ struct SmallLds {
     PathState ps;
     uint32_t w[SBLOCK / 64], w2[SBLOCK / 64];
     unsigned long long wk[SBLOCK / 64];
-    uint32_t flag;
+    uint32_t flag, walk;  // a limit passed or a check failed; a closing walk past KEPT_WALK
 };
 
 // Block-wide exclusive scan (sum, or inclusive max when MAX) of a[0, n) in
@@ -2473,7 +2473,7 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
         host->st.err = 0;
         host->st.overflow = 0;
         S.path = P;
-        S.flag = 0;
+        S.flag = S.walk = 0;
     }
     const uint32_t n_in = n_ops < SMALL_OPS ? n_ops : SMALL_OPS;
     for (uint32_t i = tid; i < SMALL_OPS; i += SBLOCK) S.op_path[i] = 0;
@@ -2521,8 +2521,10 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
     L.n_runs = n_runs;
     L.cap_points = SMALL_EVENTS;
     L.n_pairs = 0;
-    // 3. Fig ingest: the kept points in their local form (a closing walk too
-    // long for it leaves the figure to the full pipeline)
+    // 3. Fig ingest: the kept points in their local form or, where a closing
+    // walk is too long for it, with the pushed points' running maximum (a fill
+    // that ends in 40 repeats of a point: 112 us when that was left to the full
+    // pipeline, 31.7 here)
     uint32_t long_walk = 0;
     for (uint32_t e = tid; e < n_events; e += SBLOCK) {
         uint32_t first_of;
@@ -2532,8 +2534,20 @@ __global__ __launch_bounds__(SBLOCK) void k_small_front(const ft_path_op *ops, S
         S.a.ev.kept[e] = k;
         S.a.ev.idx[e] = k;
     }
-    bad |= long_walk;
+    if (long_walk) S.walk = 1;
     __syncthreads();
+    if (S.walk) {
+        uint32_t *const last = S.a.ev.idx;
+        for (uint32_t e = tid; e < n_events; e += SBLOCK)
+            ingest_event(e, L, S.a.ev.meta, S.a.ev.xy, S.run_first, S.run_path, last, bad);
+        __syncthreads();
+        (void)small_scan<true>(last, n_events, S.w);
+        for (uint32_t e = tid; e < n_events; e += SBLOCK)
+            S.a.ev.kept[e] = kept_event(e, L, S.a.ev.meta, S.a.ev.xy, S.run_first, S.run_close, last, bad);
+        __syncthreads();
+        for (uint32_t e = tid; e < n_events; e += SBLOCK) S.a.ev.idx[e] = S.a.ev.kept[e];
+        __syncthreads();
+    }
     const uint32_t n_kept = small_scan<false>(S.a.ev.idx, n_events, S.w);
     // 4. the path's counts (no cap below 65,535 points) and compaction with
     // the top (y, x) key

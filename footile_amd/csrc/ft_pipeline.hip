@@ -3378,6 +3378,10 @@ ft_status ws_launch(Workspace &ws, uint32_t mode) {
     return FT_OK;
 }
 
+// (16 long curves of 2,900 events each: k_compact takes 4.6 us so, 29.8 with
+// the six blocks that their number asks for)
+constexpr size_t ARENA_EVENTS_MIN = 256 * BLOCK;
+
 static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool with_pstate, bool copy_status,
                             bool keep_failed, HostStatus *report) {
     if (mode == MODE_STROKE) {
@@ -3496,8 +3500,11 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
     }
     if (mode == MODE_FILL || mode == MODE_STROKE) {
         // (an arena's capacity is whatever its bytes hold: the grid-stride
-        // kernels take a grid for the events a first layout expects instead)
-        const uint32_t ge = grid_for(ws.arena ? std::min(ws.cap_events, 16 * n_ops + (size_t)1024) : ws.cap_events);
+        // kernels take a grid for the events a first layout expects instead,
+        // and at least a block per CU, since few long curves may have far more)
+        const uint32_t ge =
+            grid_for(ws.arena ? std::min(ws.cap_events, std::max(16 * n_ops + (size_t)1024, ARENA_EVENTS_MIN))
+                              : ws.cap_events);
         Limits L0{};
         L0.n_ops = n_ops;
         L0.n_paths = (uint32_t)ws.n_paths;

@@ -250,28 +250,37 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t x, uint32_t *s_w, uint32
 }
 
 // The whole geometry in one launch, for layouts whose paths have at most
-// GEOM_EDGES edges and images at most GEOM_ROWS rows: a block takes `per`
-// consecutive paths, writes their vertices and counts their (edge, row)
-// pairs, takes its place in the pair list by look-back, and then per path
-// counts the rows' edges in LDS, scans them into the cells' list offsets and
-// hands out the list slots with LDS cursors.  Order within a list is free:
+// GEOM_EDGES edges: a block takes `per` consecutive paths, writes their
+// vertices and counts their (edge, row) pairs, takes its place in the pair
+// list by look-back, and then per path and GEOM_ROWS of the rows between its
+// first and last counts the rows' edges in LDS, scans them into the cells' list
+// offsets and hands out the list slots with LDS cursors; the other rows get
+// counts of 0, whose offsets nothing reads.  Order within a list is free:
 // coverage is an integer sum.  It also clears the gradients (gedge null:
 // none).  It replaces a clear over all cells, a vertex pass, atomics per edge
 // on the cells, two scans over all cells and a kernel that tested every edge
 // of a path against every row: 545 -> 168 us of a 64-image step with 17,500
 // paths, 85 us in six launches -> 19 us in two for 256 paths, 110 -> 17 us for
-// a 1000x600 image of 128 paths.  A path's work is a chain of a few barriers,
+// a 1000x600 image of 128 paths.  4,096 figures of 24 pixels in an image of
+// 9,000 rows: 63 us, 530 with counts and offsets of all rows by this kernel,
+// 290 by the general form, which took images past 8,192 rows.  A path's work is a chain of a few barriers,
 // so a launch of few paths is bound by latency.
 constexpr uint32_t GEOM_EDGES = 2048, GEOM_ROWS = 8192, GEOM_BLOCKS = 1024;
+constexpr uint32_t GEOM_SPANS = 64;  // paths of a block whose spans are kept; the others take all rows
 constexpr uint32_t EDGE_LANES = 4;  // threads per edge in the fill, on every fourth of its rows
 
 __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *points, float4 *gedge, float *gcol,
                                                     uint32_t per, unsigned long long *lb, DevStatus *st) {
-    extern __shared__ uint32_t s_row[];  // [H + 1]: differences, counts, then list cursors
+    extern __shared__ uint32_t s_row[];  // [min(H, GEOM_ROWS) + 1]: differences, counts, then list cursors
     __shared__ uint32_t s_w[BLOCK / 64], s_tk;
     __shared__ unsigned long long s_base;
+    __shared__ uint32_t s_lo[GEOM_SPANS], s_end[GEOM_SPANS];  // a path's rows [s_lo, s_end)
     const uint32_t tid = threadIdx.x;
     if (tid == 0) s_tk = lookback_ticket(lb);
+    if (tid < GEOM_SPANS) {
+        s_lo[tid] = S.H;
+        s_end[tid] = 0;
+    }
     __syncthreads();
     const uint32_t b = s_tk;
     const uint32_t k0 = b * per, k1 = k0 + per < S.n_paths ? k0 + per : S.n_paths;
@@ -290,10 +299,15 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
         const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
         for (uint32_t e = tid; e < V; e += BLOCK) {
             uint32_t r0, r1;
-            if (edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) mine += r1 - r0 + 1;
+            if (!edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) continue;
+            mine += r1 - r0 + 1;
+            if (k - k0 < GEOM_SPANS) {
+                atomicMin(&s_lo[k - k0], r0);
+                atomicMax(&s_end[k - k0], r1 + 1);
+            }
         }
     }
-    // at most GEOM_EDGES edges of GEOM_ROWS rows per path: one path's pairs fit 32 bits, a block's need not
+    // at most GEOM_EDGES edges of FT_MAX_WIDTH rows per path: one path's pairs fit 32 bits, a block's need not
     const unsigned long long wsum = wave_incl_t<unsigned long long, false>(mine);
     __shared__ unsigned long long s_sum[BLOCK / 64];
     if ((tid & 63) == 63) s_sum[tid >> 6] = wsum;
@@ -318,54 +332,68 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
     __syncthreads();
     if (s_base == ~0ull) return;  // no room: the run is repeated with more
     uint32_t base = (uint32_t)s_base;
-    const uint32_t rows_per = (S.H + BLOCK - 1) / BLOCK;
     for (uint32_t k = k0; k < k1; ++k) {
         const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
-        for (uint32_t r = tid; r <= S.H; r += BLOCK) s_row[r] = 0;
-        __syncthreads();
-        for (uint32_t e = tid; e < V; e += BLOCK) {
-            uint32_t r0, r1;
-            if (!edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) continue;
-            atomicAdd(&s_row[r0], 1u);
-            atomicAdd(&s_row[r1 + 1], 0xFFFFFFFFu);
+        // the rows [w0, w0 + h) of an edge, counted from w0
+        auto window = [&](uint32_t e, uint32_t w0, uint32_t h, uint32_t &r0, uint32_t &r1) {
+            if (!edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) return false;
+            if ((r0 >= w0 + h) | (r1 < w0)) return false;
+            r0 = r0 > w0 ? r0 - w0 : 0u;
+            r1 = r1 - w0 < h ? r1 - w0 : h - 1;
+            return true;
+        };
+        const uint32_t lo = k - k0 < GEOM_SPANS ? s_lo[k - k0] : 0u, end = k - k0 < GEOM_SPANS ? s_end[k - k0] : S.H;
+        for (uint32_t r = tid; r < lo; r += BLOCK) S.cell_cnt[(uint64_t)k * S.H + r] = 0;
+        for (uint32_t r = end > lo ? end + tid : S.H; r < S.H; r += BLOCK) S.cell_cnt[(uint64_t)k * S.H + r] = 0;
+        for (uint32_t w0 = lo; w0 < end; w0 += GEOM_ROWS) {
+            const uint32_t h = end - w0 < GEOM_ROWS ? end - w0 : GEOM_ROWS;
+            for (uint32_t r = tid; r <= h; r += BLOCK) s_row[r] = 0;
+            __syncthreads();
+            for (uint32_t e = tid; e < V; e += BLOCK) {
+                uint32_t r0, r1;
+                if (!window(e, w0, h, r0, r1)) continue;
+                atomicAdd(&s_row[r0], 1u);
+                atomicAdd(&s_row[r1 + 1], 0xFFFFFFFFu);
+            }
+            __syncthreads();
+            // thread t's rows [a, z): counts from the differences, then offsets
+            const uint32_t rows_per = (h + BLOCK - 1) / BLOCK;
+            const uint32_t a = tid * rows_per < h ? tid * rows_per : h;
+            const uint32_t z = a + rows_per < h ? a + rows_per : h;
+            uint32_t d = 0, total;
+            for (uint32_t r = a; r < z; ++r) d += s_row[r];
+            uint32_t cnt = block_excl(d, s_w, total);
+            const uint32_t before = cnt;
+            uint32_t sum = 0;
+            for (uint32_t r = a; r < z; ++r) {
+                cnt += s_row[r];
+                sum += cnt;
+            }
+            uint32_t at = base + block_excl(sum, s_w, total);
+            cnt = before;
+            const uint64_t c0 = (uint64_t)k * S.H + w0;
+            for (uint32_t r = a; r < z; ++r) {
+                cnt += s_row[r];
+                S.cell_cnt[c0 + r] = cnt;
+                S.cell_off[c0 + r] = at;
+                s_row[r] = at;
+                at += cnt;
+            }
+            __syncthreads();
+            for (uint32_t i = tid; i < V * EDGE_LANES; i += BLOCK) {
+                const uint32_t e = i / EDGE_LANES;
+                uint32_t r0, r1;
+                if (!window(e, w0, h, r0, r1)) continue;
+                for (uint32_t r = r0 + i % EDGE_LANES; r <= r1; r += EDGE_LANES)
+                    S.cell_edge[atomicAdd(&s_row[r], 1u)] = e;
+            }
+            base += total;
+            __syncthreads();
         }
-        __syncthreads();
-        // thread t's rows [a, z): counts from the differences, then offsets
-        const uint32_t a = tid * rows_per < S.H ? tid * rows_per : S.H;
-        const uint32_t z = a + rows_per < S.H ? a + rows_per : S.H;
-        uint32_t d = 0, total;
-        for (uint32_t r = a; r < z; ++r) d += s_row[r];
-        uint32_t cnt = block_excl(d, s_w, total);
-        const uint32_t before = cnt;
-        uint32_t sum = 0;
-        for (uint32_t r = a; r < z; ++r) {
-            cnt += s_row[r];
-            sum += cnt;
-        }
-        uint32_t at = base + block_excl(sum, s_w, total);
-        cnt = before;
-        const uint64_t c0 = (uint64_t)k * S.H;
-        for (uint32_t r = a; r < z; ++r) {
-            cnt += s_row[r];
-            S.cell_cnt[c0 + r] = cnt;
-            S.cell_off[c0 + r] = at;
-            s_row[r] = at;
-            at += cnt;
-        }
-        __syncthreads();
-        for (uint32_t i = tid; i < V * EDGE_LANES; i += BLOCK) {
-            const uint32_t e = i / EDGE_LANES;
-            uint32_t r0, r1;
-            if (!edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) continue;
-            for (uint32_t r = r0 + i % EDGE_LANES; r <= r1; r += EDGE_LANES)
-                S.cell_edge[atomicAdd(&s_row[r], 1u)] = e;
-        }
-        base += total;
-        __syncthreads();
     }
 }
 
-// The general form, for longer paths and taller images: k_vertices, k_rows
+// The general form, for longer paths: k_vertices, k_rows
 // (differences on the cells), two scans over the cells, and k_fill_cells.
 //
 // FILL_LANES threads per edge, each taking every FILL_LANES-th run of
@@ -484,7 +512,8 @@ __device__ void stage_row(const DScene &S, uint32_t kbase, uint32_t n, int Y, Ro
         const uint32_t p = 4 * lane + i;
         const uint64_t cell = (uint64_t)(kbase + (p < n ? p : 0u)) * S.H + (uint32_t)Y;
         c[i] = p < n ? S.cell_cnt[cell] : 0u;
-        o[i] = S.cell_off[cell];
+        o[i] = 0;
+        if (c[i]) o[i] = S.cell_off[cell];  // (most are 0 in a scene of small figures: 1,118 -> 415 us there)
     }
 #pragma unroll
     for (uint32_t i = 0; i < 5; ++i) v[i] = S.vtx_off[kbase + (4 * lane + i < n ? 4 * lane + i : n)];
@@ -1332,7 +1361,7 @@ uint32_t grid_of(uint64_t n) {
 
 // Blocks of k_geometry (0: the scene takes the general form).
 uint32_t geometry_blocks(const ft_diff *d) {
-    if (d->max_path_vtx > GEOM_EDGES || d->H > GEOM_ROWS || !d->n_paths) return 0;
+    if (d->max_path_vtx > GEOM_EDGES || !d->n_paths) return 0;
     const uint32_t per = (d->n_paths + GEOM_BLOCKS - 1) / GEOM_BLOCKS;
     return (d->n_paths + per - 1) / per;
 }
@@ -1351,7 +1380,8 @@ ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, flo
         const uint32_t per = (d->n_paths + GEOM_BLOCKS - 1) / GEOM_BLOCKS;
         if (!clean)
             k_clear_run<<<1, BLOCK, 0, s>>>(d->d_lb, (uint32_t)lookback_words(blocks), d->d_status, host_err);
-        k_geometry<<<blocks, BLOCK, (d->H + 1) * sizeof(uint32_t), s>>>(S, pts, gedge, gcol, per, d->d_lb, d->d_status);
+        const size_t lds = (std::min(d->H, GEOM_ROWS) + 1) * sizeof(uint32_t);
+        k_geometry<<<blocks, BLOCK, lds, s>>>(S, pts, gedge, gcol, per, d->d_lb, d->d_status);
         FD_HIP(hipGetLastError());
         return FT_OK;
     }

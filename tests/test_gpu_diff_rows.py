@@ -72,3 +72,31 @@ def test_paths_without_pieces_cost_little():
     more = _scene(41, 512, 512, 1024, 2, points=lambda g, n: g.uniform(600.0, 700.0, (n, 2)))
     more.points[:len(few.points)] = few.points
     assert _median_forward(more) < 2.5 * _median_forward(few)
+
+
+@pytest.mark.parametrize("h", [8191, 8192, 8193, 16384, 16385, 20000])
+def test_tall_images(oracle, h):
+    """The one-launch geometry takes 8,192 rows of a path at a time: for figures
+    in and across the windows the same canvas bytes as the general form (a path
+    of 2,081 edges outside the image sends all paths there), and the same
+    gradients but for the order of their float32 sums (at most some 1,000 terms
+    of either sign a vertex: 1e-5).  (FP64 says little here: y near 8,192 is
+    rounded at 5e-4.)"""
+    import dataclasses
+
+    from tests.test_gpu_diff_cells import _rel, _step
+    g = np.random.default_rng(h)
+    sc = _scene(h, 5, h, 6, 3)
+    tall = sc.points.reshape(6, -1, 2)
+    tall[2:] = g.uniform(-2.0, 7.0, tall[2:].shape)  # the last four small, around the windows' borders
+    tall[2:, :, 1] += np.array([8192.0, 8190.0, min(16384, h) - 3.0, h - 4.0])[:, None]
+    far = g.uniform(200.0, 300.0, size=(1 + 3 * 130, 2)).astype(np.float32)
+    more = dataclasses.replace(sc, path_image=np.append(sc.path_image, 0).astype(np.uint32),
+                               path_cubics=np.append(sc.path_cubics, 130).astype(np.uint32),
+                               points=np.concatenate([sc.points, far]),
+                               colours=np.concatenate([sc.colours, sc.colours[:1]]))
+    target = g.uniform(0, 1, size=(1, h, 5, 4)).astype(np.float32)
+    loss, canvas, gp, gc = _step(sc, target)
+    want_loss, want, want_gp, want_gc = _step(more, target)
+    assert loss == want_loss and np.array_equal(canvas, want) and np.abs(gp).max() > 0.0
+    assert _rel(gp, want_gp[:len(gp)]) < 1e-5 and _rel(gc, want_gc[:len(gc)]) < 1e-5

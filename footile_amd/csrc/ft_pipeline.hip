@@ -3232,10 +3232,17 @@ ft_status ws_set_batch(Workspace &ws, const ft_path_op *ops, size_t n_ops, const
             if ((s = ensure_event_capacity(ws, 16 * n_ops + 1024))) return s;
         }
         if (!ws.d_band_list) {
-            // (an edge lies in up to three times as many bands of default_tuning's
-            // rows as of the nominal ones)
-            size_t cap = (ws.tuned ? 4 : 12) * (16 * n_ops + 1024);
-            if ((s = dev_alloc(ws, ws.d_band_list, cap))) return s;
+            // An edge lies in up to three times as many bands of default_tuning's
+            // rows as of the nominal ones.  Where there is no room for that many
+            // pairs the list starts as the nominal rows' and grows to the need.
+            size_t cap = 4 * (16 * n_ops + 1024);
+            s = ws.tuned ? FT_ENOMEM : dev_alloc(ws, ws.d_band_list, 3 * cap);
+            if (s) {
+                (void)hipGetLastError();
+                if ((s = dev_alloc(ws, ws.d_band_list, cap))) return s;
+            } else {
+                cap *= 3;
+            }
             ws.cap_pairs = cap;
         }
         if ((s = ensure_scan_capacity(ws))) return s;

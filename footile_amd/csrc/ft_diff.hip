@@ -34,7 +34,7 @@ struct DScene {
     uint32_t n_vtx, n_cells;
     const uint32_t *pt_off;     // [n_paths + 1] first point of each path
     const uint32_t *vtx_off;    // [n_paths + 1] first vertex of each path
-    const uint32_t *vtx_path;   // [n_vtx]; general geometry only, as cell_cur
+    const uint32_t *vtx_path;   // [n_vtx]
     const uint32_t *img_first;  // [n_images + 1] first path of each image
     float2 *vtx;                // [n_vtx]
     uint32_t *cell_cnt;         // [n_cells] edges per (path, row); first the differences
@@ -1561,9 +1561,11 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
     }
     const uint64_t cells = (uint64_t)L->n_paths * L->height;
     if (cells >= 0xFFFFFFFFull) return FT_ENOTSUP;
-    std::vector<uint32_t> vtx_path, pt_path(np);
-    for (uint32_t k = 0; k < L->n_paths; ++k)
+    std::vector<uint32_t> vtx_path(nv), pt_path(np);
+    for (uint32_t k = 0; k < L->n_paths; ++k) {
+        for (uint32_t v = vtx_off[k]; v < vtx_off[k + 1]; ++v) vtx_path[v] = k;
         for (uint32_t m = pt_off[k]; m < pt_off[k + 1]; ++m) pt_path[m] = k;
+    }
     ft_diff *d = new ft_diff();
     d->n_images = L->n_images;
     d->W = L->width;
@@ -1573,12 +1575,6 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
     d->n_pts = (uint32_t)np;
     d->n_vtx = (uint32_t)nv;
     for (uint32_t k = 0; k < L->n_paths; ++k) d->max_path_vtx = std::max(d->max_path_vtx, vtx_off[k + 1] - vtx_off[k]);
-    const bool general = geometry_blocks(d) == 0;
-    if (general) {
-        vtx_path.resize(nv);
-        for (uint32_t k = 0; k < L->n_paths; ++k)
-            for (uint32_t v = vtx_off[k]; v < vtx_off[k + 1]; ++v) vtx_path[v] = k;
-    }
     d->n_cells = cells;
     d->canvas_floats = 4ull * L->n_images * L->width * L->height;
     d->ck_pitch = (d->W + 15) / 16 * 16;
@@ -1589,10 +1585,10 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
     ft_status st;
     if (hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking) != hipSuccess) st = FT_EDEVICE;
     else if ((st = dalloc(d->d_pt_off, L->n_paths + 1)) || (st = dalloc(d->d_vtx_off, L->n_paths + 1)) ||
-             (st = dalloc(d->d_vtx_path, vtx_path.size())) || (st = dalloc(d->d_pt_path, np)) ||
+             (st = dalloc(d->d_vtx_path, nv)) || (st = dalloc(d->d_pt_path, np)) ||
              (st = dalloc(d->d_img_first, L->n_images + 1)) || (st = dalloc(d->d_vtx, nv)) ||
              (st = dalloc(d->d_gedge, nv)) || (st = dalloc(d->d_cell_cnt, cells)) ||
-             (st = dalloc(d->d_cell_off, cells)) || (st = dalloc(d->d_cell_cur, general ? cells : 0)) ||
+             (st = dalloc(d->d_cell_off, cells)) || (st = dalloc(d->d_cell_cur, cells)) ||
              (st = dalloc(d->d_cell_edge, d->cap_pairs)) || (st = dalloc(d->d_lb, std::max<size_t>(4 * d->cap_tiles, lookback_words(GEOM_BLOCKS)))) ||
              (st = dalloc(d->d_ck, n_ck * d->ck_stride)) || (st = dalloc(d->d_partial, LOSS_GRID)) ||
              (st = dalloc(d->d_status, 1)) || (st = dalloc(d->d_done, 1)))
@@ -1606,8 +1602,7 @@ ft_status ft_diff_new(const ft_diff_layout *L, ft_diff **out) {
         st = FT_ENOMEM;
     else if (hipMemcpy(d->d_pt_off, pt_off.data(), pt_off.size() * 4, hipMemcpyHostToDevice) != hipSuccess ||
              hipMemcpy(d->d_vtx_off, vtx_off.data(), vtx_off.size() * 4, hipMemcpyHostToDevice) != hipSuccess ||
-             (general &&
-              hipMemcpy(d->d_vtx_path, vtx_path.data(), vtx_path.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
+             hipMemcpy(d->d_vtx_path, vtx_path.data(), nv * 4, hipMemcpyHostToDevice) != hipSuccess ||
              hipMemcpy(d->d_pt_path, pt_path.data(), np * 4, hipMemcpyHostToDevice) != hipSuccess ||
              hipMemcpy(d->d_img_first, img_first.data(), img_first.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
         st = FT_EDEVICE;

@@ -274,13 +274,10 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
     extern __shared__ uint32_t s_row[];  // [min(H, GEOM_ROWS) + 1]: differences, counts, then list cursors
     __shared__ uint32_t s_w[BLOCK / 64], s_tk;
     __shared__ unsigned long long s_base;
-    __shared__ uint32_t s_lo[GEOM_SPANS], s_end[GEOM_SPANS];  // a path's rows [s_lo, s_end)
+    __shared__ uint32_t s_up[GEOM_SPANS], s_end[GEOM_SPANS];  // a path's rows [H - s_up, s_end)
     const uint32_t tid = threadIdx.x;
     if (tid == 0) s_tk = lookback_ticket(lb);
-    if (tid < GEOM_SPANS) {
-        s_lo[tid] = S.H;
-        s_end[tid] = 0;
-    }
+    if (tid < GEOM_SPANS) s_up[tid] = s_end[tid] = 0;
     __syncthreads();
     const uint32_t b = s_tk;
     const uint32_t k0 = b * per, k1 = k0 + per < S.n_paths ? k0 + per : S.n_paths;
@@ -297,13 +294,20 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
     unsigned long long mine = 0;
     for (uint32_t k = k0; k < k1; ++k) {
         const uint32_t vb = S.vtx_off[k], V = S.vtx_off[k + 1] - vb;
+        uint32_t up = 0, end = 0;  // rows from the first on; the row after the last
         for (uint32_t e = tid; e < V; e += BLOCK) {
             uint32_t r0, r1;
             if (!edge_row_range(S.vtx[vb + e], S.vtx[vb + (e + 1 < V ? e + 1 : 0u)], S.H, r0, r1)) continue;
             mine += r1 - r0 + 1;
-            if (k - k0 < GEOM_SPANS) {
-                atomicMin(&s_lo[k - k0], r0);
-                atomicMax(&s_end[k - k0], r1 + 1);
+            up = S.H - r0 > up ? S.H - r0 : up;
+            end = r1 + 1 > end ? r1 + 1 : end;
+        }
+        if (k - k0 < GEOM_SPANS) {
+            up = wave_incl_dpp<true>(up);
+            end = wave_incl_dpp<true>(end);
+            if ((tid & 63) == 63) {
+                atomicMax(&s_up[k - k0], up);
+                atomicMax(&s_end[k - k0], end);
             }
         }
     }
@@ -342,7 +346,8 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
             r1 = r1 - w0 < h ? r1 - w0 : h - 1;
             return true;
         };
-        const uint32_t lo = k - k0 < GEOM_SPANS ? s_lo[k - k0] : 0u, end = k - k0 < GEOM_SPANS ? s_end[k - k0] : S.H;
+        const bool kept = k - k0 < GEOM_SPANS;
+        const uint32_t lo = kept ? S.H - s_up[k - k0] : 0u, end = kept ? s_end[k - k0] : S.H;
         for (uint32_t r = tid; r < lo; r += BLOCK) S.cell_cnt[(uint64_t)k * S.H + r] = 0;
         for (uint32_t r = end > lo ? end + tid : S.H; r < S.H; r += BLOCK) S.cell_cnt[(uint64_t)k * S.H + r] = 0;
         for (uint32_t w0 = lo; w0 < end; w0 += GEOM_ROWS) {
@@ -491,10 +496,10 @@ constexpr float TINY = 0x1p4f;           // of CELL_ONE: a share of 2^-22
 // us a forward and 790 a step, now 73 and 146; 256 paths across the image 113
 // and 349, now 109 and 333.)
 struct RowLds {
-    __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of their piece counts, then the total
+    __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of their piece counts; the total past the last
     __align__(16) uint8_t path[ROW_PATHS];     // their index among the staged paths; 0 past the last
     uint32_t dl[ROW_PATHS];                    // list position of a path's piece e: dl + e
-    uint32_t vb[ROW_PATHS], vn[ROW_PATHS];     // first vertex and number of vertices
+    uint2 vtx[ROW_PATHS];                      // first vertex and number of vertices
     uint32_t heavy[ROW_PATHS / SEG];           // per round: bit j, its path j has more than HEAVY pieces
     uint32_t poison[2];                        // per round parity: bit j, path j has a piece that is no number
                                                // here; bit 16 + j, one of a TINY share
@@ -512,8 +517,11 @@ __device__ void stage_row(const DScene &S, uint32_t kbase, uint32_t n, int Y, Ro
         const uint32_t p = 4 * lane + i;
         const uint64_t cell = (uint64_t)(kbase + (p < n ? p : 0u)) * S.H + (uint32_t)Y;
         c[i] = p < n ? S.cell_cnt[cell] : 0u;
+        // (of many paths most have none here, and their offsets are not loaded:
+        // 1,118 -> 415 us in a scene of small figures; with few paths the loads
+        // are cheap and a second round trip is not: 7.2 and 9.5 us for four)
         o[i] = 0;
-        if (c[i]) o[i] = S.cell_off[cell];  // (most are 0 in a scene of small figures: 1,118 -> 415 us there)
+        if (n <= 64 || c[i]) o[i] = S.cell_off[cell];
     }
 #pragma unroll
     for (uint32_t i = 0; i < 5; ++i) v[i] = S.vtx_off[kbase + (4 * lane + i < n ? 4 * lane + i : n)];
@@ -526,28 +534,26 @@ __device__ void stage_row(const DScene &S, uint32_t kbase, uint32_t n, int Y, Ro
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     const uint32_t n_live = (uint32_t)__builtin_amdgcn_readlane((int)rank1, 63);
     uint32_t pre = incl - sum, rank = rank1 - live;
+    // (one wavefront, whose LDS accesses stay in order: the entries past the
+    // last first, everywhere)
+    *reinterpret_cast<uint4 *>(&R.pb[4 * lane]) = make_uint4(total, total, total, total);
+    *reinterpret_cast<uint32_t *>(&R.path[4 * lane]) = 0;
     if (lane < ROW_PATHS / SEG) R.heavy[lane] = 0;
     if (lane < 2) R.poison[lane] = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        if (c[i]) {
-            R.pb[rank] = pre;
-            R.path[rank] = (uint8_t)(4 * lane + i);
-            R.dl[rank] = o[i] - pre;
-            R.vb[rank] = v[i];
-            R.vn[rank] = v[i + 1] - v[i];
-            if (c[i] > HEAVY) atomicOr(&R.heavy[rank / SEG], 1u << (rank % SEG));
-            ++rank;
-            pre += c[i];
-        }
-        if (4 * lane + i >= n_live) {
-            R.pb[4 * lane + i] = total;
-            R.path[4 * lane + i] = 0;
-        }
-    }
     if (lane == 63) {
         R.pb[ROW_PATHS] = total;
         R.n = n_live;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        if (!c[i]) continue;
+        R.pb[rank] = pre;
+        R.path[rank] = (uint8_t)(4 * lane + i);
+        R.dl[rank] = o[i] - pre;
+        R.vtx[rank] = make_uint2(v[i], v[i + 1] - v[i]);
+        if (c[i] > HEAVY) atomicOr(&R.heavy[rank / SEG], 1u << (rank % SEG));
+        ++rank;
+        pre += c[i];
     }
 }
 
@@ -583,7 +589,7 @@ struct PieceVtx {
 __device__ __forceinline__ PieceVtx piece_vtx(const DScene &S, const RowLds &R, uint32_t s, const PieceRef &r,
                                               uint32_t &bad) {
     const uint32_t t = s * SEG + (r.j != NO_IDX ? r.j : 0u);
-    const uint32_t vb = R.vb[t], V = R.vn[t];
+    const uint32_t vb = R.vtx[t].x, V = R.vtx[t].y;
     bad |= r.edge < V ? 0u : 1u;
     const uint32_t e = r.edge < V ? r.edge : 0u;
     PieceVtx v;
@@ -876,10 +882,10 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
                 v = piece_vtx(S, R, s + 1, ref, bad);
                 if (s + 2 < rounds) nref = piece_ref(S, R, s + 2, R.pb[(s + 2) * SEG] + threadIdx.x);
             }
+            const RoundPaths rp = round_paths(R, s, n_live);
             float A[SEG];
             round_cover<true, TW>(S, R, s, cur, first, (int)Y, xb0, s_cells, A, bad);
             const uint32_t j0 = ja + s * SEG;
-            const RoundPaths rp = round_paths(R, s, n_live);
             if (ck && j0 && in) ck[(uint64_t)(j0 / SEG) * ck_stride + slot] = C;
 #pragma unroll
             for (uint32_t j = 0; j < SEG; ++j) {

@@ -466,11 +466,14 @@ __global__ __launch_bounds__(BLOCK) void k_fill_cells(DScene S, DevStatus *st) {
 //
 // A pixel has a gradient only where its coverage is not 0, so a column that a
 // ramp touches by less than 2^-27 would lose it (the tip of a figure that
-// reaches 1e-4 into a pixel has a gradient of 1e-4 there).  A path of which a
-// ramp column is nonzero and under TINY therefore takes 64-bit cells too, of
-// 2^-56: about one round of paths in 30 has one.  (At cells of 2^-24 for all,
-// without this, gradients of a 512x512 scene were 8.2e-6 from FP64 instead of
-// 4.4e-6.)
+// reaches 1e-4 into a pixel has a gradient of 1e-4 there).  What rounding took
+// from a ramp column of a share under TINY is therefore listed, and added to
+// the column's coverage.  A path with a piece less than TINY high, or with
+// more such columns than the list has room for, takes 64-bit cells of 2^-56.
+// (At cells of 2^-24 for all, without this, gradients of a 512x512 scene were
+// 8.2e-6 from FP64 instead of 4.4e-6.  With 64-bit cells for all those paths,
+// one round in 30, a forward of 24 paths in 200x120 took 1.4 us
+// longer: its slowest row decides.)
 //
 // Every 64-column chunk of a row stands alone: a piece left of a chunk adds
 // its whole signed height to the chunk's first cell, so no carry passes
@@ -488,6 +491,7 @@ constexpr float CELL_ONE = 0x1p26f;
 constexpr float HEAVY_ONE = 0x1p38f;     // at most 2^24 pieces: |A| < 2^24
 constexpr float FINE_ONE = 0x1p56f;      // at most HEAVY pieces: |A| < 32
 constexpr float TINY = 0x1p4f;           // of CELL_ONE: a share of 2^-22
+constexpr uint32_t FIX_MAX = 32;         // listed columns per round
 
 // The paths of a staging round that have pieces in the row, in path order:
 // only they are rounded up to SEG and walked.  (A path without pieces leaves
@@ -501,8 +505,10 @@ struct RowLds {
     uint32_t dl[ROW_PATHS];                    // list position of a path's piece e: dl + e
     uint2 vtx[ROW_PATHS];                      // first vertex and number of vertices
     uint32_t heavy[ROW_PATHS / SEG];           // per round: bit j, its path j has more than HEAVY pieces
-    uint32_t poison[2];                        // per round parity: bit j, path j has a piece that is no number
-                                               // here; bit 16 + j, one of a TINY share
+    // per round parity: x: bit j, path j has a piece that is no number here,
+    // bit 16 + j, it takes 64-bit cells; y: listed columns
+    __align__(8) uint2 mark[2];
+    uint2 fix[FIX_MAX];                        // path << 16 | column; the share rounding took, in cell units
     uint32_t n;                                // how many
 };
 
@@ -539,7 +545,7 @@ __device__ void stage_row(const DScene &S, uint32_t kbase, uint32_t n, int Y, Ro
     *reinterpret_cast<uint4 *>(&R.pb[4 * lane]) = make_uint4(total, total, total, total);
     *reinterpret_cast<uint32_t *>(&R.path[4 * lane]) = 0;
     if (lane < ROW_PATHS / SEG) R.heavy[lane] = 0;
-    if (lane < 2) R.poison[lane] = 0;
+    if (lane < 2) R.mark[lane] = make_uint2(0u, 0u);
     if (lane == 63) {
         R.pb[ROW_PATHS] = total;
         R.n = n_live;
@@ -642,17 +648,17 @@ __device__ __forceinline__ float ramp_cover(const Ramp &m, float X1) {
     return ramp_mean(m, X1, a, b);
 }
 
-// v: a share in cell units, |v| at most a cell's one.
+// v rounded to a whole number: a share in cell units, |v| at most a cell's
+// one (64-bit cells: 2^56, in two exact halves, the conversion of the whole
+// being twice as long).
 template <typename T>
 __device__ __forceinline__ T cell_of(float v) {
-    if constexpr (sizeof(T) == 8)
-        return __float2ll_rn(v);
-    else
+    if constexpr (sizeof(T) == 8) {
+        const float h = rintf(v * 0x1p-28f);
+        return (T)(int)h * ((T)1 << 28) + __float2int_rn(fmaf(-h, 0x1p28f, v));
+    } else {
         return __float2int_rn(v);
-}
-// 0 < |v| < TINY
-__device__ __forceinline__ bool tiny_share(float v) {
-    return (__builtin_bit_cast(uint32_t, v) & 0x7FFFFFFFu) - 1u < __builtin_bit_cast(uint32_t, TINY) - 1u;
+    }
 }
 template <typename T>
 __device__ __forceinline__ void cell_add(T *c, T v) {
@@ -662,24 +668,26 @@ __device__ __forceinline__ void cell_add(T *c, T v) {
         atomicAdd(c, v);
 }
 
-// Adds one piece per lane to its path's row of cells (row; the wavefront's
-// lanes all call it, those without a piece with m.live false), in units of
-// 1 / one.  A ramp of more than RAMP_LANE columns is evaluated by the whole
-// wavefront, one column per lane, so that one long near-horizontal piece does
-// not hold up 63 lanes.  Returns whether a ramp column of the piece has a TINY
-// share.
-template <typename T>
-__device__ __forceinline__ bool scatter_piece(T *cells, uint32_t row_at, const Ramp &m, float xb0, int tw, float one) {
+// Adds one piece per lane to row_at of the cells (the wavefront's lanes all
+// call it, those without a piece with m.live false), in units of 1 / one.  A
+// ramp of more than RAMP_LANE columns is evaluated by the whole wavefront, one
+// column per lane, so that one long near-horizontal piece does not hold up 63
+// lanes.  fix(c, r): column c lost r to rounding (32-bit cells, TINY shares:
+// the shares of a ramp rise with its columns, so those are its first ones).
+template <typename T, class Fix>
+__device__ __forceinline__ void scatter_piece(T *cells, uint32_t row_at, const Ramp &m, float xb0, int tw, float one,
+                                              Fix &&fix) {
+    constexpr bool FIX = sizeof(T) == 4;
     const float zs = m.z * one;
     const int n = m.c1 - m.c0;
     const bool wide = m.live & (n > RAMP_LANE);
-    bool tiny = false;
     T prev = 0;
+    float least = TINY;
     if (m.live & !wide) {
         for (int c = m.c0; c < m.c1; ++c) {
             const float v = zs * ramp_cover(m, xb0 + (float)(c + 1));
             const T q = cell_of<T>(v);
-            tiny |= tiny_share(v);
+            if (FIX) least = fminf(least, fabsf(v));
             cell_add(&cells[row_at + c], q - ((c & 63) ? prev : (T)0));
             prev = q;
         }
@@ -700,24 +708,29 @@ __device__ __forceinline__ bool scatter_piece(T *cells, uint32_t row_at, const R
         const int w0 = __builtin_amdgcn_readlane(m.c0, l), w1 = __builtin_amdgcn_readlane(m.c1, l);
         const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)row_at, l);
         const int lane = threadIdx.x & 63;
-        bool any = false;
         for (int c = w0 + lane; c < w1; c += 64) {
-            const float v = wz * ramp_cover(w, xb0 + (float)(c + 1));
-            const T q = cell_of<T>(v);
+            const T q = cell_of<T>(wz * ramp_cover(w, xb0 + (float)(c + 1)));
             const T b = ((c > w0) & ((c & 63) != 0)) ? cell_of<T>(wz * ramp_cover(w, xb0 + (float)c)) : (T)0;
-            any |= tiny_share(v);
             cell_add(&cells[at + c], q - b);
         }
-        tiny |= (lane == l) & (__ballot(any) != 0ull);
     }
-    if (!m.live) return false;
-    if (wide) prev = cell_of<T>(zs * ramp_cover(m, xb0 + (float)m.c1));  // the last ramp column's value
+    if (!m.live) return;
+    if (wide) {
+        prev = cell_of<T>(zs * ramp_cover(m, xb0 + (float)m.c1));  // the last ramp column's value
+        if (FIX) least = fabsf(zs * ramp_cover(m, xb0 + (float)(m.c0 + 1)));
+    }
     // from the column after the ramp on: whole
     const T whole = cell_of<T>(zs);
     const int t = m.c1 > m.c0 ? m.c1 : m.c0;
     if (t < tw) cell_add(&cells[row_at + t], whole - ((t & 63) ? prev : (T)0));
     for (int c = (t | 63) + 1; c < tw; c += 64) cell_add(&cells[row_at + c], whole);
-    return tiny;
+    if (FIX && least < TINY) {
+        for (int c = m.c0; c < m.c1; ++c) {
+            const float v = zs * ramp_cover(m, xb0 + (float)(c + 1));
+            if (!(fabsf(v) < TINY)) break;
+            if (v != 0.0f) fix(c, v - rintf(v));
+        }
+    }
 }
 
 // Coverage A[j] of round s's paths at this thread's pixel, from the first
@@ -746,10 +759,18 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
         const uint32_t j = r.j != NO_IDX ? r.j : 0u;
         pc.live &= ((heavy >> j) & 1u) == 0u;
         const Ramp m = ramp_of(pc, xb0, tw);
-        const bool tiny = scatter_piece<int>(cells, j * pitch, m, xb0, tw, CELL_ONE);
-        if (m.nan | tiny) atomicOr(&R.poison[s & 1], (m.nan ? 1u : 0x10000u) << j);
+        const bool low = m.live & (fabsf(m.z) < TINY / CELL_ONE);
+        if (m.nan | low) atomicOr(&R.mark[s & 1].x, (m.nan ? 1u : 0x10000u) << j);
+        scatter_piece<int>(cells, j * pitch, m, xb0, tw, CELL_ONE, [&](int c, float r) {
+            const uint32_t k = atomicAdd(&R.mark[s & 1].y, 1u);
+            if (k < FIX_MAX)
+                R.fix[k] = make_uint2(j << 16 | (uint32_t)c, __builtin_bit_cast(uint32_t, r));
+            else
+                atomicOr(&R.mark[s & 1].x, 0x10000u << j);
+        });
     }
     __syncthreads();
+    const uint2 mark = R.mark[s & 1];
     uint32_t c[SEG];
 #pragma unroll
     for (uint32_t j = 0; j < SEG; ++j) {
@@ -758,43 +779,52 @@ __device__ __forceinline__ void round_cover(const DScene &S, RowLds &R, uint32_t
     }
 #pragma unroll
     for (uint32_t j = 0; j < SEG; ++j) A[j] = (float)(int)wave_incl_dpp<false>(c[j]) * (1.0f / CELL_ONE);
-    uint32_t poison = R.poison[s & 1];
-    const uint32_t wide = heavy | (poison >> 16);
-    if (wide) {  // (uniform) one path at a time, in 64-bit cells over the same LDS
-        long long *c64 = reinterpret_cast<long long *>(cells);
-        for (uint32_t j = 0; j < SEG; ++j) {
-            if (!((wide >> j) & 1u)) continue;
-            const float one = ((heavy >> j) & 1u) ? HEAVY_ONE : FINE_ONE;
-            __syncthreads();  // the cells, or the path before's, are read
-            c64[tid] = 0;
-            __syncthreads();
-            const uint32_t e0 = R.pb[s * SEG + j], e1 = R.pb[s * SEG + j + 1];
-            for (uint32_t eb = e0; eb < e1; eb += (uint32_t)tw) {  // whole blocks: scatter_piece is collective
-                const uint32_t e = eb + (uint32_t)tid;
-                PieceRef r = piece_ref(S, R, s, e < e1 ? e : NO_IDX);
-                const PieceVtx u = piece_vtx(S, R, s, r, bad);
-                Piece pc = piece_of(u.p, u.q, Y);
-                pc.live &= r.j != NO_IDX;
-                const Ramp m = ramp_of(pc, xb0, tw);
-                if (m.nan) atomicOr(&R.poison[s & 1], 1u << j);
-                (void)scatter_piece<long long>(c64, 0u, m, xb0, tw, one);
+    if (mark.x | mark.y | heavy) {  // (uniform)
+        const uint32_t n_fix = mark.y < FIX_MAX ? mark.y : FIX_MAX;
+        for (uint32_t k = 0; k < n_fix; ++k) {
+            const uint2 f = R.fix[k];
+            const float r = (f.x & 0xFFFFu) == (uint32_t)tid ? __builtin_bit_cast(float, f.y) : 0.0f;
+            const uint32_t path = (uint32_t)__builtin_amdgcn_readfirstlane((int)(f.x >> 16));
+#pragma unroll
+            for (uint32_t j = 0; j < SEG; ++j) A[j] = j == path ? fmaf(r, 1.0f / CELL_ONE, A[j]) : A[j];
+        }
+        const uint32_t wide = heavy | (mark.x >> 16);
+        uint32_t poison = mark.x;
+        if (wide) {  // one path at a time, in 64-bit cells over the same LDS
+            long long *c64 = reinterpret_cast<long long *>(cells);
+            for (uint32_t j = 0; j < SEG; ++j) {
+                if (!((wide >> j) & 1u)) continue;
+                const bool many = ((heavy >> j) & 1u) != 0;
+                const float one = many ? HEAVY_ONE : FINE_ONE;
+                __syncthreads();  // the cells, or the path before's, are read
+                c64[tid] = 0;
+                __syncthreads();
+                const uint32_t e0 = R.pb[s * SEG + j], e1 = R.pb[s * SEG + j + 1];
+                for (uint32_t eb = e0; eb < e1; eb += (uint32_t)tw) {  // whole blocks: scatter_piece is collective
+                    const uint32_t e = eb + (uint32_t)tid;
+                    PieceRef r = piece_ref(S, R, s, e < e1 ? e : NO_IDX);
+                    const PieceVtx u = piece_vtx(S, R, s, r, bad);
+                    Piece pc = piece_of(u.p, u.q, Y);
+                    pc.live &= r.j != NO_IDX;
+                    const Ramp m = ramp_of(pc, xb0, tw);
+                    if (m.nan) atomicOr(&R.mark[s & 1].x, 1u << j);
+                    scatter_piece<long long>(c64, 0u, m, xb0, tw, one, [](int, float) {});
+                }
+                __syncthreads();
+                const long long sum = (long long)wave_incl_t<unsigned long long, false>((unsigned long long)c64[tid]);
+                const float a = (float)sum * (many ? 1.0f / HEAVY_ONE : 1.0f / FINE_ONE);
+#pragma unroll
+                for (uint32_t k = 0; k < SEG; ++k) A[k] = k == j ? a : A[k];
             }
             __syncthreads();
-            const long long sum = (long long)wave_incl_t<unsigned long long, false>((unsigned long long)c64[tid]);
-            const float a = (float)sum / one;
-#pragma unroll
-            for (uint32_t k = 0; k < SEG; ++k) A[k] = k == j ? a : A[k];
+            if (ZERO) c64[tid] = 0;
+            poison = R.mark[s & 1].x;
         }
-        __syncthreads();
-        if (ZERO) c64[tid] = 0;
-        poison = R.poison[s & 1];
-    }
-    if (tid == 0) R.poison[(s + 1) & 1] = 0;
-    // a piece without an x takes its path's whole row (coverage past 1, and so no gradient)
-    if (poison & 0xFFFFu) {
+        // a piece without an x takes its path's whole row (coverage past 1, and so no gradient)
 #pragma unroll
         for (uint32_t j = 0; j < SEG; ++j) A[j] = ((poison >> j) & 1u) ? 2.0f : A[j];
     }
+    if (tid == 0) R.mark[(s + 1) & 1] = make_uint2(0u, 0u);
     if (ZERO) __syncthreads();
 }
 

@@ -85,3 +85,45 @@ def test_sliver_of_a_pixel_keeps_its_gradient(oracle, x0, eps, flip):
     assert np.abs(want_gp[own]).max() > 0.01 * eps
     assert np.abs(gp[own] - want_gp[own]).max() < 0.03 * np.abs(want_gp[own]).max()
     assert np.abs(gc[1] - want_gc[1]).max() < 0.03 * np.abs(want_gc[1]).max()
+
+
+@pytest.mark.parametrize("low", [2.0 ** -25, 2.0 ** -30, 2.0 ** -40])
+def test_low_pieces_keep_their_gradient(oracle, low):
+    """A box that reaches `low` into row 0 from above: the row's pixels are
+    covered by that much, and the gradient of the box's lower side is 1 a
+    pixel, as far as float32 has such a y.  Beside it a path whose pieces are
+    whole.  Components within 1e-5 of the largest (sums of 200 equal terms)."""
+    w, h = 260, 3
+    box = [(20.0, -2.0), (20.0, low), (220.0, low), (220.0, -2.0), (20.0, -2.0)]
+    other = [(5.0, 0.0), (5.0, 3.0), (250.0, 3.0), (250.0, 0.0), (5.0, 0.0)]
+    pts = np.concatenate([_line_cubics(other), _line_cubics(box)])
+    cot = np.zeros((1, h, w, 4), np.float32)
+    cot[0, 0] = [1.0, 0.5, -0.25, 0.75]
+    gp, _, want_gp, _ = _grads(w, h, [4, 4], pts, [[0.1, 0.3, 0.2, 0.4], [0.3, 0.2, 0.1, 0.5]], cot)
+    own = slice(13, 26)
+    assert np.abs(want_gp[own, 1]).max() > 10.0
+    assert np.abs(gp[own] - want_gp[own]).max() < 1e-5 * np.abs(want_gp[own]).max()
+
+
+@pytest.mark.parametrize("paths", [3, 15, 16, 17, 33])
+@pytest.mark.parametrize("tips", [1, 2, 3])
+def test_many_slivers_in_a_row(oracle, paths, tips):
+    """`paths` paths of `tips` tips as above in one row, two tiny shares a tip:
+    up to and past the 32 that a round of 16 paths lists.  Each path's
+    gradients, component by component (3 %, as above)."""
+    w, h, eps = 40, 9, 2.0 ** -13
+    corners = []
+    for x0 in (8, 16, 24)[:tips]:  # joined by edges along y = 4.5, which have no pieces
+        corners += [(x0 - eps, 4.5), (x0 + 6.0, 5.75), (x0 + 6.0, 3.25), (x0 - eps, 4.5)]
+    corners.append(corners[0])
+    path = _line_cubics(corners)
+    g = np.random.default_rng(paths + tips)
+    a = g.uniform(0.3, 0.9, (paths, 1))
+    colours = np.concatenate([a * g.random((paths, 3)), a], axis=1)
+    cot = np.zeros((1, h, w, 4), np.float32)
+    cot[0, 4, [7, 15, 23]] = [1.0, 0.5, 0.25, 0.75]
+    gp, gc, want_gp, want_gc = _grads(w, h, [len(corners) - 1] * paths, np.tile(path, (paths, 1)), colours, cot)
+    got, want = gp.reshape(paths, -1), want_gp.reshape(paths, -1)
+    assert (np.abs(want).max(axis=1) > 0.01 * eps).all()
+    assert (np.abs(got - want).max(axis=1) < 0.03 * np.abs(want).max(axis=1)).all()
+    assert (np.abs(gc - want_gc).max(axis=1) < 0.03 * np.abs(want_gc).max(axis=1)).all()

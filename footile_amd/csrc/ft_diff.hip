@@ -255,7 +255,8 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t x, uint32_t *s_w, uint32
 // list by look-back, and then per path and GEOM_ROWS of the rows between its
 // first and last counts the rows' edges in LDS, scans them into the cells' list
 // offsets and hands out the list slots with LDS cursors; the other rows get
-// counts of 0, whose offsets nothing reads.  Order within a list is free:
+// counts of 0, whose offsets nothing reads.  (Up to a row per thread they cost
+// nothing, and the span is not made: 0.8 of 8.3 us for 24 paths of 120 rows.)  Order within a list is free:
 // coverage is an integer sum.  It also clears the gradients (gedge null:
 // none).  It replaces a clear over all cells, a vertex pass, atomics per edge
 // on the cells, two scans over all cells and a kernel that tested every edge
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
             up = S.H - r0 > up ? S.H - r0 : up;
             end = r1 + 1 > end ? r1 + 1 : end;
         }
-        if (k - k0 < GEOM_SPANS) {
+        if ((k - k0 < GEOM_SPANS) & (S.H > BLOCK)) {
             up = wave_incl_dpp<true>(up);
             end = wave_incl_dpp<true>(end);
             if ((tid & 63) == 63) {
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
             r1 = r1 - w0 < h ? r1 - w0 : h - 1;
             return true;
         };
-        const bool kept = k - k0 < GEOM_SPANS;
+        const bool kept = (k - k0 < GEOM_SPANS) & (S.H > BLOCK);
         const uint32_t lo = kept ? S.H - s_up[k - k0] : 0u, end = kept ? s_end[k - k0] : S.H;
         for (uint32_t r = tid; r < lo; r += BLOCK) S.cell_cnt[(uint64_t)k * S.H + r] = 0;
         for (uint32_t r = end > lo ? end + tid : S.H; r < S.H; r += BLOCK) S.cell_cnt[(uint64_t)k * S.H + r] = 0;
@@ -497,11 +498,11 @@ constexpr uint32_t FIX_MAX = 32;         // listed columns per round
 // only they are rounded up to SEG and walked.  (A path without pieces leaves
 // the row's canvas as it is.  With all paths walked, a scene of small figures
 // paid for every figure in every row: 1,024 of 24 pixels in 512x512 took 271
-// us a forward and 790 a step, now 73 and 146; 256 paths across the image 113
-// and 349, now 109 and 333.)
+// us a forward and 790 a step, now 71 and 143; 256 paths across the image 113
+// and 349, now 105 and 327.)
 struct RowLds {
-    __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of their piece counts; the total past the last
-    __align__(16) uint8_t path[ROW_PATHS];     // their index among the staged paths; 0 past the last
+    __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of their piece counts; the total to the last round's end
+    __align__(16) uint8_t path[ROW_PATHS];     // their index among the staged paths; 0 to the last round's end
     uint32_t dl[ROW_PATHS];                    // list position of a path's piece e: dl + e
     uint2 vtx[ROW_PATHS];                      // first vertex and number of vertices
     uint32_t heavy[ROW_PATHS / SEG];           // per round: bit j, its path j has more than HEAVY pieces
@@ -517,50 +518,49 @@ struct RowLds {
 __device__ void stage_row(const DScene &S, uint32_t kbase, uint32_t n, int Y, RowLds &R) {
     const uint32_t lane = threadIdx.x;
     if (lane >= 64) return;
-    uint32_t c[4], o[4], v[5], sum = 0, live = 0;
+    constexpr uint32_t PER = ROW_PATHS / 64;
+    uint32_t c[PER], o[PER];
+    uint2 v[PER];
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        const uint32_t p = 4 * lane + i;
-        const uint64_t cell = (uint64_t)(kbase + (p < n ? p : 0u)) * S.H + (uint32_t)Y;
-        c[i] = p < n ? S.cell_cnt[cell] : 0u;
+    for (uint32_t i = 0; i < PER; ++i) {
+        if (64 * i >= n) break;  // (uniform)
+        const uint32_t p = 64 * i + lane, k = kbase + (p < n ? p : 0u);
+        const uint64_t cell = (uint64_t)k * S.H + (uint32_t)Y;
+        c[i] = S.cell_cnt[cell];
+        v[i] = make_uint2(S.vtx_off[k], S.vtx_off[k + 1]);
+        c[i] = p < n ? c[i] : 0u;
         // (of many paths most have none here, and their offsets are not loaded:
         // 1,118 -> 415 us in a scene of small figures; with few paths the loads
-        // are cheap and a second round trip is not: 7.2 and 9.5 us for four)
+        // are cheap and a second round trip is not)
         o[i] = 0;
         if (n <= 64 || c[i]) o[i] = S.cell_off[cell];
     }
-#pragma unroll
-    for (uint32_t i = 0; i < 5; ++i) v[i] = S.vtx_off[kbase + (4 * lane + i < n ? 4 * lane + i : n)];
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        sum += c[i];
-        live += c[i] ? 1u : 0u;
-    }
-    const uint32_t incl = wave_incl_dpp<false>(sum), rank1 = wave_incl_dpp<false>(live);
-    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-    const uint32_t n_live = (uint32_t)__builtin_amdgcn_readlane((int)rank1, 63);
-    uint32_t pre = incl - sum, rank = rank1 - live;
-    // (one wavefront, whose LDS accesses stay in order: the entries past the
-    // last first, everywhere)
-    *reinterpret_cast<uint4 *>(&R.pb[4 * lane]) = make_uint4(total, total, total, total);
-    *reinterpret_cast<uint32_t *>(&R.path[4 * lane]) = 0;
     if (lane < ROW_PATHS / SEG) R.heavy[lane] = 0;
     if (lane < 2) R.mark[lane] = make_uint2(0u, 0u);
-    if (lane == 63) {
-        R.pb[ROW_PATHS] = total;
-        R.n = n_live;
-    }
+    uint32_t first = 0, rank = 0;  // pieces and paths before
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        if (!c[i]) continue;
-        R.pb[rank] = pre;
-        R.path[rank] = (uint8_t)(4 * lane + i);
-        R.dl[rank] = o[i] - pre;
-        R.vtx[rank] = make_uint2(v[i], v[i + 1] - v[i]);
-        if (c[i] > HEAVY) atomicOr(&R.heavy[rank / SEG], 1u << (rank % SEG));
-        ++rank;
-        pre += c[i];
+    for (uint32_t i = 0; i < PER; ++i) {
+        if (64 * i >= n) break;
+        const unsigned long long live = __ballot(c[i] != 0u);
+        const uint32_t incl = wave_incl_dpp<false>(c[i]), pre = first + incl - c[i];
+        if (c[i]) {
+            const uint32_t r = rank + __builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0u));
+            R.pb[r] = pre;
+            R.path[r] = (uint8_t)(64 * i + lane);
+            R.dl[r] = o[i] - pre;
+            R.vtx[r] = make_uint2(v[i].x, v[i].y - v[i].x);
+            if (c[i] > HEAVY) atomicOr(&R.heavy[r / SEG], 1u << (r % SEG));
+        }
+        first += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        rank += (uint32_t)__popcll(live);
     }
+    // the rest of the last round
+    if (lane <= SEG && rank + lane <= ROW_PATHS) {
+        R.pb[rank + lane] = first;
+        if (rank + lane < ROW_PATHS) R.path[rank + lane] = 0;
+    }
+    if (lane == 0) R.n = rank;
 }
 
 // Piece e of round s (staged paths [s * SEG, s * SEG + SEG)).
@@ -858,6 +858,17 @@ __device__ __forceinline__ float4 round_colour(const float4 *__restrict__ staged
     return make_float4(sel(c.x), sel(c.y), sel(c.z), sel(c.w));
 }
 
+// A kernel's start: the image's first path and number of paths, and false when
+// an earlier kernel of the run failed, in one round trip to memory.
+__device__ __forceinline__ bool image_begin(const DScene &S, const DevStatus *st, uint32_t im, uint32_t &k0,
+                                            uint32_t &np) {
+    const uint32_t e = st->err, o = st->overflow, k1 = S.img_first[im + 1];
+    k0 = S.img_first[im];
+    np = k1 - k0;
+    asm volatile("" ::"s"(e), "s"(o), "s"(k0), "s"(k1));
+    return (e | o) == 0u;
+}
+
 // The canvas of one tile of one row: the image's paths with pieces there
 // composited over transparent pixels, SEG at a time, with the next round's
 // pieces loaded while a round is composited.  With ck it also leaves the
@@ -882,11 +893,11 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
         if (report) report_status(report, st, nullptr, nullptr, 0);
         for (uint32_t i = threadIdx.x; i < n_lb; i += blockDim.x) lb[i] = 0;
     }
-    if (run_failed(st)) return;
     const uint32_t tw = TW ? TW : blockDim.x, pitch = tw + 1;
     const uint32_t X = blockIdx.x * tw + threadIdx.x, Y = blockIdx.y, im = blockIdx.z;
+    uint32_t k0, np;
+    if (!image_begin(S, st, im, k0, np)) return;
     const float xb0 = (float)(blockIdx.x * tw);
-    const uint32_t k0 = S.img_first[im], np = S.img_first[im + 1] - k0;
     const uint64_t slot = ((uint64_t)im * S.H + Y) * ck_pitch + X;
     const bool in = X < S.W;
     uint32_t bad = 0;
@@ -1092,12 +1103,12 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
     extern __shared__ __align__(16) int s_cells[];  // cells, then the suffix sums of dA; then dA
     __shared__ RowLds R;
     __shared__ float s_gc[64];  // the round's colour gradients, in sum-tree order
-    if (run_failed(st)) return;
     const uint32_t tw = TW ? TW : blockDim.x, pitch = tw + 1;
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t X = blockIdx.x * tw + threadIdx.x, Y = blockIdx.y, im = blockIdx.z;
+    uint32_t k0, np;
+    if (!image_begin(S, st, im, k0, np)) return;
     const float xb0 = (float)(blockIdx.x * tw);
-    const uint32_t k0 = S.img_first[im], np = S.img_first[im + 1] - k0;
     const uint64_t slot = ((uint64_t)im * S.H + Y) * ck_pitch + X;
     const bool in = X < S.W;
     float *const s_suf = reinterpret_cast<float *>(s_cells);

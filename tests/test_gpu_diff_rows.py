@@ -24,7 +24,9 @@ def _local(h, size, rows=None):
     return points
 
 
-@pytest.mark.parametrize("paths,images", [(40, 1), (255, 1), (257, 2), (530, 1)])
+@pytest.mark.parametrize("paths,images", [
+    (40, 1), (63, 1), (64, 2), (65, 1), (127, 1), (129, 1), (193, 1),  # staged 64 at a time
+    (255, 1), (257, 2), (530, 1)])
 def test_small_figures(oracle, paths, images):
     _check(_scene(paths, 64, 48, paths, 2, images, points=_local(48, 5.0)))
 

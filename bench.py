@@ -294,8 +294,7 @@ def bench_diff(steps, warmup, check=True):
     """Differentiable workloads: one 512^2 image (256 paths x 8 cubics) and
     64 images of 256^2 (U[32,512] paths x U[4,16] cubics), fwd + loss +
     bwd per step (one ft_diff_step call, coverage recomputed in the backward);
-    gradients against the FP64 oracle.  The opt-in kept-coverage handle is
-    timed beside each as its own row."""
+    gradients against the FP64 oracle."""
     from footile_amd import diffscene as ds
     from footile_amd.diff import DiffRenderer
     out = {}
@@ -308,12 +307,6 @@ def bench_diff(steps, warmup, check=True):
                       "from params + N(0,2px) / colours + N(0,0.05); one ft_diff_step, coverage recomputed in "
                       "the backward",
           "grad_steps_per_s": 1.0 / dt, "ms_per_step": dt * 1e3, "loss": loss}
-    rk = DiffRenderer.for_scene(sc, keep_coverage=True)
-    bk = _diff_buffers(rk, sc)
-    dtk, _ = _diff_time(rk, bk, steps, warmup)
-    one["kept_coverage_variant"] = {"grad_steps_per_s": 1.0 / dtk, "ms_per_step": dtk * 1e3,
-                                   "extra_bytes": 4 * sc.n_paths * sc.width * sc.height}
-    del rk, bk
     if check:
         from oracle import pydiff as pd
         target = b["T"].download(dtype=np.float32).reshape(r.canvas_shape)
@@ -335,11 +328,6 @@ def bench_diff(steps, warmup, check=True):
     many = {"workload": "64 images 256x256 fp32 RGBA, U[32,512] paths x U[4,16] cubics (seed 4); all images "
                       "in one ft_diff_step (one host wait), coverage recomputed in the backward",
           "grad_steps_per_s": 1.0 / dt, "ms_per_step": dt * 1e3, "paths": int(sc.n_paths)}
-    rk = DiffRenderer.for_scene(sc, keep_coverage=True)
-    bk = _diff_buffers(rk, sc)
-    dtk, _ = _diff_time(rk, bk, max(2, steps // 2), 1)
-    many["kept_coverage_variant"] = {"grad_steps_per_s": 1.0 / dtk, "ms_per_step": dtk * 1e3}
-    del rk, bk
     # per-image launches of the same scenes
     per_image = 0.0
     tp, tc = ds.perturbed(sc)
@@ -397,7 +385,7 @@ def main():
     ap.add_argument("--no-extra", action="store_true", help="skip the atlas, plain and differentiable measurements")
     ap.add_argument("--no-diff-check", action="store_true", help="skip the FP64 gradient checks")
     ap.add_argument("--tuning", default=None,
-                    help="band_rows_min,lds_cells,dst_prefetch for the random-walk batch instead of autotuning "
+                    help="band_rows_min,lds_cells for the random-walk batch instead of autotuning "
                          "(profiling runs)")
     ap.add_argument("--atlas-tuning", default=None,
                     help="band_rows_min,lds_cells[,tile_groups] for the atlas instead of autotuning "
@@ -440,9 +428,9 @@ def main():
              FillDesc(len(ops), len(ops), B.ptr, W, H, W * 4, RGBA8P, rule=1, clr=clr)]
     batch = Batch(both, descs)
     if args.tuning:
-        b_rows, cells, pf = (int(v) for v in args.tuning.split(","))
-        batch.set_tuning(b_rows, cells, bool(pf))
-        tuned = {"band_rows_min": b_rows, "lds_cells": cells, "dst_prefetch": bool(pf), "tried": 0}
+        b_rows, cells = (int(v) for v in args.tuning.split(",")[:2])
+        batch.set_tuning(b_rows, cells)
+        tuned = {"band_rows_min": b_rows, "lds_cells": cells, "tried": 0}
     else:
         from footile_amd.tune import autotune
         tuned = autotune(batch, descs, len(both), cache=None)
@@ -552,7 +540,7 @@ def main():
         "edges_per_fill": int(edges[0]),
         "top_rows": [int(t) for t in tops],
         "tuning": {"band_rows_min": tuned["band_rows_min"], "lds_cells": tuned["lds_cells"],
-                   "dst_prefetch": tuned["dst_prefetch"], "candidates": tuned["tried"]},
+                   "candidates": tuned["tried"]},
     }
     if not args.no_extra:
         print("[bench] atlas", file=sys.stderr, flush=True)

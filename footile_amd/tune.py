@@ -2,9 +2,9 @@
 
 Candidates are (band_rows_min, lds_cells, dst_prefetch, tile_groups): band
 height for edge binning, the LDS cell budget that fixes the rows per raster
-block, a flag that changes nothing, and the largest path (in LDS row groups)
-the tile scheduler takes instead of the bands.  Each
-candidate is timed on the batch itself with device events (whole launch
+block, a flag that changes nothing (never varied), and the largest path (in
+LDS row groups) the tile scheduler takes instead of the bands.  Each candidate
+is timed on the batch itself with device events (whole launch
 sequence, median of a few launches after one warm-up run); the fastest wins.
 Results are cached in a JSON file keyed by a signature of the batch layout
 (path count, raster width/height histogram in powers of two, formats, op
@@ -42,7 +42,7 @@ def signature(descs, n_ops):
     return hashlib.sha1(key.encode()).hexdigest()[:16]
 
 
-def _tile_candidates(descs, prefetch):
+def _tile_candidates(descs):
     """Tile scheduler settings that move at least a tenth of the paths out of
     the bands (a path of height h and cell row stride wp takes
     ceil(h / (lds_cells // wp)) groups)."""
@@ -54,7 +54,7 @@ def _tile_candidates(descs, prefetch):
         groups = -(-h // np.maximum(1, c // np.maximum(wp, 1)))
         for tg in TILE_GROUPS:
             if np.count_nonzero(groups <= tg) * 10 >= max(len(descs), 1):
-                out += [(b, c, p, tg) for b in TILE_BAND_ROWS for p in prefetch]
+                out += [(b, c, False, tg) for b in TILE_BAND_ROWS]
     return out
 
 
@@ -83,9 +83,7 @@ def autotune(batch, descs, n_ops, cache=DEFAULT_CACHE, reps=3, candidates=None, 
         e = table[key]
         batch.set_tuning(e["band_rows_min"], e["lds_cells"], e.get("dst_prefetch", True), e.get("tile_groups", 0))
         return dict(e, cached=True, tried=0)
-    prefetch = (False,)
-    cands = candidates or ([(b, c, p, 0) for b in BAND_ROWS for c in LDS_CELLS for p in prefetch] +
-                           _tile_candidates(descs, prefetch))
+    cands = candidates or [(b, c, False, 0) for b in BAND_ROWS for c in LDS_CELLS] + _tile_candidates(descs)
     best = None
     t0 = time.perf_counter()
     for b, c, p, tg in cands:
@@ -98,7 +96,7 @@ def autotune(batch, descs, n_ops, cache=DEFAULT_CACHE, reps=3, candidates=None, 
         batch.run()
         ms = _time(batch, reps)
         if verbose:
-            print(f"[tune] band_rows_min={b} lds_cells={c} dst_prefetch={p} tile_groups={tg}: {ms:.3f} ms")
+            print(f"[tune] band_rows_min={b} lds_cells={c} tile_groups={tg}: {ms:.3f} ms")
         if best is None or ms < best[4]:
             best = (b, c, p, tg, ms)
     batch.set_tuning(*best[:4])

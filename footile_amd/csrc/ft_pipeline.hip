@@ -2078,7 +2078,7 @@ struct SmallLds {
     ft_path_op ops[SMALL_OPS];
     PathDev path;
     PathState ps;
-    uint32_t w[SBLOCK / 64], w2[SBLOCK / 64];
+    uint32_t w[SBLOCK / 64];
     unsigned long long wk[SBLOCK / 64];
     uint32_t flag, walk;  // a limit passed or a check failed; a closing walk past KEPT_WALK
 };
@@ -3434,7 +3434,7 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
     if (mode != MODE_FILL && n_ops) {
         const PenWidthSrc pw{ws.d_ops, 0u};
         scan_launch_src<uint32_t, true>(s, ws.scan_resident, pw, ws.d_op_lastpw, nullptr, n_ops, n_ops,
-                                        lb + 10 * tiles, nullptr, st, false, false, ws.tickets);
+                                        lb + 8 * tiles, nullptr, st, false, false, ws.tickets);
         lastpw = ws.d_op_lastpw;
     }
     if (n_ops) {
@@ -3476,7 +3476,7 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
         sp.tol_sq = ws.n_paths ? ws.stroke_tol_sq : 0.0f;
         const StrokeFlagSrc flags{ws.d_ev_f, 0u};
         scan_launch_src<unsigned long long, false>(s, ws.scan_resident, flags, ws.d_st_off, &st->n_events, 0, cap,
-                                                   lb + 12 * tiles, &st->st_total, st, true, false, ws.tickets);
+                                                   lb + 10 * tiles, &st->st_total, st, true, false, ws.tickets);
         k_st_compact<<<ge, BLOCK, 0, s>>>(ws.d_ev_f, ws.d_st_off, ws.d_spts, ws.d_sub_start, ws.d_sub_event, cap, st);
         EventSink em{};
         em.cap_events = ws.cap_events;
@@ -3494,12 +3494,12 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
         if (outline_blocks <= SCAN_GRID_MAX) {
             k_st_outline<<<(uint32_t)outline_blocks, BLOCK, 0, s>>>(ws.d_spts, ws.d_ev_f, ws.d_sub_start,
                                                                     ws.d_sub_event, cap, sp, ws.d_paths,
-                                                                    lb + 16 * tiles, em, st);
+                                                                    lb + 12 * tiles, em, st);
         } else {
             k_st_count<<<grid_for(cap_items), BLOCK, 0, s>>>(ws.d_spts, ws.d_ev_f, ws.d_sub_start, ws.d_sub_event,
                                                              cap, sp, ws.d_it_cnt, st);
             scan_launch<unsigned long long, false>(s, ws.scan_resident, ws.d_it_cnt, ws.d_it_off, &st->st_items, 0,
-                                                   (uint32_t)cap_items, lb + 16 * tiles, &st->stroke_total, st, true,
+                                                   (uint32_t)cap_items, lb + 12 * tiles, &st->stroke_total, st, true,
                                                    false, ws.tickets);
             k_st_emit<<<grid_for(cap_items), BLOCK, 0, s>>>(ws.d_spts, ws.d_ev_f, ws.d_sub_start, ws.d_sub_event, sp,
                                                             ws.d_it_off, ws.d_paths, em, st);
@@ -3542,12 +3542,12 @@ static ft_status ws_enqueue(Workspace &ws, uint32_t mode, hipEvent_t *ev, bool w
             if (in_scan) {
                 const IngestSrc ing{L0, ws.d_ev_meta, ws.d_ev_xy, ws.d_run_first, ws.d_run_path, 0u};
                 scan_launch_src<uint32_t, true>(s, ws.scan_resident, ing, ws.d_ev_last, &st->n_events, 0,
-                                                (uint32_t)ws.cap_events, lb + 8 * tiles, nullptr, st, true, true, ws.tickets);
+                                                (uint32_t)ws.cap_events, lb + 6 * tiles, nullptr, st, true, true, ws.tickets);
             } else {
                 k_ingest<<<ge, BLOCK, 0, s>>>(L0, ws.d_ev_meta, ws.d_ev_xy, ws.d_run_first, ws.d_run_path,
                                               ws.d_ev_last, st);
                 scan_launch<uint32_t, true>(s, ws.scan_resident, ws.d_ev_last, ws.d_ev_last, &st->n_events, 0,
-                                            (uint32_t)ws.cap_events, lb + 8 * tiles, nullptr, st, true, true, ws.tickets);
+                                            (uint32_t)ws.cap_events, lb + 6 * tiles, nullptr, st, true, true, ws.tickets);
             }
             // kept flags -> point indices
             const KeptSrc kp{L0, ws.d_ev_meta, ws.d_ev_xy, ws.d_run_first, ws.d_run_close, ws.d_ev_last,

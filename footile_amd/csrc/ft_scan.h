@@ -39,11 +39,10 @@ inline uint32_t scan_resident_blocks() {
 }
 constexpr uint32_t SCAN_GRID_MAX = 1024;  // largest scan grid
 // look-back state instances per run: 0 op counts, 1 kept points, 2 band
-// offsets, 3 band differences, 4 pushed points' running maximum, 5 PenWidth
-// indices, 6 stroker point/sub-stroke flags, 7 stroker last closes, 8 stroke
-// outline items
+// offsets, 3 pushed points' running maximum, 4 PenWidth indices, 5 stroker
+// point/sub-stroke flags, 6 stroke outline items
 constexpr uint32_t SCAN_SLOTS = N_SCAN_SLOTS;
-static_assert(SCAN_SLOTS == 9, "scan slot assignment");
+static_assert(SCAN_SLOTS == 7, "scan slot assignment");
 constexpr uint32_t SPIN_LIMIT = 1u << 24;
 
 // Device atomics for the stage code.

@@ -68,7 +68,7 @@ struct PathState {
     uint32_t fwd;               // Fig::get_dir at the top point (set before the raster)
 };
 
-constexpr uint32_t N_SCAN_SLOTS = 9;
+constexpr uint32_t N_SCAN_SLOTS = 7;
 
 // DevStatus::overflow bit: a run's closing walk was too long for the kept
 // flags' local form; the run is launched again with the ingest pass.

@@ -630,22 +630,27 @@ __device__ __forceinline__ Ramp ramp_of(const Piece &r, float xb0, int tw) {
 }
 
 // M at the pixel whose right border is X1, within the ramp: the mean of
-// clamp(u, 0, 1) for u from X1 - hi to X1 - lo; a and b are the clamped ends.
+// clamp(u, 0, 1) for u from X1 - hi to X1 - lo; a and b are the clamped ends,
+// `in` the ramp's length within the pixel and `past` that left of it.  Both
+// come from the x's and not from the u's: in column 0, where x is finer than
+// 1 - x, the u's difference over the ramp's width is off by 2^-24 / w.
 // The quotient is the correctly rounded one (a product with 1 / w corrected
 // by its remainder): M close to 0 or 1 decides whether a pixel has a
 // gradient.
-__device__ __forceinline__ float ramp_mean(const Ramp &m, float X1, float &a, float &b) {
-    const float lo = X1 - m.hi, hi = X1 - m.lo;
+__device__ __forceinline__ float ramp_mean(const Ramp &m, float X1, float &a, float &b, float &in, float &past) {
+    const float lo = X1 - m.hi, hi = X1 - m.lo, X0 = X1 - 1.0f;
     a = clamp01(lo);
     b = clamp01(hi);
+    in = fminf(m.hi, X1) - fmaxf(m.lo, X0);
+    past = fmaxf(X0 - m.lo, 0.0f);
     if (m.inv == 0.0f) return clamp01((lo + hi) * 0.5f);
-    const float I = (b - a) * (a + b) * 0.5f + fmaxf(hi - 1.0f, 0.0f);
+    const float I = in * (a + b) * 0.5f + past;
     const float q = I * m.inv;
     return fmaf(fmaf(-q, m.w, I), m.inv, q);
 }
 __device__ __forceinline__ float ramp_cover(const Ramp &m, float X1) {
-    float a, b;
-    return ramp_mean(m, X1, a, b);
+    float a, b, in, past;
+    return ramp_mean(m, X1, a, b, in, past);
 }
 
 // v rounded to a whole number: a share in cell units, |v| at most a cell's
@@ -1059,10 +1064,13 @@ __device__ __forceinline__ float chunk_right(const float *suf, int t) {
 
 // A piece's S1 = sum dA M, S2 = sum dA dM/dx_lo, S3 = sum dA dM/dx_hi terms
 // of one column (dA: the pixel's d loss / d coverage; the partials are with
-// respect to u = X1 - x, so S2 goes with the larger x).
+// respect to u = X1 - x, so S2 goes with the larger x).  The partials are
+// (M - a) / w and (b - M) / w; written out, with w = in + past + the length
+// right of the pixel, they are sums of positive terms: M - a would keep M's
+// rounding, which 1 / w multiplies.
 __device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, float &S1, float &S2, float &S3) {
-    float a, b;
-    const float M = ramp_mean(m, X1, a, b);
+    float a, b, in, past;
+    const float M = ramp_mean(m, X1, a, b, in, past);
     S1 = fmaf(g, M, S1);
     if (m.inv == 0.0f) {  // narrow: half of the slope each
         const float half = ((M > 0.0f) & (M < 1.0f)) ? 0.5f : 0.0f;
@@ -1070,8 +1078,9 @@ __device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, floa
         S3 += g * half;
         return;
     }
-    S2 = fmaf(g, (M - a) * m.inv, S2);
-    S3 = fmaf(g, (b - M) * m.inv, S3);
+    const float r = in * m.inv, even = 0.5f * r * r, g2 = g * m.inv * m.inv;
+    S2 = fmaf(g2, past * (1.0f - a), fmaf(g, even, S2));
+    S3 = fmaf(g2, fmaxf(m.hi - X1, 0.0f) * b, fmaf(g, even, S3));
 }
 
 // One tile of one row, the image's rounds of SEG paths last to first.  With f

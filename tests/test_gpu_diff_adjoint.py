@@ -127,3 +127,30 @@ def test_many_slivers_in_a_row(oracle, paths, tips):
     assert (np.abs(want).max(axis=1) > 0.01 * eps).all()
     assert (np.abs(got - want).max(axis=1) < 0.03 * np.abs(want).max(axis=1)).all()
     assert (np.abs(gc - want_gc).max(axis=1) < 0.03 * np.abs(want_gc).max(axis=1)).all()
+
+
+@pytest.mark.parametrize("x0", [0.004, 0.1, 0.3, 1.3, 60.2])  # column 0, where x is finer than 1 - x, and others
+@pytest.mark.parametrize("slope", [1.2e-5, 4.0e-5, 3.0e-4, 5.0e-3])  # ramp width a row; 1e-5 and narrower take the midpoint
+def test_near_vertical_edges(oracle, x0, slope):
+    """The canvas and the gradients of a figure whose sides lean by `slope` a
+    row.  A side's x is rounded at 2^-24 of it, a ramp's width by the same, so
+    that the partials of M, about 1/2 each, are off by 2^-23 x0 / slope
+    (half of it a side, either way) and by some 2^-22: bounds of 4 times that
+    sum, and 2e-5 for the canvas."""
+    w, h = 70, 18
+    corners = [(x0, 1.5), (x0 + 14 * slope, 15.5), (x0 + 6.0 - 14 * slope, 15.5), (x0 + 6.0, 1.5), (x0, 1.5)]
+    pts = _line_cubics(corners).astype(np.float32)
+    cubics, colours = [4], np.array([[0.3, 0.2, 0.1, 0.5]], np.float32)
+    cot = np.random.default_rng(5).uniform(0.2, 1.0, (1, h, w, 4)).astype(np.float32)
+    gp, gc, want_gp, want_gc = _grads(w, h, cubics, pts, colours, cot)
+    bound = 4.0 * (2.0 ** -23 * (x0 + 6.0) / slope + 2.0 ** -22)
+    assert np.abs(gp - want_gp).max() < bound * np.abs(want_gp).max()
+    assert np.abs(gc - want_gc).max() < 1e-5 * np.abs(want_gc).max()
+    from footile_amd.diff import DiffRenderer, device_array
+    from oracle import pydiff as pd
+    image = np.zeros(1, np.uint32)
+    r = DiffRenderer(1, w, h, image, np.asarray(cubics, np.uint32))
+    canvas = r.new_canvas()
+    r.forward(device_array(pts), device_array(colours), canvas)
+    _, want = pd.Scene(1, w, h, image, np.asarray(cubics, np.uint32)).forward(pts, colours)
+    assert np.abs(canvas.download(dtype=np.float32).reshape(r.canvas_shape) - want).max() < 2e-5

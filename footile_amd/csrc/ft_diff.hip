@@ -256,16 +256,17 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t x, uint32_t *s_w, uint32
 // first and last counts the rows' edges in LDS, scans them into the cells' list
 // offsets and hands out the list slots with LDS cursors; the other rows get
 // counts of 0, whose offsets nothing reads.  (Up to a row per thread they cost
-// nothing, and the span is not made: 0.8 of 8.3 us for 24 paths of 120 rows.)  Order within a list is free:
-// coverage is an integer sum.  It also clears the gradients (gedge null:
-// none).  It replaces a clear over all cells, a vertex pass, atomics per edge
-// on the cells, two scans over all cells and a kernel that tested every edge
-// of a path against every row: 545 -> 168 us of a 64-image step with 17,500
-// paths, 85 us in six launches -> 19 us in two for 256 paths, 110 -> 17 us for
-// a 1000x600 image of 128 paths.  4,096 figures of 24 pixels in an image of
-// 9,000 rows: 63 us, 530 with counts and offsets of all rows by this kernel,
-// 290 by the general form, which took images past 8,192 rows.  A path's work is a chain of a few barriers,
-// so a launch of few paths is bound by latency.
+// nothing, and the span is not made: 0.8 of 8.3 us for 24 paths of 120 rows.)
+// Order within a list is free: coverage is an integer sum.  It also clears the
+// gradients (gedge null: none).  It replaces a clear over all cells, a vertex
+// pass, atomics per edge on the cells, two scans over all cells and a kernel
+// that tested every edge of a path against every row: 545 -> 173 us of a
+// 64-image step with 17,500 paths, 85 us in six launches -> 18 us in one for
+// 256 paths, 110 -> 16 us for a 1000x600 image of 128 paths.  4,096 figures of
+// 24 pixels in an image of 9,000 rows: 63 us, 530 with counts and offsets of
+// all rows by this kernel, 290 by the general form, which took images past
+// 8,192 rows.  A path's work is a chain of a few barriers, so a launch of few
+// paths is bound by latency.
 constexpr uint32_t GEOM_EDGES = 2048, GEOM_ROWS = 8192, GEOM_BLOCKS = 1024;
 constexpr uint32_t GEOM_SPANS = 64;  // paths of a block whose spans are kept; the others take all rows
 constexpr uint32_t EDGE_LANES = 4;  // threads per edge in the fill, on every fourth of its rows
@@ -399,8 +400,8 @@ __global__ __launch_bounds__(BLOCK) void k_geometry(DScene S, const float2 *poin
     }
 }
 
-// The general form, for longer paths: k_vertices, k_rows
-// (differences on the cells), two scans over the cells, and k_fill_cells.
+// The general form, for longer paths: k_vertices, k_rows (differences on the
+// cells), two scans over the cells, and k_fill_cells.
 //
 // FILL_LANES threads per edge, each taking every FILL_LANES-th run of
 // FILL_ROWS rows, with the run's FILL_ROWS slot reservations (returning
@@ -455,9 +456,10 @@ __global__ __launch_bounds__(BLOCK) void k_fill_cells(DScene S, DevStatus *st) {
 // prefix sum then gives every pixel's coverage.  (Evaluating every piece that
 // touches a wavefront's columns on all of its pixels took 3.84 ms for 64
 // images of 256x256 with 17,500 paths, most of it on pixels outside the
-// ramp; this form takes 1.13 ms, and 83 us instead of 297 for one 512x512
-// image of 256 paths.  What is left is VALU work: per path and pixel about 9
-// instructions of prefix sum and 9 of composite.)
+// ramp; this form takes 1.03 ms, and 74 us instead of 297 for one 512x512
+// image of 256 paths.  What is left is VALU work, 95 % of the SIMDs' issue
+// rate for the 64 images: per path and pixel about 9 instructions of prefix
+// sum and 9 of composite.)
 //
 // Cells are integers in units of 2^-26 (an i32 add): the sum does not depend
 // on the order of the pieces, so the same inputs give the same canvas
@@ -481,9 +483,10 @@ __global__ __launch_bounds__(BLOCK) void k_fill_cells(DScene S, DevStatus *st) {
 // between wavefronts.
 // ---------------------------------------------------------------------------
 constexpr uint32_t SEG = 16;         // paths per round
-// Pixels per block.  At 93 VGPRs a SIMD holds 5 wavefronts, and blocks of 4
-// wavefronts fill them where blocks of 8 leave one empty: a 1000x600 image
-// takes 229 us a call with 256, 250 with 512, 233 with 128.
+// Pixels per block.  k_forward is held to the VGPRs with which a SIMD takes 5
+// wavefronts, and blocks of 4 wavefronts fill them where blocks of 8 leave one
+// empty: an earlier form took 229 us for a 1000x600 image with 256, 250 with
+// 512, 233 with 128.
 constexpr uint32_t TILE_MAX = 256;
 constexpr uint32_t ROW_PATHS = 256;  // paths whose cell counts are staged at once
 constexpr uint32_t HEAVY = 31;       // pieces of one path in one row past which cells are 64-bit
@@ -499,7 +502,7 @@ constexpr uint32_t FIX_MAX = 32;         // listed columns per round
 // the row's canvas as it is.  With all paths walked, a scene of small figures
 // paid for every figure in every row: 1,024 of 24 pixels in 512x512 took 271
 // us a forward and 790 a step, now 71 and 143; 256 paths across the image 113
-// and 349, now 105 and 327.)
+// and 349, now 102 and 326.)
 struct RowLds {
     __align__(16) uint32_t pb[ROW_PATHS + 4];  // exclusive scan of their piece counts; the total to the last round's end
     __align__(16) uint8_t path[ROW_PATHS];     // their index among the staged paths; 0 to the last round's end
@@ -884,8 +887,8 @@ __device__ __forceinline__ bool image_begin(const DScene &S, const DevStatus *st
 //
 // TW: the tile's width where it is TILE_MAX (any wider than 192 pixels), else
 // 0 and the block's.  As a constant it makes the LDS rows' addresses offsets of
-// one register instead of sixteen (here 1.17 -> 1.13 ms for 64 images of
-// 256x256, 86 -> 83 us for 512x512; k_backward 3.57 -> 3.19 ms).
+// one register instead of sixteen (when it came in 1.17 -> 1.13 ms for 64
+// images of 256x256, 86 -> 83 us for 512x512; k_backward 3.57 -> 3.19 ms).
 template <uint32_t TW>
 __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 *__restrict__ colours,
                                                       float4 *__restrict__ canvas, float4 *__restrict__ ck,
@@ -953,7 +956,7 @@ __global__ __launch_bounds__(TILE_MAX, 5) void k_forward(DScene S, const float4 
 // blocks, one per CU with LOSS_UNROLL loads of each kind in flight: their adds
 // to the one counter go by quickly.  (1,024 blocks of single floats and a
 // second kernel for the sum: 5.1 + 5.2 us for 512x512, 55 + 5 for 64 images of
-// 256x256; now 7.4 and 48.)
+// 256x256; now 7.5 and 46.)
 constexpr uint32_t LOSS_GRID = 256;
 constexpr int LOSS_UNROLL = 4;
 template <int VEC>
@@ -1098,11 +1101,13 @@ __device__ __forceinline__ void ramp_grad(const Ramp &m, float X1, float g, floa
 // right of it from the suffix sums (chunk_right).  (Evaluating each piece on all 64
 // pixels of every wavefront it touches and reducing the three sums over the
 // wavefront took 18.4 ms for 64 images of 256x256 with 17,500 paths; this
-// form takes 3.0 ms, and 240 us instead of 869 for one 512x512 image of 256
-// paths.  Adding four vertex gradients per piece instead of EdgeGrad's two and
-// its ends took 4.5 ms and 332 us.)  Four wavefronts per SIMD are asked for: without, the kernel takes
-// 156 VGPRs, a CU holds three blocks, and the 1,024 blocks of a 512x512 image
-// run in two passes (370 us).
+// form takes 2.86 ms, and 205-231 us instead of 869 for one 512x512 image of
+// 256 paths (where its buffers come to lie decides between the two, for a
+// reason not found).  Adding four vertex gradients per piece instead of
+// EdgeGrad's two and its ends took 4.5 ms and 332 us.)  What bounds it is VALU issue (79 % of the SIMDs' rate for
+// the 64 images, 50-56 % for the one, whose 1,024 blocks are one pass of the
+// chip) and the waits on LDS and barriers.  Four wavefronts per SIMD are asked
+// for: with three blocks per CU those 1,024 run in two passes (370 us).
 template <uint32_t TW>
 __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4 *__restrict__ colours,
                                                        const float4 *__restrict__ grad_canvas,
@@ -1156,7 +1161,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
             const RoundPaths rp = round_paths(R, s, n_live);
             float q[SEG];  // f . canvas under path j
             // f . c_j - c_j.w q_j, made again in the second pass: kept beside q it
-            // spilled 16 more registers (3.77 ms instead of 3.57 for 64 images)
+            // spilled 16 more registers (3.77 ms instead of 3.57 for 64 images when it was tried)
             auto d_of = [&](const float4 &c, float qj) {
                 return fmaf(-c.w, qj, fmaf(f.w, c.w, fmaf(f.z, c.z, fmaf(f.y, c.y, f.x * c.x))));
             };
@@ -1176,7 +1181,7 @@ __global__ __launch_bounds__(TILE_MAX, 4) void k_backward(DScene S, const float4
                 for (uint32_t h = 2; h-- > 0;) {
                     const uint32_t j = 2 * jp + h;
                     const float4 c = round_colour(staged, rp, j);
-                    // (else the first pass's alpha and d stay in registers: 3.19 ms, 3.03 so)
+                    // (else the first pass's alpha and d stay in registers: 3.19 ms, 3.03 so, when it came in)
                     asm("" : "+v"(A[j]), "+v"(q[j]));
                     const float al = alpha_cover(A[j]);
                     const float dal = T * d_of(c, q[j]), V = T * al;
@@ -1291,8 +1296,8 @@ __device__ __forceinline__ float4 edge_grad(const DScene &S, const float4 *gedge
 // cubic; a vertex's second edge is its neighbour's first.  (One thread per
 // point walked its 16 or 32 vertices one after another, a chain of loads and
 // divisions: 7.0 us for 200x120, 8.8 for 512x512 and 60 for 64 images, now
-// 4.0, 4.2 and 63.)  One block also reports the run's status, every other kernel of the
-// run being done.
+// 4.0, 4.2 and 62.)  One block also reports the run's status, every other
+// kernel of the run being done.
 __global__ __launch_bounds__(BLOCK) void k_point_grad(DScene S, const float4 *gedge, float2 *gpts, uint32_t n_pts,
                                                       const uint32_t *pt_path, const DevStatus *st,
                                                       HostStatus *report) {
@@ -1459,7 +1464,7 @@ ft_status launch_geometry(ft_diff *d, const float *points, bool clear_grads, flo
 
 // The run's one host wait.  Its kernels have written the status (and the
 // summed loss) to host memory: two copies behind the last kernel cost 8 us of
-// a 390 us step.
+// a step that then took 390.
 ft_status finish(ft_diff *d) {
     FD_HIP(hipStreamSynchronize(d->stream));
     const uint32_t late = d->h_status->late_err;
